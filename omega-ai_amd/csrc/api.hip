@@ -298,7 +298,7 @@ static int moe_reserve_backward(omega_moe *m, int T)
 
 static int moe_tile_m(const omega_moe *m, int T)
 {
-    return m->cfg.dtype == OMEGA_DTYPE_BF16 ? experts_bf16_tile_m(m, T) : experts_f32_tile_m();
+    return m->cfg.dtype == OMEGA_DTYPE_BF16 ? experts_bf16_tile_m(m, T) : experts_f32_tile_m(m, T);
 }
 
 static int moe_max_m_tiles(const omega_moe *m, int T, int bm)
@@ -319,9 +319,14 @@ static int moe_reserve(omega_moe *m, int T)
     const size_t P = (size_t)T * c.K;
     const int n_tok_tiles = ceil_div(T, router_tok_tile(c.E));
     const int bm = moe_tile_m(m, T);
-    // every expert's rows start on a row-tile boundary: the buffers hold whole tiles
+    // every expert's rows start on a row-tile boundary: the buffers hold whole tiles, of either height a batch of up to
+    // T tokens may take
     m->tiles_cap = moe_max_m_tiles(m, T, bm);
     m->rows_cap = (size_t)m->tiles_cap * bm;
+    if (c.dtype == OMEGA_DTYPE_F32) {
+        m->tiles_cap = moe_max_m_tiles(m, T, F32_TILE_M_SMALL);
+        m->rows_cap = (size_t)moe_max_m_tiles(m, T, F32_TILE_M) * F32_TILE_M;
+    }
     OMEGA_HIP_CHECK(ctx, hipMalloc((void **)&m->ids, P * 4));
     OMEGA_HIP_CHECK(ctx, hipMalloc((void **)&m->w, P * 4));
     OMEGA_HIP_CHECK(ctx, hipMalloc((void **)&m->rms, (size_t)T * 4));
@@ -644,7 +649,7 @@ static int stage_experts(omega_moe *m, const void *x, int T, int which)
     if (which == 0 && m->gather_on_load && !x) OMEGA_FAIL(m->ctx, OMEGA_ERR_INVALID_ARG, "experts: x is NULL");
     if (which == 1 && !m->a_valid) OMEGA_FAIL(m->ctx, OMEGA_ERR_INVALID_ARG, "experts_down: the up product has not run since `a` was overwritten");
     if (m->cfg.dtype == OMEGA_DTYPE_BF16) OMEGA_HIP_CHECK(m->ctx, launch_experts_bf16(m, x, T, which, m->ctx->stream));
-    else OMEGA_HIP_CHECK(m->ctx, launch_experts_f32(m, x, T, which, m->ctx->stream));
+    else OMEGA_HIP_CHECK(m->ctx, launch_product_f32(m, which == 0 ? F32_UP : F32_DOWN, (const float *)x, nullptr, T, m->ctx->stream));
     if (which == 0) m->a_valid = true;
     else m->y_valid = true;
     return OMEGA_OK;

@@ -1,152 +1,420 @@
-// Grouped expert SwiGLU products in fp32 on the matrix cores (v_mfma_f32_32x32x2_f32, fp32 operands and accumulators).
-//   up    a[r,h] = silu(xg[r,:].W1g[h,:]) * (xg[r,:].W3g[h,:])     silu(v) = v/(1+exp(-v))
-//   down  y[r,c] = a[r,:].W2g[c,:]
-// (J/engine/nn/layer/llama/LlamaMLPLayer.java:117-130; silu J/engine/nn/layer/active/gpu/activeFunction.cu:172-179;
-//  product J/engine/ad/op/gpu/OPKernel.cu:1103-1110; y = x W^T with W [out,in], J/engine/nn/layer/FullyLayer.java:181,235;
-//  the reference's product is a cuBLAS sgemm on the tensor cores, J/engine/gpu/GPUOP.java:395,405-417.)
+// Grouped products of fp32 layers on the matrix cores (v_mfma_f32_32x32x2_f32, fp32 operands and accumulators): the
+// expert SwiGLU of the forward pass and every product of the backward pass.
+//   up     a[r,h] = silu(xg[r,:].W1g[h,:]) * (xg[r,:].W3g[h,:])     silu(v) = v/(1+exp(-v))
+//   down   y[r,c] = a[r,:].W2g[c,:]
+//   da     d(a)[r,h] = dy[r,:].W2g[:,h], and from it dh1, dh3 (SwiGLU backward in the epilogue)
+//   dxg    dxg[r,c] = dh1[r,:].W1g[:,c] + dh3[r,:].W3g[:,c]
+//   wgrad  dW2g = dy^T a, dW1g = dh1^T xg, dW3g = dh3^T xg over the rows of group g
+// (J/engine/nn/layer/llama/LlamaMLPLayer.java:117-130,139-158; silu J/engine/nn/layer/active/gpu/activeFunction.cu:172-190;
+//  product J/engine/ad/op/gpu/OPKernel.cu:1103-1110; y = x W^T with W [out,in], J/engine/nn/layer/FullyLayer.java:181,235,
+//  diffW = delta^T input, diff = delta W, FullyLayer.java:292-334; the reference's product is a cuBLAS sgemm on the tensor
+//  cores, J/engine/gpu/GPUOP.java:395,405-417.)
 // Row tiles come from the tile list written by the dispatch stage: a tile never straddles two experts.
 //
-// One workgroup = 4 waves = one 64 x 64 output tile, each wave a 32 x 32 block (two accumulator blocks for the up
-// product: W1 and W3 against the same rows, so silu(h1)*h3 is applied in registers).  Operands are staged through LDS
-// k-major (As[k][row], Bs[k][col]) in steps of 32 k, so a lane's MFMA operands - A[row l32][k], B[k][col l32] for
-// k = 2*kk + lane/32 - are conflict-free 4-byte reads; the next step's rows travel from memory in registers while the
-// current step is multiplied.  Any d, H and alignment: rows that are 16-byte aligned take 16-byte loads (VEC), the
-// others scalar ones; everything past the edges of the tile is zero.
+// Bound: fp32 MFMA, 157.3 TFLOP/s (256 FLOP per clock and compute unit; 154 measured with nothing else going on).  One
+// workgroup = four waves = one tile of TM rows x TN MFMA columns, 128 x 128 or 64 x 64 (up: 64 x 128 as the smaller one;
+// half of the columns are W1's, half W3's, so a wave holds h1 and h3 of the same elements).  A wave has TM/2 x TN/2 of it
+// as 32 x 32 blocks; its row blocks alternate with the other row half's, so a ragged tile leaves both the same work.  At
+// 128 x 128 a step of 32 k is 64 MFMAs of 64 cycles per wave against 32 KiB of operands, 8 bytes per clock and compute unit.
+// A wave of such a step left to the compiler's order (barrier, LDS writes, loads, fragment reads, MFMAs) loses 2000 cycles
+// next to its 4096, and a second workgroup on the compute unit does not hide them: both run in step (MFMA busy 0.74 - 0.80,
+// whatever the number of buffers, workgroups or wave priorities).  So the order of a step is pinned: the fragments of the
+// next 8 k are read, the next step's pieces written to the other LDS buffer and the pieces of the step behind it asked for
+// between the MFMAs, a few at a time, and the one barrier of a step stands in front of MFMAs whose operands are in registers
+// (MFMA busy 0.89; 134 TFLOP/s at k = 8192).  No vector instruction but the address sums of the loads is spent per step.
+// The down and the input-gradient product, which have the fewest column tiles, take tiles of 128 x 64 (N = 1024, 8192
+// rows: 0.65 -> 0.55 and 1.26 -> 1.10 ms: 544 tiles of 128 x 128 leave the third round of two per compute unit nearly empty).
+// An operand whose rows are contiguous in k (x, W of y = x W^T) is kept [row][k] in LDS and read 16 bytes (4 k) per lane; one
+// that is contiguous across k (W of delta W, both operands of delta^T input) is kept [k][column] and read one float per
+// lane.  Both hand lane half h the k places 8j+4h .. 8j+4h+3 of every 8, so the two kinds combine freely.
+// Any width and alignment: VEC takes 16-byte loads, otherwise elements are loaded one by one.  Addresses past an edge
+// are clamped to the last valid element instead of branched over (a load in a divergent branch waits for those before
+// it); what they bring meets a zero (k past the end) or is never stored.
+//
+// T = 4096, d = 1024, H = 3584, E = 8, K = 2 (8192 rows), ms, before (64 x 64 tiles for the forward products, FMA kernels
+// for the others) and now: up 1.14 -> 0.96 (125 TFLOP/s), down 0.63 -> 0.55 (109), h1 and h3 again 1.91 -> 0.97, d(a) 1.08 -> 0.58,
+// dxg 3.00 -> 1.10, dW2 0.99 -> 0.48, dW1 and dW3 2.01 -> 0.94.
 #include "common.h"
+#include <type_traits>
 
-#define FBM 64
-#define FBN 64
 #define FBK 32
 
 typedef __attribute__((ext_vector_type(16))) float f32x16_t;
 
-int experts_f32_tile_m(void) { return FBM; }
+// LDS row stride in floats of an operand kept [row][FBK]: 16 consecutive rows start in 16 different groups of four banks
+#define F32_LD_ROW (FBK + 4)
+#define F32_LDS_FLOATS(TX, KMAJ) ((KMAJ) ? FBK * ((TX) + 4) : (TX) * F32_LD_ROW)
 
-// Stage of one operand: 64 rows x 32 k.  Thread t carries two pieces of 4 consecutive k: rows t/8 and t/8 + 32,
-// k = 4*(t%8) ...
-template <bool VEC>
-__device__ __forceinline__ void f32_fetch(const float *__restrict__ M, int rows, int Kd, int k0, int tid, float4 (&v)[2])
+// Pieces of one step that a thread carries: NV x 4 floats.  [row][k]: row r0 + (1024/FBK) u, 4 consecutive k; [k][column]: k
+// place k0 + (1024/TX) u, 4 consecutive columns.
+template <int TX, bool KMAJ>
+struct f32_piece {
+    static constexpr int NV = TX * FBK / 1024;
+    __device__ static __forceinline__ int x(int tid, int u) { return KMAJ ? 4 * (tid % (TX / 4)) : tid / (FBK / 4) + (1024 / FBK) * u; }
+    __device__ static __forceinline__ int k(int tid, int u) { return KMAJ ? tid / (TX / 4) + (1024 / TX) * u : 4 * (tid % (FBK / 4)); }
+    __device__ static __forceinline__ int lds(int tid, int u) { return KMAJ ? k(tid, u) * (TX + 4) + x(tid, u) : x(tid, u) * F32_LD_ROW + k(tid, u); }
+};
+
+// Piece u of a whole step: base = the step's first element (uniform), off = the thread's byte offset from it.  Without
+// 16-byte loads the columns of a [k][column] piece are clamped one by one (ncols of them exist).
+template <int TX, bool KMAJ, bool VEC>
+__device__ __forceinline__ float4 fetch_piece(const float *base, uint32_t off, int x, int ncols)
 {
+    const float *q = (const float *)((const unsigned char *)base + off);
+    if (VEC) return *(const float4 *)q;
+    if (!KMAJ) return make_float4(q[0], q[1], q[2], q[3]);
+    return make_float4(q[min(0, ncols - 1 - x)], q[min(1, ncols - 1 - x)], q[min(2, ncols - 1 - x)], q[min(3, ncols - 1 - x)]);
+}
+
+// The last, partial step of kleft < FBK k places: those behind read as zero, addresses are clamped
+template <int TX, bool KMAJ>
+__device__ __forceinline__ float4 fetch_partial(const float *base, uint32_t off, int tid, int u, int kleft, int ncols, int ld)
+{
+    float e[4];
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
-        const int r = (tid >> 3) + 32 * u, k = k0 + 4 * (tid & 7);
-        float4 q = {0.0f, 0.0f, 0.0f, 0.0f};
-        if (r < rows) {
-            const float *p = M + (size_t)r * Kd + k;
-            if (VEC) {
-                if (k < Kd) q = *(const float4 *)p;  // Kd % 4 == 0: a piece lies wholly inside or outside
-            } else {
-                if (k + 0 < Kd) q.x = p[0];
-                if (k + 1 < Kd) q.y = p[1];
-                if (k + 2 < Kd) q.z = p[2];
-                if (k + 3 < Kd) q.w = p[3];
+    for (int q = 0; q < 4; ++q) {
+        const int k = f32_piece<TX, KMAJ>::k(tid, u) + (KMAJ ? 0 : q), kc = min(k, kleft - 1);
+        const float *p = KMAJ ? base + (size_t)kc * ld + min(f32_piece<TX, KMAJ>::x(tid, u) + q, ncols - 1)
+                              : (const float *)((const unsigned char *)base + off) - f32_piece<TX, KMAJ>::k(tid, u) + kc;
+        const float w = *p;
+        e[q] = k < kleft ? w : 0.0f;
+    }
+    return make_float4(e[0], e[1], e[2], e[3]);
+}
+
+// four k places of one 32-row (32-column) block for this lane: LDS row / column x, k = 8 j + 4 kh ..
+template <int TX, bool KMAJ>
+__device__ __forceinline__ float4 frag(const float *S, int x, int k)
+{
+    if (!KMAJ) return *(const float4 *)&S[x * F32_LD_ROW + k];
+    return make_float4(S[k * (TX + 4) + x], S[(k + 1) * (TX + 4) + x], S[(k + 2) * (TX + 4) + x], S[(k + 3) * (TX + 4) + x]);
+}
+
+struct f32_args {
+    const float *A0, *A1;    // A operand; A1: F32_DXG second pair, F32_WG13 the second gradient's delta
+    const float *Atok;       // shared groups: token rows instead of physical rows (or null)
+    const float *B0, *B1;    // weights (F32_UP, F32_RAW: W1 and W3; F32_DXG: second pair), F32_WG*: the layer input rows
+    const float *Btok;       // F32_WG*: as Atok
+    float *C, *H1, *H3;      // output; h1 / h3 (F32_UP: kept when not null; F32_RAW: written; F32_DA: read, then dh1 / dh3)
+    const omega_tile *tiles;
+    const int32_t *tile_meta, *counts;
+    int N, Kd;               // row products: output columns and k; F32_WG*: columns and rows of one dW (k is the group's rows)
+    int E, G, T, bm;
+};
+
+#define F32_IS_WG(OP) ((OP) == F32_WG2 || (OP) == F32_WG13)
+#define F32_PAIR(OP) ((OP) == F32_UP || (OP) == F32_RAW)
+
+template <int OP, int TM, int TN, bool VEC>
+__global__ __launch_bounds__(256, 2) void f32_product_kernel(f32_args p)
+{
+    constexpr bool WG = F32_IS_WG(OP), PAIR = F32_PAIR(OP);
+    constexpr bool AK = WG, BK_ = WG || OP == F32_DA || OP == F32_DXG;  // operand contiguous across k
+    constexpr int MB = TM / 64, NB = TN / 64, NVA = TM * FBK / 1024, NVB = TN * FBK / 1024;
+    constexpr int CT = PAIR ? TN / 2 : TN;                             // output columns per tile
+    __shared__ __attribute__((aligned(16))) float As[2][F32_LDS_FLOATS(TM, AK)];
+    __shared__ __attribute__((aligned(16))) float Bs[2][F32_LDS_FLOATS(TN, BK_)];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l32 = lane & 31, kh = lane >> 5, wr = wave >> 1, wc = wave & 1;
+
+    // Tile of this workgroup.  Consecutive workgroups go round the eight XCDs: XCD x takes the x-th eighth of the tiles, and
+    // within it up to 8 row tiles walk the column tiles together, so that its workgroups share operand rows in its L2.
+    const int NT = (p.N + CT - 1) / CT;
+    const int MT = WG ? (p.Kd + TM - 1) / TM : p.tile_meta[0];  // row tiles (of one gradient matrix)
+    const int mats = OP == F32_WG13 ? 2 * p.G : OP == F32_WG2 ? p.G : 1;
+    const int total = MT * NT * mats, per = (total + 7) >> 3;
+    int t = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= per || t >= total) return;
+    const int mat = WG ? t / (MT * NT) : 0;
+    t -= mat * MT * NT;
+    const int rb = t / (8 * NT), nrb = min(8, MT - 8 * rb), ti = t - rb * 8 * NT;
+    const int mt = 8 * rb + ti % nrb, n0 = (ti / nrb) * CT;
+
+    int g, rows, K1, row0 = 0, m0 = 0;
+    const float *A0, *A1 = nullptr, *B0, *B1 = nullptr;
+    if (WG) {
+        g = OP == F32_WG13 ? mat >> 1 : mat;
+        const bool shared = g >= p.E;
+        m0 = mt * TM;
+        rows = min(TM, p.Kd - m0);
+        K1 = shared ? p.T : p.counts[g];
+        row0 = p.tile_meta[1 + g] * p.bm;
+        const float *Ad = OP == F32_WG13 && (mat & 1) ? p.A1 : p.A0;
+        A0 = shared && p.Atok ? p.Atok : Ad + (size_t)row0 * p.Kd;
+        B0 = shared && p.Btok ? p.Btok : p.B0 + (size_t)row0 * p.N;
+    } else {
+        const omega_tile tl = p.tiles[mt];
+        g = tl.g;
+        rows = tl.rows;
+        row0 = tl.row0;
+        K1 = p.Kd;
+        A0 = p.Atok && tl.xrow0 >= 0 ? p.Atok + (size_t)tl.xrow0 * p.Kd : p.A0 + (size_t)tl.row0 * p.Kd;
+        if (OP == F32_DXG) A1 = p.A1 + (size_t)tl.row0 * p.Kd;
+        B0 = p.B0 + (size_t)g * p.N * p.Kd;
+        if (PAIR || OP == F32_DXG) B1 = p.B1 + (size_t)g * p.N * p.Kd;
+    }
+
+    // Byte offsets of this thread's pieces from the step's first element (up: from W1's; the W3 columns add the distance).
+    // Rows (columns) past the tile's edge repeat the last valid ones and are never stored.
+    uint32_t oa[NVA], ob[NVB];
+#pragma unroll
+    for (int u = 0; u < NVA; ++u) {
+        const int x = f32_piece<TM, AK>::x(tid, u), k = f32_piece<TM, AK>::k(tid, u);
+        oa[u] = 4u * (AK ? (uint32_t)k * p.Kd + min(x, p.Kd - m0 - (VEC ? 4 : 1)) : (uint32_t)min(x, rows - 1) * K1 + k);
+    }
+#pragma unroll
+    for (int u = 0; u < NVB; ++u) {
+        const int x = f32_piece<TN, BK_>::x(tid, u), k = f32_piece<TN, BK_>::k(tid, u);
+        ob[u] = 4u * (BK_ ? (uint32_t)k * p.N + min(x, p.N - n0 - (VEC ? 4 : 1)) : (uint32_t)min(PAIR && x >= CT ? x - CT : x, p.N - 1 - n0) * K1 + k);
+    }
+
+    f32x16_t acc[MB][NB];
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+        for (int n = 0; n < NB; ++n)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][n][r] = 0.0f;
+
+    // this wave's row blocks: rows 32 (2 i + wr) ..; columns: TN/2 wc + 32 n (up: W1 columns 32 wc, and the same of W3)
+    const int live = max(0, min(MB, ((rows + 31) / 32 + 1 - wr) / 2));
+    const int xa = 32 * wr + l32;
+    int xb[NB];
+#pragma unroll
+    for (int n = 0; n < NB; ++n) xb[n] = (PAIR ? 32 * wc + CT * n : (TN / 2) * wc + 32 * n) + l32;
+
+    const int S1 = K1 / FBK, steps = OP == F32_DXG ? 2 * S1 : S1;  // whole steps
+    float4 va[NVA], vb[NVB];
+    const float *a_at = AK ? A0 + m0 : A0, *b_at = BK_ ? B0 + n0 : B0 + (size_t)n0 * K1, *b3_at = PAIR ? B1 + (size_t)n0 * K1 : nullptr;
+    auto fetch_a = [&](int u) { va[u] = fetch_piece<TM, AK, VEC>(a_at, oa[u], f32_piece<TM, AK>::x(tid, u), p.Kd - m0); };
+    auto fetch_b = [&](int u) {
+        vb[u] = fetch_piece<TN, BK_, VEC>(PAIR && u >= NVB / 2 ? b3_at : b_at, ob[u], f32_piece<TN, BK_>::x(tid, u), p.N - n0);
+    };
+    auto put_a = [&](int c, int u) { *(float4 *)&As[c][f32_piece<TM, AK>::lds(tid, u)] = va[u]; };
+    auto put_b = [&](int c, int u) { *(float4 *)&Bs[c][f32_piece<TN, BK_>::lds(tid, u)] = vb[u]; };
+    // the load pointers move on to step s (which the next loads bring); behind the last one they stay
+    auto advance = [&](int s) {
+        if (s >= steps) return;
+        a_at += AK ? (size_t)FBK * p.Kd : FBK;
+        b_at += BK_ ? (size_t)FBK * p.N : FBK;
+        if (PAIR) b3_at += FBK;
+        if (OP == F32_DXG && s == S1) {
+            a_at = A1;
+            b_at = B1 + n0;
+        }
+    };
+    // All steps for a wave with MBL live row blocks.  One group = 8 k of the step in buffer c: its MFMAs on the fragments
+    // read during the group before, and spread between them (pinned, a quarter of the group at a time) the reads of the
+    // next group's fragments and the group's share of the step's other work: group 0 writes the next step's pieces to the
+    // other buffer, group 1 asks for those of the step behind it; the barrier lies in front of the last group, whose
+    // fragment reads are the next step's first.  (Everything between two barriers of a step reads buffer c and writes
+    // buffer 1 - c, except that last group's reads of 1 - c, which every wave has finished writing.)
+    auto run = [&](auto mbl) {
+        constexpr int MBL = decltype(mbl)::value, NF = MBL > 0 ? MBL + NB : 0;
+        float4 fa[2][MBL > 0 ? MBL : 1], fb[2][NB];
+        auto read = [&](int set, int c, int j, int r) {
+            const int k = 8 * j + 4 * kh;
+            if (r < MBL) fa[set][r < MBL ? r : 0] = frag<TM, AK>(As[c], xa + 64 * r, k);
+            else if (r < NF) fb[set][r - MBL < NB ? r - MBL : 0] = frag<TN, BK_>(Bs[c], xb[r - MBL < NB ? r - MBL : 0], k);
+        };
+        auto group = [&](auto cc, auto jj) {
+            constexpr int c = decltype(cc)::value, j = decltype(jj)::value;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                if (NF > 0) read((j + 1) & 1, j == 3 ? 1 - c : c, (j + 1) & 3, q);
+                if (j == 0) {
+#pragma unroll
+                    for (int u = q; u < NVA; u += 4) put_a(1 - c, u);
+#pragma unroll
+                    for (int u = q; u < NVB; u += 4) put_b(1 - c, u);
+                } else if (j == 1) {
+#pragma unroll
+                    for (int u = q; u < NVA; u += 4) fetch_a(u);
+#pragma unroll
+                    for (int u = q; u < NVB; u += 4) fetch_b(u);
+                }
+#pragma unroll
+                for (int i = 0; i < MBL; ++i)
+#pragma unroll
+                    for (int n = 0; n < NB; ++n)
+                        acc[i][n] = __builtin_amdgcn_mfma_f32_32x32x2f32(((const float *)&fa[j & 1][i])[q], ((const float *)&fb[j & 1][n])[q], acc[i][n], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+        auto step = [&](auto cc, int s) {
+            group(cc, std::integral_constant<int, 0>());
+            advance(s + 2);
+            group(cc, std::integral_constant<int, 1>());
+            group(cc, std::integral_constant<int, 2>());
+            __syncthreads();
+            group(cc, std::integral_constant<int, 3>());
+        };
+        if (steps > 0) {
+#pragma unroll
+            for (int u = 0; u < NVA; ++u) { fetch_a(u); put_a(0, u); }
+#pragma unroll
+            for (int u = 0; u < NVB; ++u) { fetch_b(u); put_b(0, u); }
+            advance(1);
+#pragma unroll
+            for (int u = 0; u < NVA; ++u) fetch_a(u);
+#pragma unroll
+            for (int u = 0; u < NVB; ++u) fetch_b(u);
+            __syncthreads();
+#pragma unroll
+            for (int r = 0; r < NF; ++r) read(0, 0, 0, r);
+            int s = 0;
+            for (; s + 1 < steps; s += 2) {
+                step(std::integral_constant<int, 0>(), s);
+                step(std::integral_constant<int, 1>(), s + 1);
+            }
+            if (s < steps) step(std::integral_constant<int, 0>(), s);
+        }
+        // what is left of k (of both pairs)
+        const int kleft = K1 - S1 * FBK;
+        for (int seg = 0; kleft > 0 && seg < (OP == F32_DXG ? 2 : 1); ++seg) {
+            const float *at = (seg ? A1 : A0) + (AK ? (size_t)S1 * FBK * p.Kd + m0 : S1 * FBK);
+            const float *bt = (OP == F32_DXG && seg ? B1 : B0) + (BK_ ? (size_t)S1 * FBK * p.N + n0 : (size_t)n0 * K1 + S1 * FBK);
+            const float *b3 = PAIR ? B1 + (size_t)n0 * K1 + S1 * FBK : bt;
+            __syncthreads();
+#pragma unroll
+            for (int u = 0; u < NVA; ++u) { va[u] = fetch_partial<TM, AK>(at, oa[u], tid, u, kleft, p.Kd - m0, p.Kd); put_a(0, u); }
+#pragma unroll
+            for (int u = 0; u < NVB; ++u) {
+                vb[u] = fetch_partial<TN, BK_>(PAIR && u >= NVB / 2 ? b3 : bt, ob[u], tid, u, kleft, p.N - n0, p.N);
+                put_b(0, u);
+            }
+            __syncthreads();
+#pragma unroll
+            for (int j = 0; j < FBK / 8; ++j) {
+#pragma unroll
+                for (int r = 0; r < NF; ++r) read(0, 0, j, r);
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+#pragma unroll
+                    for (int i = 0; i < MBL; ++i)
+#pragma unroll
+                        for (int n = 0; n < NB; ++n)
+                            acc[i][n] = __builtin_amdgcn_mfma_f32_32x32x2f32(((const float *)&fa[0][i])[q], ((const float *)&fb[0][n])[q], acc[i][n], 0, 0, 0);
             }
         }
-        v[u] = q;
-    }
-}
+    };
+    if (live == MB) run(std::integral_constant<int, MB>());
+    else if (MB > 1 && live == 1) run(std::integral_constant<int, 1>());
+    else run(std::integral_constant<int, 0>());
 
-__device__ __forceinline__ void f32_stash(float (*S)[FBM + 1], int tid, const float4 (&v)[2])
-{
+    // lane: column l32 of a block; register r -> row 8*(r/4) + 4*kh + r%4
+    float *C = p.C;
+    if (OP == F32_WG2) C += (size_t)g * p.N * p.Kd;
+    if (OP == F32_WG13) C += (size_t)mat * p.N * p.Kd;
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
-        const int r = (tid >> 3) + 32 * u, k = 4 * (tid & 7);
-        S[k + 0][r] = v[u].x;
-        S[k + 1][r] = v[u].y;
-        S[k + 2][r] = v[u].z;
-        S[k + 3][r] = v[u].w;
-    }
-}
-
-// C[rows x N] = A[rows x Kd] * B[N x Kd]^T for one (row tile, column tile); FUSED adds the second
-// weight matrix and the SwiGLU epilogue.
-template <bool FUSED, bool VEC>
-__global__ __launch_bounds__(256) void experts_f32_kernel(const float *__restrict__ Axg, const float *__restrict__ Ax,
-                                                          const float *__restrict__ Wa, const float *__restrict__ Wb,
-                                                          float *__restrict__ Cout, const omega_tile *__restrict__ tiles,
-                                                          const int32_t *__restrict__ tile_meta, int N, int Kd)
-{
-    const int mt = blockIdx.y;
-    if (mt >= tile_meta[0]) return;
-    const omega_tile tl = tiles[mt];
-    const int n0 = blockIdx.x * FBN;
-    const float *A = (FUSED && tl.xrow0 >= 0) ? Ax + (size_t)tl.xrow0 * Kd : Axg + (size_t)tl.row0 * Kd;
-    const float *B1 = Wa + ((size_t)tl.g * N + n0) * Kd;
-    const float *B2 = FUSED ? Wb + ((size_t)tl.g * N + n0) * Kd : nullptr;
-    const int brows = min(FBN, N - n0);
-
-    __shared__ float As[FBK][FBM + 1];
-    __shared__ float Bs1[FBK][FBN + 1];
-    __shared__ float Bs2[FUSED ? FBK : 1][FBN + 1];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int l32 = lane & 31, kh = lane >> 5;
-    const int wr = wave >> 1, wc = wave & 1;  // this wave's 32 x 32 block of the tile
-
-    f32x16_t acc1, acc2;
+    for (int i = 0; i < MB; ++i) {
+        if (i >= live) continue;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) acc1[r] = acc2[r] = 0.0f;
-
-    float4 va[2], vb1[2], vb2[2];
-    f32_fetch<VEC>(A, tl.rows, Kd, 0, tid, va);
-    f32_fetch<VEC>(B1, brows, Kd, 0, tid, vb1);
-    if (FUSED) f32_fetch<VEC>(B2, brows, Kd, 0, tid, vb2);
-    for (int k0 = 0; k0 < Kd; k0 += FBK) {
-        f32_stash(As, tid, va);
-        f32_stash(Bs1, tid, vb1);
-        if (FUSED) f32_stash(Bs2, tid, vb2);
-        __syncthreads();
-        if (k0 + FBK < Kd) {  // the next step's rows travel while this one is multiplied
-            f32_fetch<VEC>(A, tl.rows, Kd, k0 + FBK, tid, va);
-            f32_fetch<VEC>(B1, brows, Kd, k0 + FBK, tid, vb1);
-            if (FUSED) f32_fetch<VEC>(B2, brows, Kd, k0 + FBK, tid, vb2);
-        }
+        for (int n = 0; n < (PAIR ? 1 : NB); ++n) {
+            const int col = n0 + xb[n], rbase = 32 * (2 * i + wr) + 4 * kh;
+            if (col >= p.N) continue;
+            const size_t o = (size_t)(WG ? m0 : row0) * p.N + col;
+            float h1[16], h3[16];
+            if (OP == F32_DA) {  // all of the block's h1 and h3 are asked for before any is used (clamped rows: no branches)
 #pragma unroll
-        for (int kk = 0; kk < FBK / 2; ++kk) {
-            const float a = As[2 * kk + kh][wr * 32 + l32];
-            const float b1 = Bs1[2 * kk + kh][wc * 32 + l32];
-            acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b1, acc1, 0, 0, 0);
-            if (FUSED) {
-                const float b2 = Bs2[2 * kk + kh][wc * 32 + l32];
-                acc2 = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b2, acc2, 0, 0, 0);
+                for (int r = 0; r < 16; ++r) {
+                    const size_t at = o + (size_t)min(rbase + 8 * (r >> 2) + (r & 3), rows - 1) * p.N;
+                    h1[r] = p.H1[at];
+                    h3[r] = p.H3[at];
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int row = rbase + 8 * (r >> 2) + (r & 3);
+                if (row >= rows) continue;
+                const size_t at = o + (size_t)row * p.N;
+                const float v = acc[i][n][r];
+                if (PAIR) {
+                    const float u = acc[i][NB - 1][r];
+                    if (OP == F32_UP) C[at] = (v / (1.0f + expf(-v))) * u;
+                    if (OP == F32_RAW || p.H1 != nullptr) {
+                        p.H1[at] = v;
+                        p.H3[at] = u;
+                    }
+                } else if (OP == F32_DA) {
+                    const float sg = 1.0f / (1.0f + expf(-h1[r]));
+                    p.H3[at] = v * (h1[r] * sg);
+                    p.H1[at] = (v * h3[r]) * sg * (1.0f + h1[r] * (1.0f - sg));
+                } else {
+                    C[at] = v;
+                }
             }
         }
-        __syncthreads();
-    }
-    // lane: column l32 of the block; register r -> row 8*(r/4) + 4*kh + r%4
-    const int n = n0 + wc * 32 + l32;
-    if (n >= N) return;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        const int row = wr * 32 + 8 * (r >> 2) + 4 * kh + (r & 3);
-        if (row >= tl.rows) continue;
-        float v = acc1[r];
-        if (FUSED) v = (v / (1.0f + expf(-v))) * acc2[r];
-        Cout[(size_t)(tl.row0 + row) * N + n] = v;
     }
 }
 
-hipError_t launch_experts_f32(const omega_moe *m, const void *x, int T, int which, hipStream_t s)
+int experts_f32_tile_m(const omega_moe *m, int T)
+{
+    // Row tiles of 128 once the experts hold about that many rows and the launches have a tile of 128 x 128 for every compute
+    // unit (the down product has the fewest tiles); else of 64.
+    const omega_moe_config &c = m->cfg;
+    const long long rows = (long long)T * c.K;
+    return rows >= (long long)F32_TILE_M * c.E && rows / F32_TILE_M * ceil_div(c.d, 128) >= m->ctx->num_cus ? F32_TILE_M : F32_TILE_M_SMALL;
+}
+
+template <int OP, int TM, int TN>
+static hipError_t f32_launch(const f32_args &p, bool vec, int max_tiles, hipStream_t s)
+{
+    constexpr int CT = F32_PAIR(OP) ? TN / 2 : TN;
+    const size_t tiles = (size_t)ceil_div(p.N, CT) * (F32_IS_WG(OP) ? (size_t)ceil_div(p.Kd, TM) * p.G * (OP == F32_WG13 ? 2 : 1) : max_tiles);
+    const unsigned grid = (unsigned)((tiles + 7) / 8 * 8);
+    if (vec) hipLaunchKernelGGL((f32_product_kernel<OP, TM, TN, true>), dim3(grid), dim3(256), 0, s, p);
+    else hipLaunchKernelGGL((f32_product_kernel<OP, TM, TN, false>), dim3(grid), dim3(256), 0, s, p);
+    return hipGetLastError();
+}
+
+hipError_t launch_product_f32(const omega_moe *m, int op, const float *x, const float *dout, int T, hipStream_t s)
 {
     const omega_moe_config &c = m->cfg;
-    (void)T;
-    if (which == 0) {
-        dim3 grid(ceil_div(c.H, FBN), m->max_m_tiles);
-        const bool vec = c.d % 4 == 0 && (((uintptr_t)x | (uintptr_t)m->xg | (uintptr_t)m->W1 | (uintptr_t)m->W3) % 16) == 0;
-        if (vec)
-            hipLaunchKernelGGL((experts_f32_kernel<true, true>), grid, dim3(256), 0, s, (const float *)m->xg, (const float *)x,
-                               (const float *)m->W1, (const float *)m->W3, (float *)m->a, m->tiles, m->tile_meta, c.H, c.d);
-        else
-            hipLaunchKernelGGL((experts_f32_kernel<true, false>), grid, dim3(256), 0, s, (const float *)m->xg, (const float *)x,
-                               (const float *)m->W1, (const float *)m->W3, (float *)m->a, m->tiles, m->tile_meta, c.H, c.d);
-    } else {
-        dim3 grid(ceil_div(c.d, FBN), m->max_m_tiles);
-        const bool vec = c.H % 4 == 0 && (((uintptr_t)m->a | (uintptr_t)m->W2) % 16) == 0;
-        if (vec)
-            hipLaunchKernelGGL((experts_f32_kernel<false, true>), grid, dim3(256), 0, s, (const float *)m->a, (const float *)nullptr,
-                               (const float *)m->W2, (const float *)nullptr, m->y, m->tiles, m->tile_meta, c.d, c.H);
-        else
-            hipLaunchKernelGGL((experts_f32_kernel<false, false>), grid, dim3(256), 0, s, (const float *)m->a, (const float *)nullptr,
-                               (const float *)m->W2, (const float *)nullptr, m->y, m->tiles, m->tile_meta, c.d, c.H);
+    f32_args p = {};
+    p.tiles = m->tiles;
+    p.tile_meta = m->tile_meta;
+    p.counts = m->counts;
+    p.E = c.E;
+    p.G = m->G;
+    p.T = T;
+    p.bm = m->bm;
+    const float *W1 = (const float *)m->W1, *W3 = (const float *)m->W3, *W2 = (const float *)m->W2;
+    switch (op) {
+        case F32_UP:
+        case F32_RAW:
+            p.A0 = (const float *)m->xg; p.Atok = x; p.B0 = W1; p.B1 = W3; p.N = c.H; p.Kd = c.d;
+            p.C = (float *)m->a;
+            if (op == F32_RAW) { p.H1 = m->bw_h1; p.H3 = m->bw_h3; }
+            break;
+        case F32_DOWN:
+            p.A0 = (const float *)m->a; p.B0 = W2; p.C = m->y; p.N = c.d; p.Kd = c.H;
+            break;
+        case F32_DA:
+            p.A0 = m->bw_dy; p.Atok = dout; p.B0 = W2; p.H1 = m->bw_h1; p.H3 = m->bw_h3; p.N = c.H; p.Kd = c.d;
+            break;
+        case F32_DXG:
+            p.A0 = m->bw_h1; p.A1 = m->bw_h3; p.B0 = W1; p.B1 = W3; p.C = m->bw_dxg; p.N = c.d; p.Kd = c.H;
+            break;
+        case F32_WG2:
+            p.A0 = m->bw_dy; p.Atok = dout; p.B0 = (const float *)m->a; p.C = m->dW2; p.N = c.H; p.Kd = c.d;
+            break;
+        case F32_WG13:
+            p.A0 = m->bw_h1; p.A1 = m->bw_h3; p.B0 = (const float *)m->xg; p.Btok = x; p.C = m->dW13; p.N = c.d; p.Kd = c.H;
+            break;
+        default: return hipErrorInvalidValue;
     }
-    return hipGetLastError();
+    // 16-byte loads: both widths whole multiples of four floats (every row then starts on 16 bytes) and the caller's
+    // buffers aligned (the layer's own are)
+    const bool vec = c.d % 4 == 0 && c.H % 4 == 0 && (((uintptr_t)x | (uintptr_t)dout) % 16) == 0;
+    const bool big = m->bm == 128;
+    switch (op) {
+        case F32_UP: return big ? f32_launch<F32_UP, 128, 128>(p, vec, m->max_m_tiles, s) : f32_launch<F32_UP, 64, 128>(p, vec, m->max_m_tiles, s);
+        case F32_RAW: return big ? f32_launch<F32_RAW, 128, 128>(p, vec, m->max_m_tiles, s) : f32_launch<F32_RAW, 64, 128>(p, vec, m->max_m_tiles, s);
+        case F32_DOWN: return big ? f32_launch<F32_DOWN, 128, 64>(p, vec, m->max_m_tiles, s) : f32_launch<F32_DOWN, 64, 64>(p, vec, m->max_m_tiles, s);
+        case F32_DA: return big ? f32_launch<F32_DA, 128, 128>(p, vec, m->max_m_tiles, s) : f32_launch<F32_DA, 64, 64>(p, vec, m->max_m_tiles, s);
+        case F32_DXG: return big ? f32_launch<F32_DXG, 128, 64>(p, vec, m->max_m_tiles, s) : f32_launch<F32_DXG, 64, 64>(p, vec, m->max_m_tiles, s);
+        case F32_WG2: return big ? f32_launch<F32_WG2, 128, 128>(p, vec, 0, s) : f32_launch<F32_WG2, 64, 64>(p, vec, 0, s);
+        default: return big ? f32_launch<F32_WG13, 128, 128>(p, vec, 0, s) : f32_launch<F32_WG13, 64, 64>(p, vec, 0, s);
+    }
 }

@@ -1,0 +1,32 @@
+"""The fp32 products at both row-tile heights: rows, widths and k that are no multiple of the tiles, forward and backward
+against the oracle (fp32 sums of at most a few thousand terms: relative L2 within 1e-5, as for every fp32 layer)."""
+import pytest
+
+from oracle import oracle as O
+from oracle import oracle_np as N
+from tests.synth import C
+from tests.test_gpu_backward import _check_grads, _setup
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    dict(T=1300, d=1028, H=68, E=3, K=3, Es=1),    # tiles of 128 rows: ragged row tiles, last column tiles, partial k steps
+    dict(T=1301, d=1027, H=67, E=3, K=3),          # the same without 16-byte loads
+    dict(T=300, d=260, H=132, E=2, K=2),           # tiles of 64 rows, whole and partial k steps
+    dict(T=33, d=31, H=5, E=2, K=1),               # less than one k step
+    dict(T=64, d=32, H=64, E=1, K=1),              # exactly one tile, one k step
+]
+
+
+@pytest.mark.parametrize("kw", CASES)
+def test_fp32_products_match_oracle(kw):
+    G, cfg, inp, dout, layer = _setup("c1_tiny_f32", kw, 77)
+    x = G.P.DeviceBuffer.from_numpy(G.ctx(), inp["x"], cfg.dtype)
+    g = G.P.DeviceBuffer.from_numpy(G.ctx(), dout, cfg.dtype)
+    out = layer.forward(x).to_numpy()
+    assert N.rel_l2(out, G.oracle_forward(cfg, inp)["out"]) < 1e-5
+    dx = layer.back(g).to_numpy()
+    ref = O.moe_backward(inp["x"], dout, inp["Wg"], inp["bg"], inp["W1"], inp["W3"], inp["W2"], cfg.K, cfg.renorm, cfg.Es)
+    assert N.rel_l2(dx, ref["dx"]) < 1e-5
+    _check_grads(layer, cfg, ref, 1e-5)
+    layer.close()
