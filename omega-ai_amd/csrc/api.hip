@@ -317,7 +317,8 @@ static int moe_reserve(omega_moe *m, int T)
     moe_free_workspace(m);
     const omega_moe_config &c = m->cfg;
     const size_t P = (size_t)T * c.K;
-    const int n_tok_tiles = ceil_div(T, router_tok_tile(c.E));
+    // (a smaller batch may have more, lower token tiles than the largest one: at most one per compute unit then)
+    const int n_tok_tiles = std::max(ceil_div(T, router_tok_tile(m, T)), std::min(ceil_div(T, 16), ctx->num_cus));
     const int bm = moe_tile_m(m, T);
     // every expert's rows start on a row-tile boundary: the buffers hold whole tiles, of either height a batch of up to
     // T tokens may take
@@ -404,6 +405,7 @@ int omega_moe_create(omega_ctx *ctx, const omega_moe_config *cfg, omega_moe **ou
     alloc0(&m->Wg, (size_t)c.E * c.d * m->esize);
     alloc0((void **)&m->bg, (size_t)c.E * 4);
     alloc0((void **)&m->gamma, (size_t)c.d * 4);
+    if (c.dtype == OMEGA_DTYPE_BF16 && c.E > 16) alloc0((void **)&m->gate_img, (size_t)ceil_div(c.E, 16) * 16 * c.d * 4);
     alloc0(&m->W1, wsz);
     alloc0(&m->W3, wsz);
     alloc0(&m->W2, wsz);
@@ -417,7 +419,7 @@ int omega_moe_create(omega_ctx *ctx, const omega_moe_config *cfg, omega_moe **ou
         omega_set_error(ctx, e == hipErrorOutOfMemory ? OMEGA_ERR_OOM : OMEGA_ERR_HIP, "moe_create: allocation", e,
                         __FILE__, __LINE__);
         // release whatever was allocated
-        void *ptrs[] = {m->Wg, m->bg, m->W1, m->W3, m->W2, m->counts, m->offsets, m->tile_meta, m->gamma};
+        void *ptrs[] = {m->Wg, m->bg, m->W1, m->W3, m->W2, m->counts, m->offsets, m->tile_meta, m->gamma, m->gate_img};
         for (void *p : ptrs)
             if (p) hipFree(p);
         if (m->ev0) hipEventDestroy(m->ev0);
@@ -429,7 +431,7 @@ int omega_moe_create(omega_ctx *ctx, const omega_moe_config *cfg, omega_moe **ou
         int st = moe_reserve(m, c.T_max);
         if (st != OMEGA_OK) {
             moe_free_workspace(m);
-            void *ptrs[] = {m->Wg, m->bg, m->W1, m->W3, m->W2, m->counts, m->offsets, m->tile_meta, m->gamma};
+            void *ptrs[] = {m->Wg, m->bg, m->W1, m->W3, m->W2, m->counts, m->offsets, m->tile_meta, m->gamma, m->gate_img};
             for (void *p : ptrs)
                 if (p) hipFree(p);
             hipEventDestroy(m->ev0);
@@ -449,7 +451,7 @@ int omega_moe_destroy(omega_moe *m)
     CTX_ENTER(ctx);
     hipStreamSynchronize(ctx->stream);
     moe_free_workspace(m);
-    void *ptrs[] = {m->Wg, m->bg, m->W1, m->W3, m->W2, m->counts, m->offsets, m->tile_meta, m->gamma};
+    void *ptrs[] = {m->Wg, m->bg, m->W1, m->W3, m->W2, m->counts, m->offsets, m->tile_meta, m->gamma, m->gate_img};
     for (void *p : ptrs)
         if (p) hipFree(p);
     if (m->dWg) hipFree(m->dWg);
@@ -503,6 +505,7 @@ int omega_moe_set_weights(omega_moe *m, int which, int expert, const void *src, 
     void *p; size_t bytes;
     if (!src || weight_slot(m, which, expert, &p, &bytes) != OMEGA_OK)
         OMEGA_FAIL(ctx, OMEGA_ERR_INVALID_ARG, "set_weights: bad kind, expert index or source");
+    if (which == OMEGA_W_GATE) m->gate_img_valid = false;
     m->master_valid = false;  // fp32 master copies of a bf16 layer are remade from the weights at the next update
     // the activations (and, in training mode, the h1 / h3 records) of the last forward belong to the old weights: a
     // backward pass needs a new forward first
@@ -914,7 +917,7 @@ int omega_moe_update(omega_moe *m, float lr)
         OMEGA_HIP_CHECK(ctx, launch_update_bf16(m, m->master, lr, 0, ctx->stream));
         if (c.has_gate_bias) OMEGA_HIP_CHECK(ctx, launch_axpy_f32(m->bg, m->dbg, -lr, (size_t)c.E, ctx->stream));
         if (m->gamma_set) OMEGA_HIP_CHECK(ctx, launch_axpy_f32(m->gamma, m->dgamma, -lr, (size_t)c.d, ctx->stream));
-        m->wT_valid = false;
+        m->wT_valid = m->gate_img_valid = false;
         stage_invalidates(m);
         return OMEGA_OK;
     }
@@ -963,7 +966,7 @@ int omega_moe_update_adamw(omega_moe *m, float lr, float beta1, float beta2, flo
             OMEGA_HIP_CHECK(ctx, launch_update_bf16(m, m->master, 0.0f, 1, ctx->stream));
             m->master_valid = true;
         }
-        m->wT_valid = false;
+        m->wT_valid = m->gate_img_valid = false;
     }
     OMEGA_HIP_CHECK(ctx, launch_update_adamw(m, m->master, m->adam_m, m->adam_v, p, ctx->stream));
     stage_invalidates(m);  // the weights changed: a backward pass needs a new forward

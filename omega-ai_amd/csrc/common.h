@@ -57,6 +57,8 @@ struct omega_moe {
     // weights (layer dtype except bg)
     void *Wg = nullptr;   // [E,d]
     float *bg = nullptr;  // [E]
+    float *gate_img = nullptr;            // bf16 layers with more than 16 experts: fp32 image of Wg for the router (router.hip) ...
+    mutable bool gate_img_valid = false;  // ... made by the next router launch after Wg has changed
     void *W1 = nullptr;   // [G,H,d]
     void *W3 = nullptr;   // [G,H,d]
     void *W2 = nullptr;   // [G,d,H]
@@ -161,7 +163,7 @@ struct omega_moe {
 
 // Tokens per router workgroup = per row of tile_counts and per workgroup of the dispatch kernel: 16 for layers
 // with at most 16 experts, else 32 (router.hip).
-int router_tok_tile(int E);
+int router_tok_tile(const omega_moe *m, int T);
 #define ROUTER_TOK_TILE_MAX 32
 
 // Size of the last-level (memory-side) cache of the device: streams larger than this are written / read around it.

@@ -776,7 +776,7 @@ hipError_t launch_dispatch_index(const omega_moe *m, int T, int bm, hipStream_t 
     const bool rows = x != nullptr && c.dtype == OMEGA_DTYPE_BF16;
     // from half the last-level cache of gathered rows on, the rows are written around it
     const int nt_stores = (size_t)T * c.K * c.d * 2 > OMEGA_LLC_BYTES / 2 ? 1 : 0;
-    const int tok_tile = router_tok_tile(c.E);
+    const int tok_tile = router_tok_tile(m, T);
     const int n_tiles = ceil_div(T, tok_tile);
     const int n_sched = m->desc_up != nullptr ? SCHED_WGS : 0;  // bf16 layers
     hipLaunchKernelGGL(dispatch_rank_kernel, dim3(n_tiles + n_sched), dim3(rows ? 1024 : 256), 0, s, m->ids, m->tile_counts, m->counts,

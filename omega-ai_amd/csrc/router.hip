@@ -11,7 +11,7 @@
 //  phase 2  softmax as the reference's thread-per-row kernel (J/engine/gpu/SoftmaxKernel.cu:4-24, CPU twin
 //           J/engine/gpu/SoftmaxKernel.java:69-87): max, e=(float)exp((double)(z-max)), sum in expert order,
 //           divide -- the experts of a token live in the lanes of a wave (or of an 8/16/32-lane group),
-//           the ordered sum is taken through cross-lane reads;
+//           the ordered sum is taken by one lane per token;
 //           top-k: K rounds of a cross-lane (value,index) butterfly arg-max, "greater value, or equal
 //           value and lower index" so ties go to the lowest expert; winners are masked out.
 //  phase 3  LDS-atomic histogram of the selected experts, flushed as row `tile` of tile_counts[.,E].
@@ -26,9 +26,6 @@ typedef __attribute__((ext_vector_type(8))) __bf16 rt_bf16x8;
 typedef __attribute__((ext_vector_type(16))) float rt_f32x16;
 
 #define ROUTER_EPT(EP) ((EP) >= 128 ? 4 : (EP) >= 32 ? 2 : 1)
-// MFMA form of the exact sums (bf16 layers with more than 16 experts): a unit = 16 tokens x 64 experts, one
-// v_mfma_f32_16x16x1_4b_f32 per k; a workgroup of 32 tokens has 2 * ceil(EP/64) units, dealt to its 4 waves
-#define ROUTER_MU(EP) ((EP) > 128 ? 2 : 1)
 // token tile and threads per workgroup for EP (padded) experts
 #define ROUTER_TT(EP) ((EP) <= 16 ? 16 : 32)
 #define ROUTER_NTHR(EP) ((EP) <= 8 ? 128 : 256)
@@ -36,7 +33,13 @@ typedef __attribute__((ext_vector_type(16))) float rt_f32x16;
 // next chunk's loads need to arrive, and the kernel is bound by one memory latency per chunk: 512-k chunks halve their
 // number (Mixtral shape, 4096 tokens: 32-token tiles 42 us; 16-token tiles 54 us with 256-k chunks, 34 us with 512)
 #define ROUTER_KC_SMALL 512
-int router_tok_tile(int E) { return E <= 16 ? 16 : 32; }
+static bool router_on_mfma(const omega_moe *m) { return m->cfg.dtype == OMEGA_DTYPE_BF16 && m->cfg.E > 16; }
+int router_tok_tile(const omega_moe *m, int T)
+{
+    if (m->cfg.E <= 16) return 16;
+    // (matrix-core form: tiles of 16 tokens while they find a compute unit each)
+    return router_on_mfma(m) && m->cfg.router_mode == OMEGA_ROUTER_EXACT && ceil_div(T, 16) <= m->ctx->num_cus ? 16 : 32;
+}
 
 // Phase 1 for the tokens t0.. of one workgroup: acc[x*NT + i] = logit of (token tg + i*TPP, expert e1 + x*EL), bias
 // not yet added.  A thread owns EPT experts (2 from 128 experts on: each x value read from LDS then feeds two sums,
@@ -47,16 +50,10 @@ int router_tok_tile(int E) { return E <= 16 ? 16 : 32; }
 // every load is a whole 16-byte vector; rows beyond T or E are redirected to the last valid row (their sums are
 // never used), which keeps the loads free of branches - and with that really asynchronous: a load issued inside
 // a divergent branch makes the compiler wait for all earlier ones first.
-// MFMA: the sums run on the matrix cores instead (macc; acc is not touched): v_mfma_f32_16x16x1_4b_f32 takes ONE k per
-// instruction - D = C + a*b per element, one product and one addition - so a chain of them over k = 0, 1, 2, ... is
-// the sequential sum, term for term: with bf16 operands every product is exact in fp32 and the addition rounds once,
-// exactly as the fused multiply-add of the vector path does.  A unit of 16 tokens x 64 experts is four 16 x 16 blocks
-// (lane l supplies x[token l % 16][k] and Wg[expert l of the unit][k]); the chain of one unit keeps a SIMD's matrix
-// pipe busy at twice the rate of the vector units, and a lane reads 32 bytes of LDS per 4 k instead of 128.
-template <int EP, int KC, bool EXACT, bool XBF, bool FAST_IO, bool MFMA = false>
+template <int EP, int KC, bool EXACT, bool XBF, bool FAST_IO>
 __device__ __forceinline__ void router_sums(const void *__restrict__ x, const void *__restrict__ Wg, int T, int d, int E,
                                             int t0, float (*xs)[KC + 4], float (*ws)[KC + 4],
-                                            float (&acc)[ROUTER_TT(EP) * EP / ROUTER_NTHR(EP)], rt_f32x16 (&macc)[ROUTER_MU(EP)])
+                                            float (&acc)[ROUTER_TT(EP) * EP / ROUTER_NTHR(EP)])
 {
     constexpr int TOK_TILE = ROUTER_TT(EP), NTHR = ROUTER_NTHR(EP);
     constexpr int EPT = ROUTER_EPT(EP);           // experts per thread
@@ -179,31 +176,7 @@ __device__ __forceinline__ void router_sums(const void *__restrict__ x, const vo
             }                                                                          \
         }                                                                              \
     } while (0)
-        if (MFMA) {
-            constexpr int UNITS = 2 * ((EP + 63) / 64), MU = ROUTER_MU(EP);
-            const int lane = tid & 63, wave = tid >> 6;
-            const float *xrow[MU], *wrow[MU];
-#pragma unroll
-            for (int j = 0; j < MU; ++j) {
-                const int u = min(wave + 4 * j, UNITS - 1);  // (waves without a unit do not enter the loop below)
-                xrow[j] = &xs[(u & 1) * 16 + (lane & 15)][0];
-                wrow[j] = &ws[min((u >> 1) * 64 + lane, EP - 1)][0];
-            }
-            if (wave < UNITS) {  // uniform over the wave
-#pragma unroll 4
-                for (int k4 = 0; k4 < KC / 4; ++k4) {  // (beyond d the staged chunk is zero: a +0 term changes nothing)
-#pragma unroll
-                    for (int j = 0; j < MU; ++j) {
-                        if (wave + 4 * j >= UNITS) continue;
-                        const float4 xv = *(const float4 *)(xrow[j] + k4 * 4), wv = *(const float4 *)(wrow[j] + k4 * 4);
-                        macc[j] = __builtin_amdgcn_mfma_f32_16x16x1f32(xv.x, wv.x, macc[j], 0, 0, 0);
-                        macc[j] = __builtin_amdgcn_mfma_f32_16x16x1f32(xv.y, wv.y, macc[j], 0, 0, 0);
-                        macc[j] = __builtin_amdgcn_mfma_f32_16x16x1f32(xv.z, wv.z, macc[j], 0, 0, 0);
-                        macc[j] = __builtin_amdgcn_mfma_f32_16x16x1f32(xv.w, wv.w, macc[j], 0, 0, 0);
-                    }
-                }
-            }
-        } else if (!wave_live) {
+        if (!wave_live) {
             // every token of this wave lies beyond T: it only stages and keeps the barriers
         } else if (FAST_IO || kend == KC) {
             // whole chunk: no exit test inside, so the LDS reads of later steps are issued ahead of the sums
@@ -227,6 +200,22 @@ __device__ __forceinline__ void router_sums(const void *__restrict__ x, const vo
 // LPT lanes combine by a butterfly on (value, index) with "greater value, or equal value and lower index", so ties go
 // to the lowest expert; the winner is masked out.  RELAXED (the matrix-core FAST path, tolerance mode) takes the
 // exponentials in single precision.
+// The value another lane of the token's 8 or 16 holds, in the lane's own pipeline (DPP) instead of through the LDS crossbar:
+// step 1 and 2 pair the lanes of a quad, 4 the two quads of eight lanes and 8 the two eights of sixteen, each mirrored - after
+// the steps before, the lanes that a mirror exchanges hold the same values, so a butterfly over steps 1, 2, 4 (, 8) leaves every
+// lane with the result of all.  (Worth 1 us of a launch with 6 or 8 rounds.)
+template <int STEP>
+__device__ __forceinline__ int token_lane(int v)
+{
+    constexpr int ctrl = STEP == 1 ? 0xB1 : STEP == 2 ? 0x4E : STEP == 4 ? 0x141 : 0x140;  // quad_perm [1,0,3,2], [2,3,0,1]; row_half_mirror; row_mirror
+    return __builtin_amdgcn_update_dpp(v, v, ctrl, 0xF, 0xF, true);
+}
+template <int STEP>
+__device__ __forceinline__ float token_lane(float v)
+{
+    return __int_as_float(token_lane<STEP>(__float_as_int(v)));
+}
+
 template <int EP, bool RELAXED = false, int TOK_TILE = 32, int NTHR = 256>
 __device__ __forceinline__ void router_select(float (*lg)[EP], int *hist, int t0, int tile, int T, int E, int K, int renorm,
                                               int32_t *__restrict__ ids, float *__restrict__ wout,
@@ -248,8 +237,10 @@ __device__ __forceinline__ void router_select(float (*lg)[EP], int *hist, int t0
         p[q] = (e < E && e < EP) ? lg[tt][e] : -INFINITY;
         mx = fmaxf(mx, p[q]);
     }
-#pragma unroll
-    for (int m = LPT / 2; m >= 1; m >>= 1) mx = fmaxf(mx, __shfl_xor(mx, m, LPT));
+    mx = fmaxf(mx, token_lane<1>(mx));
+    mx = fmaxf(mx, token_lane<2>(mx));
+    mx = fmaxf(mx, token_lane<4>(mx));
+    if (LPT == 16) mx = fmaxf(mx, token_lane<8>(mx));
 #pragma unroll
     for (int q = 0; q < VPL; ++q) {
         const int e = sub + q * LPT;
@@ -258,8 +249,17 @@ __device__ __forceinline__ void router_select(float (*lg)[EP], int *hist, int t0
     }
     __syncthreads();
     float s = 0.0f;
-    if (sub == 0 && live)
-        for (int e = 0; e < E; ++e) s = s + lg[tt][e];
+    if (sub == 0 && live) {
+        int e = 0;
+        for (; e + 16 <= E; e += 16) {  // sixteen reads in flight; the additions stay in expert order
+            float v[16];
+#pragma unroll
+            for (int q = 0; q < 16; ++q) v[q] = lg[tt][e + q];
+#pragma unroll
+            for (int q = 0; q < 16; ++q) s = s + v[q];
+        }
+        for (; e < E; ++e) s = s + lg[tt][e];
+    }
     s = __shfl(s, 0, LPT);
 #pragma unroll
     for (int q = 0; q < VPL; ++q) {
@@ -280,12 +280,13 @@ __device__ __forceinline__ void router_select(float (*lg)[EP], int *hist, int t0
 #pragma unroll
         for (int q = 1; q < VPL; ++q)
             if (p[q] > bv) { bv = p[q]; bi = sub + q * LPT; }
-#pragma unroll
-        for (int m = LPT / 2; m >= 1; m >>= 1) {
-            const float ov = __shfl_xor(bv, m, LPT);
-            const int oi = __shfl_xor(bi, m, LPT);
+        auto meet = [&](float ov, int oi) {
             if (ov > bv || (ov == bv && oi < bi)) { bv = ov; bi = oi; }
-        }
+        };
+        meet(token_lane<1>(bv), token_lane<1>(bi));
+        meet(token_lane<2>(bv), token_lane<2>(bi));
+        meet(token_lane<4>(bv), token_lane<4>(bi));
+        if (LPT == 16) meet(token_lane<8>(bv), token_lane<8>(bi));
         rs = rs + bv;
 #pragma unroll
         for (int u = 0; u < KPL; ++u)
@@ -307,7 +308,7 @@ __device__ __forceinline__ void router_select(float (*lg)[EP], int *hist, int t0
     for (int e = tid; e < E; e += NTHR) tile_counts[(size_t)tile * E + e] = hist[e];
 }
 
-template <int EP, int KC, bool EXACT, bool MFMA = false>
+template <int EP, int KC, bool EXACT>
 __global__ __launch_bounds__(ROUTER_NTHR(EP)) void router_kernel(const void *__restrict__ x, int dtype, const void *__restrict__ Wg,
                                                      const float *__restrict__ bg, int T, int d, int E, int K,
                                                      int renorm, int32_t *__restrict__ ids,
@@ -339,48 +340,16 @@ __global__ __launch_bounds__(ROUTER_NTHR(EP)) void router_kernel(const void *__r
 #pragma unroll
     for (int i = 0; i < NT * EPT; ++i) acc[i] = 0.0f;
 
-    rt_f32x16 macc[ROUTER_MU(EP)];
-#pragma unroll
-    for (int j = 0; j < ROUTER_MU(EP); ++j)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) macc[j][r] = 0.0f;
-
     const bool fast_io = (d % KC == 0) && (((uintptr_t)x | (uintptr_t)Wg) % 16 == 0);
-    if (MFMA) {  // bf16 layers only (the launcher sees to it)
-        if (fast_io) router_sums<EP, KC, EXACT, true, true, true>(x, Wg, T, d, E, t0, xs, ws, acc, macc);
-        else router_sums<EP, KC, EXACT, true, false, true>(x, Wg, T, d, E, t0, xs, ws, acc, macc);
-    } else if (dtype == OMEGA_DTYPE_BF16) {
-        if (fast_io) router_sums<EP, KC, EXACT, true, true>(x, Wg, T, d, E, t0, xs, ws, acc, macc);
-        else router_sums<EP, KC, EXACT, true, false>(x, Wg, T, d, E, t0, xs, ws, acc, macc);
+    if (dtype == OMEGA_DTYPE_BF16) {
+        if (fast_io) router_sums<EP, KC, EXACT, true, true>(x, Wg, T, d, E, t0, xs, ws, acc);
+        else router_sums<EP, KC, EXACT, true, false>(x, Wg, T, d, E, t0, xs, ws, acc);
     } else {
-        if (fast_io) router_sums<EP, KC, EXACT, false, true>(x, Wg, T, d, E, t0, xs, ws, acc, macc);
-        else router_sums<EP, KC, EXACT, false, false>(x, Wg, T, d, E, t0, xs, ws, acc, macc);
-    }
-    if (MFMA) {
-        // unit u = (token half u % 2, expert group u / 2); lane: expert l % 16 of block b, register 4*b + r -> token 4*(l/16) + r
-        constexpr int UNITS = 2 * ((EP + 63) / 64);
-        const int lane = tid & 63, wave = tid >> 6;
-#pragma unroll
-        for (int j = 0; j < ROUTER_MU(EP); ++j) {
-            const int u = wave + 4 * j;
-            if (u >= UNITS) continue;
-#pragma unroll
-            for (int b = 0; b < 4; ++b) {
-                const int e = (u >> 1) * 64 + 16 * b + (lane & 15);
-                if (e >= EP) continue;
-                const float bias = (bg != nullptr && e < E) ? bg[e] : 0.0f;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int tt = (u & 1) * 16 + 4 * (lane >> 4) + r;
-                    const float z = bg != nullptr ? macc[j][4 * b + r] + bias : macc[j][4 * b + r];
-                    lg[tt][e] = z;
-                    if (logits_out != nullptr && t0 + tt < T && e < E) logits_out[(size_t)(t0 + tt) * E + e] = z;
-                }
-            }
-        }
+        if (fast_io) router_sums<EP, KC, EXACT, false, true>(x, Wg, T, d, E, t0, xs, ws, acc);
+        else router_sums<EP, KC, EXACT, false, false>(x, Wg, T, d, E, t0, xs, ws, acc);
     }
 #pragma unroll
-    for (int x_ = 0; x_ < (MFMA ? 0 : EPT); ++x_) {
+    for (int x_ = 0; x_ < EPT; ++x_) {
         const int e = e1 + x_ * EL;
         const float b = (bg != nullptr && e < E) ? bg[e] : 0.0f;
 #pragma unroll
@@ -487,6 +456,153 @@ __global__ __launch_bounds__(256) void router_mfma_kernel(const bf16_t *__restri
     }
     __syncthreads();
     router_select<EP, true>(lg, hist, t0, tile, T, E, K, renorm, ids, wout, tile_counts, probs_out);
+}
+
+// Exact sums of bf16 layers with more than 16 experts on the matrix cores.  v_mfma_f32_16x16x4_f32 forms each element of
+// its result as fma(a3, b3, fma(a2, b2, fma(a1, b1, fma(a0, b0, c)))): a chain of them over k = 0..3, 4..7, ... is the
+// sequential sum, term for term (checked bit for bit against fmaf, exponents from one end of the range to the other); the
+// products of bf16 operands are exact in fp32, so it is also the unfused sum of the exact mode.  An instruction takes four k
+// of 16 tokens x 16 experts where v_mfma_f32_16x16x1_4b_f32 takes one k of 16 x 64: the same rate per matrix core, but
+// chains a quarter as long (d/4 instructions of 44 cycles; 32 where a SIMD has two chains), and four times as many of them.
+// Bound: the chain while the tiles find a SIMD per unit (d = 2048: 512 x 44 cycles = 10 us), then the fp32 matrix rate
+// (16384 tokens x 128 experts: 62 us).  A wave holds CE expert units x CT token units; the workgroup has TT tokens.  Operands: lane
+// l supplies token (expert) l % 16 and k = 4 q + l / 16 of instruction q.  x passes through LDS as fp32, two buffers of RM_KC
+// columns, every 16 columns stored [k % 4][k / 4] so that a lane's four instructions' worth is one 16-byte read; the gate
+// comes from an fp32 image in that very order (router_pack_gate_kernel, made when the weights change), 1 KiB per wave and 16
+// k straight from the L2, up to 16 such loads ahead.
+// Router launch, us, one k per instruction -> four: 48 and 1500 tokens, d = 2048, 64 experts: 50 -> 18.5; 8192 tokens: 53 -> 34;
+// 16384 tokens, 128 experts: 100 -> 88; 300 tokens, 128 experts: 58 -> 29.5; 8192 tokens, 200 experts: 164 -> 82; 4096 tokens,
+// d = 1024, 32 experts: 26 -> 11.  The tolerance mode's kernel (router_mfma_kernel) is as fast up to 1500 tokens and faster
+// behind (8192 tokens 20, 16384 tokens 67), where this one is bound by the fp32 matrix rate.
+#define RM_KC 256
+#define RM_LDW (RM_KC + 4)
+typedef __attribute__((ext_vector_type(4))) float rt_f32x4;
+
+// Wg [E,d] bf16 -> fp32 [unit of 16 experts][k / 16][lane][4]: lane l, value q = Wg[16 unit + l % 16][16 (k/16) + 4 q + l / 16]
+__global__ __launch_bounds__(256) void router_pack_gate_kernel(const bf16_t *__restrict__ Wg, int E, int d, int units, float4 *__restrict__ img)
+{
+    const int KB = d >> 4;
+    for (int i = blockIdx.x * 256 + threadIdx.x; i < units * KB * 64; i += gridDim.x * 256) {
+        const int l = i & 63, kb = (i >> 6) % KB, e = (i >> 6) / KB * 16 + (l & 15), k = 16 * kb + (l >> 4);
+        float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if (e < E) {
+            const bf16_t *w = Wg + (size_t)e * d + k;
+            v = make_float4(bf16_to_f32(w[0]), bf16_to_f32(w[4]), bf16_to_f32(w[8]), bf16_to_f32(w[12]));
+        }
+        img[i] = v;
+    }
+}
+
+template <int EP, int TT, int NW, int CE, int CT>
+__global__ __launch_bounds__(64 * NW) void router_units_kernel(const bf16_t *__restrict__ x, const float4 *__restrict__ img,
+                                                               const float *__restrict__ bg, int T, int d, int E, int K, int renorm,
+                                                               int32_t *__restrict__ ids, float *__restrict__ wout,
+                                                               int32_t *__restrict__ tile_counts, float *__restrict__ logits_out,
+                                                               float *__restrict__ probs_out)
+{
+    constexpr int NTHR = 64 * NW, EU = EP / 16, NWE = EU / CE;  // waves across the experts
+    static_assert(NWE * (TT / 16 / CT) == NW, "every unit has one wave");
+    constexpr int XV = TT * RM_KC / 8 / NTHR;                    // 16-byte pieces of x per thread and chunk
+    static_assert(XV * NTHR * 8 == TT * RM_KC, "whole pieces per thread");
+    constexpr int PD = CE > 2 ? 2 : 16 / CE, BPC = RM_KC / 16;         // gate loads in flight; 16-k blocks per chunk
+    __shared__ __attribute__((aligned(16))) float xs[2][TT][RM_LDW];
+    __shared__ int hist[EP];
+    static_assert(EP <= RM_LDW, "the logits take the place of the staged rows");
+    float(*lg)[EP] = (float(*)[EP]) & xs[0][0][0];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l16 = lane & 15, lq = lane >> 4;
+    const int tile = blockIdx.x, t0 = tile * TT;
+    for (int i = tid; i < EP; i += NTHR) hist[i] = 0;
+    const int u0 = (wave % NWE) * CE, tu0 = (wave / NWE) * CT;   // first expert unit, first token unit of this wave
+    const int KB = d >> 4, nch = d / RM_KC;
+    const bool live = 16 * u0 < E && t0 + 16 * tu0 < T;          // a wave without experts or tokens only stages
+    const bool aligned = ((uintptr_t)x & 15) == 0;
+
+    uint4 xr[XV];
+    auto fetch = [&](int c) {
+#pragma unroll
+        for (int v = 0; v < XV; ++v) {
+            const int i = tid + v * NTHR;
+            const bf16_t *p = x + (size_t)min(t0 + i / (RM_KC / 8), T - 1) * d + c * RM_KC + (i % (RM_KC / 8)) * 8;
+            if (aligned) xr[v] = *(const uint4 *)p;
+            else xr[v] = make_uint4(p[0] | (uint32_t)p[1] << 16, p[2] | (uint32_t)p[3] << 16, p[4] | (uint32_t)p[5] << 16, p[6] | (uint32_t)p[7] << 16);
+        }
+    };
+    auto stash = [&](int c) {
+#pragma unroll
+        for (int v = 0; v < XV; ++v) {
+            const int i = tid + v * NTHR, k8 = i % (RM_KC / 8);
+            float *o = &xs[c & 1][i / (RM_KC / 8)][(k8 >> 1) * 16 + (k8 & 1) * 2];  // k = 8 k8 + j: [j % 4][2 (k8 % 2) + j / 4]
+            *(float2 *)(o + 0) = make_float2(__uint_as_float(xr[v].x << 16), __uint_as_float(xr[v].z << 16));
+            *(float2 *)(o + 4) = make_float2(__uint_as_float(xr[v].x & 0xffff0000u), __uint_as_float(xr[v].z & 0xffff0000u));
+            *(float2 *)(o + 8) = make_float2(__uint_as_float(xr[v].y << 16), __uint_as_float(xr[v].w << 16));
+            *(float2 *)(o + 12) = make_float2(__uint_as_float(xr[v].y & 0xffff0000u), __uint_as_float(xr[v].w & 0xffff0000u));
+        }
+    };
+    const float4 *wp[CE];
+#pragma unroll
+    for (int e = 0; e < CE; ++e) wp[e] = img + (size_t)min(u0 + e, (E - 1) >> 4) * KB * 64 + lane;
+    float4 wb[PD][CE];
+    rt_f32x4 acc[CT][CE];
+#pragma unroll
+    for (int t = 0; t < CT; ++t)
+#pragma unroll
+        for (int e = 0; e < CE; ++e)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[t][e][r] = 0.0f;
+
+    fetch(0);
+    if (live)
+#pragma unroll
+        for (int b = 0; b < PD; ++b)
+#pragma unroll
+            for (int e = 0; e < CE; ++e) wb[b][e] = wp[e][(size_t)b * 64];
+    stash(0);
+    for (int c = 0; c < nch; ++c) {
+        __syncthreads();  // chunk c is staged, and chunk c - 1 summed
+        if (c + 1 < nch) fetch(c + 1);
+        if (live) {
+            const float *xp = &xs[c & 1][16 * tu0 + l16][4 * lq];
+#pragma unroll
+            for (int b = 0; b < BPC; ++b) {
+                float4 xa[CT], w[CE];
+#pragma unroll
+                for (int t = 0; t < CT; ++t) xa[t] = *(const float4 *)(xp + t * 16 * RM_LDW + b * 16);
+#pragma unroll
+                for (int e = 0; e < CE; ++e) {
+                    w[e] = wb[b % PD][e];
+                    wb[b % PD][e] = wp[e][(size_t)min(c * BPC + b + PD, KB - 1) * 64];
+                }
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+#pragma unroll
+                    for (int t = 0; t < CT; ++t)
+#pragma unroll
+                        for (int e = 0; e < CE; ++e)
+                            acc[t][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(((const float *)&xa[t])[q], ((const float *)&w[e])[q], acc[t][e], 0, 0, 0);
+            }
+        }
+        if (c + 1 < nch) stash(c + 1);
+    }
+    __syncthreads();
+    // lane: expert l16 of unit u0 + e; register r -> token 4 lq + r of unit tu0 + t
+    if (live)
+#pragma unroll
+        for (int t = 0; t < CT; ++t)
+#pragma unroll
+            for (int e = 0; e < CE; ++e) {
+                const int ex = 16 * (u0 + e) + l16;
+                const float bias = bg != nullptr && ex < E ? bg[ex] : 0.0f;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int tt = 16 * (tu0 + t) + 4 * lq + r;
+                    const float z = bg != nullptr ? acc[t][e][r] + bias : acc[t][e][r];
+                    lg[tt][ex] = z;
+                    if (logits_out != nullptr && t0 + tt < T && ex < E) logits_out[(size_t)(t0 + tt) * E + ex] = z;
+                }
+            }
+    __syncthreads();
+    router_select<EP, false, TT, NTHR>(lg, hist, t0, tile, T, E, K, renorm, ids, wout, tile_counts, probs_out);
 }
 
 // Batches of at most one 16-token tile per compute unit, bf16, at most 16 experts, d a multiple of 512: the whole
@@ -626,10 +742,10 @@ hipError_t router_init(void)
 hipError_t launch_router(const omega_moe *m, const void *x, int T, float *logits_out, float *probs_out, hipStream_t s)
 {
     const omega_moe_config &c = m->cfg;
-    const int tiles = ceil_div(T, router_tok_tile(c.E));
+    const int tiles = ceil_div(T, router_tok_tile(m, T));
     const int exact = c.router_mode == OMEGA_ROUTER_EXACT;
     const float *bg = c.has_gate_bias ? m->bg : nullptr;
-    if (!exact && c.dtype == OMEGA_DTYPE_BF16 && c.E > 16 && ((uintptr_t)x % 16) == 0) {
+    if (!exact && router_on_mfma(m) && ((uintptr_t)x % 16) == 0) {
 #define ROUTER_MFMA_LAUNCH(EPV)                                                                                          \
     hipLaunchKernelGGL(router_mfma_kernel<EPV>, dim3(tiles), dim3(256), 0, s, (const bf16_t *)x, (const bf16_t *)m->Wg, bg, T, \
                        c.d, c.E, c.K, c.renorm, m->ids, m->w, m->tile_counts, logits_out, probs_out)
@@ -638,6 +754,26 @@ hipError_t launch_router(const omega_moe *m, const void *x, int T, float *logits
         else if (c.E <= 128) ROUTER_MFMA_LAUNCH(128);
         else ROUTER_MFMA_LAUNCH(256);
 #undef ROUTER_MFMA_LAUNCH
+        return hipGetLastError();
+    }
+    if (router_on_mfma(m)) {
+        const int units = ceil_div(c.E, 16), tt = router_tok_tile(m, T);
+        if (!m->gate_img_valid) {
+            const int n = units * (c.d / 16) * 64;
+            hipLaunchKernelGGL(router_pack_gate_kernel, dim3(ceil_div(n, 256)), dim3(256), 0, s, (const bf16_t *)m->Wg, c.E, c.d, units,
+                               (float4 *)m->gate_img);
+            hipError_t e = hipGetLastError();
+            if (e != hipSuccess) return e;
+            m->gate_img_valid = true;
+        }
+#define ROUTER_UNITS(EPV, TTV, NWV, CEV, CTV)                                                                            \
+    hipLaunchKernelGGL((router_units_kernel<EPV, TTV, NWV, CEV, CTV>), dim3(tiles), dim3(64 * NWV), 0, s, (const bf16_t *)x, \
+                       (const float4 *)m->gate_img, bg, T, c.d, c.E, c.K, c.renorm, m->ids, m->w, m->tile_counts, logits_out, probs_out)
+        if (c.E <= 32) { if (tt == 16) ROUTER_UNITS(32, 16, 2, 1, 1); else ROUTER_UNITS(32, 32, 4, 1, 1); }
+        else if (c.E <= 64) { if (tt == 16) ROUTER_UNITS(64, 16, 4, 1, 1); else ROUTER_UNITS(64, 32, 4, 1, 2); }
+        else if (c.E <= 128) { if (tt == 16) ROUTER_UNITS(128, 16, 4, 2, 1); else ROUTER_UNITS(128, 32, 8, 1, 2); }
+        else { if (tt == 16) ROUTER_UNITS(256, 16, 4, 4, 1); else ROUTER_UNITS(256, 32, 8, 2, 2); }
+#undef ROUTER_UNITS
         return hipGetLastError();
     }
     // at most 16 experts, bf16, at most one tile per compute unit: chains fed by staging waves (either mode: same bits)
@@ -653,14 +789,9 @@ hipError_t launch_router(const omega_moe *m, const void *x, int T, float *logits
                                m->tile_counts, logits_out, probs_out);
         return hipGetLastError();
     }
-    // exact sums of bf16 layers with more than 16 experts: on the matrix cores, one k per instruction
-    const bool exact_mfma = exact && c.dtype == OMEGA_DTYPE_BF16 && c.E > 16;
 #define ROUTER_LAUNCH(EPV, KCV)                                                                                    \
     do {                                                                                                           \
-        if (exact_mfma)                                                                                            \
-            hipLaunchKernelGGL((router_kernel<EPV, KCV, true, (EPV > 16)>), dim3(tiles), dim3(ROUTER_NTHR(EPV)), 0, s, x, c.dtype, m->Wg, bg, \
-                               T, c.d, c.E, c.K, c.renorm, m->ids, m->w, m->tile_counts, logits_out, probs_out);   \
-        else if (exact)                                                                                            \
+        if (exact)                                                                                            \
             hipLaunchKernelGGL((router_kernel<EPV, KCV, true>), dim3(tiles), dim3(ROUTER_NTHR(EPV)), 0, s, x, c.dtype, m->Wg, bg, \
                                T, c.d, c.E, c.K, c.renorm, m->ids, m->w, m->tile_counts, logits_out, probs_out);   \
         else                                                                                                       \
