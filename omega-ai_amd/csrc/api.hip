@@ -255,7 +255,7 @@ static int moe_reserve_backward(omega_moe *m, int T)
     OMEGA_HIP_CHECK(ctx, hipMalloc((void **)&m->bw_probs, (size_t)Tc * c.E * 4));
     OMEGA_HIP_CHECK(ctx, hipMalloc((void **)&m->bw_dw, (size_t)Tc * c.K * 4));
     OMEGA_HIP_CHECK(ctx, hipMalloc((void **)&m->bw_dlogits, (size_t)Tc * c.E * 4));
-    OMEGA_HIP_CHECK(ctx, hipMalloc((void **)&m->bw_gpart, (size_t)32 * c.E * c.d * 4));
+    OMEGA_HIP_CHECK(ctx, hipMalloc((void **)&m->bw_gpart, (size_t)bw_gate_slices(m) * c.E * c.d * 4));
     OMEGA_HIP_CHECK(ctx, hipMalloc(&m->bw_dhx, (size_t)Tc * c.d * m->esize));
     OMEGA_HIP_CHECK(ctx, hipMalloc((void **)&m->bw_h1, rc * c.H * 4));
     OMEGA_HIP_CHECK(ctx, hipMalloc((void **)&m->bw_h3, rc * c.H * 4));

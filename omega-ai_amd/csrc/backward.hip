@@ -19,6 +19,7 @@
 //   bw_dx_kernel        dx[t,:] = sum_j dxg[row(t,j),:] + shared rows + dlogits[t,:] . Wg
 #include "common.h"
 #include "pack.h"
+#include <algorithm>
 
 __device__ __forceinline__ float block_sum_256(float v, float *red)
 {
@@ -53,14 +54,15 @@ __global__ __launch_bounds__(256) void bw_combine_kernel(const float *__restrict
     }
 }
 
-// One thread per token: dw -> gradient of the selected probabilities (through the renormalisation w = q / sum q when
-// enabled) -> softmax_back over the E experts.  Only the selected experts have a non-zero probability gradient, so
-// sum_e p_e*dp_e runs over the K slots.
+// dw -> gradient of the selected probabilities (through the renormalisation w = q / sum q when enabled) -> softmax_back
+// over the E experts.  Only the selected experts have a non-zero probability gradient, so sum_e p_e*dp_e runs over the K
+// slots.  16 lanes per token: each forms the K-slot sums, then every 16th row element (a thread per token wrote its row
+// alone: 3000 tokens, 16 experts 11.7 -> 5 us).
 __global__ __launch_bounds__(256) void bw_router_kernel(const float *__restrict__ probs, const int32_t *__restrict__ ids,
                                                         const float *__restrict__ w, const float *__restrict__ dw, int T,
                                                         int E, int K, int renorm, float *__restrict__ dlogits)
 {
-    const int t = blockIdx.x * 256 + threadIdx.x;
+    const int t = blockIdx.x * 16 + (threadIdx.x >> 4), sub = threadIdx.x & 15;
     if (t >= T) return;
     const float *p = probs + (size_t)t * E;
     const int32_t *id = ids + (size_t)t * K;
@@ -77,83 +79,138 @@ __global__ __launch_bounds__(256) void bw_router_kernel(const float *__restrict_
         sum = fmaf(p[id[j]], g, sum);
     }
     float *dl = dlogits + (size_t)t * E;
-    for (int e = 0; e < E; ++e) dl[e] = (0.0f - sum) * p[e];
-    for (int j = 0; j < K; ++j) {
-        float g = dw[(size_t)t * K + j];
-        if (renorm) g = (g - dot) / S;
-        dl[id[j]] = (g - sum) * p[id[j]];
+    for (int e = sub; e < E; e += 16) {
+        float g = 0.0f;
+        for (int j = 0; j < K; ++j)
+            if (id[j] == e) {
+                g = dw[(size_t)t * K + j];
+                if (renorm) g = (g - dot) / S;
+            }
+        dl[e] = (g - sum) * p[e];
     }
 }
 
 // Gate weight gradient dWg[e,k] = sum_t dlogits[t,e] * x[t,k] (diffW = delta^T . input) in two steps, both with a fixed
-// order of additions: partial sums over slices of the tokens, then their sum.  Workgroup (column chunk of 256, token
-// slice, expert chunk of 32): a thread owns one column and up to 32 experts; the slice's dlogits pass through LDS.
-#define GW_EC 32
-template <bool XBF>
+// order of additions: partial sums over slices of the tokens, then their sum.  A wave takes a slice of the tokens, 256
+// columns and 32 experts on the fp32 matrix cores (v_mfma_f32_32x32x2: two tokens per instruction): lane l supplies
+// dlogits[token, e0 + l % 32] and, from one piece of 8 adjacent columns of x per token, the operands of eight column blocks
+// {8 c + j}, so nothing passes through LDS.  Bound: reading x (and the matrix rate from 32 experts on); with one thread per
+// column and 32 sums in registers the launch was one load latency per token: 4096 tokens x 4096 columns x 8 experts
+// 89 -> 25 us, 3000 x 2048 x 16: 82 -> 18 us.
+typedef __attribute__((ext_vector_type(16))) float gw_f32x16;
+template <bool XBF, bool VEC>
 __global__ __launch_bounds__(256) void bw_gate_partial_kernel(const float *__restrict__ dlogits, const void *__restrict__ x,
                                                               int T, int d, int E, int tslice, float *__restrict__ part)
 {
-    __shared__ __attribute__((aligned(16))) float dl[64][GW_EC];
-    const int k = blockIdx.x * 256 + threadIdx.x, e0 = blockIdx.z * GW_EC;
-    const int t0 = blockIdx.y * tslice, t1 = min(T, t0 + tslice);
-    float acc[GW_EC];
+    const int lane = threadIdx.x & 63, sl = blockIdx.y * 4 + (threadIdx.x >> 6);
+    const int l32 = lane & 31, kh = lane >> 5;
+    const int c = blockIdx.x * 256 + 8 * l32, e0 = blockIdx.z * 32;
+    const int t0 = sl * tslice, t1 = min(T, t0 + tslice);
+    if (t0 >= T) return;
+    gw_f32x16 acc[8];
 #pragma unroll
-    for (int e = 0; e < GW_EC; ++e) acc[e] = 0.0f;
-    for (int tb = t0; tb < t1; tb += 64) {
-        __syncthreads();
-        for (int i = threadIdx.x; i < 64 * GW_EC; i += 256) {
-            const int tt = tb + i / GW_EC, e = e0 + i % GW_EC;
-            dl[i / GW_EC][i % GW_EC] = (tt < t1 && e < E) ? dlogits[(size_t)tt * E + e] : 0.0f;
-        }
-        __syncthreads();
-        if (k < d) {
-            const int n = min(64, t1 - tb);
-            for (int tt = 0; tt < n; ++tt) {
-                const float xv = XBF ? bf16_to_f32(((const bf16_t *)x)[(size_t)(tb + tt) * d + k])
-                                     : ((const float *)x)[(size_t)(tb + tt) * d + k];
+    for (int j = 0; j < 8; ++j)
 #pragma unroll
-                for (int e4 = 0; e4 < GW_EC / 4; ++e4) {  // the whole wave reads the same 16 bytes: one broadcast read
-                    const float4 v = *(const float4 *)&dl[tt][e4 * 4];
-                    acc[e4 * 4 + 0] = fmaf(v.x, xv, acc[e4 * 4 + 0]);
-                    acc[e4 * 4 + 1] = fmaf(v.y, xv, acc[e4 * 4 + 1]);
-                    acc[e4 * 4 + 2] = fmaf(v.z, xv, acc[e4 * 4 + 2]);
-                    acc[e4 * 4 + 3] = fmaf(v.w, xv, acc[e4 * 4 + 3]);
+        for (int r = 0; r < 16; ++r) acc[j][r] = 0.0f;
+    constexpr int U = 8;  // token pairs in flight
+    for (int tb = t0; tb < t1; tb += 2 * U) {
+        float dl[U], xv[U][8];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int t = tb + 2 * u + kh, tc = min(t, t1 - 1);
+            dl[u] = dlogits[(size_t)tc * E + min(e0 + l32, E - 1)];
+            if (t >= t1) dl[u] = 0.0f;
+            if (VEC && XBF) {
+                const uint4 v = *(const uint4 *)((const bf16_t *)x + (size_t)tc * d + min(c, d - 8));
+                const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    xv[u][2 * q] = __uint_as_float(w[q] << 16);
+                    xv[u][2 * q + 1] = __uint_as_float(w[q] & 0xffff0000u);
+                }
+            } else if (VEC) {
+                const float *p = (const float *)x + (size_t)tc * d + min(c, d - 8);
+                *(float4 *)&xv[u][0] = *(const float4 *)p;
+                *(float4 *)&xv[u][4] = *(const float4 *)(p + 4);
+            } else {
+#pragma unroll
+                for (int q = 0; q < 8; ++q) {
+                    const size_t o = (size_t)tc * d + min(c + q, d - 1);
+                    xv[u][q] = XBF ? bf16_to_f32(((const bf16_t *)x)[o]) : ((const float *)x)[o];
                 }
             }
         }
-    }
-    if (k < d)
 #pragma unroll
-        for (int e = 0; e < GW_EC; ++e)
-            if (e0 + e < E) part[((size_t)blockIdx.y * E + e0 + e) * d + k] = acc[e];
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(dl[u], xv[u][j], acc[j], 0, 0, 0);
+    }
+    // register r of block j: expert e0 + 8*(r/4) + 4*kh + r%4, column c + j
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const int e = e0 + 8 * (r >> 2) + 4 * kh + (r & 3);
+        if (e >= E) continue;
+        float *o = part + ((size_t)sl * E + e) * d + c;
+        if (VEC) {
+            if (c < d) {
+                *(float4 *)o = make_float4(acc[0][r], acc[1][r], acc[2][r], acc[3][r]);
+                *(float4 *)(o + 4) = make_float4(acc[4][r], acc[5][r], acc[6][r], acc[7][r]);
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                if (c + j < d) o[j] = acc[j][r];
+        }
+    }
 }
 
-__global__ __launch_bounds__(256) void bw_gate_reduce_kernel(const float *__restrict__ part, int nslices, size_t n,
-                                                             float *__restrict__ dWg)
+// out[i] = sum_q part[q][i]: 64 elements per workgroup, four threads each with a quarter of the slices
+__global__ __launch_bounds__(256) void bw_part_sums_kernel(const float *__restrict__ part, int nsl, size_t n, float *__restrict__ out)
 {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
+    __shared__ float red[4][64];
+    const int l = threadIdx.x & 63, sg = threadIdx.x >> 6;
+    const size_t i = (size_t)blockIdx.x * 64 + l;
+    const int per = (nsl + 3) / 4, q0 = sg * per, q1 = min(nsl, q0 + per);
     float s = 0.0f;
-    for (int q = 0; q < nslices; ++q) s += part[(size_t)q * n + i];
-    dWg[i] = s;
+    if (i < n) {
+        int q = q0;
+        for (; q + 16 <= q1; q += 16) {
+            float v[16];
+#pragma unroll
+            for (int u = 0; u < 16; ++u) v[u] = part[(size_t)(q + u) * n + i];
+#pragma unroll
+            for (int u = 0; u < 16; ++u) s += v[u];
+        }
+        for (; q < q1; ++q) s += part[(size_t)q * n + i];
+    }
+    red[sg][l] = s;
+    __syncthreads();
+    if (sg == 0 && i < n) out[i] = (red[0][l] + red[1][l]) + (red[2][l] + red[3][l]);
 }
 
-#define GW_SLICES 32
+hipError_t launch_part_sums(const float *part, int nsl, size_t n, float *out, hipStream_t s)
+{
+    hipLaunchKernelGGL(bw_part_sums_kernel, dim3((unsigned)((n + 63) / 64)), dim3(256), 0, s, part, nsl, n, out);
+    return hipGetLastError();
+}
+
 static hipError_t launch_gate_wgrad(const omega_moe *m, const void *x, int T, hipStream_t s)
 {
     const omega_moe_config &c = m->cfg;
-    const int tslice = ceil_div(ceil_div(T, GW_SLICES), 64) * 64, nsl = ceil_div(T, tslice);
-    const dim3 grid(ceil_div(c.d, 256), nsl, ceil_div(c.E, GW_EC));
-    if (c.dtype == OMEGA_DTYPE_BF16)
-        hipLaunchKernelGGL(bw_gate_partial_kernel<true>, grid, dim3(256), 0, s, (const float *)m->bw_dlogits, x, T, c.d, c.E,
-                           tslice, m->bw_gpart);
-    else
-        hipLaunchKernelGGL(bw_gate_partial_kernel<false>, grid, dim3(256), 0, s, (const float *)m->bw_dlogits, x, T, c.d, c.E,
-                           tslice, m->bw_gpart);
-    const size_t n = (size_t)c.E * c.d;
-    hipLaunchKernelGGL(bw_gate_reduce_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, (const float *)m->bw_gpart, nsl,
-                       n, m->dWg);
-    return hipGetLastError();
+    const int cb = ceil_div(c.d, 256), eb = ceil_div(c.E, 32);
+    // token slices: about 2048 waves in all, 16 tokens or more each
+    int nsl = std::min({bw_gate_slices(m), std::max(4, 2048 / (cb * eb)), ceil_div(T, 16)});
+    const int tslice = ceil_div(ceil_div(T, nsl), 2) * 2;
+    nsl = ceil_div(T, tslice);
+    const dim3 grid(cb, ceil_div(nsl, 4), eb);
+    const bool vec = c.d % 8 == 0 && ((uintptr_t)x % 16) == 0;
+#define GATE_PARTIAL(BF, V) hipLaunchKernelGGL((bw_gate_partial_kernel<BF, V>), grid, dim3(256), 0, s, (const float *)m->bw_dlogits, x, T, c.d, c.E, tslice, m->bw_gpart)
+    if (c.dtype == OMEGA_DTYPE_BF16) { if (vec) GATE_PARTIAL(true, true); else GATE_PARTIAL(true, false); }
+    else { if (vec) GATE_PARTIAL(false, true); else GATE_PARTIAL(false, false); }
+#undef GATE_PARTIAL
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    return launch_part_sums(m->bw_gpart, nsl, (size_t)c.E * c.d, m->dWg, s);
 }
 
 // dbg[e] = sum_t dlogits[t,e]: one workgroup per expert.
@@ -233,7 +290,10 @@ __global__ __launch_bounds__(256) void bw_dx_kernel(const float *__restrict__ dx
 
 // bf16 layers (d is a multiple of 256): four adjacent columns per thread (16-byte loads of the fp32 rows, 8-byte loads
 // of the gate weights), the row indices of the workgroup's tokens staged in LDS so that the loads of a token's rows do
-// not wait for index loads one by one.  Same sums in the same order as bw_dx_kernel.
+// not wait for index loads one by one.  Same sums in the same order as bw_dx_kernel.  KU: rows of a token fetched together
+// (slots past K re-read the last row), of 8 / KU tokens at a time.  Bound: the fp32 rows of dxg; 4096 tokens x 4096 columns, K = 2:
+// 64 -> 60 us with two rows instead of eight per token, 39 us straight behind the product that writes them.
+template <int KU>
 __global__ __launch_bounds__(256) void bw_dx4_bf16_kernel(const float *__restrict__ dxg, const int32_t *__restrict__ dstp,
                                                           const float *__restrict__ dlogits, const bf16_t *__restrict__ Wg,
                                                           const int32_t *__restrict__ tile_meta, int T, int K, int d, int E,
@@ -266,30 +326,40 @@ __global__ __launch_bounds__(256) void bw_dx4_bf16_kernel(const float *__restric
 #pragma unroll
             for (int v = 0; v < 4; ++v) g[v][tt] = fmaf(dv[tt], w[v], g[v][tt]);
     }
+    constexpr int TG = 8 / KU;  // tokens whose rows are fetched together
 #pragma unroll
-    for (int tt = 0; tt < DX_TT; ++tt) {
-        if (tt >= nt) break;
-        const int t = t0 + tt;
-        float a[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-        for (int j0 = 0; j0 < K; j0 += 8) {
-            float4 v[8];
+    for (int tg = 0; tg < DX_TT; tg += TG) {
+        if (tg >= nt) break;
+        float a[TG][4];
 #pragma unroll
-            for (int u = 0; u < 8; ++u)  // slots past K re-read the last row and are not added
-                v[u] = *(const float4 *)(dxg + (size_t)rows_s[tt * K + min(j0 + u, K - 1)] * d + c);
+        for (int u = 0; u < TG; ++u) a[u][0] = a[u][1] = a[u][2] = a[u][3] = 0.0f;
+        for (int j0 = 0; j0 < K; j0 += KU) {
+            float4 v[TG][KU];
 #pragma unroll
-            for (int u = 0; u < 8; ++u)
-                if (j0 + u < K) { a[0] += v[u].x; a[1] += v[u].y; a[2] += v[u].z; a[3] += v[u].w; }
+            for (int u = 0; u < TG; ++u)
+#pragma unroll
+                for (int w = 0; w < KU; ++w) v[u][w] = *(const float4 *)(dxg + (size_t)rows_s[min(tg + u, nt - 1) * K + min(j0 + w, K - 1)] * d + c);
+#pragma unroll
+            for (int u = 0; u < TG; ++u)
+#pragma unroll
+                for (int w = 0; w < KU; ++w)
+                    if (j0 + w < K) { a[u][0] += v[u][w].x; a[u][1] += v[u][w].y; a[u][2] += v[u][w].z; a[u][3] += v[u][w].w; }
         }
-        for (int s = 0; s < Es; ++s) {
-            const float4 v = *(const float4 *)(dxg + ((size_t)tile_meta[1 + E + s] * bm + t) * d + c);
-            a[0] += v.x; a[1] += v.y; a[2] += v.z; a[3] += v.w;
-        }
 #pragma unroll
-        for (int q = 0; q < 4; ++q) a[q] += g[q][tt];
-        uint2 o;
-        o.x = (uint32_t)f32_to_bf16(a[0]) | ((uint32_t)f32_to_bf16(a[1]) << 16);
-        o.y = (uint32_t)f32_to_bf16(a[2]) | ((uint32_t)f32_to_bf16(a[3]) << 16);
-        *(uint2 *)(dx + (size_t)t * d + c) = o;
+        for (int u = 0; u < TG; ++u) {
+            const int tt = tg + u, t = t0 + tt;
+            if (tt >= nt) break;
+            for (int s = 0; s < Es; ++s) {
+                const float4 v = *(const float4 *)(dxg + ((size_t)tile_meta[1 + E + s] * bm + t) * d + c);
+                a[u][0] += v.x; a[u][1] += v.y; a[u][2] += v.z; a[u][3] += v.w;
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q) a[u][q] += g[q][tt];
+            uint2 o;
+            o.x = (uint32_t)f32_to_bf16(a[u][0]) | ((uint32_t)f32_to_bf16(a[u][1]) << 16);
+            o.y = (uint32_t)f32_to_bf16(a[u][2]) | ((uint32_t)f32_to_bf16(a[u][3]) << 16);
+            *(uint2 *)(dx + (size_t)t * d + c) = o;
+        }
     }
 }
 
@@ -522,7 +592,7 @@ hipError_t launch_backward_f32(const omega_moe *m, const void *xv, const void *d
     for (int op : {F32_RAW, F32_DA, F32_DXG, F32_WG2, F32_WG13})
         if ((e = launch_product_f32(m, op, x, dout, T, s)) != hipSuccess) return e;
     // router and gate
-    hipLaunchKernelGGL(bw_router_kernel, dim3(ceil_div(T, 256)), dim3(256), 0, s, (const float *)m->bw_probs, m->ids, m->w,
+    hipLaunchKernelGGL(bw_router_kernel, dim3(ceil_div(T, 16)), dim3(256), 0, s, (const float *)m->bw_probs, m->ids, m->w,
                        (const float *)m->bw_dw, T, c.E, c.K, c.renorm, m->bw_dlogits);
     if ((e = launch_gate_wgrad(m, x, T, s)) != hipSuccess) return e;
     if (c.has_gate_bias)
@@ -623,6 +693,23 @@ hipError_t launch_backward_bf16(const omega_moe *m, const void *x, const void *d
     STEP(launch_product_bf16(m, MODE_DOWN, m->bw_dh16, nullptr, m->W13T, nullptr, m->bw_dxg, sliced ? (void *)m->y_slabs : nullptr,
                              nullptr, m->wq_down, c.d, 2 * c.H, s));
     if (sliced) STEP(launch_down_slab_reduce(m, m->bw_dxg, s));
+    // router and gate, and the input gradient while the rows of dxg are in the last-level cache (behind the weight
+    // gradients, which write 5.6 GB at the Mixtral shape, the launch took 60 us there)
+    hipLaunchKernelGGL(bw_router_kernel, dim3(ceil_div(T, 16)), dim3(256), 0, s, (const float *)m->bw_probs, m->ids, m->w,
+                       (const float *)m->bw_dw, T, c.E, c.K, c.renorm, m->bw_dlogits);
+    STEP(launch_gate_wgrad(m, x, T, s));
+    if (c.has_gate_bias)
+        hipLaunchKernelGGL(bw_gate_bias_kernel, dim3(c.E), dim3(256), 0, s, (const float *)m->bw_dlogits, T, c.E, m->dbg);
+#define DX4(KU)                                                                                                          \
+    hipLaunchKernelGGL(bw_dx4_bf16_kernel<KU>, dim3(ceil_div(T, DX_TT), ceil_div(c.d, 1024)), dim3(256),                  \
+                       (c.E * DX_TT + DX_TT * c.K) * sizeof(float), s, (const float *)m->bw_dxg, m->dstp,                 \
+                       (const float *)m->bw_dlogits, (const bf16_t *)m->Wg, m->tile_meta, T, c.K, c.d, c.E, c.Es, m->bm,   \
+                       (bf16_t *)dx)
+    if (c.K <= 2) DX4(2);
+    else if (c.K <= 4) DX4(4);
+    else DX4(8);
+#undef DX4
+    STEP(hipGetLastError());
     // weight gradients: the experts' rows become the K axis of transposed images
     STEP(launch_transpose_groups(m, m->bw_dy16, m->bw_dys16, c.d, m->bw_dyT, T, s));
     STEP(launch_transpose_groups(m, m->a, nullptr, c.H, m->bw_aT, T, s));
@@ -635,16 +722,6 @@ hipError_t launch_backward_bf16(const omega_moe *m, const void *x, const void *d
     hipLaunchKernelGGL(bw_zero_empty_kernel, dim3(G, 128), dim3(256), 0, s, m->counts, c.E, T, m->dW13, m->dW2, HD,
                        (const int32_t *)(m->bw_zero_state + (m->bw_zero_phase ? G : 0)), m->bw_zero_state + (m->bw_zero_phase ? 0 : G),
                        m->bw_zero_valid ? 0 : 1);
-    // router and gate
-    hipLaunchKernelGGL(bw_router_kernel, dim3(ceil_div(T, 256)), dim3(256), 0, s, (const float *)m->bw_probs, m->ids, m->w,
-                       (const float *)m->bw_dw, T, c.E, c.K, c.renorm, m->bw_dlogits);
-    STEP(launch_gate_wgrad(m, x, T, s));
-    if (c.has_gate_bias)
-        hipLaunchKernelGGL(bw_gate_bias_kernel, dim3(c.E), dim3(256), 0, s, (const float *)m->bw_dlogits, T, c.E, m->dbg);
-    hipLaunchKernelGGL(bw_dx4_bf16_kernel, dim3(ceil_div(T, DX_TT), ceil_div(c.d, 1024)), dim3(256),
-                       (c.E * DX_TT + DX_TT * c.K) * sizeof(float), s, (const float *)m->bw_dxg, m->dstp,
-                       (const float *)m->bw_dlogits, (const bf16_t *)m->Wg, m->tile_meta, T, c.K, c.d, c.E, c.Es, m->bm,
-                       (bf16_t *)dx);
 #undef STEP
     return hipGetLastError();
 }

@@ -123,7 +123,7 @@ struct omega_moe {
     float *bw_probs = nullptr;       // [T,E] softmax of the gate logits
     float *bw_dw = nullptr;          // [T,K] gradient of the combine weights
     float *bw_dlogits = nullptr;     // [T,E]
-    float *bw_gpart = nullptr;       // [32][E,d] partial sums of the gate weight gradient over token slices
+    float *bw_gpart = nullptr;       // [bw_gate_slices][E,d] partial sums of the gate weight gradient over token slices
     float *bw_dy = nullptr;          // [rows_cap,d] gradient of the expert outputs
     float *bw_h1 = nullptr;          // [rows_cap,H] h1, then dh1
     float *bw_h3 = nullptr;          // [rows_cap,H] h3, then dh3
@@ -215,6 +215,11 @@ hipError_t launch_update_bf16(const omega_moe *m, float *master, float lr, int i
 hipError_t launch_zero_f32(float *dst, size_t n, hipStream_t s);
 hipError_t launch_axpy_f32(float *dst, const float *src, float scale, size_t n, hipStream_t s);
 #define OMEGA_SUMSQ_SLOTS 2049  // doubles of scratch launch_sumsq_f32 needs; the result is the last one
+// out[i] = sum over q < nsl of part[q*n + i], in a fixed order
+hipError_t launch_part_sums(const float *part, int nsl, size_t n, float *out, hipStream_t s);
+// Partial sums of the gate and norm weight gradients (bw_gpart): slices of [E,d], or of [d], which fit the same room
+static inline int bw_gate_slices(const omega_moe *m) { return m->cfg.E <= 32 ? 128 : 64; }
+static inline int bw_norm_slices(const omega_moe *m) { return m->cfg.E > 1 ? 256 : 128; }
 hipError_t launch_sumsq_f32(const float *src, size_t n, double *part, hipStream_t s);
 hipError_t launch_scale_f32(float *dst, float coef, size_t n, hipStream_t s);
 struct omega_adamw {
