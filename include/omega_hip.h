@@ -165,9 +165,9 @@ int omega_moe_backward(omega_moe *moe, const void *x_dev, const void *dout_dev, 
 int omega_moe_backward_block(omega_moe *moe, const void *x_dev, const void *dout_dev, int T, void *dx_dev);
 /* Training mode (off at creation).  The reference's layers keep their outputs for back() (LlamaMLPLayer.diff reads
  * active.getOutput() and getLinear3().getOutput(), J/engine/nn/layer/llama/LlamaMLPLayer.java:148-152); with training
- * on, omega_moe_forward of a bf16 layer likewise stores h1 and h3 (fp32, from the accumulators of its up product) and
+ * on, omega_moe_forward likewise stores h1 and h3 (fp32, from the accumulators of its up product) and
  * omega_moe_backward reads them instead of recomputing them.  Same results either way; the forward pass writes
- * 8*H bytes more per expert row.  fp32 layers ignore the switch. */
+ * 8*H bytes more per expert row and allocates what the backward pass works on. */
 int omega_moe_set_training(omega_moe *moe, int on);
 /* How the rows of x reach the experts of a bf16 layer.  The reference has no dispatch (its row gathers, e.g.
  * img_token_drop, J/engine/nn/layer/dit/kernel/TokenDropKernel.cu:147-160, always write the gathered copy).

@@ -588,8 +588,8 @@ static void stage_invalidates(omega_moe *m)
 
 static int stage_router(omega_moe *m, const void *x, int T)
 {
-    // training mode (bf16 layers, backward workspace in place): the probabilities are kept for the backward pass
-    float *probs = (m->training && m->cfg.dtype == OMEGA_DTYPE_BF16 && m->bw_T_cap >= T) ? m->bw_probs : nullptr;
+    // training mode (backward workspace in place): the probabilities are kept for the backward pass
+    float *probs = m->training && m->bw_T_cap >= T ? m->bw_probs : nullptr;
     m->routed_T = m->dispatched_T = -1;
     OMEGA_HIP_CHECK(m->ctx, launch_router(m, x, T, nullptr, probs, m->ctx->stream));
     m->routed_T = T;
@@ -689,11 +689,19 @@ static int forward_impl(omega_moe *m, const void *x, int T, void *out, int block
     const void *xin = block ? m->hbuf : x;
     m->fwd_T = T;
     m->fwd_block = block != 0;
-    // training mode (bf16 layers): the up product also leaves h1 / h3 for the backward pass
-    const bool keep = m->training && m->cfg.dtype == OMEGA_DTYPE_BF16;
+    // training mode: the up product also leaves h1 / h3 for the backward pass
+    bool keep = m->training;
     if (keep) {
         m->bm = moe_tile_m(m, T);
-        RUN(moe_reserve_backward(m, T));
+        const int st = moe_reserve_backward(m, T);
+        // an fp32 layer's forward pass does without its backward workspace if there is no room for it (the backward pass
+        // then asks again, and recomputes); what was allocated before the failure is given back
+        keep = st == OMEGA_OK;
+        if (!keep) {
+            if (st != OMEGA_ERR_OOM || m->cfg.dtype == OMEGA_DTYPE_BF16) return st;
+            (void)hipGetLastError();
+            moe_free_backward_workspace(m);
+        }
     }
     m->rec_valid = false;
     if (m->profiling) {
@@ -775,6 +783,7 @@ static int backward_impl(omega_moe *m, const void *x, const void *dout, int T, v
                                                      : "backward: no omega_moe_forward has run for this T");
     if (!dout || !dx) OMEGA_FAIL(ctx, OMEGA_ERR_INVALID_ARG, "backward: dout or dx is NULL");
     RUN(moe_reserve_backward(m, T));
+    m->bw_started = true;
     const bool bf = m->cfg.dtype == OMEGA_DTYPE_BF16;
     // block form: the layer ran on the normalised rows it still holds; its input gradient then passes the norm backwards
     // and meets the gradient of the residual branch
@@ -810,6 +819,7 @@ int omega_moe_time_backward(omega_moe *m, const void *x, const void *dout, int T
     if (T <= 0 || T != m->fwd_T || m->fwd_block) OMEGA_FAIL(ctx, OMEGA_ERR_INVALID_ARG, "time_backward: no omega_moe_forward has run for this T");
     if (!dout || !dx || !ms_avg || iters <= 0 || warmup < 0) OMEGA_FAIL(ctx, OMEGA_ERR_INVALID_ARG, "time_backward: bad argument");
     RUN(moe_reserve_backward(m, T));
+    m->bw_started = true;
     const bool bf = m->cfg.dtype == OMEGA_DTYPE_BF16;
     if (bf) RUN(ensure_gathered(m, x, T));
     for (int i = 0; i < warmup + iters; ++i) {
@@ -846,10 +856,13 @@ static int grad_slot(omega_moe *m, int which, int expert, float **ptr, size_t *f
     }
 }
 
+// (a training forward of a bf16 layer leaves zeros to read before any backward pass, one of an fp32 layer does not)
+static bool has_grads(const omega_moe *m) { return m->dWg && (m->bw_started || m->cfg.dtype == OMEGA_DTYPE_BF16); }
+
 int omega_moe_get_grad(omega_moe *m, int which, int expert, void *dst, int is_device)
 {
     MOE_ENTER(m);
-    if (!m->dWg) OMEGA_FAIL(ctx, OMEGA_ERR_INVALID_ARG, "get_grad: no backward has run");
+    if (!has_grads(m)) OMEGA_FAIL(ctx, OMEGA_ERR_INVALID_ARG, "get_grad: no backward has run");
     float *p; size_t n;
     if (!dst || grad_slot(m, which, expert, &p, &n) != OMEGA_OK)
         OMEGA_FAIL(ctx, OMEGA_ERR_INVALID_ARG, "get_grad: bad kind, expert index or destination");
@@ -861,7 +874,7 @@ int omega_moe_get_grad(omega_moe *m, int which, int expert, void *dst, int is_de
 int omega_moe_acc_grad(omega_moe *m, float scale)
 {
     MOE_ENTER(m);
-    if (!m->dWg) OMEGA_FAIL(ctx, OMEGA_ERR_INVALID_ARG, "acc_grad: no backward has run");
+    if (!has_grads(m)) OMEGA_FAIL(ctx, OMEGA_ERR_INVALID_ARG, "acc_grad: no backward has run");
     const size_t n = grad_block_floats(m);
     if (!m->acc_grad) OMEGA_HIP_CHECK(ctx, hipMalloc((void **)&m->acc_grad, n * 4));
     if (!m->acc_valid) {
@@ -876,7 +889,7 @@ int omega_moe_acc_grad(omega_moe *m, float scale)
 int omega_moe_grad_sumsq(omega_moe *m, float *sumsq_host)
 {
     MOE_ENTER(m);
-    if (!m->dWg) OMEGA_FAIL(ctx, OMEGA_ERR_INVALID_ARG, "grad_sumsq: no backward has run");
+    if (!has_grads(m)) OMEGA_FAIL(ctx, OMEGA_ERR_INVALID_ARG, "grad_sumsq: no backward has run");
     if (!sumsq_host) OMEGA_FAIL(ctx, OMEGA_ERR_INVALID_ARG, "grad_sumsq: destination is NULL");
     if (!m->sumsq_part) OMEGA_HIP_CHECK(ctx, hipMalloc((void **)&m->sumsq_part, OMEGA_SUMSQ_SLOTS * sizeof(double)));
     // the gradients lie in one block whose padding is zero, so one pass covers every tensor
@@ -891,7 +904,7 @@ int omega_moe_grad_sumsq(omega_moe *m, float *sumsq_host)
 int omega_moe_scale_grad(omega_moe *m, float coef)
 {
     MOE_ENTER(m);
-    if (!m->dWg) OMEGA_FAIL(ctx, OMEGA_ERR_INVALID_ARG, "scale_grad: no backward has run");
+    if (!has_grads(m)) OMEGA_FAIL(ctx, OMEGA_ERR_INVALID_ARG, "scale_grad: no backward has run");
     OMEGA_HIP_CHECK(ctx, launch_scale_f32(m->acc_valid ? m->acc_grad : m->dWg, coef, grad_block_floats(m), ctx->stream));
     return OMEGA_OK;
 }
@@ -899,7 +912,7 @@ int omega_moe_scale_grad(omega_moe *m, float coef)
 int omega_moe_update(omega_moe *m, float lr)
 {
     MOE_ENTER(m);
-    if (!m->dWg) OMEGA_FAIL(ctx, OMEGA_ERR_INVALID_ARG, "update: no backward has run");
+    if (!has_grads(m)) OMEGA_FAIL(ctx, OMEGA_ERR_INVALID_ARG, "update: no backward has run");
     const omega_moe_config &c = m->cfg;
     if (m->acc_valid) {
         OMEGA_HIP_CHECK(ctx, hipMemcpyAsync(m->dWg, m->acc_grad, grad_block_floats(m) * 4, hipMemcpyDeviceToDevice, ctx->stream));
@@ -937,7 +950,7 @@ int omega_moe_update(omega_moe *m, float lr)
 int omega_moe_update_adamw(omega_moe *m, float lr, float beta1, float beta2, float weight_decay, int train_time)
 {
     MOE_ENTER(m);
-    if (!m->dWg) OMEGA_FAIL(ctx, OMEGA_ERR_INVALID_ARG, "update_adamw: no backward has run");
+    if (!has_grads(m)) OMEGA_FAIL(ctx, OMEGA_ERR_INVALID_ARG, "update_adamw: no backward has run");
     if (train_time < 1 || !(beta1 >= 0.0f && beta1 < 1.0f) || !(beta2 >= 0.0f && beta2 < 1.0f))
         OMEGA_FAIL(ctx, OMEGA_ERR_INVALID_ARG, "update_adamw: train_time starts at 1 and the betas lie in [0, 1)");
     const omega_moe_config &c = m->cfg;

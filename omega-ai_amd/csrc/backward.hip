@@ -579,17 +579,25 @@ hipError_t launch_update_bf16(const omega_moe *m, float *master, float lr, int i
     return hipGetLastError();
 }
 
-hipError_t launch_backward_f32(const omega_moe *m, const void *xv, const void *doutv, int T, void *dxv, hipStream_t s)
+hipError_t launch_backward_f32(omega_moe *m, const void *xv, const void *doutv, int T, void *dxv, hipStream_t s)
 {
     const omega_moe_config &c = m->cfg;
     const float *x = (const float *)xv, *dout = (const float *)doutv;
     hipError_t e;
-    // probabilities of the forward pass (the router leaves ids and w as they are: same inputs, same arithmetic)
-    if ((e = launch_router(m, x, T, nullptr, m->bw_probs, s)) != hipSuccess) return e;
+    // A training forward kept the probabilities, h1 and h3; else they are computed once more (the router leaves ids and w as
+    // they are: same inputs, same arithmetic).  The d(a) product puts dh1 and dh3 where h1 and h3 were, so a second
+    // backward pass of the same forward computes them again.  T = 4096, d = 1024, H = 3584, 8 experts, top 2: the product
+    // that makes h1 and h3 takes 1.0 ms of a training step, writing them from the forward's accumulators 0.1.
+    const bool kept = m->rec_valid;
+    m->rec_valid = false;
+    if (!kept) {
+        if ((e = launch_router(m, x, T, nullptr, m->bw_probs, s)) != hipSuccess) return e;
+        if ((e = launch_product_f32(m, F32_RAW, x, dout, T, s)) != hipSuccess) return e;
+    }
     hipLaunchKernelGGL(bw_combine_kernel, dim3(T), dim3(256), 0, s, dout, m->y, m->dstp, m->w, c.K, c.d, m->bw_dy, m->bw_dw);
-    // h1, h3 (recomputed), then d(a) = dy . W2 with the SwiGLU backward in its epilogue: bw_h1 <- dh1, bw_h3 <- dh3
+    // d(a) = dy . W2 with the SwiGLU backward in its epilogue: bw_h1 <- dh1, bw_h3 <- dh3
     // dxg = dh1 . W1 + dh3 . W3;  weight gradients: dW2 = dy^T a [d,H]; dW1 = dh1^T xg, dW3 = dh3^T xg [H,d]
-    for (int op : {F32_RAW, F32_DA, F32_DXG, F32_WG2, F32_WG13})
+    for (int op : {F32_DA, F32_DXG, F32_WG2, F32_WG13})
         if ((e = launch_product_f32(m, op, x, dout, T, s)) != hipSuccess) return e;
     // router and gate
     hipLaunchKernelGGL(bw_router_kernel, dim3(ceil_div(T, 16)), dim3(256), 0, s, (const float *)m->bw_probs, m->ids, m->w,

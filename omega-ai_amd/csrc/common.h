@@ -152,7 +152,8 @@ struct omega_moe {
     bool a_valid = true, y_valid = true;  // false once omega_moe_fill_workspace has overwritten the buffer
     bool fwd_block = false;          // ... and whether it was the block form
     void *bw_dhx = nullptr;          // [T,d] layer dtype: input gradient of the layer inside the block form
-    bool training = false;           // forward keeps h1 / h3 (bf16 layers: as block records in bw_h1 / bw_h3)
+    bool training = false;           // forward keeps h1 / h3 in bw_h1 / bw_h3 (bf16 layers: as block records)
+    bool bw_started = false;         // a backward pass has been asked for: there are gradients to read
     bool rec_valid = false;          // bw_h1 / bw_h3 hold h1 / h3 of the last forward
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     // per-stage event profiling of forward calls (6 events per call), off by default
@@ -200,7 +201,7 @@ hipError_t launch_product_f32(const omega_moe *m, int op, const float *x, const 
 hipError_t launch_experts_bf16(const omega_moe *m, const void *x, int T, int which, hipStream_t s);
 // resid != nullptr: out = resid + layer output (one rounding of the fp32 sum)
 hipError_t launch_combine(const omega_moe *m, int T, void *out, const void *resid, hipStream_t s);
-hipError_t launch_backward_f32(const omega_moe *m, const void *x, const void *dout, int T, void *dx, hipStream_t s);
+hipError_t launch_backward_f32(omega_moe *m, const void *x, const void *dout, int T, void *dx, hipStream_t s);
 hipError_t launch_backward_bf16(const omega_moe *m, const void *x, const void *dout, int T, void *dx, hipStream_t s);
 hipError_t launch_backward_tables(const omega_moe *m, int T, hipStream_t s);
 hipError_t launch_transpose_groups(const omega_moe *m, const void *src, const void *src_alt, int cols, void *dst, int T,

@@ -385,7 +385,7 @@ hipError_t launch_product_f32(const omega_moe *m, int op, const float *x, const 
         case F32_RAW:
             p.A0 = (const float *)m->xg; p.Atok = x; p.B0 = W1; p.B1 = W3; p.N = c.H; p.Kd = c.d;
             p.C = (float *)m->a;
-            if (op == F32_RAW) { p.H1 = m->bw_h1; p.H3 = m->bw_h3; }
+            if (op == F32_RAW || m->training) { p.H1 = m->bw_h1; p.H3 = m->bw_h3; }  // (null: no backward workspace)
             break;
         case F32_DOWN:
             p.A0 = (const float *)m->a; p.B0 = W2; p.C = m->y; p.N = c.d; p.Kd = c.H;

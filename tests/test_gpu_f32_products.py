@@ -1,5 +1,8 @@
 """The fp32 products at both row-tile heights: rows, widths and k that are no multiple of the tiles, forward and backward
 against the oracle (fp32 sums of at most a few thousand terms: relative L2 within 1e-5, as for every fp32 layer)."""
+import importlib
+
+import numpy as np
 import pytest
 
 from oracle import oracle as O
@@ -8,6 +11,7 @@ from tests.synth import C
 from tests.test_gpu_backward import _check_grads, _setup
 
 pytestmark = pytest.mark.gpu
+L = importlib.import_module("omega-ai_amd._lib")
 
 CASES = [
     dict(T=1300, d=1028, H=68, E=3, K=3, Es=1),    # tiles of 128 rows: ragged row tiles, last column tiles, partial k steps
@@ -29,4 +33,36 @@ def test_fp32_products_match_oracle(kw):
     ref = O.moe_backward(inp["x"], dout, inp["Wg"], inp["bg"], inp["W1"], inp["W3"], inp["W2"], cfg.K, cfg.renorm, cfg.Es)
     assert N.rel_l2(dx, ref["dx"]) < 1e-5
     _check_grads(layer, cfg, ref, 1e-5)
+    layer.close()
+
+
+@pytest.mark.parametrize("kw", [CASES[0], CASES[1], CASES[3], dict(T=50, d=48, H=40, E=16, K=2, zipf_bias=1.2)])
+def test_fp32_training_mode_keeps_h1_h3(kw):
+    """The backward pass reads the h1, h3 and probabilities that a training forward left: the same bits as computing them
+    again, once; a second backward pass, whose d(a) product has overwritten them, computes them again."""
+    G, cfg, inp, dout, layer = _setup("c1_tiny_f32", kw, 78)
+    x = G.P.DeviceBuffer.from_numpy(G.ctx(), inp["x"], cfg.dtype)
+    g = G.P.DeviceBuffer.from_numpy(G.ctx(), dout, cfg.dtype)
+
+    def grads():
+        return [layer.back(g).to_numpy(), layer.grad(L.W_GATE)] + [
+            layer.grad(w, e) for e in range(cfg.E + cfg.Es) for w in (L.W_W1, L.W_W3, L.W_W2)]
+
+    def same(a, b):
+        return all(np.array_equal(u, v) for u, v in zip(a, b))
+
+    out = layer.forward(x).to_numpy()
+    want = grads()
+    layer.set_training(True)
+    assert np.array_equal(layer.forward(x).to_numpy(), out)
+    assert same(grads(), want) and same(grads(), want)
+    layer.forward(x)
+    layer.set_training(False)      # what was kept no longer counts
+    assert same(grads(), want)
+    fresh = G.build_layer(cfg, inp)
+    fresh.set_training(True)
+    fresh.forward(x)
+    with pytest.raises(RuntimeError):      # no backward pass yet: no gradients, as without training mode
+        fresh.grad(L.W_GATE)
+    fresh.close()
     layer.close()
