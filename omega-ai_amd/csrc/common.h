@@ -197,7 +197,8 @@ hipError_t launch_dispatch_index(const omega_moe *m, int T, int bm, hipStream_t 
 hipError_t launch_dispatch_gather(const omega_moe *m, const void *x, int T, hipStream_t s);
 // products of fp32 layers (experts_f32.hip describes each); x / dout: token rows the shared experts read
 enum { F32_UP = 0, F32_DOWN, F32_RAW, F32_DA, F32_DXG, F32_WG2, F32_WG13 };
-hipError_t launch_product_f32(const omega_moe *m, int op, const float *x, const float *dout, int T, hipStream_t s);
+// (gather: F32_UP fetches the routed rows from x and leaves the gathered copy beside it)
+hipError_t launch_product_f32(const omega_moe *m, int op, const float *x, const float *dout, int T, hipStream_t s, bool gather = false);
 hipError_t launch_experts_bf16(const omega_moe *m, const void *x, int T, int which, hipStream_t s);
 // resid != nullptr: out = resid + layer output (one rounding of the fp32 sum)
 hipError_t launch_combine(const omega_moe *m, int T, void *out, const void *resid, hipStream_t s);
@@ -231,7 +232,7 @@ hipError_t launch_pack_rows(void *dst_packed, const void *src_rowmajor, int R, i
 hipError_t launch_unpack_rows(void *dst_rowmajor, const void *src_packed, int R, int Kd, hipStream_t s);
 int experts_bf16_tile_m(const omega_moe *m, int T);
 #define F32_TILE_M 128       // row-tile heights of fp32 layers: experts_f32_tile_m chooses one per batch
-#define F32_TILE_M_SMALL 64
+#define F32_TILE_M_SMALL 32
 int experts_f32_tile_m(const omega_moe *m, int T);
 hipError_t experts_bf16_init(void);
 hipError_t launch_down_slab_reduce(const omega_moe *m, float *y, hipStream_t s);  // y += partial results of k-sliced items

@@ -12,8 +12,8 @@
 // Row tiles come from the tile list written by the dispatch stage: a tile never straddles two experts.
 //
 // Bound: fp32 MFMA, 157.3 TFLOP/s (256 FLOP per clock and compute unit; 154 measured with nothing else going on).  One
-// workgroup = four waves = one tile of TM rows x TN MFMA columns, 128 x 128 or 64 x 64 (up: 64 x 128 as the smaller one;
-// half of the columns are W1's, half W3's, so a wave holds h1 and h3 of the same elements).  A wave has TM/2 x TN/2 of it
+// workgroup = four waves = one tile of TM rows x TN MFMA columns, 128 x 128 or, for small batches, 32 x 32 (up: 32 x 64;
+// half of the columns are W1's, half W3's, so a wave holds h1 and h3 of the same elements; weight gradients: 64 x 64).  A wave has TM/2 x TN/2 of it
 // as 32 x 32 blocks; its row blocks alternate with the other row half's, so a ragged tile leaves both the same work.  At
 // 128 x 128 a step of 32 k is 64 MFMAs of 64 cycles per wave against 32 KiB of operands, 8 bytes per clock and compute unit.
 // A wave of such a step left to the compiler's order (barrier, LDS writes, loads, fragment reads, MFMAs) loses 2000 cycles
@@ -24,9 +24,13 @@
 // (MFMA busy 0.89; 134 TFLOP/s at k = 8192).  No vector instruction but the address sums of the loads is spent per step.
 // The down and the input-gradient product, which have the fewest column tiles, take tiles of 128 x 64 (N = 1024, 8192
 // rows: 0.65 -> 0.55 and 1.26 -> 1.10 ms: 544 tiles of 128 x 128 leave the third round of two per compute unit nearly empty).
+// A small batch leaves compute units idle and is as long as the chain of one wave: its tiles are 32 x 32 of four waves with
+// one block of v_mfma_f32_16x16x4 each (the same rate, four k in 32 cycles instead of two in 64) and steps of 64 k, so a wave's
+// chain is a quarter of that of the 64 x 64 tiles they replace.  Forward pass of 8 experts, top 2, us: 256 tokens x 128 x 256
+// 33 -> 26, 1 token x 1024 x 3584 109 -> 56, 256 tokens 206 -> 164; forward + backward of 64 tokens x 256 x 1024 137 -> 101.
 // An operand whose rows are contiguous in k (x, W of y = x W^T) is kept [row][k] in LDS and read 16 bytes (4 k) per lane; one
 // that is contiguous across k (W of delta W, both operands of delta^T input) is kept [k][column] and read one float per
-// lane.  Both hand lane half h the k places 8j+4h .. 8j+4h+3 of every 8, so the two kinds combine freely.
+// lane.  Both hand lane half (quarter) h the k places 4h .. 4h+3 of every 8 (16), so the two kinds combine freely.
 // Any width and alignment: VEC takes 16-byte loads, otherwise elements are loaded one by one.  Addresses past an edge
 // are clamped to the last valid element instead of branched over (a load in a divergent branch waits for those before
 // it); what they bring meets a zero (k past the end) or is never stored.
@@ -35,19 +39,28 @@
 // for the others) and now: up 1.14 -> 0.96 (125 TFLOP/s), down 0.63 -> 0.55 (109), h1 and h3 again 1.91 -> 0.97, d(a) 1.08 -> 0.58,
 // dxg 3.00 -> 1.10, dW2 0.99 -> 0.48, dW1 and dW3 2.01 -> 0.94.
 #include "common.h"
+#include <algorithm>
 #include <type_traits>
 
-#define FBK 32
-
-typedef __attribute__((ext_vector_type(16))) float f32x16_t;
+// matrix-core blocks of BS x BS: v_mfma_f32_32x32x2 (two k at a time, lane half = k) or v_mfma_f32_16x16x4 (four, lane
+// quarter = k)
+template <int BS> struct f32_block;
+template <> struct f32_block<32> {
+    typedef __attribute__((ext_vector_type(16))) float acc_t;
+    static __device__ __forceinline__ acc_t mfma(float a, float b, acc_t c) { return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0); }
+};
+template <> struct f32_block<16> {
+    typedef __attribute__((ext_vector_type(4))) float acc_t;
+    static __device__ __forceinline__ acc_t mfma(float a, float b, acc_t c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+};
 
 // LDS row stride in floats of an operand kept [row][FBK]: 16 consecutive rows start in 16 different groups of four banks
 #define F32_LD_ROW (FBK + 4)
 #define F32_LDS_FLOATS(TX, KMAJ) ((KMAJ) ? FBK * ((TX) + 4) : (TX) * F32_LD_ROW)
 
-// Pieces of one step that a thread carries: NV x 4 floats.  [row][k]: row r0 + (1024/FBK) u, 4 consecutive k; [k][column]: k
-// place k0 + (1024/TX) u, 4 consecutive columns.
-template <int TX, bool KMAJ>
+// Pieces of one step of FBK k places that a thread carries: NV x 4 floats.  [row][k]: row r0 + (1024/FBK) u, 4 consecutive
+// k; [k][column]: k place k0 + (1024/TX) u, 4 consecutive columns.
+template <int TX, bool KMAJ, int FBK>
 struct f32_piece {
     static constexpr int NV = TX * FBK / 1024;
     __device__ static __forceinline__ int x(int tid, int u) { return KMAJ ? 4 * (tid % (TX / 4)) : tid / (FBK / 4) + (1024 / FBK) * u; }
@@ -57,7 +70,7 @@ struct f32_piece {
 
 // Piece u of a whole step: base = the step's first element (uniform), off = the thread's byte offset from it.  Without
 // 16-byte loads the columns of a [k][column] piece are clamped one by one (ncols of them exist).
-template <int TX, bool KMAJ, bool VEC>
+template <bool KMAJ, bool VEC>
 __device__ __forceinline__ float4 fetch_piece(const float *base, uint32_t off, int x, int ncols)
 {
     const float *q = (const float *)((const unsigned char *)base + off);
@@ -67,23 +80,23 @@ __device__ __forceinline__ float4 fetch_piece(const float *base, uint32_t off, i
 }
 
 // The last, partial step of kleft < FBK k places: those behind read as zero, addresses are clamped
-template <int TX, bool KMAJ>
+template <int TX, bool KMAJ, int FBK>
 __device__ __forceinline__ float4 fetch_partial(const float *base, uint32_t off, int tid, int u, int kleft, int ncols, int ld)
 {
     float e[4];
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-        const int k = f32_piece<TX, KMAJ>::k(tid, u) + (KMAJ ? 0 : q), kc = min(k, kleft - 1);
-        const float *p = KMAJ ? base + (size_t)kc * ld + min(f32_piece<TX, KMAJ>::x(tid, u) + q, ncols - 1)
-                              : (const float *)((const unsigned char *)base + off) - f32_piece<TX, KMAJ>::k(tid, u) + kc;
+        const int k = f32_piece<TX, KMAJ, FBK>::k(tid, u) + (KMAJ ? 0 : q), kc = min(k, kleft - 1);
+        const float *p = KMAJ ? base + (size_t)kc * ld + min(f32_piece<TX, KMAJ, FBK>::x(tid, u) + q, ncols - 1)
+                              : (const float *)((const unsigned char *)base + off) - f32_piece<TX, KMAJ, FBK>::k(tid, u) + kc;
         const float w = *p;
         e[q] = k < kleft ? w : 0.0f;
     }
     return make_float4(e[0], e[1], e[2], e[3]);
 }
 
-// four k places of one 32-row (32-column) block for this lane: LDS row / column x, k = 8 j + 4 kh ..
-template <int TX, bool KMAJ>
+// four k places of one block for this lane: LDS row / column x, places k .. k + 3
+template <int TX, bool KMAJ, int FBK>
 __device__ __forceinline__ float4 frag(const float *S, int x, int k)
 {
     if (!KMAJ) return *(const float4 *)&S[x * F32_LD_ROW + k];
@@ -93,6 +106,10 @@ __device__ __forceinline__ float4 frag(const float *S, int x, int k)
 struct f32_args {
     const float *A0, *A1;    // A operand; A1: F32_DXG second pair, F32_WG13 the second gradient's delta
     const float *Atok;       // shared groups: token rows instead of physical rows (or null)
+    const int32_t *tokp;     // F32_UP: routed rows come from Atok through this row -> token table (or null: from A0) ...
+    float *xg;               // ... and the launch's last `copy_wgs` workgroups leave the gathered rows here
+    const int32_t *dstp;     // pair -> row
+    int copy_wgs, K;
     const float *B0, *B1;    // weights (F32_UP, F32_RAW: W1 and W3; F32_DXG: second pair), F32_WG*: the layer input rows
     const float *Btok;       // F32_WG*: as Atok
     float *C, *H1, *H3;      // output; h1 / h3 (F32_UP: kept when not null; F32_RAW: written; F32_DA: read, then dh1 / dh3)
@@ -105,17 +122,50 @@ struct f32_args {
 #define F32_IS_WG(OP) ((OP) == F32_WG2 || (OP) == F32_WG13)
 #define F32_PAIR(OP) ((OP) == F32_UP || (OP) == F32_RAW)
 
+// Gathered rows of a launch whose product workgroups fetch theirs from the tokens (a wave per token, the row read once and
+// written to its K places): the backward pass reads them.  Beside the products instead of a launch in front of them.
+template <bool VEC>
+__device__ __forceinline__ void copy_gathered(const f32_args &p, int wg, int lane, int wave)
+{
+    const int d = p.Kd;
+    for (int t = 4 * wg + wave; t < p.T; t += 4 * p.copy_wgs) {
+        const int row = lane < p.K ? p.dstp[(size_t)t * p.K + lane] : 0;
+        const float *src = p.Atok + (size_t)t * d;
+        for (int c0 = 0; c0 < d; c0 += VEC ? 256 : 64) {  // (every lane makes every trip: the cross-lane reads need them all)
+            const int c = c0 + (VEC ? 4 : 1) * lane;
+            float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            if (c < d) {
+                if (VEC) v = *(const float4 *)(src + c);
+                else v.x = src[c];
+            }
+            for (int j = 0; j < p.K; ++j) {
+                float *o = p.xg + (size_t)__shfl(row, j, 64) * d + c;
+                if (c < d) {
+                    if (VEC) *(float4 *)o = v;
+                    else *o = v.x;
+                }
+            }
+        }
+    }
+}
+
 template <int OP, int TM, int TN, bool VEC>
 __global__ __launch_bounds__(256, 2) void f32_product_kernel(f32_args p)
 {
     constexpr bool WG = F32_IS_WG(OP), PAIR = F32_PAIR(OP);
     constexpr bool AK = WG, BK_ = WG || OP == F32_DA || OP == F32_DXG;  // operand contiguous across k
-    constexpr int MB = TM / 64, NB = TN / 64, NVA = TM * FBK / 1024, NVB = TN * FBK / 1024;
+    constexpr int BS = TM == F32_TILE_M_SMALL ? 16 : 32, GK = 256 / BS, FBK = 4 * GK;  // blocks; k places of a group and of a step
+    constexpr int MB = TM / (2 * BS), NB = TN / (2 * BS), NVA = TM * FBK / 1024, NVB = TN * FBK / 1024, NR = BS * BS / 64;
+    typedef typename f32_block<BS>::acc_t acc_t;
     constexpr int CT = PAIR ? TN / 2 : TN;                             // output columns per tile
     __shared__ __attribute__((aligned(16))) float As[2][F32_LDS_FLOATS(TM, AK)];
     __shared__ __attribute__((aligned(16))) float Bs[2][F32_LDS_FLOATS(TN, BK_)];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int l32 = lane & 31, kh = lane >> 5, wr = wave >> 1, wc = wave & 1;
+    const int lb = lane % BS, kh = lane / BS, wr = wave >> 1, wc = wave & 1;
+    if (OP == F32_UP && (int)blockIdx.x >= (int)gridDim.x - p.copy_wgs) {
+        copy_gathered<VEC>(p, blockIdx.x - (gridDim.x - p.copy_wgs), lane, wave);
+        return;
+    }
 
     // Tile of this workgroup.  Consecutive workgroups go round the eight XCDs: XCD x takes the x-th eighth of the tiles, and
     // within it up to 8 row tiles walk the column tiles together, so that its workgroups share operand rows in its L2.
@@ -132,6 +182,7 @@ __global__ __launch_bounds__(256, 2) void f32_product_kernel(f32_args p)
 
     int g, rows, K1, row0 = 0, m0 = 0;
     const float *A0, *A1 = nullptr, *B0, *B1 = nullptr;
+    bool fetch_rows = false;
     if (WG) {
         g = OP == F32_WG13 ? mat >> 1 : mat;
         const bool shared = g >= p.E;
@@ -149,6 +200,8 @@ __global__ __launch_bounds__(256, 2) void f32_product_kernel(f32_args p)
         row0 = tl.row0;
         K1 = p.Kd;
         A0 = p.Atok && tl.xrow0 >= 0 ? p.Atok + (size_t)tl.xrow0 * p.Kd : p.A0 + (size_t)tl.row0 * p.Kd;
+        fetch_rows = OP == F32_UP && p.tokp != nullptr && tl.xrow0 < 0;
+        if (fetch_rows) A0 = p.Atok;
         if (OP == F32_DXG) A1 = p.A1 + (size_t)tl.row0 * p.Kd;
         B0 = p.B0 + (size_t)g * p.N * p.Kd;
         if (PAIR || OP == F32_DXG) B1 = p.B1 + (size_t)g * p.N * p.Kd;
@@ -159,39 +212,39 @@ __global__ __launch_bounds__(256, 2) void f32_product_kernel(f32_args p)
     uint32_t oa[NVA], ob[NVB];
 #pragma unroll
     for (int u = 0; u < NVA; ++u) {
-        const int x = f32_piece<TM, AK>::x(tid, u), k = f32_piece<TM, AK>::k(tid, u);
-        oa[u] = 4u * (AK ? (uint32_t)k * p.Kd + min(x, p.Kd - m0 - (VEC ? 4 : 1)) : (uint32_t)min(x, rows - 1) * K1 + k);
+        const int x = f32_piece<TM, AK, FBK>::x(tid, u), k = f32_piece<TM, AK, FBK>::k(tid, u);
+        oa[u] = 4u * (AK ? (uint32_t)k * p.Kd + min(x, p.Kd - m0 - (VEC ? 4 : 1)) : (uint32_t)(fetch_rows ? p.tokp[row0 + min(x, rows - 1)] : min(x, rows - 1)) * K1 + k);
     }
 #pragma unroll
     for (int u = 0; u < NVB; ++u) {
-        const int x = f32_piece<TN, BK_>::x(tid, u), k = f32_piece<TN, BK_>::k(tid, u);
+        const int x = f32_piece<TN, BK_, FBK>::x(tid, u), k = f32_piece<TN, BK_, FBK>::k(tid, u);
         ob[u] = 4u * (BK_ ? (uint32_t)k * p.N + min(x, p.N - n0 - (VEC ? 4 : 1)) : (uint32_t)min(PAIR && x >= CT ? x - CT : x, p.N - 1 - n0) * K1 + k);
     }
 
-    f32x16_t acc[MB][NB];
+    acc_t acc[MB][NB];
 #pragma unroll
     for (int i = 0; i < MB; ++i)
 #pragma unroll
         for (int n = 0; n < NB; ++n)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][n][r] = 0.0f;
+            for (int r = 0; r < NR; ++r) acc[i][n][r] = 0.0f;
 
-    // this wave's row blocks: rows 32 (2 i + wr) ..; columns: TN/2 wc + 32 n (up: W1 columns 32 wc, and the same of W3)
-    const int live = max(0, min(MB, ((rows + 31) / 32 + 1 - wr) / 2));
-    const int xa = 32 * wr + l32;
+    // this wave's row blocks: rows BS (2 i + wr) ..; columns: TN/2 wc + BS n (up: W1 columns BS wc, and the same of W3)
+    const int live = max(0, min(MB, ((rows + BS - 1) / BS + 1 - wr) / 2));
+    const int xa = BS * wr + lb;
     int xb[NB];
 #pragma unroll
-    for (int n = 0; n < NB; ++n) xb[n] = (PAIR ? 32 * wc + CT * n : (TN / 2) * wc + 32 * n) + l32;
+    for (int n = 0; n < NB; ++n) xb[n] = (PAIR ? BS * wc + CT * n : (TN / 2) * wc + BS * n) + lb;
 
     const int S1 = K1 / FBK, steps = OP == F32_DXG ? 2 * S1 : S1;  // whole steps
     float4 va[NVA], vb[NVB];
     const float *a_at = AK ? A0 + m0 : A0, *b_at = BK_ ? B0 + n0 : B0 + (size_t)n0 * K1, *b3_at = PAIR ? B1 + (size_t)n0 * K1 : nullptr;
-    auto fetch_a = [&](int u) { va[u] = fetch_piece<TM, AK, VEC>(a_at, oa[u], f32_piece<TM, AK>::x(tid, u), p.Kd - m0); };
+    auto fetch_a = [&](int u) { va[u] = fetch_piece<AK, VEC>(a_at, oa[u], f32_piece<TM, AK, FBK>::x(tid, u), p.Kd - m0); };
     auto fetch_b = [&](int u) {
-        vb[u] = fetch_piece<TN, BK_, VEC>(PAIR && u >= NVB / 2 ? b3_at : b_at, ob[u], f32_piece<TN, BK_>::x(tid, u), p.N - n0);
+        vb[u] = fetch_piece<BK_, VEC>(PAIR && u >= NVB / 2 ? b3_at : b_at, ob[u], f32_piece<TN, BK_, FBK>::x(tid, u), p.N - n0);
     };
-    auto put_a = [&](int c, int u) { *(float4 *)&As[c][f32_piece<TM, AK>::lds(tid, u)] = va[u]; };
-    auto put_b = [&](int c, int u) { *(float4 *)&Bs[c][f32_piece<TN, BK_>::lds(tid, u)] = vb[u]; };
+    auto put_a = [&](int c, int u) { *(float4 *)&As[c][f32_piece<TM, AK, FBK>::lds(tid, u)] = va[u]; };
+    auto put_b = [&](int c, int u) { *(float4 *)&Bs[c][f32_piece<TN, BK_, FBK>::lds(tid, u)] = vb[u]; };
     // the load pointers move on to step s (which the next loads bring); behind the last one they stay
     auto advance = [&](int s) {
         if (s >= steps) return;
@@ -203,7 +256,7 @@ __global__ __launch_bounds__(256, 2) void f32_product_kernel(f32_args p)
             b_at = B1 + n0;
         }
     };
-    // All steps for a wave with MBL live row blocks.  One group = 8 k of the step in buffer c: its MFMAs on the fragments
+    // All steps for a wave with MBL live row blocks.  One group = GK k of the step in buffer c: its MFMAs on the fragments
     // read during the group before, and spread between them (pinned, a quarter of the group at a time) the reads of the
     // next group's fragments and the group's share of the step's other work: group 0 writes the next step's pieces to the
     // other buffer, group 1 asks for those of the step behind it; the barrier lies in front of the last group, whose
@@ -213,9 +266,9 @@ __global__ __launch_bounds__(256, 2) void f32_product_kernel(f32_args p)
         constexpr int MBL = decltype(mbl)::value, NF = MBL > 0 ? MBL + NB : 0;
         float4 fa[2][MBL > 0 ? MBL : 1], fb[2][NB];
         auto read = [&](int set, int c, int j, int r) {
-            const int k = 8 * j + 4 * kh;
-            if (r < MBL) fa[set][r < MBL ? r : 0] = frag<TM, AK>(As[c], xa + 64 * r, k);
-            else if (r < NF) fb[set][r - MBL < NB ? r - MBL : 0] = frag<TN, BK_>(Bs[c], xb[r - MBL < NB ? r - MBL : 0], k);
+            const int k = GK * j + 4 * kh;
+            if (r < MBL) fa[set][r < MBL ? r : 0] = frag<TM, AK, FBK>(As[c], xa + 2 * BS * r, k);
+            else if (r < NF) fb[set][r - MBL < NB ? r - MBL : 0] = frag<TN, BK_, FBK>(Bs[c], xb[r - MBL < NB ? r - MBL : 0], k);
         };
         auto group = [&](auto cc, auto jj) {
             constexpr int c = decltype(cc)::value, j = decltype(jj)::value;
@@ -237,7 +290,7 @@ __global__ __launch_bounds__(256, 2) void f32_product_kernel(f32_args p)
                 for (int i = 0; i < MBL; ++i)
 #pragma unroll
                     for (int n = 0; n < NB; ++n)
-                        acc[i][n] = __builtin_amdgcn_mfma_f32_32x32x2f32(((const float *)&fa[j & 1][i])[q], ((const float *)&fb[j & 1][n])[q], acc[i][n], 0, 0, 0);
+                        acc[i][n] = f32_block<BS>::mfma(((const float *)&fa[j & 1][i])[q], ((const float *)&fb[j & 1][n])[q], acc[i][n]);
                 __builtin_amdgcn_sched_barrier(0);
             }
         };
@@ -277,15 +330,15 @@ __global__ __launch_bounds__(256, 2) void f32_product_kernel(f32_args p)
             const float *b3 = PAIR ? B1 + (size_t)n0 * K1 + S1 * FBK : bt;
             __syncthreads();
 #pragma unroll
-            for (int u = 0; u < NVA; ++u) { va[u] = fetch_partial<TM, AK>(at, oa[u], tid, u, kleft, p.Kd - m0, p.Kd); put_a(0, u); }
+            for (int u = 0; u < NVA; ++u) { va[u] = fetch_partial<TM, AK, FBK>(at, oa[u], tid, u, kleft, p.Kd - m0, p.Kd); put_a(0, u); }
 #pragma unroll
             for (int u = 0; u < NVB; ++u) {
-                vb[u] = fetch_partial<TN, BK_>(PAIR && u >= NVB / 2 ? b3 : bt, ob[u], tid, u, kleft, p.N - n0, p.N);
+                vb[u] = fetch_partial<TN, BK_, FBK>(PAIR && u >= NVB / 2 ? b3 : bt, ob[u], tid, u, kleft, p.N - n0, p.N);
                 put_b(0, u);
             }
             __syncthreads();
 #pragma unroll
-            for (int j = 0; j < FBK / 8; ++j) {
+            for (int j = 0; j < 4; ++j) {
 #pragma unroll
                 for (int r = 0; r < NF; ++r) read(0, 0, j, r);
 #pragma unroll
@@ -294,7 +347,7 @@ __global__ __launch_bounds__(256, 2) void f32_product_kernel(f32_args p)
                     for (int i = 0; i < MBL; ++i)
 #pragma unroll
                         for (int n = 0; n < NB; ++n)
-                            acc[i][n] = __builtin_amdgcn_mfma_f32_32x32x2f32(((const float *)&fa[0][i])[q], ((const float *)&fb[0][n])[q], acc[i][n], 0, 0, 0);
+                            acc[i][n] = f32_block<BS>::mfma(((const float *)&fa[0][i])[q], ((const float *)&fb[0][n])[q], acc[i][n]);
             }
         }
     };
@@ -302,7 +355,7 @@ __global__ __launch_bounds__(256, 2) void f32_product_kernel(f32_args p)
     else if (MB > 1 && live == 1) run(std::integral_constant<int, 1>());
     else run(std::integral_constant<int, 0>());
 
-    // lane: column l32 of a block; register r -> row 8*(r/4) + 4*kh + r%4
+    // lane: column lb of a block; register r -> row 8*(r/4) + 4*kh + r%4
     float *C = p.C;
     if (OP == F32_WG2) C += (size_t)g * p.N * p.Kd;
     if (OP == F32_WG13) C += (size_t)mat * p.N * p.Kd;
@@ -311,20 +364,20 @@ __global__ __launch_bounds__(256, 2) void f32_product_kernel(f32_args p)
         if (i >= live) continue;
 #pragma unroll
         for (int n = 0; n < (PAIR ? 1 : NB); ++n) {
-            const int col = n0 + xb[n], rbase = 32 * (2 * i + wr) + 4 * kh;
+            const int col = n0 + xb[n], rbase = BS * (2 * i + wr) + 4 * kh;
             if (col >= p.N) continue;
             const size_t o = (size_t)(WG ? m0 : row0) * p.N + col;
-            float h1[16], h3[16];
+            float h1[NR], h3[NR];
             if (OP == F32_DA) {  // all of the block's h1 and h3 are asked for before any is used (clamped rows: no branches)
 #pragma unroll
-                for (int r = 0; r < 16; ++r) {
+                for (int r = 0; r < NR; ++r) {
                     const size_t at = o + (size_t)min(rbase + 8 * (r >> 2) + (r & 3), rows - 1) * p.N;
                     h1[r] = p.H1[at];
                     h3[r] = p.H3[at];
                 }
             }
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
+            for (int r = 0; r < NR; ++r) {
                 const int row = rbase + 8 * (r >> 2) + (r & 3);
                 if (row >= rows) continue;
                 const size_t at = o + (size_t)row * p.N;
@@ -351,7 +404,8 @@ __global__ __launch_bounds__(256, 2) void f32_product_kernel(f32_args p)
 int experts_f32_tile_m(const omega_moe *m, int T)
 {
     // Row tiles of 128 once the experts hold about that many rows and the launches have a tile of 128 x 128 for every compute
-    // unit (the down product has the fewest tiles); else of 64.
+    // unit (the down product has the fewest tiles); else of 32.  (Forward pass with 2048 rows of 8 experts, d = 1024, H = 3584:
+    // small tiles 460 us, 64 x 64 ones 469; with 4096 rows the large ones take 887, small ones twice the 460.)
     const omega_moe_config &c = m->cfg;
     const long long rows = (long long)T * c.K;
     return rows >= (long long)F32_TILE_M * c.E && rows / F32_TILE_M * ceil_div(c.d, 128) >= m->ctx->num_cus ? F32_TILE_M : F32_TILE_M_SMALL;
@@ -362,13 +416,13 @@ static hipError_t f32_launch(const f32_args &p, bool vec, int max_tiles, hipStre
 {
     constexpr int CT = F32_PAIR(OP) ? TN / 2 : TN;
     const size_t tiles = (size_t)ceil_div(p.N, CT) * (F32_IS_WG(OP) ? (size_t)ceil_div(p.Kd, TM) * p.G * (OP == F32_WG13 ? 2 : 1) : max_tiles);
-    const unsigned grid = (unsigned)((tiles + 7) / 8 * 8);
+    const unsigned grid = (unsigned)((tiles + 7) / 8 * 8) + p.copy_wgs;
     if (vec) hipLaunchKernelGGL((f32_product_kernel<OP, TM, TN, true>), dim3(grid), dim3(256), 0, s, p);
     else hipLaunchKernelGGL((f32_product_kernel<OP, TM, TN, false>), dim3(grid), dim3(256), 0, s, p);
     return hipGetLastError();
 }
 
-hipError_t launch_product_f32(const omega_moe *m, int op, const float *x, const float *dout, int T, hipStream_t s)
+hipError_t launch_product_f32(const omega_moe *m, int op, const float *x, const float *dout, int T, hipStream_t s, bool gather)
 {
     const omega_moe_config &c = m->cfg;
     f32_args p = {};
@@ -385,6 +439,10 @@ hipError_t launch_product_f32(const omega_moe *m, int op, const float *x, const 
         case F32_RAW:
             p.A0 = (const float *)m->xg; p.Atok = x; p.B0 = W1; p.B1 = W3; p.N = c.H; p.Kd = c.d;
             p.C = (float *)m->a;
+            if (gather) {
+                p.tokp = m->tokp; p.dstp = m->dstp; p.xg = (float *)m->xg; p.K = c.K;
+                p.copy_wgs = std::min(ceil_div(T, 4), m->ctx->num_cus);
+            }
             if (op == F32_RAW || m->training) { p.H1 = m->bw_h1; p.H3 = m->bw_h3; }  // (null: no backward workspace)
             break;
         case F32_DOWN:
@@ -407,14 +465,18 @@ hipError_t launch_product_f32(const omega_moe *m, int op, const float *x, const 
     // 16-byte loads: both widths whole multiples of four floats (every row then starts on 16 bytes) and the caller's
     // buffers aligned (the layer's own are)
     const bool vec = c.d % 4 == 0 && c.H % 4 == 0 && (((uintptr_t)x | (uintptr_t)dout) % 16) == 0;
-    const bool big = m->bm == 128;
+    const bool big = m->bm == F32_TILE_M;
+#define F32_ROWS(OP, TN_BIG, TN_SMALL)                                                         \
+    (big ? f32_launch<OP, F32_TILE_M, TN_BIG>(p, vec, m->max_m_tiles, s)                       \
+         : f32_launch<OP, F32_TILE_M_SMALL, TN_SMALL>(p, vec, m->max_m_tiles, s))
     switch (op) {
-        case F32_UP: return big ? f32_launch<F32_UP, 128, 128>(p, vec, m->max_m_tiles, s) : f32_launch<F32_UP, 64, 128>(p, vec, m->max_m_tiles, s);
-        case F32_RAW: return big ? f32_launch<F32_RAW, 128, 128>(p, vec, m->max_m_tiles, s) : f32_launch<F32_RAW, 64, 128>(p, vec, m->max_m_tiles, s);
-        case F32_DOWN: return big ? f32_launch<F32_DOWN, 128, 64>(p, vec, m->max_m_tiles, s) : f32_launch<F32_DOWN, 64, 64>(p, vec, m->max_m_tiles, s);
-        case F32_DA: return big ? f32_launch<F32_DA, 128, 128>(p, vec, m->max_m_tiles, s) : f32_launch<F32_DA, 64, 64>(p, vec, m->max_m_tiles, s);
-        case F32_DXG: return big ? f32_launch<F32_DXG, 128, 64>(p, vec, m->max_m_tiles, s) : f32_launch<F32_DXG, 64, 64>(p, vec, m->max_m_tiles, s);
+        case F32_UP: return F32_ROWS(F32_UP, 128, 64);
+        case F32_RAW: return F32_ROWS(F32_RAW, 128, 64);
+        case F32_DOWN: return F32_ROWS(F32_DOWN, 64, 32);
+        case F32_DA: return F32_ROWS(F32_DA, 128, 32);
+        case F32_DXG: return F32_ROWS(F32_DXG, 64, 32);
         case F32_WG2: return big ? f32_launch<F32_WG2, 128, 128>(p, vec, 0, s) : f32_launch<F32_WG2, 64, 64>(p, vec, 0, s);
         default: return big ? f32_launch<F32_WG13, 128, 128>(p, vec, 0, s) : f32_launch<F32_WG13, 64, 64>(p, vec, 0, s);
     }
+#undef F32_ROWS
 }

@@ -16,9 +16,13 @@ L = importlib.import_module("omega-ai_amd._lib")
 CASES = [
     dict(T=1300, d=1028, H=68, E=3, K=3, Es=1),    # tiles of 128 rows: ragged row tiles, last column tiles, partial k steps
     dict(T=1301, d=1027, H=67, E=3, K=3),          # the same without 16-byte loads
-    dict(T=300, d=260, H=132, E=2, K=2),           # tiles of 64 rows, whole and partial k steps
+    dict(T=300, d=260, H=132, E=2, K=2),           # tiles of 32 rows, whole and partial k steps
+    dict(T=77, d=68, H=60, E=5, K=3, Es=1),        # ragged tiles of 32 rows, one k step and a part, less than one
+    dict(T=77, d=67, H=65, E=5, K=3, Es=1),        # the same without 16-byte loads
+    dict(T=1, d=128, H=256, E=8, K=2),             # a row per expert
     dict(T=33, d=31, H=5, E=2, K=1),               # less than one k step
-    dict(T=64, d=32, H=64, E=1, K=1),              # exactly one tile, one k step
+    dict(T=64, d=32, H=64, E=1, K=1),              # whole row tiles, half a k step and one
+    dict(T=32, d=32, H=64, E=1, K=1),              # exactly one row tile, one k step of the down product
 ]
 
 
@@ -36,7 +40,7 @@ def test_fp32_products_match_oracle(kw):
     layer.close()
 
 
-@pytest.mark.parametrize("kw", [CASES[0], CASES[1], CASES[3], dict(T=50, d=48, H=40, E=16, K=2, zipf_bias=1.2)])
+@pytest.mark.parametrize("kw", [CASES[0], CASES[1], CASES[6], dict(T=50, d=48, H=40, E=16, K=2, zipf_bias=1.2)])
 def test_fp32_training_mode_keeps_h1_h3(kw):
     """The backward pass reads the h1, h3 and probabilities that a training forward left: the same bits as computing them
     again, once; a second backward pass, whose d(a) product has overwritten them, computes them again."""
@@ -65,4 +69,25 @@ def test_fp32_training_mode_keeps_h1_h3(kw):
     with pytest.raises(RuntimeError):      # no backward pass yet: no gradients, as without training mode
         fresh.grad(L.W_GATE)
     fresh.close()
+    layer.close()
+
+
+@pytest.mark.parametrize("kw", [dict(T=77, d=68, H=60, E=5, K=3, Es=1), dict(T=1301, d=1027, H=67, E=3, K=3)])
+def test_fp32_gather_beside_the_up_product(kw):
+    """A forward pass fetches the rows of the up product from x and leaves the gathered copy beside it; the stages run one by
+    one gather first.  Same bits, and the up product can run again on the copy."""
+    G, cfg, inp, _, layer = _setup("c1_tiny_f32", kw, 79)
+    x = G.P.DeviceBuffer.from_numpy(G.ctx(), inp["x"], cfg.dtype)
+    out = layer.forward(x).to_numpy()
+    xg, a = layer.workspace("xg", cfg.T), layer.workspace("a", cfg.T)
+    assert np.array_equal(xg, inp["x"][layer.routing(cfg.T)["src_row"]])
+    lib, ctx, h = layer.lib, layer.ctx, layer.handle
+    xp = x.ptr if cfg.Es else None          # (shared experts read the token rows)
+    ctx.check(lib.omega_moe_experts_up(h, xp, cfg.T))
+    assert np.array_equal(layer.workspace("a", cfg.T), a)
+    o2 = G.P.DeviceBuffer(ctx, (cfg.T, cfg.d), cfg.dtype)
+    for st in (lib.omega_moe_router(h, x.ptr, cfg.T), lib.omega_moe_dispatch(h, x.ptr, cfg.T), lib.omega_moe_experts_up(h, xp, cfg.T),
+               lib.omega_moe_experts_down(h, cfg.T), lib.omega_moe_combine(h, cfg.T, o2.ptr)):
+        ctx.check(st)
+    assert np.array_equal(o2.to_numpy(), out) and np.array_equal(layer.workspace("xg", cfg.T), xg)
     layer.close()
