@@ -76,7 +76,8 @@ __device__ __forceinline__ float4 fetch_piece(const float *base, uint32_t off, i
     const float *q = (const float *)((const unsigned char *)base + off);
     if (VEC) return *(const float4 *)q;
     if (!KMAJ) return make_float4(q[0], q[1], q[2], q[3]);
-    return make_float4(q[min(0, ncols - 1 - x)], q[min(1, ncols - 1 - x)], q[min(2, ncols - 1 - x)], q[min(3, ncols - 1 - x)]);
+    const int last = max(0, ncols - 1 - x);  // (q is the last column already where x lies past it)
+    return make_float4(q[0], q[min(1, last)], q[min(2, last)], q[min(3, last)]);
 }
 
 // The last, partial step of kleft < FBK k places: those behind read as zero, addresses are clamped

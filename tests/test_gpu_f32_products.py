@@ -21,6 +21,7 @@ CASES = [
     dict(T=77, d=67, H=65, E=5, K=3, Es=1),        # the same without 16-byte loads
     dict(T=1, d=128, H=256, E=8, K=2),             # a row per expert
     dict(T=33, d=31, H=5, E=2, K=1),               # less than one k step
+    dict(T=200, d=33, H=5, E=2, K=2),              # whole k steps of weight gradients far narrower than a tile
     dict(T=64, d=32, H=64, E=1, K=1),              # whole row tiles, half a k step and one
     dict(T=32, d=32, H=64, E=1, K=1),              # exactly one row tile, one k step of the down product
 ]
