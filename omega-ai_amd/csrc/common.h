@@ -231,6 +231,7 @@ hipError_t launch_update_adamw(const omega_moe *m, float *master, float *mw, flo
 hipError_t launch_pack_rows(void *dst_packed, const void *src_rowmajor, int R, int Kd, hipStream_t s);
 hipError_t launch_unpack_rows(void *dst_rowmajor, const void *src_packed, int R, int Kd, hipStream_t s);
 int experts_bf16_tile_m(const omega_moe *m, int T);
+bool wgrad_on_four_waves(const omega_moe *m, int M, int N);  // which kernel takes the weight gradients of M x N per expert
 #define F32_TILE_M 128       // row-tile heights of fp32 layers: experts_f32_tile_m chooses one per batch
 #define F32_TILE_M_SMALL 32
 int experts_f32_tile_m(const omega_moe *m, int T);

@@ -843,9 +843,9 @@ hipError_t launch_unpack_rows(void *dst_rowmajor, const void *src_packed, int R,
 
 // ---- work-item tables of the backward products (bf16 layers) ----
 // k space of the weight gradients: the experts' rows, expert after expert, each expert's share rounded up to 64 rows
-// and to at least 192 (a product item must be longer than the load ring of the product kernel); kt0[g] = first k step
+// and to at least 192 or 256 (an item of the eight-wave kernel has at least 6 k steps, one of the four-wave kernel 8); kt0[g] = first k step
 // (32 rows) of group g, kt0[G] = all of them.  Empty groups take no space and get no items.
-__device__ __forceinline__ int kspace_steps(int rows) { return rows > 0 ? max((rows + 63) / 64 * 2, 6) : 0; }
+__device__ __forceinline__ int kspace_steps(int rows, int least) { return rows > 0 ? max((rows + 63) / 64 * 2, least) : 0; }
 
 // One workgroup per group g: the items of the d(a) product (256-column tiles over H, table as the forward ones), the
 // group's place in k space, and its items of the two weight-gradient products (all 256 x 256 tiles of dW_g;
@@ -854,7 +854,7 @@ __global__ __launch_bounds__(256) void bw_tables_kernel(int32_t *__restrict__ ti
                                                         int E, int Es, int T, int bm, omega_tile_desc *__restrict__ desc_da,
                                                         int nt_da, int32_t *__restrict__ kt0,
                                                         omega_tile_desc *__restrict__ desc_w2, int M2, int NT2,
-                                                        omega_tile_desc *__restrict__ desc_w13, int M13, int NT13)
+                                                        omega_tile_desc *__restrict__ desc_w13, int M13, int NT13, int least_ks)
 {
     __shared__ int red_k[4], red_n[4];
     const int G = E + Es, g = blockIdx.x, tid = threadIdx.x;
@@ -866,7 +866,7 @@ __global__ __launch_bounds__(256) void bw_tables_kernel(int32_t *__restrict__ ti
     int ks = 0, ne = 0;
     for (int q = tid; q < g; q += 256) {
         const int r = q < E ? counts[q] : T;
-        ks += kspace_steps(r);
+        ks += kspace_steps(r, least_ks);
         ne += r > 0 ? 1 : 0;
     }
 #pragma unroll
@@ -878,7 +878,7 @@ __global__ __launch_bounds__(256) void bw_tables_kernel(int32_t *__restrict__ ti
     __syncthreads();
     ks = red_k[0] + red_k[1] + red_k[2] + red_k[3];
     ne = red_n[0] + red_n[1] + red_n[2] + red_n[3];
-    const int my_ks = kspace_steps(rows);
+    const int my_ks = kspace_steps(rows, least_ks);
     if (tid == 0) {
         kt0[g] = ks;
         if (g == G - 1) {
@@ -926,7 +926,8 @@ hipError_t launch_backward_tables(const omega_moe *m, int T, hipStream_t s)
     const omega_moe_config &c = m->cfg;
     const int G = c.E + c.Es;
     hipLaunchKernelGGL(bw_tables_kernel, dim3(G), dim3(256), 0, s, m->tile_meta, m->counts, c.E, c.Es, T, m->bm, m->desc_da,
-                       ceil_div(c.H, 256), m->bw_kt0, m->desc_w2, c.d, ceil_div(c.H, 256), m->desc_w13, 2 * c.H, c.d / 256);
+                       ceil_div(c.H, 256), m->bw_kt0, m->desc_w2, c.d, ceil_div(c.H, 256), m->desc_w13, 2 * c.H, c.d / 256,
+                       wgrad_on_four_waves(m, c.d, c.H) || wgrad_on_four_waves(m, 2 * c.H, c.d) ? 8 : 6);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     sched_args sa = {{m->desc_da, m->desc_w2, m->desc_w13}, {m->wq_da, m->wq_w2, m->wq_w13}, {G + 4, G + 5, G + 6}, {0, 1, 1},

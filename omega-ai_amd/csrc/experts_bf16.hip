@@ -652,7 +652,8 @@ struct Up4Tok {
 
 // DOWN: the plain product y = a . W2^T: 256 columns of W2 (W1 = W2, W3 unused), A = the packed a; an item may be a k
 // slice of a tile (a_rg slices, slice kt0, partial result xrow0: see make_ctx) - slices start on even k steps here
-template <bool GATHER, bool DOWN = false>
+// WG (with DOWN): dW = A^T . B over the rows of one expert, both operands transposed packed images (MODE_WGRAD)
+template <bool GATHER, bool DOWN = false, bool WG = false>
 __device__ __forceinline__ Up4Item up4_item(const omega_tile_desc &d, const bf16_t *Axg, const bf16_t *Ax, const bf16_t *W1,
                                             const bf16_t *W3, int N, int Kd, int wave, int lane, const Up4Tok &tk, bool slices = false)
 {
@@ -664,6 +665,19 @@ __device__ __forceinline__ Up4Item up4_item(const omega_tile_desc &d, const bf16
     c.n0 = d.n0;
     c.kt = KT;
     c.slab = 0;
+    if (WG) {
+        const size_t k0 = (size_t)d.kt0 * 8192;
+        c.kt = d.xrow0;
+        c.A = uniform_ptr((const unsigned char *)Axg + (size_t)d.a_rg * rg_bytes + k0);
+        c.B0 = uniform_ptr((const unsigned char *)W1 + (size_t)d.b_rg * rg_bytes + k0);
+        c.B1 = uniform_ptr(c.B0 + rg_bytes);
+#pragma unroll
+        for (int n = 0; n < 4; ++n) {
+            const int q = wave + 4 * n;
+            c.va[n] = (uint32_t)(q >> 3) * (uint32_t)rg_bytes + (uint32_t)(q & 7) * 1024u + (uint32_t)lane * 16u;
+        }
+        return c;
+    }
     const size_t wrg = (size_t)d.g * (N >> 7) + (d.n0 >> 7);
     if (DOWN) {
         size_t k0 = 0;
@@ -733,11 +747,12 @@ struct Up4State {
     bf16x8_t fa0[8], fb0[8], fa1[8], fb1[8];
     const unsigned char *lA, *lB0, *lB1;
     uint32_t va[4];
+    bool stored;  // (weight gradients) the last 64 instructions that vmcnt counts are stores
 };
 
 // One work item for a wave with NU units of valid rows (units beyond them issue no MFMAs; the accumulators live for
 // one item, so every NU is its own straight-line code with NU * 32 accumulator registers).
-template <int NU, bool WNT, bool GATHER, bool DOWN>
+template <int NU, bool WNT, bool GATHER, bool DOWN, bool WG>
 __device__ __forceinline__ void up4_run_item(unsigned char *smem, Up4State &st, const Up4Item &it, Up4Item &nxt_it,
                                              const omega_tile_desc &dn, const bf16_t *Axg, const bf16_t *Ax, const bf16_t *W1,
                                              const bf16_t *W3, void *Cout, void *slabs, int N, int Kd, int wave, int lane,
@@ -777,7 +792,7 @@ __device__ __forceinline__ void up4_run_item(unsigned char *smem, Up4State &st, 
             asm volatile("global_load_dword %0, %1, %2" : "=&v"(ntk.t[n]) : "v"(o), "s"(tokp) : "memory");
         }
     }
-    if (!GATHER && has_next) nxt_it = up4_item<false, DOWN>(dn, Axg, Ax, W1, W3, N, Kd, wave, lane, Up4Tok{}, slabs != nullptr);
+    if (!GATHER && has_next) nxt_it = up4_item<false, DOWN, WG>(dn, Axg, Ax, W1, W3, N, Kd, wave, lane, Up4Tok{}, slabs != nullptr);
 
 // fragment read r (0..7: B fragment r, 8..15: A fragment r - 8) of the stage whose read addresses are ra / rb0 / rb1
 #define U4_READ(FA, FB, r)                                                                                              \
@@ -801,7 +816,7 @@ __device__ __forceinline__ void up4_run_item(unsigned char *smem, Up4State &st, 
 #define U4_MFMA(PA, PB, Z, iu, c)                                                                                       \
     do {                                                                                                                \
         if ((iu) < NU)                                                                                                  \
-            acc[(iu) % NA][c] = DOWN ? __builtin_amdgcn_mfma_f32_16x16x32_bf16(PA[iu], PB[c], (Z) ? zero4 : acc[(iu) % NA][c], 0, 0, 0) \
+            acc[(iu) % NA][c] = DOWN && !WG ? __builtin_amdgcn_mfma_f32_16x16x32_bf16(PA[iu], PB[c], (Z) ? zero4 : acc[(iu) % NA][c], 0, 0, 0) \
                                      : __builtin_amdgcn_mfma_f32_16x16x32_bf16(PB[c], PA[iu], (Z) ? zero4 : acc[(iu) % NA][c], 0, 0, 0); \
     } while (0)
 // A wave issues one instruction every four cycles and an MFMA of this shape occupies the matrix core for sixteen: up
@@ -852,7 +867,8 @@ __device__ __forceinline__ void up4_run_item(unsigned char *smem, Up4State &st, 
             rb1 = sn + pb[1];                                                                                           \
         }                                                                                                               \
         __builtin_amdgcn_sched_barrier(0);                                                                              \
-        asm volatile("s_waitcnt vmcnt(24) lgkmcnt(0)" ::: "memory");                                                    \
+        if (WG && late) asm volatile("s_waitcnt vmcnt(63) lgkmcnt(0)" ::: "memory");                                    \
+        else asm volatile("s_waitcnt vmcnt(24) lgkmcnt(0)" ::: "memory");                                               \
         __syncthreads();                                                                                                \
     } while (0)
 
@@ -870,9 +886,18 @@ __device__ __forceinline__ void up4_run_item(unsigned char *smem, Up4State &st, 
     // KT steps (even, at least 8), two at a time.  The loads issued during steps 0 .. KT - 6 are the item's own (its steps
     // 5 .. KT - 1), those of the last five steps the next item's first five (behind the last item of a queue this item's
     // once more: nobody reads them).
+    // (WG: the 64 stores of the item before lie between the loads that steps 0 .. 2 wait for and the younger ones: 16 to
+    // 24 loads and the stores may be in flight there, 80 instructions and more, of which the counter can tell 63)
+    bool late = WG && st.stored;
     U4_STEP(st.fa0, st.fb0, st.fa1, st.fb1, true);
     U4_STEP(st.fa1, st.fb1, st.fa0, st.fb0, false);
-    for (int k = 2; k < KT - 6; k += 2) {
+    if (WG && KT > 8) {
+        U4_STEP(st.fa0, st.fb0, st.fa1, st.fb1, false);
+        late = false;
+        U4_STEP(st.fa1, st.fb1, st.fa0, st.fb0, false);
+    }
+    late = false;
+    for (int k = WG ? 4 : 2; k < KT - 6; k += 2) {
         U4_STEP(st.fa0, st.fb0, st.fa1, st.fb1, false);
         U4_STEP(st.fa1, st.fb1, st.fa0, st.fb0, false);
     }
@@ -908,6 +933,17 @@ __device__ __forceinline__ void up4_run_item(unsigned char *smem, Up4State &st, 
         // register r row 4 (l / 16) + r of the unit, so 16 lanes store 64 consecutive bytes of a row
         float *Cbase = (float *)Cout + (size_t)it.row0 * N + it.n0;
         int ld = N;
+        if (WG) {
+            // columns first: lane l holds row l % 16 of the unit, register r column 4 (l / 16) + r of fragment c's 16
+            st.stored = it.n0 + wn * 128 < N;
+            if (!st.stored) return;  // last column tile of a width that is not a multiple of 256
+            float *out = Cbase + (size_t)(16 * wm + l16) * N + wn * 128 + 4 * lq;
+#pragma unroll
+            for (int iu = 0; iu < NU; ++iu)
+#pragma unroll
+                for (int c = 0; c < 8; ++c) *(f32x4_t *)(out + (size_t)(32 * iu) * N + 16 * c) = acc[iu][c];
+            return;
+        }
         if (it.slab > 0) {
             Cbase = (float *)slabs + (size_t)it.slab * (BM * 256);
             ld = 256;
@@ -952,7 +988,7 @@ __device__ __forceinline__ void up4_run_item(unsigned char *smem, Up4State &st, 
 }
 
 // DOWN: the plain down product on the same kernel (W1 = W2, slabs = room for the partial results of k slices or null)
-template <bool WNT, bool GATHER, bool DOWN = false>
+template <bool WNT, bool GATHER, bool DOWN = false, bool WG = false>
 __global__ __launch_bounds__(U4_WAVES * 64) void experts_up4_kernel(const bf16_t *__restrict__ Axg, const bf16_t *__restrict__ Ax,
                                                                     const bf16_t *__restrict__ W1, const bf16_t *__restrict__ W3,
                                                                     void *__restrict__ Cout, const omega_tile_desc *__restrict__ wq,
@@ -972,7 +1008,7 @@ __global__ __launch_bounds__(U4_WAVES * 64) void experts_up4_kernel(const bf16_t
 
     omega_tile_desc d = wq[wg];
     if (d.rows <= 0) return;
-    Up4Item it = up4_item<GATHER, DOWN>(d, Axg, Ax, W1, W3, N, Kd, wave, lane, GATHER ? up4_tokens(d, tokp, wave, lane) : Up4Tok{},
+    Up4Item it = up4_item<GATHER, DOWN, WG>(d, Axg, Ax, W1, W3, N, Kd, wave, lane, GATHER ? up4_tokens(d, tokp, wave, lane) : Up4Tok{},
                                         slabs != nullptr);
     Up4State st;
     st.lA = it.A;
@@ -1017,6 +1053,7 @@ __global__ __launch_bounds__(U4_WAVES * 64) void experts_up4_kernel(const bf16_t
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __syncthreads();
     st.cur = 0;
+    st.stored = false;
 
     for (int q = 1;; ++q) {
         const omega_tile_desc dn = wq[(size_t)q * n_wg + wg];
@@ -1024,8 +1061,9 @@ __global__ __launch_bounds__(U4_WAVES * 64) void experts_up4_kernel(const bf16_t
         const int units = (it.rows + 15) >> 4;
         const int nu = __builtin_amdgcn_readfirstlane(max(0, min(8, (units + 1 - wm) >> 1)));
         Up4Item nxt_it = it;
-#define U4_RUN(NU) up4_run_item<NU, WNT, GATHER, DOWN>(smem, st, it, nxt_it, dn, Axg, Ax, W1, W3, Cout, slabs, N, Kd, wave, lane, tokp)
-        switch (nu) {
+#define U4_RUN(NU) up4_run_item<NU, WNT, GATHER, DOWN, WG>(smem, st, it, nxt_it, dn, Axg, Ax, W1, W3, Cout, slabs, N, Kd, wave, lane, tokp)
+        if (WG) U4_RUN(8);  // (every row of a weight gradient is there)
+        else switch (nu) {
             case 8: U4_RUN(8); break;
             case 7: U4_RUN(7); break;
             case 6: U4_RUN(6); break;
@@ -1104,7 +1142,8 @@ hipError_t experts_bf16_init(void)
                          (const void *)experts_bf16_kernel<MODE_DOWN, true>,
                          (const void *)experts_up4_kernel<false, false>, (const void *)experts_up4_kernel<true, false>,
                          (const void *)experts_up4_kernel<false, true>, (const void *)experts_up4_kernel<true, true>,
-                         (const void *)experts_up4_kernel<false, false, true>, (const void *)experts_up4_kernel<true, false, true>};
+                         (const void *)experts_up4_kernel<false, false, true>, (const void *)experts_up4_kernel<true, false, true>,
+                         (const void *)experts_up4_kernel<false, false, true, true>};
     for (const void *f : fns) {
         hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM_BYTES);
         if (e != hipSuccess) return e;
@@ -1172,6 +1211,17 @@ hipError_t launch_experts_bf16(const omega_moe *m, const void *x, int T, int whi
     return hipGetLastError();
 }
 
+// Weight gradients (dW of M x N per expert) with one wave per SIMD, from 24 tiles per workgroup on: the k steps are cheaper and
+// the first three of an item do not wait for the stores of the one before, but nothing hides the lone waves' start and last
+// tile, and with few tiles two waves per SIMD even out better.  dW1 and dW3 / dW2, us, eight waves -> four (tiles per workgroup):
+// d = 4096, H = 14336, 8 experts, top 2 (56 / 28), 4096 tokens 2027 -> 1903 / 1141 -> 1073, 2048 tokens 1525 -> 1477 / 837 -> 807, 1024
+// tokens 1082 -> 1049 / 625 -> 620; not taken: d = 2048, H = 1408, 64 experts, top 6 (22 / 12), 4096 tokens 464 -> 466 / 226 -> 243;
+// 16 experts, top 4 (5.5 / 3), 3000 tokens 164 -> 177 / 85 -> 88.
+bool wgrad_on_four_waves(const omega_moe *m, int M, int N)
+{
+    return (long long)m->G * (M / 256) * ceil_div(N, 256) >= 24LL * m->n_wg;
+}
+
 // One product of the backward pass on the same kernel; `mode` as the enum above, operands and outputs as its comment says.
 hipError_t launch_product_bf16(const omega_moe *m, int mode, const void *A, const void *Aalt, const void *Wa, const void *Wb,
                                void *Cout, void *Aux1, void *Aux2, const omega_tile_desc *wq, int N, int Kd, hipStream_t s)
@@ -1182,6 +1232,12 @@ hipError_t launch_product_bf16(const omega_moe *m, int mode, const void *A, cons
         hipLaunchKernelGGL((experts_up4_kernel<false, false, true>), dim3(m->n_wg), dim3(U4_WAVES * 64), SMEM_BYTES, s, (const bf16_t *)A,
                            (const bf16_t *)nullptr, (const bf16_t *)Wa, (const bf16_t *)nullptr, Cout, wq, N, Kd, (const int32_t *)nullptr,
                            Aux1);
+        return hipGetLastError();
+    }
+    if (mode == MODE_WGRAD && wgrad_on_four_waves(m, Cout == m->dW2 ? m->cfg.d : 2 * m->cfg.H, N)) {
+        hipLaunchKernelGGL((experts_up4_kernel<false, false, true, true>), dim3(m->n_wg), dim3(U4_WAVES * 64), SMEM_BYTES, s,
+                           (const bf16_t *)A, (const bf16_t *)nullptr, (const bf16_t *)Wa, (const bf16_t *)nullptr, Cout, wq, N, Kd,
+                           (const int32_t *)nullptr, (void *)nullptr);
         return hipGetLastError();
     }
 #define LAUNCH(MODE)                                                                                                   \
