@@ -990,17 +990,21 @@ __global__ __launch_bounds__(256) void transpose_packed_kernel(const unsigned ch
             const int c = c0 + ch * 8;
             v = *(const uint4 *)(sp + pk_chunk_off(r0 + rb + rr, c >> 5, (c & 31) >> 3, KTs));
         }
-        *(uint4 *)&tile[rr][ch * 8] = v;
+        *(uint4 *)&tile[rr][(ch ^ (2 * (rr >> 3) & 6)) * 8] = v;
     }
     __syncthreads();
-    // store: 64 destination rows x 8 chunks of 8 k places
+    // store: 64 destination rows x 8 chunks of 8 k places, a wave one whole 1 KiB block (16 rows x 4 chunks) at a time.  (The
+    // column chunks of the tile are swapped by row group, so that the four chunks of a destination row sit in different banks.
+    // Bound: the bytes.  With 64 rows x 1 chunk per wave, i.e. 16 of every 64 bytes, 8192 rows of 28672 columns took 234 us instead
+    // of 186, of 14336 120 instead of 83, of 4096 41 instead of 32.)
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
-        const int idx = tid + u * 256;
-        const int cc = idx & 63, kc = idx >> 6;  // destination row c0 + cc, k places kc*8 .. kc*8+7 of the 64
+        const int blk = (tid >> 6) + 4 * u, l = tid & 63;
+        const int cc = (blk & 3) * 16 + (l >> 2), kc = (blk >> 2) * 4 + (l & 3);  // destination row c0 + cc, k places kc*8 .. kc*8+7 of the 64
+        const int col = ((cc >> 3) ^ (2 * kc & 6)) * 8 + (cc & 7);
         uint16_t e[8];
 #pragma unroll
-        for (int q = 0; q < 8; ++q) e[q] = tile[kc * 8 + q][cc];
+        for (int q = 0; q < 8; ++q) e[q] = tile[kc * 8 + q][col];
         uint4 v;
         v.x = e[0] | ((uint32_t)e[1] << 16);
         v.y = e[2] | ((uint32_t)e[3] << 16);
