@@ -947,10 +947,8 @@ int omega_moe_update(omega_moe *m, float lr)
     OMEGA_HIP_CHECK(ctx, launch_axpy_f32((float *)m->Wg, m->dWg, -lr, (size_t)c.E * c.d, ctx->stream));
     if (c.has_gate_bias) OMEGA_HIP_CHECK(ctx, launch_axpy_f32(m->bg, m->dbg, -lr, (size_t)c.E, ctx->stream));
     if (m->gamma_set) OMEGA_HIP_CHECK(ctx, launch_axpy_f32(m->gamma, m->dgamma, -lr, (size_t)c.d, ctx->stream));
-    for (int g = 0; g < m->G; ++g) {
-        OMEGA_HIP_CHECK(ctx, launch_axpy_f32((float *)m->W1 + per * g, m->dW13 + per * 2 * g, -lr, per, ctx->stream));
-        OMEGA_HIP_CHECK(ctx, launch_axpy_f32((float *)m->W3 + per * g, m->dW13 + per * (2 * g + 1), -lr, per, ctx->stream));
-    }
+    OMEGA_HIP_CHECK(ctx, launch_axpy_groups_f32((float *)m->W1, per, m->dW13, 2 * per, -lr, per, m->G, ctx->stream));
+    OMEGA_HIP_CHECK(ctx, launch_axpy_groups_f32((float *)m->W3, per, m->dW13 + per, 2 * per, -lr, per, m->G, ctx->stream));
     OMEGA_HIP_CHECK(ctx, launch_axpy_f32((float *)m->W2, m->dW2, -lr, per * m->G, ctx->stream));
     stage_invalidates(m);  // the weights changed: a backward pass needs a new forward
     return OMEGA_OK;

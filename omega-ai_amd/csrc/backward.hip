@@ -384,9 +384,13 @@ __global__ __launch_bounds__(256) void bw_dx_scalar_kernel(const float *__restri
 }
 
 // dst += scale * src (accGrad: axpy_gpu, J/engine/nn/layer/FullyLayer.java:593-607);  w -= lr * g (update without an updater,
-// FullyLayer.java:581-586)
-__global__ __launch_bounds__(256) void bw_axpy_kernel(float *__restrict__ dst, const float *__restrict__ src, float scale, size_t n)
+// FullyLayer.java:581-586).  Group blockIdx.y of n elements at dst + y*dstride, src + y*sstride: the experts of a layer in one
+// launch (a training step of 64 tokens x 256 x 512, 16 experts: 803 -> 740 us; 512 x 512 x 1024, 8 experts: 594 -> 562).
+__global__ __launch_bounds__(256) void bw_axpy_kernel(float *__restrict__ dst, size_t dstride, const float *__restrict__ src,
+                                                      size_t sstride, float scale, size_t n)
 {
+    dst += blockIdx.y * dstride;
+    src += blockIdx.y * sstride;
     // 16-byte accesses when both pointers allow them
     if ((((uintptr_t)dst | (uintptr_t)src) & 15) == 0) {
         const size_t n4 = n >> 2;
@@ -421,12 +425,18 @@ hipError_t launch_zero_f32(float *dst, size_t n, hipStream_t s)
     return hipGetLastError();
 }
 
+hipError_t launch_axpy_groups_f32(float *dst, size_t dstride, const float *src, size_t sstride, float scale, size_t n, int groups,
+                                  hipStream_t s)
+{
+    if (n == 0 || groups == 0) return hipSuccess;
+    const int grid = (int)((n + 255) / 256 < 4096 ? (n + 255) / 256 : 4096);
+    hipLaunchKernelGGL(bw_axpy_kernel, dim3(grid, groups), dim3(256), 0, s, dst, dstride, src, sstride, scale, n);
+    return hipGetLastError();
+}
+
 hipError_t launch_axpy_f32(float *dst, const float *src, float scale, size_t n, hipStream_t s)
 {
-    if (n == 0) return hipSuccess;
-    const int grid = (int)((n + 255) / 256 < 4096 ? (n + 255) / 256 : 4096);
-    hipLaunchKernelGGL(bw_axpy_kernel, dim3(grid), dim3(256), 0, s, dst, src, scale, n);
-    return hipGetLastError();
+    return launch_axpy_groups_f32(dst, 0, src, 0, scale, n, 1, s);
 }
 
 // ---- global gradient norm and clipping (Network.clipGradNorm, J/engine/nn/network/Network.java:379-432) ----

@@ -216,6 +216,8 @@ hipError_t launch_product_bf16(const omega_moe *m, int mode, const void *A, cons
 hipError_t launch_update_bf16(const omega_moe *m, float *master, float lr, int init, hipStream_t s);
 hipError_t launch_zero_f32(float *dst, size_t n, hipStream_t s);
 hipError_t launch_axpy_f32(float *dst, const float *src, float scale, size_t n, hipStream_t s);
+hipError_t launch_axpy_groups_f32(float *dst, size_t dstride, const float *src, size_t sstride, float scale, size_t n, int groups,
+                                  hipStream_t s);
 #define OMEGA_SUMSQ_SLOTS 2049  // doubles of scratch launch_sumsq_f32 needs; the result is the last one
 // out[i] = sum over q < nsl of part[q*n + i], in a fixed order
 hipError_t launch_part_sums(const float *part, int nsl, size_t n, float *out, hipStream_t s);

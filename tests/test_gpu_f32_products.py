@@ -92,3 +92,18 @@ def test_fp32_gather_beside_the_up_product(kw):
         ctx.check(st)
     assert np.array_equal(o2.to_numpy(), out) and np.array_equal(layer.workspace("xg", cfg.T), xg)
     layer.close()
+
+
+@pytest.mark.parametrize("d,H", [(33, 5), (68, 60)])  # groups that start on any float / on 16 bytes
+def test_update_steps_every_expert(d, H):
+    """w - lr * g with one rounding, every tensor of every expert (float64 rounds it twice: within 1e-7)."""
+    G, cfg, inp, dout, layer = _setup("c1_tiny_f32", dict(T=40, d=d, H=H, E=5, K=2, Es=1), 3)
+    layer.forward(G.P.DeviceBuffer.from_numpy(G.ctx(), inp["x"], cfg.dtype))
+    layer.back(G.P.DeviceBuffer.from_numpy(G.ctx(), dout, cfg.dtype))
+    kinds = ((L.W_W1, "W1", (H, d)), (L.W_W3, "W3", (H, d)), (L.W_W2, "W2", (d, H)))
+    grads = {(k, g): layer.grad(w, g).astype(np.float64) for w, k, _ in kinds for g in range(cfg.E + cfg.Es)}
+    layer.update(0.25)
+    for w, k, shape in kinds:
+        for g in range(cfg.E + cfg.Es):
+            assert N.rel_l2(layer._download_weight(w, g, shape), inp[k][g] - 0.25 * grads[k, g]) < 1e-7, (k, g)
+    layer.close()
