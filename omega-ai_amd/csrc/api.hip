@@ -214,7 +214,7 @@ static size_t grad_block_floats(const omega_moe *m)
 }
 
 // Gradient buffers (once) and the workspace of the backward pass for the current forward workspace.
-static int moe_reserve_backward(omega_moe *m, int T)
+static int moe_alloc_backward(omega_moe *m, int T)
 {
     omega_ctx *ctx = m->ctx;
     const omega_moe_config &c = m->cfg;
@@ -294,6 +294,36 @@ static int moe_reserve_backward(omega_moe *m, int T)
     m->bw_T_cap = Tc;
     m->bw_rows_cap = rc;
     return OMEGA_OK;
+}
+
+// The same, whole or not at all: where it fails, what this call allocated is given back (the gradients of an earlier
+// backward pass stay), so that no pointer of the workspace is left without the others, and the runtime's record of the
+// failure is fetched, which the next launch would else report as its own.
+static int moe_reserve_backward(omega_moe *m, int T)
+{
+    const bool had_grads = m->dWg != nullptr, had_wT = m->W2T != nullptr;
+    const int st = moe_alloc_backward(m, T);
+    if (st == OMEGA_OK) return OMEGA_OK;
+    (void)hipGetLastError();
+    moe_free_backward_workspace(m);
+    if (!had_grads) {
+        if (m->dWg) hipFree(m->dWg);
+        if (m->bw_zero_state) hipFree(m->bw_zero_state);
+        m->dWg = m->dbg = m->dgamma = m->dW13 = m->dW2 = nullptr;
+        m->bw_zero_state = nullptr;
+    }
+    if (!had_wT) {
+        if (m->W2T) hipFree(m->W2T);
+        if (m->W13T) hipFree(m->W13T);
+        m->W2T = m->W13T = nullptr;
+    }
+    return st;
+}
+
+// Whether the router and the up product leave the probabilities, h1 and h3 for the backward pass
+static bool keeps_for_backward(const omega_moe *m, int T)
+{
+    return m->training && m->bw_T_cap >= T && m->bw_rows_cap >= m->rows_cap;
 }
 
 static int moe_tile_m(const omega_moe *m, int T)
@@ -589,7 +619,7 @@ static void stage_invalidates(omega_moe *m)
 static int stage_router(omega_moe *m, const void *x, int T)
 {
     // training mode (backward workspace in place): the probabilities are kept for the backward pass
-    float *probs = m->training && m->bw_T_cap >= T ? m->bw_probs : nullptr;
+    float *probs = keeps_for_backward(m, T) ? m->bw_probs : nullptr;
     m->routed_T = m->dispatched_T = -1;
     OMEGA_HIP_CHECK(m->ctx, launch_router(m, x, T, nullptr, probs, m->ctx->stream));
     m->routed_T = T;
@@ -655,11 +685,12 @@ static int stage_experts(omega_moe *m, const void *x, int T, int which)
         OMEGA_FAIL(m->ctx, OMEGA_ERR_INVALID_ARG, "experts: dispatch has not run for this T");
     if (which == 0 && m->gather_on_load && !x) OMEGA_FAIL(m->ctx, OMEGA_ERR_INVALID_ARG, "experts: x is NULL");
     if (which == 1 && !m->a_valid) OMEGA_FAIL(m->ctx, OMEGA_ERR_INVALID_ARG, "experts_down: the up product has not run since `a` was overwritten");
-    if (m->cfg.dtype == OMEGA_DTYPE_BF16) OMEGA_HIP_CHECK(m->ctx, launch_experts_bf16(m, x, T, which, m->ctx->stream));
+    const bool keep = which == 0 && keeps_for_backward(m, T);
+    if (m->cfg.dtype == OMEGA_DTYPE_BF16) OMEGA_HIP_CHECK(m->ctx, launch_experts_bf16(m, x, T, which, m->ctx->stream, keep));
     else if (which == 0) {
         const bool gather = !m->xg_valid;
         if (gather && !x) OMEGA_FAIL(m->ctx, OMEGA_ERR_INVALID_ARG, "experts: x is NULL");
-        OMEGA_HIP_CHECK(m->ctx, launch_product_f32(m, F32_UP, (const float *)x, nullptr, T, m->ctx->stream, gather));
+        OMEGA_HIP_CHECK(m->ctx, launch_product_f32(m, F32_UP, (const float *)x, nullptr, T, m->ctx->stream, gather, keep));
         m->xg_valid = true;
     } else OMEGA_HIP_CHECK(m->ctx, launch_product_f32(m, F32_DOWN, nullptr, nullptr, T, m->ctx->stream));
     if (which == 0) m->a_valid = true;
@@ -704,13 +735,9 @@ static int forward_impl(omega_moe *m, const void *x, int T, void *out, int block
         m->bm = moe_tile_m(m, T);
         const int st = moe_reserve_backward(m, T);
         // an fp32 layer's forward pass does without its backward workspace if there is no room for it (the backward pass
-        // then asks again, and recomputes); what was allocated before the failure is given back
+        // then asks again, and recomputes)
         keep = st == OMEGA_OK;
-        if (!keep) {
-            if (st != OMEGA_ERR_OOM || m->cfg.dtype == OMEGA_DTYPE_BF16) return st;
-            (void)hipGetLastError();
-            moe_free_backward_workspace(m);
-        }
+        if (!keep && (st != OMEGA_ERR_OOM || m->cfg.dtype == OMEGA_DTYPE_BF16)) return st;
     }
     m->rec_valid = false;
     if (m->profiling) {

@@ -197,9 +197,11 @@ hipError_t launch_dispatch_index(const omega_moe *m, int T, int bm, hipStream_t 
 hipError_t launch_dispatch_gather(const omega_moe *m, const void *x, int T, hipStream_t s);
 // products of fp32 layers (experts_f32.hip describes each); x / dout: token rows the shared experts read
 enum { F32_UP = 0, F32_DOWN, F32_RAW, F32_DA, F32_DXG, F32_WG2, F32_WG13 };
-// (gather: F32_UP fetches the routed rows from x and leaves the gathered copy beside it)
-hipError_t launch_product_f32(const omega_moe *m, int op, const float *x, const float *dout, int T, hipStream_t s, bool gather = false);
-hipError_t launch_experts_bf16(const omega_moe *m, const void *x, int T, int which, hipStream_t s);
+// (gather: F32_UP fetches the routed rows from x and leaves the gathered copy beside it; keep: it leaves h1 and h3 in
+// bw_h1 / bw_h3, as launch_experts_bf16 does)
+hipError_t launch_product_f32(const omega_moe *m, int op, const float *x, const float *dout, int T, hipStream_t s, bool gather = false,
+                              bool keep = false);
+hipError_t launch_experts_bf16(const omega_moe *m, const void *x, int T, int which, hipStream_t s, bool keep);
 // resid != nullptr: out = resid + layer output (one rounding of the fp32 sum)
 hipError_t launch_combine(const omega_moe *m, int T, void *out, const void *resid, hipStream_t s);
 hipError_t launch_backward_f32(omega_moe *m, const void *x, const void *dout, int T, void *dx, hipStream_t s);

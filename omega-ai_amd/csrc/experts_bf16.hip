@@ -1151,7 +1151,7 @@ hipError_t experts_bf16_init(void)
     return hipSuccess;
 }
 
-hipError_t launch_experts_bf16(const omega_moe *m, const void *x, int T, int which, hipStream_t s)
+hipError_t launch_experts_bf16(const omega_moe *m, const void *x, int T, int which, hipStream_t s, bool keep)
 {
     const omega_moe_config &c = m->cfg;
     // the ring must be shorter than an item: K >= (NSTAGE + 1) * BK (guaranteed at creation: d, H >= 256)
@@ -1161,7 +1161,7 @@ hipError_t launch_experts_bf16(const omega_moe *m, const void *x, int T, int whi
     // 16 / 64 tokens 9 % faster, 256 tokens equal, 512 tokens 5 % slower; at d = 2048, H = 1408, E = 64, K = 6: 64 and
     // 512 tokens 4-6 % faster, 2048 tokens 2 % slower.
     const bool wnt = (long long)T * c.K <= 64LL * c.E;
-    if (which == 0 && m->training && m->bw_h1 != nullptr) {
+    if (which == 0 && keep) {
         // training mode: h1 and h3 are kept for the backward pass, as the reference's layers keep their outputs
         hipLaunchKernelGGL(experts_bf16_kernel<MODE_UPREC>, dim3(m->n_wg), dim3(NWAVES * 64), SMEM_BYTES, s,
                            (const bf16_t *)m->xg, (const bf16_t *)m->xs, (const bf16_t *)m->W1, (const bf16_t *)m->W3, m->a,

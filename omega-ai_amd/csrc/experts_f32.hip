@@ -423,7 +423,7 @@ static hipError_t f32_launch(const f32_args &p, bool vec, int max_tiles, hipStre
     return hipGetLastError();
 }
 
-hipError_t launch_product_f32(const omega_moe *m, int op, const float *x, const float *dout, int T, hipStream_t s, bool gather)
+hipError_t launch_product_f32(const omega_moe *m, int op, const float *x, const float *dout, int T, hipStream_t s, bool gather, bool keep)
 {
     const omega_moe_config &c = m->cfg;
     f32_args p = {};
@@ -444,7 +444,7 @@ hipError_t launch_product_f32(const omega_moe *m, int op, const float *x, const 
                 p.tokp = m->tokp; p.dstp = m->dstp; p.xg = (float *)m->xg; p.K = c.K;
                 p.copy_wgs = std::min(ceil_div(T, 4), m->ctx->num_cus);
             }
-            if (op == F32_RAW || m->training) { p.H1 = m->bw_h1; p.H3 = m->bw_h3; }  // (null: no backward workspace)
+            if (op == F32_RAW || keep) { p.H1 = m->bw_h1; p.H3 = m->bw_h3; }
             break;
         case F32_DOWN:
             p.A0 = (const float *)m->a; p.B0 = W2; p.C = m->y; p.N = c.d; p.Kd = c.H;

@@ -1,0 +1,110 @@
+"""Host logic of the C ABI without a GPU: api.hip compiled for the host against stand-ins for the HIP runtime and the kernel
+launchers (host_runtime.cpp).  What is allocated, given back, kept and refused; nothing is computed."""
+import ctypes as C
+import os
+import subprocess
+
+import pytest
+
+from tests.conftest import ROOT, load_pkg
+
+L = load_pkg("_lib")
+OOM = 2      # OMEGA_ERR_OOM
+
+
+@pytest.fixture(scope="module")
+def lib(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("host") / "host_logic.so")
+    csrc = os.path.join(ROOT, "omega-ai_amd", "csrc")
+    subprocess.check_call(["g++", "-std=c++17", "-O1", "-g", "-w", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__",
+                           "-D__align__(n)=__attribute__((aligned(n)))", "-DHIP_SYMBOL(x)=((const void *)(x))",
+                           "-I/opt/rocm/include", "-I" + os.path.join(ROOT, "include"), "-I" + csrc, "-o", so,
+                           "-x", "c++", os.path.join(csrc, "api.hip"), os.path.join(ROOT, "tests", "host_runtime.cpp")])
+    lib = C.CDLL(so)
+    for name, (res, args) in L.SIGNATURES.items():
+        if hasattr(lib, name):
+            getattr(lib, name).restype, getattr(lib, name).argtypes = res, args
+    lib.host_live_bytes.restype = C.c_size_t
+    lib.host_take_log.restype = C.c_char_p
+    return lib
+
+
+class Layer:
+    """A layer over the stand-ins; the buffers of its caller are addresses that nothing follows."""
+
+    def __init__(self, lib, dtype="f32", d=256, H=256, E=4, K=2, Es=1, T_max=0):
+        self.lib, self.ctx, self.h = lib, C.c_void_p(), C.c_void_p()
+        assert lib.omega_hip_ctx_create(0, C.byref(self.ctx)) == 0
+        cfg = L.MoEConfigStruct(T_max, d, E, K, H, Es, 1, 1, L.DTYPE_BF16 if dtype == "bf16" else L.DTYPE_F32, L.ROUTER_EXACT)
+        assert lib.omega_moe_create(self.ctx, C.byref(cfg), C.byref(self.h)) == 0
+        self.x, self.g, self.out = 0x1000, 0x2000, 0x3000
+
+    def forward(self, T):
+        return self.lib.omega_moe_forward(self.h, self.x, T, self.out)
+
+    def back(self, T):
+        return self.lib.omega_moe_backward(self.h, self.x, self.g, T, self.out)
+
+    def stages(self, T):
+        """The stages up to the up product, one by one."""
+        return [self.lib.omega_moe_router(self.h, self.x, T), self.lib.omega_moe_dispatch(self.h, self.x, T),
+                self.lib.omega_moe_experts_up(self.h, self.x, T)]
+
+    def grad_status(self):
+        import numpy as np
+        return self.lib.omega_moe_get_grad(self.h, L.W_GATE_BIAS, 0, np.empty(64, np.float32).ctypes.data, 0)
+
+    def log(self):
+        return self.lib.host_take_log().decode().splitlines()
+
+    def close(self):
+        assert self.lib.omega_moe_destroy(self.h) == 0 and self.lib.omega_hip_ctx_destroy(self.ctx) == 0
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_a_backward_workspace_is_there_whole_or_not_at_all(lib, dtype):
+    """Whichever allocation of the backward pass runs out of memory, everything that it took before is given back, nothing that
+    follows works on a part of it, and the next call finds no error left behind."""
+    for n in range(1, 100):
+        m = Layer(lib, dtype)
+        assert m.forward(8) == 0
+        before = lib.host_live_count(), lib.host_live_bytes()
+        lib.host_fail_allocation(n)
+        st = m.back(8)
+        lib.host_fail_allocation(0)
+        if st == 0:
+            break
+        assert st == OOM and (lib.host_live_count(), lib.host_live_bytes()) == before, n
+        assert m.lib.omega_moe_set_training(m.h, 1) == 0
+        m.log()
+        assert m.stages(8) == [0, 0, 0], n          # no error of the failed allocation, and ...
+        assert not any("keep=1" in s or "without" in s for s in m.log()), n    # ... nothing kept where there is no room
+        assert m.forward(8) == 0 and m.back(8) == 0 and "without" not in "".join(m.log()) and m.grad_status() == 0
+        m.close()
+    assert n > 10      # (every allocation had its turn)
+    m.close()
+    assert lib.host_live_count() == 0
+
+
+def test_an_fp32_training_forward_without_room_keeps_nothing(lib):
+    """... and the gradients of an earlier backward pass, which are not part of the workspace."""
+    for n in range(1, 100):
+        m = Layer(lib)
+        assert m.forward(8) == 0
+        before = lib.host_live_count(), lib.host_live_bytes()
+        assert lib.omega_moe_set_training(m.h, 1) == 0
+        lib.host_fail_allocation(n)
+        assert m.forward(8) == 0, n
+        lib.host_fail_allocation(0)
+        if any("keep=1" in s for s in m.log()):
+            break
+        assert (lib.host_live_count(), lib.host_live_bytes()) == before, n
+        assert m.grad_status() != 0          # no backward pass has run
+        assert m.forward(8) == 0 and m.back(8) == 0 and "backward_f32 kept=1" in m.log()
+        lib.host_fail_allocation(20)         # (a forward pass of more tokens: its own workspace, then the backward pass's)
+        assert m.forward(64) == 0 and m.grad_status() == 0
+        lib.host_fail_allocation(0)
+        assert "product_f32 op=0 gather=1 keep=0" in m.log()
+        m.close()
+    assert n > 8
+    m.close()
