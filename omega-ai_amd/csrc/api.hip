@@ -727,8 +727,7 @@ static int forward_impl(omega_moe *m, const void *x, int T, void *out, int block
     // block form: the layer runs on the normalised rows h (one small kernel writes them and rms), the combine adds x back
     const void *resid = block ? x : nullptr;
     const void *xin = block ? m->hbuf : x;
-    m->fwd_T = T;
-    m->fwd_block = block != 0;
+    stage_invalidates(m);  // (until every stage is launched there is no batch that a backward pass may follow)
     // training mode: the up product also leaves h1 / h3 for the backward pass
     bool keep = m->training;
     if (keep) {
@@ -739,7 +738,12 @@ static int forward_impl(omega_moe *m, const void *x, int T, void *out, int block
         keep = st == OMEGA_OK;
         if (!keep && (st != OMEGA_ERR_OOM || m->cfg.dtype == OMEGA_DTYPE_BF16)) return st;
     }
-    m->rec_valid = false;
+    auto done = [&]() {
+        m->fwd_T = T;
+        m->fwd_block = block != 0;
+        m->rec_valid = keep;
+        return OMEGA_OK;
+    };
     if (m->profiling) {
         // six events bracket the five stages; durations are read back by omega_moe_get_profile
         if (m->prof_used + 6 > m->prof_events.size()) {
@@ -763,8 +767,7 @@ static int forward_impl(omega_moe *m, const void *x, int T, void *out, int block
         RUN(stage_combine(m, T, out, resid));
         OMEGA_HIP_CHECK(ctx, hipEventRecord(ev[5], ctx->stream));
         m->prof_used += 6;
-        m->rec_valid = keep;
-        return OMEGA_OK;
+        return done();
     }
     if (block) OMEGA_HIP_CHECK(ctx, launch_rmsnorm(m, x, T, m->hbuf, ctx->stream));
     RUN(stage_router(m, xin, T));
@@ -772,8 +775,7 @@ static int forward_impl(omega_moe *m, const void *x, int T, void *out, int block
     RUN(stage_experts(m, xin, T, 0));
     RUN(stage_experts(m, xin, T, 1));
     RUN(stage_combine(m, T, out, resid));
-    m->rec_valid = keep;
-    return OMEGA_OK;
+    return done();
 }
 
 int omega_moe_set_training(omega_moe *m, int on)

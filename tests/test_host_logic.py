@@ -108,3 +108,16 @@ def test_an_fp32_training_forward_without_room_keeps_nothing(lib):
         m.close()
     assert n > 8
     m.close()
+
+
+def test_a_failed_forward_leaves_no_batch_to_go_back_through(lib):
+    """A training forward that found no room for the backward workspace routed nothing: the index buffers are an earlier
+    batch's, and a backward pass that formed its addresses from them would read past their end.  It is refused."""
+    m = Layer(lib, "bf16", T_max=32)
+    assert m.forward(8) == 0 and lib.omega_moe_set_training(m.h, 1) == 0
+    lib.host_fail_allocation(3)
+    assert m.forward(16) == OOM
+    lib.host_fail_allocation(0)
+    assert m.back(16) == 1 and m.back(8) == 1
+    assert m.forward(16) == 0 and m.back(16) == 0
+    m.close()
