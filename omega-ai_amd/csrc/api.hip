@@ -189,6 +189,7 @@ static void moe_free_backward_workspace(omega_moe *m)
     m->bw_T_cap = 0;
     m->bw_rows_cap = 0;
     m->bw_ksteps_cap = 0;
+    m->bw_ran = false;
 }
 
 static void moe_free_workspace(omega_moe *m)
@@ -821,7 +822,7 @@ static int backward_impl(omega_moe *m, const void *x, const void *dout, int T, v
                                                      : "backward: no omega_moe_forward has run for this T");
     if (!dout || !dx) OMEGA_FAIL(ctx, OMEGA_ERR_INVALID_ARG, "backward: dout or dx is NULL");
     RUN(moe_reserve_backward(m, T));
-    m->bw_started = true;
+    m->bw_started = m->bw_ran = true;
     const bool bf = m->cfg.dtype == OMEGA_DTYPE_BF16;
     // block form: the layer ran on the normalised rows it still holds; its input gradient then passes the norm backwards
     // and meets the gradient of the residual branch
@@ -857,7 +858,7 @@ int omega_moe_time_backward(omega_moe *m, const void *x, const void *dout, int T
     if (T <= 0 || T != m->fwd_T || m->fwd_block) OMEGA_FAIL(ctx, OMEGA_ERR_INVALID_ARG, "time_backward: no omega_moe_forward has run for this T");
     if (!dout || !dx || !ms_avg || iters <= 0 || warmup < 0) OMEGA_FAIL(ctx, OMEGA_ERR_INVALID_ARG, "time_backward: bad argument");
     RUN(moe_reserve_backward(m, T));
-    m->bw_started = true;
+    m->bw_started = m->bw_ran = true;
     const bool bf = m->cfg.dtype == OMEGA_DTYPE_BF16;
     if (bf) RUN(ensure_gathered(m, x, T));
     for (int i = 0; i < warmup + iters; ++i) {
@@ -1186,7 +1187,7 @@ int omega_moe_get_workspace(omega_moe *m, int which, int T, void *host_dst)
     if (!host_dst || which < 0 || which > 4 || T <= 0 || T > m->T_cap || m->bm == 0)
         OMEGA_FAIL(ctx, OMEGA_ERR_INVALID_ARG, "get_workspace: bad selector, T, or no dispatch has run");
     const omega_moe_config &c = m->cfg;
-    if (which >= 3 && (T > m->bw_T_cap || (which == 3 && !m->bw_dh16)))
+    if (which >= 3 && (!m->bw_ran || T > m->bw_T_cap || (which == 3 && !m->bw_dh16)))
         OMEGA_FAIL(ctx, OMEGA_ERR_INVALID_ARG, "get_workspace: no backward has run (selector 3: of a bf16 layer)");
     if (which == 4) {
         OMEGA_HIP_CHECK(ctx, hipMemcpyAsync(host_dst, m->bw_dlogits, (size_t)T * c.E * 4, hipMemcpyDeviceToHost, ctx->stream));

@@ -153,7 +153,8 @@ struct omega_moe {
     bool fwd_block = false;          // ... and whether it was the block form
     void *bw_dhx = nullptr;          // [T,d] layer dtype: input gradient of the layer inside the block form
     bool training = false;           // forward keeps h1 / h3 in bw_h1 / bw_h3 (bf16 layers: as block records)
-    bool bw_started = false;         // a backward pass has been asked for: there are gradients to read
+    bool bw_started = false;         // a backward pass has been asked for: there are gradients to read ...
+    bool bw_ran = false;             // ... and, until the workspace is freed, what the pass left in it
     bool rec_valid = false;          // bw_h1 / bw_h3 hold h1 / h3 of the last forward
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     // per-stage event profiling of forward calls (6 events per call), off by default

@@ -121,3 +121,26 @@ def test_a_failed_forward_leaves_no_batch_to_go_back_through(lib):
     assert m.back(16) == 1 and m.back(8) == 1
     assert m.forward(16) == 0 and m.back(16) == 0
     m.close()
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_backward_rows_can_be_read_behind_a_backward_pass_only(lib, dtype):
+    """dh (bf16 layers) and dlogits of a workspace that a training forward allocated, and of one that has grown since the last
+    backward pass, hold nothing yet."""
+    import numpy as np
+    m = Layer(lib, dtype)
+    host = np.empty(1 << 18, np.float32)
+
+    def read():
+        return {w: lib.omega_moe_get_workspace(m.h, w, 8, host.ctypes.data) for w in ((3, 4) if dtype == "bf16" else (4,))}
+
+    assert lib.omega_moe_set_training(m.h, 1) == 0 and m.forward(8) == 0
+    assert set(read().values()) == {1}
+    assert m.back(8) == 0
+    assert set(read().values()) == {0}
+    assert m.forward(8) == 0 and set(read().values()) == {0}     # the last backward pass's, until the next
+    assert m.forward(64) == 0
+    assert set(read().values()) == {1}
+    ms = C.c_float()
+    assert lib.omega_moe_time_backward(m.h, m.x, m.g, 64, m.out, 0, 1, C.byref(ms)) == 0 and set(read().values()) == {0}
+    m.close()
