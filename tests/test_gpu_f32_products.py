@@ -107,3 +107,24 @@ def test_update_steps_every_expert(d, H):
         for g in range(cfg.E + cfg.Es):
             assert N.rel_l2(layer._download_weight(w, g, shape), inp[k][g] - 0.25 * grads[k, g]) < 1e-7, (k, g)
     layer.close()
+
+
+@pytest.mark.parametrize("training", [False, True])
+def test_one_layer_at_both_tile_heights(training):
+    """Batches with tiles of 128 rows, then 32, then 128 again on one layer's workspace: the bits of a layer that sees the batch
+    alone."""
+    G, cfg, inp, dout, layer = _setup("c1_tiny_f32", CASES[0], 80)
+
+    def step(lay, T):
+        lay.set_training(training)
+        x = G.P.DeviceBuffer.from_numpy(G.ctx(), inp["x"][:T], cfg.dtype)
+        g = G.P.DeviceBuffer.from_numpy(G.ctx(), dout[:T], cfg.dtype)
+        out = lay.forward(x).to_numpy()
+        return [out, lay.back(g).to_numpy(), lay.grad(L.W_GATE)] + [
+            lay.grad(w, e) for e in range(cfg.E + cfg.Es) for w in (L.W_W1, L.W_W3, L.W_W2)]
+
+    for T in (cfg.T, 77, 1, cfg.T):
+        alone = G.build_layer(cfg, inp)
+        assert all(np.array_equal(a, b) for a, b in zip(step(layer, T), step(alone, T))), T
+        alone.close()
+    layer.close()

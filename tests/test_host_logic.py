@@ -144,3 +144,19 @@ def test_backward_rows_can_be_read_behind_a_backward_pass_only(lib, dtype):
     ms = C.c_float()
     assert lib.omega_moe_time_backward(m.h, m.x, m.g, 64, m.out, 0, 1, C.byref(ms)) == 0 and set(read().values()) == {0}
     m.close()
+
+
+@pytest.mark.parametrize("T,tile", [(1, 32), (1023, 32), (1024, 128), (3000, 128)])
+def test_fp32_rows_are_padded_to_the_tile_in_use(lib, T, tile):
+    """xg, a and y hold every expert's rows in whole tiles of the height that a batch of T tokens takes; batches of fewer
+    tokens, which may take the lower one, need no more."""
+    d, H, E, K, Es = 64, 32, 48, 3, 2
+    m = Layer(lib, d=d, H=H, E=E, K=K, Es=Es)
+    before = lib.host_live_bytes()
+    assert m.forward(T) == 0
+    per_row = (2 * d + H) * 4 + 4       # xg, y, a and the row's token
+    rest = T * (5 * K * 4 + d * 4 + 4) + (T // 16 + 17) * E * 4 + (T * K // 32 + E + Es * (T // 32 + 1)) * 16
+    rows = (T * K // tile + E + Es * -(-T // tile)) * tile
+    assert rows * per_row <= lib.host_live_bytes() - before <= rows * per_row + rest
+    assert rows >= max((t * K // h + E + Es * -(-t // h)) * h for t in (T, 1000, 1) if t <= T for h in ([32, 128] if t >= 1024 else [32]))
+    m.close()
