@@ -128,3 +128,32 @@ def test_one_layer_at_both_tile_heights(training):
         assert all(np.array_equal(a, b) for a, b in zip(step(layer, T), step(alone, T))), T
         alone.close()
     layer.close()
+
+
+def _chain(A, B):
+    """A . B as one fp32 chain of fused multiply-adds over k, element by element."""
+    s = np.zeros((A.shape[0], B.shape[1]), np.float32)
+    for k in range(A.shape[1]):
+        s = (A[:, k:k + 1].astype(np.float64) * B[k:k + 1].astype(np.float64) + s).astype(np.float32)
+    return s
+
+
+@pytest.mark.parametrize("T,d,H", [(64, 64, 3584), (64, 63, 3551), (32768, 128, 3584), (32768, 128, 3620)])
+def test_input_gradient_adds_two_sums(T, d, H):
+    """dxg = dh1 . W1 + dh3 . W3 is the sum of two sums of H terms (tiles of 32 rows, of 128; an odd number of k steps; k left
+    over), not a chain of 2 H: against float64 the error is that of two chains on the same operands (1.2: the roundings of
+    dh itself, three sums of d terms, add at most sqrt(1 + 3 d / H) = 1.05, and 4096 elements scatter by a few percent), where
+    one chain has 1.41 times it."""
+    G, cfg, inp, dout, layer = _setup("c1_tiny_f32", dict(T=T, d=d, H=H, E=1, K=1), 81)
+    layer.forward(G.P.DeviceBuffer.from_numpy(G.ctx(), inp["x"], cfg.dtype))
+    dx = layer.back(G.P.DeviceBuffer.from_numpy(G.ctx(), dout, cfg.dtype)).to_numpy()
+    rows = np.linspace(0, T - 1, 64).astype(int)
+    x, g, W1, W3, W2 = (a.astype(np.float64) for a in (inp["x"][rows], dout[rows], inp["W1"][0], inp["W3"][0], inp["W2"][0]))
+    h1, h3, da = x @ W1.T, x @ W3.T, g @ W2        # one expert: combine weight 1, no gradient through the gate
+    s = 1.0 / (1.0 + np.exp(-h1))
+    dh1, dh3 = da * h3 * s * (1.0 + h1 * (1.0 - s)), da * h1 * s
+    exact = dh1 @ W1 + dh3 @ W3
+    two = _chain(dh1.astype(np.float32), inp["W1"][0]) + _chain(dh3.astype(np.float32), inp["W3"][0])
+    err, two_err = N.rel_l2(dx[rows], exact), N.rel_l2(two, exact)
+    assert err < 1.2 * two_err
+    layer.close()
