@@ -198,8 +198,10 @@ static hipError_t launch_gate_wgrad(const omega_moe *m, const void *x, int T, hi
 {
     const omega_moe_config &c = m->cfg;
     const int cb = ceil_div(c.d, 256), eb = ceil_div(c.E, 32);
-    // token slices: about 2048 waves in all, 16 tokens or more each
-    int nsl = std::min({bw_gate_slices(m), std::max(4, 2048 / (cb * eb)), ceil_div(T, 16)});
+    // token slices: about 2048 waves in all, but 32 slices or more, which bounds a chain's rounding error (4096 tokens, 256
+    // experts, relative to float64: 16384 columns in 4 slices 6.1e-7, in 32 2.1e-7; 4096 columns in 16 2.9e-7, in 32 2.1e-7), and
+    // 16 tokens or more each
+    int nsl = std::min({bw_gate_slices(m), std::max(32, 2048 / (cb * eb)), ceil_div(T, 16)});
     const int tslice = ceil_div(ceil_div(T, nsl), 2) * 2;
     nsl = ceil_div(T, tslice);
     const dim3 grid(cb, ceil_div(nsl, 4), eb);
