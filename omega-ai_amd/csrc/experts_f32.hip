@@ -496,9 +496,12 @@ hipError_t launch_product_f32(const omega_moe *m, int op, const float *x, const 
             break;
         default: return hipErrorInvalidValue;
     }
-    // 16-byte loads: both widths whole multiples of four floats (every row then starts on 16 bytes) and the caller's
-    // buffers aligned (the layer's own are)
-    const bool vec = c.d % 4 == 0 && c.H % 4 == 0 && (((uintptr_t)x | (uintptr_t)dout) % 16) == 0;
+    // 16-byte loads, where every row of either operand starts on 16 bytes: the rows of the layer's buffers and weights are d or
+    // H floats long, those of the caller (x or dout, where the product reads it) need their buffer aligned as well.  Up and down
+    // read rows of one width only.   (Forward pass
+    // of 4096 tokens, 8 experts, top 2, us, both widths asked of every product and now: d = 1024, H = 2731 1238 -> 1214; d = 512, H = 1001 305 -> 299.)
+    const bool d4 = c.d % 4 == 0, H4 = c.H % 4 == 0;
+    const bool vec = (op == F32_DOWN || d4) && (op == F32_UP || op == F32_RAW || H4) && (((uintptr_t)p.Atok | (uintptr_t)p.Btok) % 16) == 0;
     const bool big = m->bm == F32_TILE_M;
 #define F32_ROWS(OP, TN_BIG, TN_SMALL)                                                         \
     (big ? f32_launch<OP, F32_TILE_M, TN_BIG>(p, vec, m->max_m_tiles, s)                       \

@@ -1,5 +1,6 @@
 """The fp32 products at both row-tile heights: rows, widths and k that are no multiple of the tiles, forward and backward
 against the oracle (fp32 sums of at most a few thousand terms: relative L2 within 1e-5, as for every fp32 layer)."""
+import ctypes
 import importlib
 
 import numpy as np
@@ -24,6 +25,10 @@ CASES = [
     dict(T=200, d=33, H=5, E=2, K=2),              # whole k steps of weight gradients far narrower than a tile
     dict(T=64, d=32, H=64, E=1, K=1),              # whole row tiles, half a k step and one
     dict(T=32, d=32, H=64, E=1, K=1),              # exactly one row tile, one k step of the down product
+    dict(T=1300, d=1028, H=67, E=3, K=3, Es=1),    # 16-byte loads in the up product alone, tiles of 128 rows
+    dict(T=77, d=68, H=61, E=5, K=3, Es=1),        # and of 32
+    dict(T=1301, d=1025, H=68, E=3, K=3),          # in the down product alone
+    dict(T=77, d=67, H=60, E=5, K=3, Es=1),
 ]
 
 
@@ -156,4 +161,23 @@ def test_input_gradient_adds_two_sums(T, d, H):
     two = _chain(dh1.astype(np.float32), inp["W1"][0]) + _chain(dh3.astype(np.float32), inp["W3"][0])
     err, two_err = N.rel_l2(dx[rows], exact), N.rel_l2(two, exact)
     assert err < 1.2 * two_err
+    layer.close()
+
+
+@pytest.mark.parametrize("kw", [CASES[0], dict(T=77, d=68, H=61, E=5, K=3, Es=1), dict(T=77, d=68, H=60, E=5, K=3)])
+def test_rows_that_start_off_a_16_byte_boundary(kw):
+    """The caller's x and dout one float behind an aligned address: loads element by element, the same bits."""
+    G, cfg, inp, dout, layer = _setup("c1_tiny_f32", kw, 83)
+    ctx, lib, n = layer.ctx, layer.lib, cfg.T * cfg.d
+    got = []
+    for skip in (0, 1):
+        x, g = (G.P.DeviceBuffer.from_numpy(ctx, np.concatenate([np.zeros(skip, np.float32), a.reshape(-1)]), "f32")
+                for a in (inp["x"], dout))
+        out, dx = (G.P.DeviceBuffer(ctx, (cfg.T, cfg.d), "f32") for _ in range(2))
+        xp, gp = (ctypes.c_void_p(b.ptr.value + 4 * skip) for b in (x, g))
+        ctx.check(lib.omega_moe_forward(layer.handle, xp, cfg.T, out.ptr))
+        ctx.check(lib.omega_moe_backward(layer.handle, xp, gp, cfg.T, dx.ptr))
+        got.append([out.to_numpy(), dx.to_numpy(), layer.grad(L.W_GATE)] + [
+            layer.grad(w, e) for e in range(cfg.E + cfg.Es) for w in (L.W_W1, L.W_W3, L.W_W2)])
+    assert all(np.array_equal(a, b) for a, b in zip(*got))
     layer.close()
