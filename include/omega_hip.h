@@ -277,7 +277,8 @@ int omega_moe_time_stage(omega_moe *moe, int stage, const void *x_dev, int T, vo
                          float *ms_avg);
 
 /* Average duration in milliseconds of omega_moe_backward, measured like omega_moe_time_stage; the forward pass for
- * x_dev and T must have run. */
+ * x_dev and T must have run.  After a training forward every repetition is the pass of a training step: what such a pass
+ * uses up is computed again between them, outside the time. */
 int omega_moe_time_backward(omega_moe *moe, const void *x_dev, const void *dout_dev, int T, void *dx_dev, int warmup,
                             int iters, float *ms_avg);
 

@@ -181,3 +181,19 @@ def test_rows_that_start_off_a_16_byte_boundary(kw):
             layer.grad(w, e) for e in range(cfg.E + cfg.Es) for w in (L.W_W1, L.W_W3, L.W_W2)])
     assert all(np.array_equal(a, b) for a, b in zip(*got))
     layer.close()
+
+
+def test_timed_backward_passes_leave_the_gradients_of_one():
+    """What a timed pass of a training step uses up is computed again in front of the next: every pass gives the same bits."""
+    G, cfg, inp, dout, layer = _setup("c1_tiny_f32", CASES[0], 84)
+    x = G.P.DeviceBuffer.from_numpy(G.ctx(), inp["x"], cfg.dtype)
+    g = G.P.DeviceBuffer.from_numpy(G.ctx(), dout, cfg.dtype)
+    dx = G.P.DeviceBuffer(G.ctx(), (cfg.T, cfg.d), cfg.dtype)
+    layer.set_training(True)
+    layer.forward(x)
+    want = [layer.back(g).to_numpy(), layer.grad(L.W_GATE), layer.grad(L.W_W1, 1), layer.grad(L.W_W2, 3)]
+    layer.forward(x)
+    assert layer.time_backward(x, g, cfg.T, dx, warmup=1, iters=2) > 0
+    got = [dx.to_numpy(), layer.grad(L.W_GATE), layer.grad(L.W_W1, 1), layer.grad(L.W_W2, 3)]
+    assert all(np.array_equal(a, b) for a, b in zip(got, want))
+    layer.close()

@@ -160,3 +160,19 @@ def test_fp32_rows_are_padded_to_the_tile_in_use(lib, T, tile):
     assert rows * per_row <= lib.host_live_bytes() - before <= rows * per_row + rest
     assert rows >= max((t * K // h + E + Es * -(-t // h)) * h for t in (T, 1000, 1) if t <= T for h in ([32, 128] if t >= 1024 else [32]))
     m.close()
+
+
+@pytest.mark.parametrize("dtype,training", [("f32", 1), ("f32", 0), ("bf16", 1), ("bf16", 0)])
+def test_time_backward_times_the_pass_of_its_mode(lib, dtype, training):
+    """After a training forward every timed pass finds h1, h3 and the probabilities kept, also in an fp32 layer, whose pass
+    uses them up; computing them again between the passes is not timed (the stand-in's clock counts launches: one a pass)."""
+    m = Layer(lib, dtype)
+    assert lib.omega_moe_set_training(m.h, training) == 0 and m.forward(8) == 0
+    m.log()
+    ms = C.c_float()
+    for warmup, iters in ((2, 3), (0, 1)):
+        assert lib.omega_moe_time_backward(m.h, m.x, m.g, 8, m.out, warmup, iters, C.byref(ms)) == 0
+        passes = [s for s in m.log() if s.startswith("backward_")]
+        assert passes == [f"backward_{dtype} kept={training}"] * (warmup + iters) and ms.value == 1.0
+        assert m.forward(8) == 0 and m.log()
+    m.close()
