@@ -341,7 +341,7 @@ __global__ __launch_bounds__(ROUTER_NTHR(EP)) void router_kernel(const void *__r
     for (int i = 0; i < NT * EPT; ++i) acc[i] = 0.0f;
 
     const bool fast_io = (d % KC == 0) && (((uintptr_t)x | (uintptr_t)Wg) % 16 == 0);
-    if (dtype == OMEGA_DTYPE_BF16) {
+    if (EP <= 16 && dtype == OMEGA_DTYPE_BF16) {  // (bf16 layers with more experts run on the matrix cores)
         if (fast_io) router_sums<EP, KC, EXACT, true, true>(x, Wg, T, d, E, t0, xs, ws, acc);
         else router_sums<EP, KC, EXACT, true, false>(x, Wg, T, d, E, t0, xs, ws, acc);
     } else {
