@@ -215,7 +215,8 @@ hipError_t launch_transpose_images(const void *src, int R, int cols, void *dst, 
 // products of the matrix-core kernel (experts_bf16.hip describes each)
 enum { MODE_UP = 0, MODE_DOWN = 1, MODE_UPRAW = 2, MODE_DA = 3, MODE_WGRAD = 4, MODE_UPREC = 5 };
 hipError_t launch_product_bf16(const omega_moe *m, int mode, const void *A, const void *Aalt, const void *Wa, const void *Wb,
-                               void *Cout, void *Aux1, void *Aux2, const omega_tile_desc *wq, int N, int Kd, hipStream_t s);
+                               void *Cout, void *Aux1, void *Aux2, const omega_tile_desc *wq, int N, int Kd, hipStream_t s,
+                               int M = 0);  // M: rows of one expert's gradient (MODE_WGRAD)
 hipError_t launch_update_bf16(const omega_moe *m, float *master, float lr, int init, hipStream_t s);
 hipError_t launch_zero_f32(float *dst, size_t n, hipStream_t s);
 hipError_t launch_axpy_f32(float *dst, const float *src, float scale, size_t n, hipStream_t s);

@@ -1224,7 +1224,7 @@ bool wgrad_on_four_waves(const omega_moe *m, int M, int N)
 
 // One product of the backward pass on the same kernel; `mode` as the enum above, operands and outputs as its comment says.
 hipError_t launch_product_bf16(const omega_moe *m, int mode, const void *A, const void *Aalt, const void *Wa, const void *Wb,
-                               void *Cout, void *Aux1, void *Aux2, const omega_tile_desc *wq, int N, int Kd, hipStream_t s)
+                               void *Cout, void *Aux1, void *Aux2, const omega_tile_desc *wq, int N, int Kd, hipStream_t s, int M)
 {
     if (Kd < (NSTAGE + 1) * BK) return hipErrorInvalidValue;
     if (mode == MODE_DOWN && m->down_cols == 256 && Kd % 64 == 0 && Kd >= 8 * BK) {
@@ -1234,7 +1234,7 @@ hipError_t launch_product_bf16(const omega_moe *m, int mode, const void *A, cons
                            Aux1);
         return hipGetLastError();
     }
-    if (mode == MODE_WGRAD && wgrad_on_four_waves(m, Cout == m->dW2 ? m->cfg.d : 2 * m->cfg.H, N)) {
+    if (mode == MODE_WGRAD && wgrad_on_four_waves(m, M, N)) {
         hipLaunchKernelGGL((experts_up4_kernel<false, false, true, true>), dim3(m->n_wg), dim3(U4_WAVES * 64), SMEM_BYTES, s,
                            (const bf16_t *)A, (const bf16_t *)nullptr, (const bf16_t *)Wa, (const bf16_t *)nullptr, Cout, wq, N, Kd,
                            (const int32_t *)nullptr, (void *)nullptr);
