@@ -572,15 +572,15 @@ __global__ __launch_bounds__(256) void bw_update_rows_bf16_kernel(float *__restr
     }
 }
 
-// masters laid out like the gradient block: mWg at `master`, mW13 and mW2 at the offsets of dW13 and dW2
+// masters laid out like the gradient block
 hipError_t launch_update_bf16(const omega_moe *m, float *master, float lr, int init, hipStream_t s)
 {
     const omega_moe_config &c = m->cfg;
     const size_t HD = (size_t)c.H * c.d;
-    float *mW13 = master + (m->dW13 - m->dWg), *mW2 = master + (m->dW2 - m->dWg);
+    float *mWg = master + (m->dWg - m->grads), *mW13 = master + (m->dW13 - m->grads), *mW2 = master + (m->dW2 - m->grads);
     const size_t nWg = (size_t)c.E * c.d;
     hipLaunchKernelGGL(bw_update_rows_bf16_kernel, dim3((unsigned)((nWg + 255) / 256 < 1024 ? (nWg + 255) / 256 : 1024)), dim3(256), 0,
-                       s, master, (const float *)m->dWg, (bf16_t *)m->Wg, nWg, lr, init);
+                       s, mWg, (const float *)m->dWg, (bf16_t *)m->Wg, nWg, lr, init);
     const dim3 grid(512, m->G);
     hipLaunchKernelGGL(bw_update_packed_kernel, grid, dim3(256), 0, s, mW13, 2 * HD, (const float *)m->dW13, 2 * HD,
                        (unsigned char *)m->W1, HD * 2, c.H, c.d, lr, init);

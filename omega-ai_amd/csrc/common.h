@@ -110,7 +110,8 @@ struct omega_moe {
     // their weights, the accumulators of accGrad, and the workspace of the pass, indexed by physical rows like xg / a / y
     // (dW13: [G][2][H,d], the gradients of W1 and W3 of an expert back to back)
     float *dWg = nullptr, *dbg = nullptr, *dgamma = nullptr, *dW13 = nullptr, *dW2 = nullptr;
-    float *acc_grad = nullptr;       // accumulators, one block in the order dWg, dbg, dgamma, dW13, dW2
+    float *grads = nullptr;          // the block they are part of, in the order dW13, dW2, dWg, dbg, dgamma
+    float *acc_grad = nullptr;       // accumulators, laid out like the gradient block
     bool acc_valid = false;          // accGrad has run since the last update
     int32_t *bw_zero_state = nullptr;  // [2][G]: which groups' weight-gradient blocks are known to be zero (two copies, used in turn)
     int bw_zero_phase = 0;           // which copy the next backward pass reads

@@ -93,19 +93,19 @@ static inline unsigned grid_for(size_t n, unsigned cap)
     return (unsigned)(b < cap ? (b ? b : 1) : cap);
 }
 
-// mw, vw (and master for bf16 layers) are laid out like the gradient block that starts at m->dWg
+// mw, vw (and master for bf16 layers) are laid out like the gradient block
 hipError_t launch_update_adamw(const omega_moe *m, float *master, float *mw, float *vw, const omega_adamw &p, hipStream_t s)
 {
     const omega_moe_config &c = m->cfg;
     const size_t HD = (size_t)c.H * c.d, nWg = (size_t)c.E * c.d;
-    const size_t o_bg = m->dbg - m->dWg, o_gm = m->dgamma - m->dWg, o13 = m->dW13 - m->dWg, o2 = m->dW2 - m->dWg;
+    const size_t o_g = m->dWg - m->grads, o_bg = m->dbg - m->grads, o_gm = m->dgamma - m->grads, o13 = m->dW13 - m->grads, o2 = m->dW2 - m->grads;
     const bool bf = c.dtype == OMEGA_DTYPE_BF16;
     if (bf)
-        hipLaunchKernelGGL(adamw_rows_bf16_kernel, dim3(grid_for(nWg, 1024)), dim3(256), 0, s, master, (const float *)m->dWg, mw,
-                           vw, (bf16_t *)m->Wg, nWg, p);
+        hipLaunchKernelGGL(adamw_rows_bf16_kernel, dim3(grid_for(nWg, 1024)), dim3(256), 0, s, master + o_g, (const float *)m->dWg,
+                           mw + o_g, vw + o_g, (bf16_t *)m->Wg, nWg, p);
     else
         hipLaunchKernelGGL(adamw_f32_kernel, dim3(grid_for(nWg, 1024)), dim3(256), 0, s, (float *)m->Wg, (size_t)0,
-                           (const float *)m->dWg, mw, vw, (size_t)0, nWg, p);
+                           (const float *)m->dWg, mw + o_g, vw + o_g, (size_t)0, nWg, p);
     if (c.has_gate_bias)
         hipLaunchKernelGGL(adamw_f32_kernel, dim3(grid_for(c.E, 1024)), dim3(256), 0, s, m->bg, (size_t)0, (const float *)m->dbg,
                            mw + o_bg, vw + o_bg, (size_t)0, (size_t)c.E, p);

@@ -48,7 +48,8 @@ hipError_t hipMalloc(void **p, size_t n)
 {
     *p = nullptr;
     if (g_fail_in > 0 && --g_fail_in == 0) return g_last = hipErrorOutOfMemory;
-    *p = calloc(n ? n : 1, 1);
+    *p = aligned_alloc(256, (n + 256) / 256 * 256);  // (as the device's allocations are aligned)
+    memset(*p, 0, n);
     g_live[*p] = n;
     g_bytes += n;
     return hipSuccess;
@@ -128,7 +129,14 @@ hipError_t launch_transpose_images(const void *, int, int, void *dst, int, int, 
     return line(dst ? "transpose" : "transpose into nothing");
 }
 hipError_t launch_update_bf16(const omega_moe *, float *, float, int, hipStream_t) { return line("update"); }
-hipError_t launch_update_adamw(const omega_moe *, float *, float *, float *, const omega_adamw &, hipStream_t) { return line("adamw"); }
+hipError_t launch_update_adamw(const omega_moe *m, float *master, float *mw, float *vw, const omega_adamw &, hipStream_t)
+{
+    const size_t o13 = m->dW13 - m->grads;
+    uintptr_t at = (uintptr_t)m->dW13 | (uintptr_t)(mw + o13) | (uintptr_t)(vw + o13);
+    if (master) at |= (uintptr_t)(master + o13);
+    uintptr_t block = (uintptr_t)m->grads | (uintptr_t)mw | (uintptr_t)vw | (uintptr_t)master;
+    return line("adamw block %d experts %d", (int)(block % 16), (int)(at % 128));
+}
 hipError_t launch_zero_f32(float *, size_t, hipStream_t) { return line("zero"); }
 hipError_t launch_axpy_f32(float *, const float *, float, size_t, hipStream_t) { return line("axpy"); }
 hipError_t launch_axpy_groups_f32(float *, size_t, const float *, size_t, float, size_t, int, hipStream_t) { return line("axpy"); }

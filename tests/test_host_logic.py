@@ -176,3 +176,20 @@ def test_time_backward_times_the_pass_of_its_mode(lib, dtype, training):
         assert passes == [f"backward_{dtype} kept={training}"] * (warmup + iters) and ms.value == 1.0
         assert m.forward(8) == 0 and m.log()
     m.close()
+
+
+@pytest.mark.parametrize("dtype,d,E", [("bf16", 256, 4), ("bf16", 4096, 8), ("bf16", 2048, 16), ("bf16", 768, 7), ("f32", 68, 5),
+                                       ("f32", 33, 3)])
+def test_expert_blocks_of_the_optimiser_start_on_a_cache_line(lib, dtype, d, E):
+    """Gradients, moments and master weights of the experts start on 128 bytes, the blocks they are part of on 16, whatever the
+    widths of the gate; the layer gives all of them back."""
+    m = Layer(lib, dtype, d=d, E=E)
+    assert m.forward(8) == 0 and m.back(8) == 0
+    for step in (1, 2):
+        assert lib.omega_moe_acc_grad(m.h, 1.0) == 0
+        m.log()
+        assert lib.omega_moe_update_adamw(m.h, 1e-3, 0.9, 0.999, 0.0, step) == 0
+        assert m.log()[-1] == "adamw block 0 experts 0"
+        assert m.forward(8) == 0 and m.back(8) == 0
+    m.close()
+    assert lib.host_live_count() == 0
