@@ -736,9 +736,9 @@ hipError_t launch_backward_bf16(const omega_moe *m, const void *x, const void *d
     STEP(launch_transpose_groups(m, m->xg, m->xs, c.d, m->bw_xgT, T, s));
     STEP(launch_transpose_groups(m, m->bw_dh16, nullptr, 2 * c.H, m->bw_dhT, T, s));
     STEP(launch_product_bf16(m, MODE_WGRAD, m->bw_dyT, nullptr, m->bw_aT, nullptr, m->dW2, nullptr, nullptr, m->wq_w2, c.H,
-                             m->bw_ksteps_cap * 32, s, c.d));
+                             m->bw_ksteps_cap * 32, s, wgrad_on_four_waves(m, T, c.d, c.H)));
     STEP(launch_product_bf16(m, MODE_WGRAD, m->bw_dhT, nullptr, m->bw_xgT, nullptr, m->dW13, nullptr, nullptr, m->wq_w13, c.d,
-                             m->bw_ksteps_cap * 32, s, 2 * c.H));
+                             m->bw_ksteps_cap * 32, s, wgrad_on_four_waves(m, T, 2 * c.H, c.d)));
     hipLaunchKernelGGL(bw_zero_empty_kernel, dim3(G, 128), dim3(256), 0, s, m->counts, c.E, T, m->dW13, m->dW2, HD,
                        (const int32_t *)(m->bw_zero_state + (m->bw_zero_phase ? G : 0)), m->bw_zero_state + (m->bw_zero_phase ? 0 : G),
                        m->bw_zero_valid ? 0 : 1);

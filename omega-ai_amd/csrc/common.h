@@ -217,7 +217,7 @@ hipError_t launch_transpose_images(const void *src, int R, int cols, void *dst, 
 enum { MODE_UP = 0, MODE_DOWN = 1, MODE_UPRAW = 2, MODE_DA = 3, MODE_WGRAD = 4, MODE_UPREC = 5 };
 hipError_t launch_product_bf16(const omega_moe *m, int mode, const void *A, const void *Aalt, const void *Wa, const void *Wb,
                                void *Cout, void *Aux1, void *Aux2, const omega_tile_desc *wq, int N, int Kd, hipStream_t s,
-                               int M = 0);  // M: rows of one expert's gradient (MODE_WGRAD)
+                               bool four_waves = false);  // (MODE_WGRAD: wgrad_on_four_waves)
 hipError_t launch_update_bf16(const omega_moe *m, float *master, float lr, int init, hipStream_t s);
 hipError_t launch_zero_f32(float *dst, size_t n, hipStream_t s);
 hipError_t launch_axpy_f32(float *dst, const float *src, float scale, size_t n, hipStream_t s);
@@ -238,7 +238,7 @@ hipError_t launch_update_adamw(const omega_moe *m, float *master, float *mw, flo
 hipError_t launch_pack_rows(void *dst_packed, const void *src_rowmajor, int R, int Kd, hipStream_t s);
 hipError_t launch_unpack_rows(void *dst_rowmajor, const void *src_packed, int R, int Kd, hipStream_t s);
 int experts_bf16_tile_m(const omega_moe *m, int T);
-bool wgrad_on_four_waves(const omega_moe *m, int M, int N);  // which kernel takes the weight gradients of M x N per expert
+bool wgrad_on_four_waves(const omega_moe *m, int T, int M, int N);  // which kernel takes the weight gradients of M x N per expert
 #define F32_TILE_M 128       // row-tile heights of fp32 layers: experts_f32_tile_m chooses one per batch
 #define F32_TILE_M_SMALL 32
 int experts_f32_tile_m(const omega_moe *m, int T);

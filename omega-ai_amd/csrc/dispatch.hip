@@ -927,7 +927,7 @@ hipError_t launch_backward_tables(const omega_moe *m, int T, hipStream_t s)
     const int G = c.E + c.Es;
     hipLaunchKernelGGL(bw_tables_kernel, dim3(G), dim3(256), 0, s, m->tile_meta, m->counts, c.E, c.Es, T, m->bm, m->desc_da,
                        ceil_div(c.H, 256), m->bw_kt0, m->desc_w2, c.d, ceil_div(c.H, 256), m->desc_w13, 2 * c.H, c.d / 256,
-                       wgrad_on_four_waves(m, c.d, c.H) || wgrad_on_four_waves(m, 2 * c.H, c.d) ? 8 : 6);
+                       wgrad_on_four_waves(m, T, c.d, c.H) || wgrad_on_four_waves(m, T, 2 * c.H, c.d) ? 8 : 6);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     sched_args sa = {{m->desc_da, m->desc_w2, m->desc_w13}, {m->wq_da, m->wq_w2, m->wq_w13}, {G + 4, G + 5, G + 6}, {0, 1, 1},

@@ -1211,20 +1211,24 @@ hipError_t launch_experts_bf16(const omega_moe *m, const void *x, int T, int whi
     return hipGetLastError();
 }
 
-// Weight gradients (dW of M x N per expert) with one wave per SIMD, from 24 tiles per workgroup on: the k steps are cheaper and
-// the first three of an item do not wait for the stores of the one before, but nothing hides the lone waves' start and last
-// tile, and with few tiles two waves per SIMD even out better.  dW1 and dW3 / dW2, us, eight waves -> four (tiles per workgroup):
-// d = 4096, H = 14336, 8 experts, top 2 (56 / 28), 4096 tokens 2027 -> 1903 / 1141 -> 1073, 2048 tokens 1525 -> 1477 / 837 -> 807, 1024
-// tokens 1082 -> 1049 / 625 -> 620; not taken: d = 2048, H = 1408, 64 experts, top 6 (22 / 12), 4096 tokens 464 -> 466 / 226 -> 243;
-// 16 experts, top 4 (5.5 / 3), 3000 tokens 164 -> 177 / 85 -> 88.
-bool wgrad_on_four_waves(const omega_moe *m, int M, int N)
+// Weight gradients (dW of M x N per expert) with one wave per SIMD where an expert has 1024 rows or more (32 k steps), 2 tiles or
+// more per workgroup, and all of them 32: the k steps are cheaper and the first three of an item wait for a few of the stores of
+// the item before only, but nothing else hides those stores or the lone waves' start, and an item has at least 8 k steps
+// where the eight waves take 6.  dW1 and dW3, us, eight waves -> four (rows and tiles per expert / 256): d = 4096, H = 14336, 8
+// experts 4096 tokens (1024, 7) 1987 -> 1951, 6000 tokens 2667 -> 2544, 8192 tokens 3463 -> 3402; d = 4096, H = 4096, 16 experts, 16000
+// tokens (2000, 2) 1896 -> 1829; d = 2048, H = 8192, the same 1852 -> 1800.  Not taken: d = 4096, H = 14336, 1024 tokens (256, 7) 967 ->
+// 1028, 3000 tokens (750, 7) 1580 -> 1590; d = 4096, H = 2048, 64 experts, top 6, 16000 tokens (1500, 1) 3185 -> 3263; 256 experts, top 4, d
+// = 2048, H = 768, 30000 tokens (468, 0.2) 1034 -> 1155; dW2 of d = 4096, H = 14336 (28 tiles per workgroup in all), 4096 tokens 1080 ->
+// 1086, 8192 tokens 1711 -> 1770.  A training step of 64 tokens x 4096 x 14336 took 2586 us on eight waves, 2732 on four.
+bool wgrad_on_four_waves(const omega_moe *m, int T, int M, int N)
 {
-    return (long long)m->G * (M / 256) * ceil_div(N, 256) >= 24LL * m->n_wg;
+    const long long tiles = (long long)(M / 256) * ceil_div(N, 256);
+    return (long long)T * m->cfg.K >= 1024LL * m->cfg.E && tiles >= 2 * m->n_wg && m->G * tiles >= 32LL * m->n_wg;
 }
 
 // One product of the backward pass on the same kernel; `mode` as the enum above, operands and outputs as its comment says.
 hipError_t launch_product_bf16(const omega_moe *m, int mode, const void *A, const void *Aalt, const void *Wa, const void *Wb,
-                               void *Cout, void *Aux1, void *Aux2, const omega_tile_desc *wq, int N, int Kd, hipStream_t s, int M)
+                               void *Cout, void *Aux1, void *Aux2, const omega_tile_desc *wq, int N, int Kd, hipStream_t s, bool four_waves)
 {
     if (Kd < (NSTAGE + 1) * BK) return hipErrorInvalidValue;
     if (mode == MODE_DOWN && m->down_cols == 256 && Kd % 64 == 0 && Kd >= 8 * BK) {
@@ -1234,7 +1238,7 @@ hipError_t launch_product_bf16(const omega_moe *m, int mode, const void *A, cons
                            Aux1);
         return hipGetLastError();
     }
-    if (mode == MODE_WGRAD && wgrad_on_four_waves(m, M, N)) {
+    if (mode == MODE_WGRAD && four_waves) {
         hipLaunchKernelGGL((experts_up4_kernel<false, false, true, true>), dim3(m->n_wg), dim3(U4_WAVES * 64), SMEM_BYTES, s,
                            (const bf16_t *)A, (const bf16_t *)nullptr, (const bf16_t *)Wa, (const bf16_t *)nullptr, Cout, wq, N, Kd,
                            (const int32_t *)nullptr, (void *)nullptr);

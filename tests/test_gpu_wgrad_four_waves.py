@@ -1,6 +1,7 @@
-"""Weight gradients on the four-wave kernel (24 tiles per workgroup and more): an H of 128 mod 256, experts without rows, with
-less than one item's k steps and with several row tiles.  The products' operands are bf16 rows of the workspace, so float64
-gives them exactly; the sums are fp32 over at most a few hundred rows (relative L2 far below 1e-5)."""
+"""Weight gradients of many tiles on either kernel - four waves from 1024 rows per expert, 2 tiles per workgroup and expert and 32 in
+all on, else eight: an H of 128 mod 256, experts without rows, with less than one item's k steps and with several row tiles.
+The products' operands are bf16 rows of the workspace, so float64 gives them exactly; the sums are fp32 over at most a few thousand
+rows, added in up to 1000 products of 32 terms (relative L2 below 1e-5)."""
 import importlib
 
 import numpy as np
@@ -15,8 +16,9 @@ L = importlib.import_module("omega-ai_amd._lib")
 
 
 @pytest.mark.parametrize("kw", [
-    dict(T=600, d=2048, H=896, E=192, K=4, zipf_bias=1.2),   # both products
-    dict(T=70, d=1024, H=896, E=224, K=2, zipf_bias=0.0),    # dW1 and dW3 only: dW2 has 14 tiles per workgroup
+    dict(T=600, d=2048, H=896, E=192, K=4, zipf_bias=1.2),   # few rows per expert: eight waves
+    dict(T=70, d=1024, H=896, E=224, K=2, zipf_bias=0.0),
+    dict(T=8200, d=4096, H=8064, E=16, K=2, zipf_bias=1.2),  # both products on four waves (512 and 1008 tiles per expert)
 ])
 def test_weight_gradients_of_many_tiles(kw):
     from tests import gpu_util as G
@@ -32,14 +34,21 @@ def test_weight_gradients_of_many_tiles(kw):
     layer.forward(x)
     layer.back(g)
     r = layer.routing()
-    a, xg, dh = (layer.workspace(n, T).astype(np.float64) for n in ("a", "xg", "dh"))
-    dy = np.empty((T * K, d))
-    dy[r["dst"]] = O.round_bf16(r["w"].reshape(-1)[:, None] * np.repeat(g.to_numpy(), K, axis=0))
+    a, xg, dh = (layer.workspace(n, T) for n in ("a", "xg", "dh"))
+    dout = g.to_numpy()
     off, n = r["offsets"], np.diff(r["offsets"])
+    token, w = r["src_row"], np.empty(T * K, np.float32)
+    w[r["dst"]] = r["w"].reshape(-1)
+    # columns of every width: all of them, or of a wide layer the first and last 64 and 64 around the middle
+    cols = lambda size: np.arange(size) if size <= 2048 else np.r_[0:64, size // 2 - 32:size // 2 + 32, size - 64:size]
+    cd, cH = cols(d), cols(H)
     for e in sorted({int(n.argmin()), int(n.argmax()), int(np.argsort(n)[E // 2]), E - 1}):
         s = slice(off[e], off[e + 1])
-        for got, want in ((layer.grad(L.W_W2, e), dy[s].T @ a[s]), (layer.grad(L.W_W1, e), dh[s, :H].T @ xg[s]),
-                          (layer.grad(L.W_W3, e), dh[s, H:].T @ xg[s])):
+        dy = O.round_bf16(w[s, None] * dout[token[s]][:, cd]).astype(np.float64)
+        ae, xe = a[s][:, cH].astype(np.float64), xg[s][:, cd].astype(np.float64)
+        d1, d3 = dh[s][:, cH].astype(np.float64), dh[s][:, H + cH].astype(np.float64)
+        for got, want in ((layer.grad(L.W_W2, e)[np.ix_(cd, cH)], dy.T @ ae), (layer.grad(L.W_W1, e)[np.ix_(cH, cd)], d1.T @ xe),
+                          (layer.grad(L.W_W3, e)[np.ix_(cH, cd)], d3.T @ xe)):
             if n[e] == 0:
                 assert not got.any(), e
             else:
