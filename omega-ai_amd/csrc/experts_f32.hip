@@ -475,7 +475,9 @@ hipError_t launch_product_f32(const omega_moe *m, int op, const float *x, const 
             p.C = (float *)m->a;
             if (gather) {
                 p.tokp = m->tokp; p.dstp = m->dstp; p.xg = (float *)m->xg; p.K = c.K;
-                p.copy_wgs = std::min(ceil_div(T, 4), m->ctx->num_cus);
+                // (a token per wave until there are four workgroups per compute unit: a wave with several waits for each in
+                // turn behind the last product; 4096 tokens x 64 x 64, 64 experts, top 6, forward pass: 48.0 -> 46.4 us)
+                p.copy_wgs = std::min(ceil_div(T, 4), 4 * m->ctx->num_cus);
             }
             if (op == F32_RAW || keep) { p.H1 = m->bw_h1; p.H3 = m->bw_h3; }
             break;
