@@ -352,10 +352,9 @@ static int moe_reserve(omega_moe *m, int T)
     const size_t P = (size_t)T * c.K;
     // (a smaller batch may have more, lower token tiles than the largest one: at most one per compute unit then)
     const int n_tok_tiles = std::max(ceil_div(T, router_tok_tile(m, T)), std::min(ceil_div(T, 16), ctx->num_cus));
-    const int bm = moe_tile_m(m, T);
-    // every expert's rows start on a row-tile boundary: the buffers hold whole tiles.  fp32 layers: of the height that T
-    // tokens take, which is the largest any batch of up to T takes, and as many as there are of the smaller height (whose
-    // padding is the smaller too)
+    const int bm = c.dtype == OMEGA_DTYPE_F32 ? experts_f32_tile_m_max(m, T) : moe_tile_m(m, T);
+    // every expert's rows start on a row-tile boundary: the buffers hold whole tiles.  fp32 layers: of the largest height that
+    // any batch of up to T tokens takes, and as many as there are of the smaller height (whose padding is the smaller too)
     m->rows_cap = (size_t)moe_max_m_tiles(m, T, bm) * bm;
     m->tiles_cap = moe_max_m_tiles(m, T, c.dtype == OMEGA_DTYPE_F32 ? F32_TILE_M_SMALL : bm);
     OMEGA_HIP_CHECK(ctx, hipMalloc((void **)&m->ids, P * 4));

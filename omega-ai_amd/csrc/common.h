@@ -242,6 +242,7 @@ bool wgrad_on_four_waves(const omega_moe *m, int T, int M, int N);  // which ker
 #define F32_TILE_M 128       // row-tile heights of fp32 layers: experts_f32_tile_m chooses one per batch
 #define F32_TILE_M_SMALL 32
 int experts_f32_tile_m(const omega_moe *m, int T);
+int experts_f32_tile_m_max(const omega_moe *m, int T);  // no batch of up to T tokens takes a larger one
 hipError_t experts_bf16_init(void);
 hipError_t launch_down_slab_reduce(const omega_moe *m, float *y, hipStream_t s);  // y += partial results of k-sliced items
 hipError_t router_init(void);  // kernel attributes of the router (LDS beyond 64 KiB), once per device

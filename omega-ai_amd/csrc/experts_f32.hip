@@ -40,6 +40,7 @@
 // dxg 3.00 -> 1.10, dW2 0.99 -> 0.48, dW1 and dW3 2.01 -> 0.94.
 #include "common.h"
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 // matrix-core blocks of BS x BS: v_mfma_f32_32x32x2 (two k at a time, lane half = k) or v_mfma_f32_16x16x4 (four, lane
@@ -435,14 +436,36 @@ __global__ __launch_bounds__(256, 2) void f32_product_kernel(f32_args p)
     }
 }
 
-int experts_f32_tile_m(const omega_moe *m, int T)
+// The largest row-tile height that a batch of up to T tokens takes: 128 once the experts hold about that many rows and the down
+// product has a tile of 128 x 128 for every compute unit.  Weight gradients take their tiles of 128 x 128 from there on.
+int experts_f32_tile_m_max(const omega_moe *m, int T)
 {
-    // Row tiles of 128 once the experts hold about that many rows and the launches have a tile of 128 x 128 for every compute
-    // unit (the down product has the fewest tiles); else of 32.  (Forward pass with 2048 rows of 8 experts, d = 1024, H = 3584:
-    // small tiles 460 us, 64 x 64 ones 469; with 4096 rows the large ones take 887, small ones twice the 460.)
     const omega_moe_config &c = m->cfg;
     const long long rows = (long long)T * c.K;
     return rows >= (long long)F32_TILE_M * c.E && rows / F32_TILE_M * ceil_div(c.d, 128) >= m->ctx->num_cus ? F32_TILE_M : F32_TILE_M_SMALL;
+}
+
+// Within that, tiles of 32 rows where those of 128 would leave compute units idle for longer than they are worth: the up and
+// the down product in rounds of one tile per compute unit (a tile takes its k places and 32 more; an expert's last one counts
+// a quarter) against tiles of 32 at 0.86 of the large ones' rate.  Forward pass, us, 128 rows / 32 (/ the 64 x 64 tiles
+// before either): 2048 tokens x 1024 x 1024, 16 experts, top 2 358 / 267 (329), 4096 tokens x 512 x 1024, the same 316 / 269 (302), 64
+// experts, top 4, x 256 x 1024 354 / 316 (316), 2723 tokens x 1992 x 64, 6 experts, top 4 230 / 170 (206); the other way 4096 tokens x
+// 1024 x 3584, 8 experts, top 2 1524 / 1660 (1705), x 512 x 1024, 16 experts, top 4 483 / 506 (527).  Where elements are loaded one by one
+// the larger tile is the faster one (2981 tokens x 1287 x 111, 7 experts, top 5: 0.81 of the time).
+int experts_f32_tile_m(const omega_moe *m, int T)
+{
+    const omega_moe_config &c = m->cfg;
+    const int most = experts_f32_tile_m_max(m, T);
+    if (most == F32_TILE_M_SMALL || c.d % 4 != 0 || c.H % 4 != 0) return most;
+    // the last, partial round takes half a round and half of its share
+    auto rounds = [&](double tiles) {
+        const double n = tiles / m->ctx->num_cus, whole = std::floor(n);
+        return whole + (n > whole ? 0.5 + 0.5 * (n - whole) : 0.0);
+    };
+    const double rows = (double)T * c.K, tiles_m = rows / F32_TILE_M + c.E / 4.0;
+    const double large = rounds(tiles_m * ceil_div(c.H, 64)) * (c.d + 32.0) + rounds(tiles_m * ceil_div(c.d, 64)) * (c.H + 32.0) / 2.0;
+    const double small = 3.0 * rows * c.H * c.d / (m->ctx->num_cus * 128.0 * 128.0) / 0.86;
+    return large > 1.05 * small ? F32_TILE_M_SMALL : F32_TILE_M;
 }
 
 template <int OP, int TM, int TN>
@@ -504,7 +527,7 @@ hipError_t launch_product_f32(const omega_moe *m, int op, const float *x, const 
     // of 4096 tokens, 8 experts, top 2, us, both widths asked of every product and now: d = 1024, H = 2731 1238 -> 1214; d = 512, H = 1001 305 -> 299.)
     const bool d4 = c.d % 4 == 0, H4 = c.H % 4 == 0;
     const bool vec = (op == F32_DOWN || d4) && (op == F32_UP || op == F32_RAW || H4) && (((uintptr_t)p.Atok | (uintptr_t)p.Btok) % 16) == 0;
-    const bool big = m->bm == F32_TILE_M;
+    const bool big = (F32_IS_WG(op) ? experts_f32_tile_m_max(m, T) : m->bm) == F32_TILE_M;
 #define F32_ROWS(OP, TN_BIG, TN_SMALL)                                                         \
     (big ? f32_launch<OP, F32_TILE_M, TN_BIG>(p, vec, m->max_m_tiles, s)                       \
          : f32_launch<OP, F32_TILE_M_SMALL, TN_SMALL>(p, vec, m->max_m_tiles, s))

@@ -93,6 +93,7 @@ hipError_t router_init(void) { return hipSuccess; }
 hipError_t experts_bf16_init(void) { return hipSuccess; }
 int router_tok_tile(const omega_moe *m, int) { return m->cfg.E <= 16 ? 16 : 32; }
 int experts_bf16_tile_m(const omega_moe *, int) { return 256; }
+int experts_f32_tile_m_max(const omega_moe *, int T) { return T >= 1024 ? F32_TILE_M : F32_TILE_M_SMALL; }
 int experts_f32_tile_m(const omega_moe *, int T) { return T >= 1024 ? F32_TILE_M : F32_TILE_M_SMALL; }  // (a rule of the same kind)
 
 hipError_t launch_fill_normal(void *, uint64_t, uint64_t, uint64_t, double, uint64_t, int, hipStream_t) { return line("fill"); }

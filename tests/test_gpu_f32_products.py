@@ -14,9 +14,11 @@ from tests.test_gpu_backward import _check_grads, _setup
 pytestmark = pytest.mark.gpu
 L = importlib.import_module("omega-ai_amd._lib")
 
+# tiles of 128 rows with 16-byte loads: ragged row tiles, last column tiles, partial k steps
+ROWS_128 = dict(T=5073, d=380, H=124, E=3, K=3, Es=1)
 CASES = [
-    dict(T=1300, d=1028, H=68, E=3, K=3, Es=1),    # tiles of 128 rows: ragged row tiles, last column tiles, partial k steps
-    dict(T=1301, d=1027, H=67, E=3, K=3),          # the same without 16-byte loads
+    dict(T=1300, d=1028, H=68, E=3, K=3, Es=1),    # tiles of 32 rows, and of 128 x 128 in the weight gradients
+    dict(T=1301, d=1027, H=67, E=3, K=3),          # tiles of 128 rows without 16-byte loads
     dict(T=300, d=260, H=132, E=2, K=2),           # tiles of 32 rows, whole and partial k steps
     dict(T=77, d=68, H=60, E=5, K=3, Es=1),        # ragged tiles of 32 rows, one k step and a part, less than one
     dict(T=77, d=67, H=65, E=5, K=3, Es=1),        # the same without 16-byte loads
@@ -29,6 +31,7 @@ CASES = [
     dict(T=77, d=68, H=61, E=5, K=3, Es=1),        # and of 32
     dict(T=1301, d=1025, H=68, E=3, K=3),          # in the down product alone
     dict(T=77, d=67, H=60, E=5, K=3, Es=1),
+    ROWS_128,
 ]
 
 
@@ -46,7 +49,7 @@ def test_fp32_products_match_oracle(kw):
     layer.close()
 
 
-@pytest.mark.parametrize("kw", [CASES[0], CASES[1], CASES[6], dict(T=50, d=48, H=40, E=16, K=2, zipf_bias=1.2)])
+@pytest.mark.parametrize("kw", [CASES[0], CASES[1], CASES[6], ROWS_128, dict(T=50, d=48, H=40, E=16, K=2, zipf_bias=1.2)])
 def test_fp32_training_mode_keeps_h1_h3(kw):
     """The backward pass reads the h1, h3 and probabilities that a training forward left: the same bits as computing them
     again, once; a second backward pass, whose d(a) product has overwritten them, computes them again."""
@@ -118,7 +121,7 @@ def test_update_steps_every_expert(d, H):
 def test_one_layer_at_both_tile_heights(training):
     """Batches with tiles of 128 rows, then 32, then 128 again on one layer's workspace: the bits of a layer that sees the batch
     alone."""
-    G, cfg, inp, dout, layer = _setup("c1_tiny_f32", CASES[0], 80)
+    G, cfg, inp, dout, layer = _setup("c1_tiny_f32", ROWS_128, 80)
 
     def step(lay, T):
         lay.set_training(training)
@@ -143,7 +146,7 @@ def _chain(A, B):
     return s
 
 
-@pytest.mark.parametrize("T,d,H", [(64, 64, 3584), (64, 63, 3551), (32768, 128, 3584), (32768, 128, 3620)])
+@pytest.mark.parametrize("T,d,H", [(64, 64, 3584), (64, 63, 3551), (49088, 128, 3584), (49088, 128, 3620)])
 def test_input_gradient_adds_two_sums(T, d, H):
     """dxg = dh1 . W1 + dh3 . W3 is the sum of two sums of H terms (tiles of 32 rows, of 128; an odd number of k steps; k left
     over), not a chain of 2 H: against float64 the error is that of two chains on the same operands (1.2: the roundings of
@@ -164,7 +167,7 @@ def test_input_gradient_adds_two_sums(T, d, H):
     layer.close()
 
 
-@pytest.mark.parametrize("kw", [CASES[0], dict(T=77, d=68, H=61, E=5, K=3, Es=1), dict(T=77, d=68, H=60, E=5, K=3)])
+@pytest.mark.parametrize("kw", [CASES[0], ROWS_128, dict(T=77, d=68, H=61, E=5, K=3, Es=1), dict(T=77, d=68, H=60, E=5, K=3)])
 def test_rows_that_start_off_a_16_byte_boundary(kw):
     """The caller's x and dout one float behind an aligned address: loads element by element, the same bits."""
     G, cfg, inp, dout, layer = _setup("c1_tiny_f32", kw, 83)
@@ -185,7 +188,7 @@ def test_rows_that_start_off_a_16_byte_boundary(kw):
 
 def test_timed_backward_passes_leave_the_gradients_of_one():
     """What a timed pass of a training step uses up is computed again in front of the next: every pass gives the same bits."""
-    G, cfg, inp, dout, layer = _setup("c1_tiny_f32", CASES[0], 84)
+    G, cfg, inp, dout, layer = _setup("c1_tiny_f32", ROWS_128, 84)
     x = G.P.DeviceBuffer.from_numpy(G.ctx(), inp["x"], cfg.dtype)
     g = G.P.DeviceBuffer.from_numpy(G.ctx(), dout, cfg.dtype)
     dx = G.P.DeviceBuffer(G.ctx(), (cfg.T, cfg.d), cfg.dtype)
