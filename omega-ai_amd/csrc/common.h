@@ -240,6 +240,7 @@ hipError_t launch_unpack_rows(void *dst_rowmajor, const void *src_packed, int R,
 int experts_bf16_tile_m(const omega_moe *m, int T);
 bool wgrad_on_four_waves(const omega_moe *m, int T, int M, int N);  // which kernel takes the weight gradients of M x N per expert
 #define F32_TILE_M 128       // row-tile heights of fp32 layers: experts_f32_tile_m chooses one per batch
+#define F32_TILE_M_MID 64
 #define F32_TILE_M_SMALL 32
 int experts_f32_tile_m(const omega_moe *m, int T);
 int experts_f32_tile_m_max(const omega_moe *m, int T);  // no batch of up to T tokens takes a larger one

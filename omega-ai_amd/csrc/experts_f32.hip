@@ -12,7 +12,7 @@
 // Row tiles come from the tile list written by the dispatch stage: a tile never straddles two experts.
 //
 // Bound: fp32 MFMA, 157.3 TFLOP/s (256 FLOP per clock and compute unit; 154 measured with nothing else going on).  One
-// workgroup = four waves = one tile of TM rows x TN MFMA columns, 128 x 128 or, for small batches, 32 x 32 (up: 32 x 64;
+// workgroup = four waves = one tile of TM rows x TN MFMA columns, 128 x 128, 64 x 64 (up: 64 x 128) or, for small batches, 32 x 32 (up: 32 x 64;
 // half of the columns are W1's, half W3's, so a wave holds h1 and h3 of the same elements; weight gradients: 64 x 64).  A wave has TM/2 x TN/2 of it
 // as 32 x 32 blocks; its row blocks alternate with the other row half's, so a ragged tile leaves both the same work.  At
 // 128 x 128 a step of 32 k is 64 MFMAs of 64 cycles per wave against 32 KiB of operands, 8 bytes per clock and compute unit.
@@ -436,36 +436,46 @@ __global__ __launch_bounds__(256, 2) void f32_product_kernel(f32_args p)
     }
 }
 
-// The largest row-tile height that a batch of up to T tokens takes: 128 once the experts hold about that many rows and the down
-// product has a tile of 128 x 128 for every compute unit.  Weight gradients take their tiles of 128 x 128 from there on.
+// The largest row-tile height that a batch of up to T tokens takes: with fewer than 128 rows per expert always 32 (160 shapes of
+// 1 to 4096 tokens, d = 64 .. 1024, H = 64 .. 3584, 2 to 16 experts: tiles of 64 took 0.97 to 1.90 times as long)
 int experts_f32_tile_m_max(const omega_moe *m, int T)
 {
-    const omega_moe_config &c = m->cfg;
-    const long long rows = (long long)T * c.K;
-    return rows >= (long long)F32_TILE_M * c.E && rows / F32_TILE_M * ceil_div(c.d, 128) >= m->ctx->num_cus ? F32_TILE_M : F32_TILE_M_SMALL;
+    return (long long)T * m->cfg.K >= 128LL * m->cfg.E ? F32_TILE_M : F32_TILE_M_SMALL;
 }
 
-// Within that, tiles of 32 rows where those of 128 would leave compute units idle for longer than they are worth: the up and
-// the down product in rounds of one tile per compute unit (a tile takes its k places and 32 more; an expert's last one counts
-// a quarter) against tiles of 32 at 0.86 of the large ones' rate.  Forward pass, us, 128 rows / 32 (/ the 64 x 64 tiles
-// before either): 2048 tokens x 1024 x 1024, 16 experts, top 2 358 / 267 (329), 4096 tokens x 512 x 1024, the same 316 / 269 (302), 64
-// experts, top 4, x 256 x 1024 354 / 316 (316), 2723 tokens x 1992 x 64, 6 experts, top 4 230 / 170 (206); the other way 4096 tokens x
-// 1024 x 3584, 8 experts, top 2 1524 / 1660 (1705), x 512 x 1024, 16 experts, top 4 483 / 506 (527).  Where elements are loaded one by one
-// the larger tile is the faster one (2981 tokens x 1287 x 111, 7 experts, top 5: 0.81 of the time).
+// From there on the height whose forward products are the shortest by this estimate.  A tile takes its k places in whole steps, a
+// fixed number more and, for a last partial step, `rest` more, at a rate that falls a little with its size (`a`: time per
+// column of k); a product takes rounds of one tile per compute unit, its last, partial round `part` of one and that share of the
+// rest, all of them `least` rounds or more; an expert has `pad` tiles more than its rows.  The numbers are fitted to 540 forward
+// passes of the range above at all three heights, of which the estimate takes the best or one within 5 % (0.4 % in the mean).
+// Forward pass, us, at 32 / 64 / 128 rows: 2048 tokens x 1024 x 1024, 16 experts, top 2 272 / 281 / 361, 1001 tokens x 124 x 1676, 6 experts,
+// top 5 and 2 shared 196 / 143 / 160, 3496 tokens x 120 x 452, 9 experts, top 7 192 / 148 / 144, 4096 tokens x 1024 x 3584, 8 experts, top 2
+// 1654 / 1547 / 1535.  (The 64 x 64 tiles of an earlier kernel: 330, 143, 142, 1715.)
 int experts_f32_tile_m(const omega_moe *m, int T)
 {
+    if (experts_f32_tile_m_max(m, T) == F32_TILE_M_SMALL) return F32_TILE_M_SMALL;
     const omega_moe_config &c = m->cfg;
-    const int most = experts_f32_tile_m_max(m, T);
-    if (most == F32_TILE_M_SMALL || c.d % 4 != 0 || c.H % 4 != 0) return most;
-    // the last, partial round takes half a round and half of its share
-    auto rounds = [&](double tiles) {
-        const double n = tiles / m->ctx->num_cus, whole = std::floor(n);
-        return whole + (n > whole ? 0.5 + 0.5 * (n - whole) : 0.0);
-    };
-    const double rows = (double)T * c.K, tiles_m = rows / F32_TILE_M + c.E / 4.0;
-    const double large = rounds(tiles_m * ceil_div(c.H, 64)) * (c.d + 32.0) + rounds(tiles_m * ceil_div(c.d, 64)) * (c.H + 32.0) / 2.0;
-    const double small = 3.0 * rows * c.H * c.d / (m->ctx->num_cus * 128.0 * 128.0) / 0.86;
-    return large > 1.05 * small ? F32_TILE_M_SMALL : F32_TILE_M;
+    static const struct { int bm, step, cols; double a, more, rest, pad, least, part; } form[] = {
+        {F32_TILE_M_SMALL, 64, 32, 1.0, 104, 64, 1.0, 0.6, 0.15},
+        {F32_TILE_M_MID, 32, 64, 4.0, 60, 42, 0.55, 0.95, 0.4},
+        {F32_TILE_M, 32, 64, 7.3, 64, 52, 0.65, 0.8, 0.5}};
+    int best = F32_TILE_M_SMALL;
+    double least_time = 0.0;
+    for (const auto &f : form) {
+        const double tiles_m = (double)T * c.K / f.bm + f.pad * c.E + (double)c.Es * ceil_div(T, f.bm);
+        auto product = [&](int k, int n) {
+            const double all = tiles_m * ceil_div(n, f.cols) / m->ctx->num_cus, whole = std::floor(all);
+            const double rounds = all < f.least ? f.least : whole + (all > whole ? f.part + (1.0 - f.part) * (all - whole) : 0.0);
+            return rounds * (ceil_div(k, f.step) * f.step + f.more + (k % f.step != 0 ? f.rest : 0.0));
+        };
+        // (the up product's tiles hold two columns of weights for each of their own)
+        const double time = f.a * (product(c.d, c.H) + 0.56 * product(c.H, c.d));
+        if (f.bm == F32_TILE_M_SMALL || time < least_time) {
+            best = f.bm;
+            least_time = time;
+        }
+    }
+    return best;
 }
 
 template <int OP, int TM, int TN>
@@ -527,18 +537,22 @@ hipError_t launch_product_f32(const omega_moe *m, int op, const float *x, const 
     // of 4096 tokens, 8 experts, top 2, us, both widths asked of every product and now: d = 1024, H = 2731 1238 -> 1214; d = 512, H = 1001 305 -> 299.)
     const bool d4 = c.d % 4 == 0, H4 = c.H % 4 == 0;
     const bool vec = (op == F32_DOWN || d4) && (op == F32_UP || op == F32_RAW || H4) && (((uintptr_t)p.Atok | (uintptr_t)p.Btok) % 16) == 0;
-    const bool big = (F32_IS_WG(op) ? experts_f32_tile_m_max(m, T) : m->bm) == F32_TILE_M;
-#define F32_ROWS(OP, TN_BIG, TN_SMALL)                                                         \
-    (big ? f32_launch<OP, F32_TILE_M, TN_BIG>(p, vec, m->max_m_tiles, s)                       \
-         : f32_launch<OP, F32_TILE_M_SMALL, TN_SMALL>(p, vec, m->max_m_tiles, s))
+    // weight gradients, whose tiles do not depend on the row tiles: of 128 x 128 from 128 rows per expert on, once the down product
+    // would have such a tile for every compute unit
+    const long long rows = (long long)T * c.K;
+    const bool wide = rows >= 128LL * c.E && rows / 128 * ceil_div(c.d, 128) >= m->ctx->num_cus;
+#define F32_ROWS(OP, TN_BIG, TN_MID, TN_SMALL)                                                 \
+    (m->bm == F32_TILE_M ? f32_launch<OP, F32_TILE_M, TN_BIG>(p, vec, m->max_m_tiles, s)       \
+     : m->bm == F32_TILE_M_MID ? f32_launch<OP, F32_TILE_M_MID, TN_MID>(p, vec, m->max_m_tiles, s) \
+                               : f32_launch<OP, F32_TILE_M_SMALL, TN_SMALL>(p, vec, m->max_m_tiles, s))
     switch (op) {
-        case F32_UP: return F32_ROWS(F32_UP, 128, 64);
-        case F32_RAW: return F32_ROWS(F32_RAW, 128, 64);
-        case F32_DOWN: return F32_ROWS(F32_DOWN, 64, 32);
-        case F32_DA: return F32_ROWS(F32_DA, 128, 32);
-        case F32_DXG: return F32_ROWS(F32_DXG, 64, 32);
-        case F32_WG2: return big ? f32_launch<F32_WG2, 128, 128>(p, vec, 0, s) : f32_launch<F32_WG2, 64, 64>(p, vec, 0, s);
-        default: return big ? f32_launch<F32_WG13, 128, 128>(p, vec, 0, s) : f32_launch<F32_WG13, 64, 64>(p, vec, 0, s);
+        case F32_UP: return F32_ROWS(F32_UP, 128, 128, 64);
+        case F32_RAW: return F32_ROWS(F32_RAW, 128, 128, 64);
+        case F32_DOWN: return F32_ROWS(F32_DOWN, 64, 64, 32);
+        case F32_DA: return F32_ROWS(F32_DA, 128, 64, 32);
+        case F32_DXG: return F32_ROWS(F32_DXG, 64, 64, 32);
+        case F32_WG2: return wide ? f32_launch<F32_WG2, 128, 128>(p, vec, 0, s) : f32_launch<F32_WG2, 64, 64>(p, vec, 0, s);
+        default: return wide ? f32_launch<F32_WG13, 128, 128>(p, vec, 0, s) : f32_launch<F32_WG13, 64, 64>(p, vec, 0, s);
     }
 #undef F32_ROWS
 }

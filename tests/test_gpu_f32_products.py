@@ -1,4 +1,4 @@
-"""The fp32 products at both row-tile heights: rows, widths and k that are no multiple of the tiles, forward and backward
+"""The fp32 products at the three row-tile heights: rows, widths and k that are no multiple of the tiles, forward and backward
 against the oracle (fp32 sums of at most a few thousand terms: relative L2 within 1e-5, as for every fp32 layer)."""
 import ctypes
 import importlib
@@ -14,11 +14,12 @@ from tests.test_gpu_backward import _check_grads, _setup
 pytestmark = pytest.mark.gpu
 L = importlib.import_module("omega-ai_amd._lib")
 
-# tiles of 128 rows with 16-byte loads: ragged row tiles, last column tiles, partial k steps
-ROWS_128 = dict(T=5073, d=380, H=124, E=3, K=3, Es=1)
+# tiles of 128 and of 64 rows with 16-byte loads: ragged row tiles, last column tiles, partial k steps
+ROWS_128 = dict(T=1333, d=228, H=228, E=3, K=3, Es=1)
+ROWS_64 = dict(T=1955, d=100, H=132, E=3, K=3, Es=1)
 CASES = [
     dict(T=1300, d=1028, H=68, E=3, K=3, Es=1),    # tiles of 32 rows, and of 128 x 128 in the weight gradients
-    dict(T=1301, d=1027, H=67, E=3, K=3),          # tiles of 128 rows without 16-byte loads
+    dict(T=1301, d=1027, H=67, E=3, K=3),          # the same without 16-byte loads
     dict(T=300, d=260, H=132, E=2, K=2),           # tiles of 32 rows, whole and partial k steps
     dict(T=77, d=68, H=60, E=5, K=3, Es=1),        # ragged tiles of 32 rows, one k step and a part, less than one
     dict(T=77, d=67, H=65, E=5, K=3, Es=1),        # the same without 16-byte loads
@@ -27,11 +28,14 @@ CASES = [
     dict(T=200, d=33, H=5, E=2, K=2),              # whole k steps of weight gradients far narrower than a tile
     dict(T=64, d=32, H=64, E=1, K=1),              # whole row tiles, half a k step and one
     dict(T=32, d=32, H=64, E=1, K=1),              # exactly one row tile, one k step of the down product
-    dict(T=1300, d=1028, H=67, E=3, K=3, Es=1),    # 16-byte loads in the up product alone, tiles of 128 rows
+    dict(T=1333, d=228, H=235, E=3, K=3, Es=1),    # 16-byte loads in the up product alone, tiles of 128 rows
     dict(T=77, d=68, H=61, E=5, K=3, Es=1),        # and of 32
-    dict(T=1301, d=1025, H=68, E=3, K=3),          # in the down product alone
+    dict(T=1333, d=235, H=228, E=3, K=3, Es=1),    # in the down product alone, tiles of 128 rows
     dict(T=77, d=67, H=60, E=5, K=3, Es=1),
     ROWS_128,
+    dict(ROWS_128, d=193, H=235),                  # tiles of 128 rows without 16-byte loads
+    ROWS_64,
+    dict(ROWS_64, d=99, H=131),                    # of 64
 ]
 
 
@@ -49,7 +53,7 @@ def test_fp32_products_match_oracle(kw):
     layer.close()
 
 
-@pytest.mark.parametrize("kw", [CASES[0], CASES[1], CASES[6], ROWS_128, dict(T=50, d=48, H=40, E=16, K=2, zipf_bias=1.2)])
+@pytest.mark.parametrize("kw", [CASES[0], CASES[1], CASES[6], ROWS_128, ROWS_64, dict(T=50, d=48, H=40, E=16, K=2, zipf_bias=1.2)])
 def test_fp32_training_mode_keeps_h1_h3(kw):
     """The backward pass reads the h1, h3 and probabilities that a training forward left: the same bits as computing them
     again, once; a second backward pass, whose d(a) product has overwritten them, computes them again."""
@@ -118,8 +122,8 @@ def test_update_steps_every_expert(d, H):
 
 
 @pytest.mark.parametrize("training", [False, True])
-def test_one_layer_at_both_tile_heights(training):
-    """Batches with tiles of 128 rows, then 32, then 128 again on one layer's workspace: the bits of a layer that sees the batch
+def test_one_layer_at_every_tile_height(training):
+    """Batches with tiles of 128 rows, then 64, 32 and 128 again on one layer's workspace: the bits of a layer that sees the batch
     alone."""
     G, cfg, inp, dout, layer = _setup("c1_tiny_f32", ROWS_128, 80)
 
@@ -131,7 +135,7 @@ def test_one_layer_at_both_tile_heights(training):
         return [out, lay.back(g).to_numpy(), lay.grad(L.W_GATE)] + [
             lay.grad(w, e) for e in range(cfg.E + cfg.Es) for w in (L.W_W1, L.W_W3, L.W_W2)]
 
-    for T in (cfg.T, 77, 1, cfg.T):
+    for T in (cfg.T, 900, 77, 1, cfg.T):
         alone = G.build_layer(cfg, inp)
         assert all(np.array_equal(a, b) for a, b in zip(step(layer, T), step(alone, T))), T
         alone.close()
@@ -146,10 +150,10 @@ def _chain(A, B):
     return s
 
 
-@pytest.mark.parametrize("T,d,H", [(64, 64, 3584), (64, 63, 3551), (49088, 128, 3584), (49088, 128, 3620)])
+@pytest.mark.parametrize("T,d,H", [(64, 64, 3584), (64, 63, 3551), (4096, 96, 3596), (49088, 128, 3584), (49088, 128, 3620)])
 def test_input_gradient_adds_two_sums(T, d, H):
-    """dxg = dh1 . W1 + dh3 . W3 is the sum of two sums of H terms (tiles of 32 rows, of 128; an odd number of k steps; k left
-    over), not a chain of 2 H: against float64 the error is that of two chains on the same operands (1.2: the roundings of
+    """dxg = dh1 . W1 + dh3 . W3 is the sum of two sums of H terms (tiles of 32 rows, of 64 and of 128; an odd number of k
+    steps; k left over), not a chain of 2 H: against float64 the error is that of two chains on the same operands (1.2: the roundings of
     dh itself, three sums of d terms, add at most sqrt(1 + 3 d / H) = 1.05, and 4096 elements scatter by a few percent), where
     one chain has 1.41 times it."""
     G, cfg, inp, dout, layer = _setup("c1_tiny_f32", dict(T=T, d=d, H=H, E=1, K=1), 81)
@@ -167,7 +171,7 @@ def test_input_gradient_adds_two_sums(T, d, H):
     layer.close()
 
 
-@pytest.mark.parametrize("kw", [CASES[0], ROWS_128, dict(T=77, d=68, H=61, E=5, K=3, Es=1), dict(T=77, d=68, H=60, E=5, K=3)])
+@pytest.mark.parametrize("kw", [CASES[0], ROWS_128, ROWS_64, dict(T=77, d=68, H=61, E=5, K=3, Es=1), dict(T=77, d=68, H=60, E=5, K=3)])
 def test_rows_that_start_off_a_16_byte_boundary(kw):
     """The caller's x and dout one float behind an aligned address: loads element by element, the same bits."""
     G, cfg, inp, dout, layer = _setup("c1_tiny_f32", kw, 83)
