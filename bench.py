@@ -198,7 +198,7 @@ def main():
         "config": {"workload": f"{cfg.name}: T={cfg.T} ({cfg.batch}x{cfg.seq}) d={cfg.d} E={cfg.E} K={cfg.K} H={cfg.H} "
                                f"Es={cfg.Es} renorm={int(cfg.renorm)} {cfg.dtype}, fp32 accumulate",
                    "router_mode": a.router, "seed": a.seed},
-        "roofline": {"bound": "mfma", "kernel": ("experts_up4_kernel" if cfg.dtype == "bf16" else "experts_f32_kernel<true>") + " (up product): a = silu(xg W1^T) * (xg W3^T)",
+        "roofline": {"bound": "mfma", "kernel": ("experts_up4_kernel" if cfg.dtype == "bf16" else "f32_product_kernel<0>") + " (up product): a = silu(xg W1^T) * (xg W3^T)",
                      "achieved": up_tflops, "peak": peak, "unit": "TFLOP/s", "frac": up_tflops / peak,
                      "algorithmic_flops_per_launch": up_flops, "avg_launch_ms": stage_ms["experts_up"],
                      "traffic": traffic, "traffic_source": traffic_src,
@@ -246,8 +246,9 @@ def main():
             ids, w = O.topk(p, cfg.K, cfg.renorm)
             counts, offsets, dst, src = O.dispatch(ids, cfg.E)
             # a token of every row tile of every expert (first row of the tile, last row of the expert), so that the
-            # sample touches every row tile the grouped products schedule, plus 16 evenly spaced tokens
-            bm = 256 if bf else 64
+            # sample touches every row tile the grouped products schedule (fp32: of the smallest height), plus 16 evenly
+            # spaced tokens
+            bm = 256 if bf else 32
             pick = set(np.linspace(0, cfg.T - 1, 16).astype(np.int64).tolist())
             for e in range(cfg.E):
                 n, l0 = int(counts[e]), int(offsets[e])

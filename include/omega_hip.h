@@ -177,7 +177,7 @@ int omega_moe_set_training(omega_moe *moe, int on);
  *     row -> token table of the dispatch stage.  Same results bit for bit.  The loads then read 64-byte pieces of
  *     rows instead of whole lines, which costs the product 1-8 %, and K row copies per token are saved: AUTO takes
  *     this form while H/128 <= 2 K (a row tile is read H/128 times).
- * Training mode and fp32 layers always copy.  x must stay unchanged until the forward pass has finished either way;
+ * Training mode and fp32 layers always leave the copy.  x must stay unchanged until the forward pass has finished either way;
  * with ON_LOAD, omega_moe_get_workspace(moe, 0, ...) and a backward pass gather the rows when they are asked for,
  * from the x of the last dispatch, which must still hold that batch. */
 #define OMEGA_GATHER_AUTO 0

@@ -8,10 +8,10 @@
 //                  (silu_backward, J/engine/nn/layer/active/gpu/activeFunction.cu:182-190)
 //   softmax        sum = sum_e out*delta; diff = (delta - sum) * out   (softmax_back, J/engine/gpu/SoftmaxKernel.cu:101-112)
 // The routing of the forward pass (ids, permutation, row tiles) is reused as it was left in the workspace, together
-// with the activations a and the expert outputs y; h1 and h3 are recomputed.  Expert rows keep their forward places:
-// dy, dh1, dh3 and dxg are indexed by the same physical rows as xg, a and y.
+// with the activations a and the expert outputs y; h1 and h3 are computed again unless a training forward kept
+// them.  Expert rows keep their forward places: dy, dh1, dh3 and dxg are indexed by the same physical rows as xg, a and y.
 //
-// bf16 layers run every product on the matrix-core kernel of the forward pass (launch_backward_bf16 at the end of this
+// bf16 layers run every product on the matrix-core kernels of the forward pass (launch_backward_bf16 at the end of this
 // file; the products themselves are described in experts_bf16.hip, their tables and the transposes in dispatch.hip).
 // fp32 layers run theirs on the fp32 matrix-core kernel (experts_f32.hip).  Here:
 //   bw_combine_kernel   dy[r,:] = w[t,j] * dout[t,:],  dw[t,j] = dout[t,:] . y[r,:]

@@ -164,8 +164,8 @@ struct omega_moe {
     size_t prof_used = 0;
 };
 
-// Tokens per router workgroup = per row of tile_counts and per workgroup of the dispatch kernel: 16 for layers
-// with at most 16 experts, else 32 (router.hip).
+// Tokens per router workgroup = per row of tile_counts and per workgroup of the dispatch kernel: 16 for layers with at most
+// 16 experts and for exact bf16 layers with more while such tiles find a compute unit each, else 32 (router.hip).
 int router_tok_tile(const omega_moe *m, int T);
 #define ROUTER_TOK_TILE_MAX 32
 

@@ -843,8 +843,8 @@ hipError_t launch_unpack_rows(void *dst_rowmajor, const void *src_packed, int R,
 
 // ---- work-item tables of the backward products (bf16 layers) ----
 // k space of the weight gradients: the experts' rows, expert after expert, each expert's share rounded up to 64 rows
-// and to at least 192 or 256 (an item of the eight-wave kernel has at least 6 k steps, one of the four-wave kernel 8); kt0[g] = first k step
-// (32 rows) of group g, kt0[G] = all of them.  Empty groups take no space and get no items.
+// and to at least 192, or 256 where the four-wave kernel takes one of the products (its items have at least 8 k steps, those of
+// the eight-wave kernel 6); kt0[g] = first k step (32 rows) of group g, kt0[G] = all of them.  Empty groups take no space and get no items.
 __device__ __forceinline__ int kspace_steps(int rows, int least) { return rows > 0 ? max((rows + 63) / 64 * 2, least) : 0; }
 
 // One workgroup per group g: the items of the d(a) product (256-column tiles over H, table as the forward ones), the

@@ -12,11 +12,12 @@
 //                        reads per 64 MFMAs, the instruction order of a k step pinned (a lone wave issues one instruction
 //                        every four cycles, an MFMA occupies the matrix core for sixteen).  The forward pass's up
 //                        product (it can fetch its rows from x through the row -> token table), the down product with
-//                        256-column items and the backward pass's input-gradient product: 2-3 % faster than eight waves.
+//                        256-column items, the backward pass's input-gradient product (2-3 % faster than eight waves) and the
+//                        weight gradients of many tiles and rows (wgrad_on_four_waves).
 //   experts_bf16_kernel  eight waves (2 row halves x 4 column quarters, two per SIMD, 128 accumulator registers each;
 //                        the 32-row blocks of the tile alternate between the row halves, so a ragged tile splits
-//                        evenly): the products that keep or read h1 / h3 records, the weight gradients, and down
-//                        products with 128-column items.
+//                        evenly): the products that keep or read h1 / h3 records, the other weight gradients, and
+//                        down products with 128-column items.
 //
 // Data movement: global -> LDS directly (global_load_lds_dwordx4, no staging registers) into a ring of five
 // stages of (A 256x32 + B 256x32) bf16 = 160 KiB, i.e. all of a CU's LDS.  A wave-wide direct load fills 1 KiB

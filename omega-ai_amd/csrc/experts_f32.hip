@@ -21,7 +21,8 @@
 // whatever the number of buffers, workgroups or wave priorities).  So the order of a step is pinned: the fragments of the
 // next 8 k are read, the next step's pieces written to the other LDS buffer and the pieces of the step behind it asked for
 // between the MFMAs, a few at a time, and the one barrier of a step stands in front of MFMAs whose operands are in registers
-// (MFMA busy 0.89; 134 TFLOP/s at k = 8192).  No vector instruction but the address sums of the loads is spent per step.
+// (up product, ragged tiles and the last round included: MFMA busy 0.80 and 125 TFLOP/s at k = 1024, 0.82 and 124 at k =
+// 8192).  No vector instruction but the address sums of the loads is spent per step.
 // The down and the input-gradient product, which have the fewest column tiles, take tiles of 128 x 64 (N = 1024, 8192
 // rows: 0.65 -> 0.55 and 1.26 -> 1.10 ms: 544 tiles of 128 x 128 leave the third round of two per compute unit nearly empty).
 // A small batch leaves compute units idle and is as long as the chain of one wave: its tiles are 32 x 32 of four waves with

@@ -1,10 +1,10 @@
 // Router: gate projection, row softmax, wave-level top-k, per-token-tile expert histogram.
 //
-// One workgroup routes a tile of TT tokens: 32 (256 threads), or 16 for layers with at most 16 experts (one thread per
-// token and expert, 128 or 256 threads: the sums are bound by LDS reads per compute unit, so such a layer spreads its
-// tokens over twice as many workgroups).
+// One workgroup routes a tile of TT tokens: 32, or 16 for layers with at most 16 experts (one thread per token and expert, 128
+// or 256 threads: the sums are bound by LDS reads per compute unit, so such a layer spreads its tokens over twice as many
+// workgroups) and for exact bf16 layers with more while tiles of 16 find a compute unit each.
 //  phase 1  logits[t,e] = sum_k x[t,k]*Wg[e,k] (+bg[e]): one lane per (token, expert); x and Wg are
-//           staged through LDS in chunks of 64..256 k.  EXACT mode adds the products one k at a time with
+//           staged through LDS in chunks of 64..512 k.  EXACT mode adds the products one k at a time with
 //           a separate multiply and add (this file is compiled with -ffp-contract=off), which is the
 //           summation order of the reference's CPU dot (J/common/utils/MatrixOperation.java:1472-1478);
 //           FAST mode uses fused multiply-adds (same order, one rounding per step).
@@ -15,7 +15,8 @@
 //           top-k: K rounds of a cross-lane (value,index) butterfly arg-max, "greater value, or equal
 //           value and lower index" so ties go to the lowest expert; winners are masked out.
 //  phase 3  LDS-atomic histogram of the selected experts, flushed as row `tile` of tile_counts[.,E].
-// FAST mode of bf16 layers with more than 16 experts takes phase 1 to the matrix cores (router_mfma_kernel below).
+// bf16 layers with more than 16 experts take phase 1 to the matrix cores: router_units_kernel with the same bits, in FAST mode
+// router_mfma_kernel (both below).
 // bf16 layers with at most 16 experts and at most one tile per compute unit take router_pipe_kernel: phase 1 is then as
 // long as one chain of d dependent multiply-adds, and separate staging waves keep everything else out of the waves that
 // run the chains (Mixtral shape: 4096 tokens 33 -> 29 us, 64 tokens 27 -> 22 us; of the 22, 11 are the chain itself at
@@ -791,7 +792,7 @@ hipError_t launch_router(const omega_moe *m, const void *x, int T, float *logits
     }
 #define ROUTER_LAUNCH(EPV, KCV)                                                                                    \
     do {                                                                                                           \
-        if (exact)                                                                                            \
+        if (exact)                                                                                                 \
             hipLaunchKernelGGL((router_kernel<EPV, KCV, true>), dim3(tiles), dim3(ROUTER_NTHR(EPV)), 0, s, x, c.dtype, m->Wg, bg, \
                                T, c.d, c.E, c.K, c.renorm, m->ids, m->w, m->tile_counts, logits_out, probs_out);   \
         else                                                                                                       \

@@ -37,9 +37,10 @@ __global__ __launch_bounds__(256) void adamw_f32_kernel(float *__restrict__ w, s
 
 // bf16 expert weights: the step is taken on the fp32 master, the packed bf16 image is re-rounded from it.  A thread takes four
 // adjacent columns of a row of expert blockIdx.y, so that every load and store of a wave is one contiguous kilobyte (master,
-// gradient and moments share one layout; the image gets 8 bytes of a 16-byte chunk).  Bound: the 30 bytes per weight (49
-// million of them: 347 us with two 16-byte halves of a chunk per thread and 64-bit indices, 293 now, 5.0 TB/s), which pass the
-// last-level cache by.
+// gradient and moments share one layout; the image gets 8 bytes of a 16-byte chunk).  Bound: the 30 bytes per weight, which
+// pass the last-level cache by.  Two 16-byte halves of a chunk per thread and 64-bit indices -> now: 49 million weights 347
+// -> 269 us (5.5 TB/s), 470 million 3633 -> 3246 us (4.3 TB/s).  All of it with the blocks on cache lines: 64 bytes off the
+// line the new form took 293 us, 32 bytes off 3850.
 typedef __attribute__((ext_vector_type(4))) float adamw_f32x4;
 __global__ __launch_bounds__(256) void adamw_packed_kernel(float *__restrict__ master, const float *__restrict__ grad,
                                                            float *__restrict__ mw, float *__restrict__ vw, size_t stride,
