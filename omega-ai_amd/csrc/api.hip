@@ -195,12 +195,12 @@ static void moe_free_backward_workspace(omega_moe *m)
 static void moe_free_workspace(omega_moe *m)
 {
     void *ptrs[] = {m->ids, m->w, m->tile_counts, m->dst, m->dstp, m->src_row, m->tiles, m->xg, m->xs, m->a, m->y,
-                    m->desc_up, m->desc_down, m->wq_up, m->wq_down, m->rms, m->hbuf, m->tokp};
+                    m->desc_up, m->desc_down, m->wq_up, m->wq_down, m->rms, m->hbuf, m->tokp, m->slab_tab};
     for (void *p : ptrs)
         if (p) hipFree(p);
     m->ids = nullptr; m->w = nullptr; m->tile_counts = nullptr; m->dst = nullptr; m->dstp = nullptr; m->src_row = nullptr; m->xs = nullptr; m->desc_up = nullptr; m->desc_down = nullptr; m->wq_up = nullptr; m->wq_down = nullptr; m->rms = nullptr; m->hbuf = nullptr;
-    m->tiles = nullptr; m->xg = nullptr; m->a = nullptr; m->y = nullptr; m->tokp = nullptr;
-    m->xg_valid = false;
+    m->tiles = nullptr; m->xg = nullptr; m->a = nullptr; m->y = nullptr; m->tokp = nullptr; m->slab_tab = nullptr;
+    m->xg_valid = m->y_partial = false;
     m->T_cap = 0;
     moe_free_backward_workspace(m);
     m->fwd_T = -1;
@@ -385,6 +385,7 @@ static int moe_reserve(omega_moe *m, int T)
         OMEGA_HIP_CHECK(ctx, hipMalloc((void **)&m->wq_down, q_down * m->n_wg * sizeof(omega_tile_desc)));
         // partial results of k-sliced items of the down product: sliced entries never exceed 256, each a tile of 256 x 256
         if (!m->y_slabs) OMEGA_HIP_CHECK(ctx, hipMalloc((void **)&m->y_slabs, (size_t)256 * 256 * 256 * 4));
+        OMEGA_HIP_CHECK(ctx, hipMalloc((void **)&m->slab_tab, m->rows_cap / 32 * (c.d / 256) * 4));
         // an all-zero queue is an empty one: the product kernels return at once if no dispatch has run yet
         OMEGA_HIP_CHECK(ctx, hipMemsetAsync(m->wq_up, 0, q_up * m->n_wg * sizeof(omega_tile_desc), ctx->stream));
         OMEGA_HIP_CHECK(ctx, hipMemsetAsync(m->wq_down, 0, q_down * m->n_wg * sizeof(omega_tile_desc), ctx->stream));
@@ -624,10 +625,21 @@ static int stage_router(omega_moe *m, const void *x, int T)
     m->routed_T = T;
     return OMEGA_OK;
 }
+// y with the k slices of its down product added, for whatever reads y other than the combine kernel
+static int ensure_y_whole(omega_moe *m)
+{
+    if (!m->y_partial) return OMEGA_OK;
+    OMEGA_HIP_CHECK(m->ctx, launch_down_slab_reduce(m, m->y, m->ctx->stream));
+    m->y_partial = false;
+    return OMEGA_OK;
+}
 // up_follows: the up product is launched right behind on the same x
 static int stage_dispatch(omega_moe *m, const void *x, int T, bool up_follows = false)
 {
     if (m->routed_T != T) OMEGA_FAIL(m->ctx, OMEGA_ERR_INVALID_ARG, "dispatch: the router has not run for this T");
+    // (the tables that say where the slices of y are get overwritten; in a forward pass y itself follows)
+    if (up_follows) m->y_partial = false;
+    else if (ensure_y_whole(m) != OMEGA_OK) return OMEGA_ERR_HIP;
     m->dispatched_T = -1;
     const int bm = moe_tile_m(m, T);
     m->bm = bm;
@@ -692,14 +704,22 @@ static int stage_experts(omega_moe *m, const void *x, int T, int which)
         OMEGA_HIP_CHECK(m->ctx, launch_product_f32(m, F32_UP, (const float *)x, nullptr, T, m->ctx->stream, gather, keep));
         m->xg_valid = true;
     } else OMEGA_HIP_CHECK(m->ctx, launch_product_f32(m, F32_DOWN, nullptr, nullptr, T, m->ctx->stream));
-    if (which == 0) m->a_valid = true;
-    else m->y_valid = true;
-    return OMEGA_OK;
+    if (which == 0) {
+        m->a_valid = true;
+        return OMEGA_OK;
+    }
+    m->y_valid = true;
+    // (the backward pass behind a training forward reads y)
+    return keeps_for_backward(m, T) ? ensure_y_whole(m) : OMEGA_OK;
 }
 static int stage_combine(omega_moe *m, int T, void *out, const void *resid)
 {
     if (m->dispatched_T != T) OMEGA_FAIL(m->ctx, OMEGA_ERR_INVALID_ARG, "combine: dispatch has not run for this T");
     if (!m->y_valid) OMEGA_FAIL(m->ctx, OMEGA_ERR_INVALID_ARG, "combine: the down product has not run since `y` was overwritten");
+    if (!combine_by_vectors(m, out, resid)) {
+        const int st = ensure_y_whole(m);
+        if (st != OMEGA_OK) return st;
+    }
     OMEGA_HIP_CHECK(m->ctx, launch_combine(m, T, out, resid, m->ctx->stream));
     return OMEGA_OK;
 }
@@ -827,6 +847,7 @@ static int backward_impl(omega_moe *m, const void *x, const void *dout, int T, v
     const void *xin = block ? m->hbuf : x;
     void *dxl = block ? m->bw_dhx : dx;
     if (bf) RUN(ensure_gathered(m, xin, T));
+    RUN(ensure_y_whole(m));
     OMEGA_HIP_CHECK(ctx, bf ? launch_backward_bf16(m, xin, dout, T, dxl, ctx->stream) : launch_backward_f32(m, xin, dout, T, dxl, ctx->stream));
     if (bf) {  // the pass wrote the states of the weight-gradient blocks into the other copy
         m->bw_zero_phase ^= 1;
@@ -859,6 +880,7 @@ int omega_moe_time_backward(omega_moe *m, const void *x, const void *dout, int T
     m->bw_started = m->bw_ran = true;
     const bool bf = m->cfg.dtype == OMEGA_DTYPE_BF16;
     if (bf) RUN(ensure_gathered(m, x, T));
+    RUN(ensure_y_whole(m));
     // A pass of an fp32 layer uses up what a training forward kept (the d(a) product overwrites h1 and h3): it is put back in
     // front of every further one, outside the time, so that each is the pass of a training step.
     const bool put_back = !bf && m->rec_valid;
@@ -1212,6 +1234,7 @@ int omega_moe_get_workspace(omega_moe *m, int which, int T, void *host_dst)
         if (m->dispatched_T != T) OMEGA_FAIL(ctx, OMEGA_ERR_INVALID_ARG, "get_workspace: dispatch has not run for this T");
         RUN(ensure_gathered(m, m->last_x, T));
     }
+    if (which == 2) RUN(ensure_y_whole(m));
     const void *src = which == 0 ? m->xg : which == 1 ? m->a : which == 3 ? m->bw_dh16 : (const void *)m->y;
     const size_t bytes = m->rows_cap * cols * es;
     std::vector<int32_t> meta(G + 2), off(c.E + 1);
@@ -1253,6 +1276,7 @@ int omega_moe_fill_workspace(omega_moe *m, int which, int byte_value)
     stage_invalidates(m);
     if (which == 1) m->a_valid = false;
     m->y_valid = false;
+    if (which == 2) m->y_partial = false;
     OMEGA_HIP_CHECK(ctx, hipMemsetAsync(p, byte_value, bytes, ctx->stream));
     return OMEGA_OK;
 }
@@ -1287,6 +1311,7 @@ int omega_moe_time_stage(omega_moe *m, int stage, const void *x, int T, void *ou
                 OMEGA_HIP_CHECK(ctx, launch_rmsnorm(m, x, T, m->hbuf, ctx->stream));
                 return OMEGA_OK;
             default:
+                m->y_partial = false;  // (y is written again below)
                 RUN(stage_router(m, x, T));
                 RUN(stage_dispatch(m, x, T));
                 RUN(stage_experts(m, x, T, 0));

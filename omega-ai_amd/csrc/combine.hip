@@ -9,18 +9,77 @@
 
 #define MAXK 64
 
-// KU: slots whose rows are fetched together before any of them is used (all loads of a group are in flight at
-// once; slots beyond K re-read the last row and are ignored).
+// The slices of KU rows of y (SL below) added to what the lane holds of them, VEC columns from c0 on.  Lanes whose tile has fewer
+// slices than others' read a row again and drop it: no branch keeps the loads from being in flight together.
+template <int KU, int VEC>
+__device__ __forceinline__ void add_slices(float4 (&v)[KU][VEC / 4], const int (&rows)[KU], int d, int c0, const float *__restrict__ y,
+                                           const float *__restrict__ slabs, const int32_t *__restrict__ slab_tab)
+{
+    const int nct = d >> 8, ct = c0 >> 8;
+    int ent[KU], most = 0;
+#pragma unroll
+    for (int u = 0; u < KU; ++u) ent[u] = slab_tab[(size_t)(rows[u] >> 5) * nct + ct];
+#pragma unroll
+    for (int u = 0; u < KU; ++u) most = max(most, (ent[u] >> 9) & 15);
+    if (__ballot(most > 1) == 0) return;
+    const bool more = __ballot(most > 5) != 0;
+    constexpr int SB = KU <= 4 ? KU : (KU + 1) / 2;  // rows whose slices are in flight together
+#pragma unroll
+    for (int u0 = 0; u0 < KU; u0 += SB) {
+        for (int s0 = 1; s0 < (more ? 8 : 4); s0 += 4) {
+            float4 w[SB][4][VEC / 4];  // slices s0 .. s0 + 3
+#pragma unroll
+            for (int u = 0; u < SB && u0 + u < KU; ++u) {
+                const int e = ent[u0 + u], row = rows[u0 + u], ks = (e >> 9) & 15;
+                const float *tile = slabs + (size_t)(e & 511) * 65536 + (size_t)((e >> 13) * 32 + (row & 31)) * 256 + (c0 & 255);
+#pragma unroll
+                for (int s = 0; s < 4; ++s) {
+                    const float *p = s0 + s < ks ? tile + (size_t)(s0 + s) * 65536 : y + (size_t)row * d + c0;
+#pragma unroll
+                    for (int q = 0; q < VEC / 4; ++q) w[u][s][q] = ((const float4 *)p)[q];
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < SB && u0 + u < KU; ++u) {
+                const int ks = (ent[u0 + u] >> 9) & 15;
+#pragma unroll
+                for (int s = 0; s < 4; ++s)
+                    if (s0 + s < ks) {
+#pragma unroll
+                        for (int q = 0; q < VEC / 4; ++q) {
+                            v[u0 + u][q].x = v[u0 + u][q].x + w[u][s][q].x;
+                            v[u0 + u][q].y = v[u0 + u][q].y + w[u][s][q].y;
+                            v[u0 + u][q].z = v[u0 + u][q].z + w[u][s][q].z;
+                            v[u0 + u][q].w = v[u0 + u][q].w + w[u][s][q].w;
+                        }
+                    }
+            }
+        }
+    }
+}
+
+// KU: slots (and shared experts behind them) whose rows are fetched together before any of them is used (all loads of a
+// group are in flight at once).  Their number is exact up to eight: a row read twice costs what it weighs when y passes the cache
+// by (9978 tokens, a routed and two shared rows each, four reads instead of three: pass 982 -> 998 us; groups of exact size 994 against 1005
+// with the shared rows one after the other).
 // resid != nullptr (block form): the row of x is added to the fp32 sum before the output is rounded
 // (Tensor_OP().add(mlp out, tmp1, tmp2), J/engine/nn/layer/llama/LlamaTransformerBlock.java:136).
 // NT: the rows of y are read with non-temporal loads.  They are read exactly once; when y is larger than the last-level
 // cache (256 MiB) letting them pass it by is worth 13 % (8192 tokens, 64 experts: 0.143 -> 0.125 ms; 16384 tokens, 128
 // experts: 0.260 -> 0.225 ms), below that size nothing.
-template <int VEC, bool BF16, int KU, bool NT>
+// SL: the batch's down product left k slices of some tiles in `slabs` (y_slabs) and `slab_tab` says which: entry [32-row block of
+// the buffer][column tile] = first slice's place | slices << 9 | block within the tile << 13, 0 for a tile that is whole in y.
+// They are added here, to the row of y and in slice order - the sums down_slab_reduce_kernel forms -, while the rows are in
+// registers anyway: a launch and a round trip of y less.  (That kernel is left to what reads y itself: training, backward
+// passes, omega_moe_get_workspace.)  Whole passes, reduce and combine -> combine, d = 4096, H = 14336, 8 experts, top 2, us: 1 token
+// 144.6 -> 142.5, 64 tokens 488 -> 484, 777 tokens (block form; 2 slices of every tile) 639 -> 625, 4096 tokens (4 of the last 64)
+// 2240 -> 2230.
+template <int VEC, bool BF16, int KU, bool NT, bool SL>
 __global__ __launch_bounds__(256) void combine_kernel(const float *__restrict__ y, const int32_t *__restrict__ dst,
                                                       const float *__restrict__ w, int T, int K, int d, int Es,
                                                       const int32_t *__restrict__ tile_meta, int E, int bm,
-                                                      const void *__restrict__ resid, void *__restrict__ out, int split)
+                                                      const void *__restrict__ resid, void *__restrict__ out, int split,
+                                                      const float *__restrict__ slabs, const int32_t *__restrict__ slab_tab)
 {
     // `split` waves share a token, each taking d / split consecutive columns (more waves, more loads in flight, when
     // the batch has few tokens for the compute units there are)
@@ -29,27 +88,32 @@ __global__ __launch_bounds__(256) void combine_kernel(const float *__restrict__ 
     const int t = wv / split, part = wv - t * split;
     if (t >= T) return;
     const int dc = d / split;
-    // lane j < K holds row index and weight of slot j; broadcast through cross-lane reads
-    int myrow = 0;
+    // lane j < K holds row index and weight of slot j, lane j < Es the row of shared expert j; handed out by lane reads
+    int myrow = 0, shrow = 0;
     float myw = 0.0f;
     if (lane < K) {
         myrow = dst[(size_t)t * K + lane];
         myw = w[(size_t)t * K + lane];
     }
-    // every lane makes every trip (lanes past the row's end work on column 0 and store nothing): the cross-lane reads
-    // of the slot rows and weights below must find their source lanes active
+    if (lane < Es) shrow = tile_meta[1 + E + lane] * bm + t;
+    const bool sliced = SL && tile_meta[E + Es + 9] > 0;  // (the host knows bounds of the number of tiles only)
+    const int n = K + Es;
+    // (lanes past the row's end work on column 0 and store nothing)
     for (int cb = part * dc; cb < (part + 1) * dc; cb += 64 * VEC) {
         const bool on = cb + lane * VEC < (part + 1) * dc;
         const int c0 = on ? cb + lane * VEC : 0;
         float acc[VEC];
 #pragma unroll
         for (int v = 0; v < VEC; ++v) acc[v] = 0.0f;
-        for (int j0 = 0; j0 < K; j0 += KU) {
+        // the rows of the slots, then those of the shared experts, KU at a time
+        for (int j0 = 0; j0 < n; j0 += KU) {
             float4 buf[KU][VEC / 4];
+            int rows[KU];
 #pragma unroll
             for (int u = 0; u < KU; ++u) {
-                const int row = __shfl(myrow, min(j0 + u, K - 1), 64);
-                const float4 *src = (const float4 *)(y + (size_t)row * d + c0);
+                const int j = min(j0 + u, n - 1);  // (a last group with a row too few reads that of the last again)
+                rows[u] = j < K ? __builtin_amdgcn_readlane(myrow, j) : __builtin_amdgcn_readlane(shrow, j - K);
+                const float4 *src = (const float4 *)(y + (size_t)rows[u] * d + c0);
 #pragma unroll
                 for (int q = 0; q < VEC / 4; ++q) {
                     if (NT) {
@@ -61,10 +125,11 @@ __global__ __launch_bounds__(256) void combine_kernel(const float *__restrict__ 
                     }
                 }
             }
+            if (SL && sliced) add_slices<KU, VEC>(buf, rows, d, c0, y, slabs, slab_tab);
 #pragma unroll
             for (int u = 0; u < KU; ++u) {
                 if (j0 + u < K) {
-                    const float wj = __shfl(myw, j0 + u, 64);
+                    const float wj = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(myw), j0 + u));
 #pragma unroll
                     for (int q = 0; q < VEC / 4; ++q) {
                         const float4 v4 = buf[u][q];
@@ -74,18 +139,16 @@ __global__ __launch_bounds__(256) void combine_kernel(const float *__restrict__ 
                         term = wj * v4.z; acc[q * 4 + 2] = acc[q * 4 + 2] + term;
                         term = wj * v4.w; acc[q * 4 + 3] = acc[q * 4 + 3] + term;
                     }
-                }
-            }
-        }
-        for (int s = 0; s < Es; ++s) {
-            const float4 *src = (const float4 *)(y + ((size_t)tile_meta[1 + E + s] * bm + t) * d + c0);
+                } else if (j0 + u < n) {
 #pragma unroll
-            for (int q = 0; q < VEC / 4; ++q) {
-                const float4 v4 = src[q];
-                acc[q * 4 + 0] = acc[q * 4 + 0] + v4.x;
-                acc[q * 4 + 1] = acc[q * 4 + 1] + v4.y;
-                acc[q * 4 + 2] = acc[q * 4 + 2] + v4.z;
-                acc[q * 4 + 3] = acc[q * 4 + 3] + v4.w;
+                    for (int q = 0; q < VEC / 4; ++q) {
+                        const float4 v4 = buf[u][q];
+                        acc[q * 4 + 0] = acc[q * 4 + 0] + v4.x;
+                        acc[q * 4 + 1] = acc[q * 4 + 1] + v4.y;
+                        acc[q * 4 + 2] = acc[q * 4 + 2] + v4.z;
+                        acc[q * 4 + 3] = acc[q * 4 + 3] + v4.w;
+                    }
+                }
             }
         }
         if (resid != nullptr) {
@@ -139,37 +202,52 @@ __global__ __launch_bounds__(256) void combine_scalar_kernel(const float *__rest
     }
 }
 
+// 16-byte loads and stores (the only form that adds the k slices of a down product)
+bool combine_by_vectors(const omega_moe *m, const void *out, const void *resid)
+{
+    const int vec = m->cfg.dtype == OMEGA_DTYPE_BF16 ? 8 : 4;
+    return m->cfg.d % vec == 0 && (((uintptr_t)out | (uintptr_t)resid) % 16) == 0 && m->cfg.K <= MAXK;
+}
+
 hipError_t launch_combine(const omega_moe *m, int T, void *out, const void *resid, hipStream_t s)
 {
     const omega_moe_config &c = m->cfg;
     const bool bf = c.dtype == OMEGA_DTYPE_BF16;
     const int vec = bf ? 8 : 4;
-    if (c.d % vec == 0 && (((uintptr_t)out | (uintptr_t)resid) % 16) == 0 && c.K <= MAXK) {
+    if (combine_by_vectors(m, out, resid)) {
         const bool nt = (size_t)T * (c.K + c.Es) * c.d * 4 > OMEGA_LLC_BYTES;
         // several waves per token, each with a share of the columns, until the launch has 256 waves per compute unit:
         // more loads in flight (4096 tokens x 4096 columns: 36.3 -> 30.6 us with 8 waves per token; 64 tokens:
         // 12.0 -> 6.9 us; 8192 tokens x 2048 columns x 8 rows: 122.6 -> 113.8 us with 4; 16384 tokens: 228 -> 210 us)
         int split = 1;
         while (split < 8 && (long long)T * split < 256LL * m->ctx->num_cus && c.d % (64 * vec * split * 2) == 0) split *= 2;
-#define COMBINE_LAUNCH2(KUV, NTV)                                                                                      \
-    do {                                                                                                              \
-        if (bf)                                                                                                       \
-            hipLaunchKernelGGL((combine_kernel<8, true, KUV, NTV>), dim3(ceil_div(T * split, 4)), dim3(256), 0, s, m->y, m->dstp, m->w, \
-                               T, c.K, c.d, c.Es, m->tile_meta, c.E, m->bm, resid, out, split);                              \
-        else                                                                                                          \
-            hipLaunchKernelGGL((combine_kernel<4, false, KUV, NTV>), dim3(ceil_div(T * split, 4)), dim3(256), 0, s, m->y, m->dstp, \
-                               m->w, T, c.K, c.d, c.Es, m->tile_meta, c.E, m->bm, resid, out, split);                        \
+        const bool sl = m->y_partial;
+        const int n = c.K + c.Es, ku = ceil_div(n, ceil_div(n, 8));  // rows of a token in groups of one size, eight at most
+        const int grid = ceil_div(T * split, 4);
+#define COMBINE_LAUNCH(VECV, BFV, KUV, NTV, SLV)                                                                                       \
+    hipLaunchKernelGGL((combine_kernel<VECV, BFV, KUV, NTV, SLV>), dim3(grid), dim3(256), 0, s, m->y, m->dstp, m->w, T, c.K, c.d, c.Es, \
+                       m->tile_meta, c.E, m->bm, resid, out, split, m->y_slabs, m->slab_tab)
+#define COMBINE_SLOTS(VECV, BFV, NTV, SLV)                  \
+    do {                                                     \
+        switch (ku) {                                        \
+        case 1: COMBINE_LAUNCH(VECV, BFV, 1, NTV, SLV); break; \
+        case 2: COMBINE_LAUNCH(VECV, BFV, 2, NTV, SLV); break; \
+        case 3: COMBINE_LAUNCH(VECV, BFV, 3, NTV, SLV); break; \
+        case 4: COMBINE_LAUNCH(VECV, BFV, 4, NTV, SLV); break; \
+        case 5: COMBINE_LAUNCH(VECV, BFV, 5, NTV, SLV); break; \
+        case 6: COMBINE_LAUNCH(VECV, BFV, 6, NTV, SLV); break; \
+        case 7: COMBINE_LAUNCH(VECV, BFV, 7, NTV, SLV); break; \
+        default: COMBINE_LAUNCH(VECV, BFV, 8, NTV, SLV);      \
+        }                                                    \
     } while (0)
-#define COMBINE_LAUNCH(KUV)              \
-    do {                                 \
-        if (nt) COMBINE_LAUNCH2(KUV, true); \
-        else COMBINE_LAUNCH2(KUV, false);   \
-    } while (0)
-        if (c.K <= 2) COMBINE_LAUNCH(2);
-        else if (c.K <= 4) COMBINE_LAUNCH(4);
-        else COMBINE_LAUNCH(8);
+        if (sl && nt) COMBINE_SLOTS(8, true, true, true);
+        else if (sl) COMBINE_SLOTS(8, true, false, true);
+        else if (bf && nt) COMBINE_SLOTS(8, true, true, false);
+        else if (bf) COMBINE_SLOTS(8, true, false, false);
+        else if (nt) COMBINE_SLOTS(4, false, true, false);
+        else COMBINE_SLOTS(4, false, false, false);
+#undef COMBINE_SLOTS
 #undef COMBINE_LAUNCH
-#undef COMBINE_LAUNCH2
     } else {
         if (bf)
             hipLaunchKernelGGL(combine_scalar_kernel<true>, dim3(T), dim3(256), 0, s, m->y, m->dstp, m->w, T, c.K, c.d,

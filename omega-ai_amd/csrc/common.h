@@ -98,6 +98,10 @@ struct omega_moe {
     int down_cols = 256;
     int down_ks_max = 1;             // > 1: the down table of this batch may hold k slices of every tile (small batches)
     int down_tail_ks = 1;            // > 1: the last tiles of the down table may be cut into up to this many k slices
+    // the down product of the batch in y has left k slices in y_slabs that are not in y: the combine kernel adds them on its
+    // way (combine.hip), whatever else reads y has them added first (ensure_y_whole)
+    bool y_partial = false;
+    int32_t *slab_tab = nullptr;     // which tiles those are: [32-row block of y][column tile of 256] (combine.hip describes an entry)
     float *y_slabs = nullptr;        // partial results of the k slices: 256 tiles of 256 x 256 floats, one per sliced entry
     void *xg = nullptr;              // [rows_cap,d]  gathered tokens (bf16: packed tile image, see pack.h)
     void *xs = nullptr;              // bf16 with shared experts: packed copy of x, [ceil(T/bm)*bm,d]
@@ -203,8 +207,9 @@ enum { F32_UP = 0, F32_DOWN, F32_RAW, F32_DA, F32_DXG, F32_WG2, F32_WG13 };
 // bw_h1 / bw_h3, as launch_experts_bf16 does)
 hipError_t launch_product_f32(const omega_moe *m, int op, const float *x, const float *dout, int T, hipStream_t s, bool gather = false,
                               bool keep = false);
-hipError_t launch_experts_bf16(const omega_moe *m, const void *x, int T, int which, hipStream_t s, bool keep);
+hipError_t launch_experts_bf16(omega_moe *m, const void *x, int T, int which, hipStream_t s, bool keep);
 // resid != nullptr: out = resid + layer output (one rounding of the fp32 sum)
+bool combine_by_vectors(const omega_moe *m, const void *out, const void *resid);
 hipError_t launch_combine(const omega_moe *m, int T, void *out, const void *resid, hipStream_t s);
 hipError_t launch_backward_f32(omega_moe *m, const void *x, const void *dout, int T, void *dx, hipStream_t s);
 hipError_t launch_backward_bf16(const omega_moe *m, const void *x, const void *dout, int T, void *dx, hipStream_t s);

@@ -435,7 +435,7 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8, 8))) vo
                                                             omega_tile_desc *__restrict__ wq_down, int n_wg,
                                                             const unsigned char *__restrict__ x, int d,
                                                             unsigned char *__restrict__ xg, unsigned char *__restrict__ xs,
-                                                            int nt_stores, int n_sched)
+                                                            int nt_stores, int n_sched, int32_t *__restrict__ slab_tab)
 {
     __shared__ int off_s[MAXE + 1];        // logical first row of each expert
     __shared__ int mt_s[MAXE + 64 + 1];    // first row tile of each group (routed, then shared)
@@ -699,8 +699,14 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8, 8))) vo
             for (int ent = tile * nthr + tid; ent < tsu.entries(); ent += n_tiles * nthr)
                 desc_up[ent] = item_desc(ent, tpu, tsu, mt_s, off_s, E, G, T, bm);
         if (desc_down != nullptr)
-            for (int ent = tile * nthr + tid; ent < tsd.entries(); ent += n_tiles * nthr)
-                desc_down[ent] = item_desc(ent, tpd, tsd, mt_s, off_s, E, G, T, bm);
+            for (int ent = tile * nthr + tid; ent < tsd.entries(); ent += n_tiles * nthr) {
+                const omega_tile_desc e = item_desc(ent, tpd, tsd, mt_s, off_s, E, G, T, bm);
+                desc_down[ent] = e;
+                // where the combine kernel finds the k slices of a tile (combine.hip): slice 0 speaks for all of them
+                if (slab_tab != nullptr && !(e.a_rg > 1 && e.kt0 > 0))
+                    for (int b = 0; 32 * b < e.rows; ++b)
+                        slab_tab[(size_t)((e.row0 >> 5) + b) * nt_down + (e.n0 >> 8)] = e.a_rg > 1 ? e.xrow0 | e.a_rg << 9 | b << 13 : 0;
+            }
     }
 
     // ---- row copies (bf16 layers whose up product reads a gathered copy) ----
@@ -783,7 +789,8 @@ hipError_t launch_dispatch_index(const omega_moe *m, int T, int bm, hipStream_t 
                        n_tiles, T, tok_tile, c.K, c.E, c.Es, bm, m->offsets, m->dst, m->dstp, m->src_row, m->tokp, m->tiles,
                        m->tile_meta, m->desc_up, c.H / 128, 128, m->desc_down, c.d / m->down_cols, m->down_cols,
                        m->down_ks_max, c.H / 32, m->down_tail_ks, m->wq_up, m->wq_down, m->n_wg, (const unsigned char *)x, c.d,
-                       (unsigned char *)(rows ? m->xg : nullptr), (unsigned char *)(rows ? m->xs : nullptr), nt_stores, n_sched);
+                       (unsigned char *)(rows ? m->xg : nullptr), (unsigned char *)(rows ? m->xs : nullptr), nt_stores, n_sched,
+                       m->down_ks_max > 1 || m->down_tail_ks > 1 ? m->slab_tab : nullptr);
     return hipGetLastError();
 }
 

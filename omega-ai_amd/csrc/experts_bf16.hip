@@ -1152,7 +1152,7 @@ hipError_t experts_bf16_init(void)
     return hipSuccess;
 }
 
-hipError_t launch_experts_bf16(const omega_moe *m, const void *x, int T, int which, hipStream_t s, bool keep)
+hipError_t launch_experts_bf16(omega_moe *m, const void *x, int T, int which, hipStream_t s, bool keep)
 {
     const omega_moe_config &c = m->cfg;
     // the ring must be shorter than an item: K >= (NSTAGE + 1) * BK (guaranteed at creation: d, H >= 256)
@@ -1183,7 +1183,7 @@ hipError_t launch_experts_bf16(const omega_moe *m, const void *x, int T, int whi
 #undef UP4_LAUNCH
     } else {
         // the table may hold k slices (every tile of a small batch, or the last tiles of a large one): their partial
-        // results go to y_slabs and are added into y right behind the product
+        // results go to y_slabs, for the combine kernel or down_slab_reduce_kernel to add (omega_moe::y_partial)
         void *slabs = (m->down_ks_max > 1 || m->down_tail_ks > 1) ? (void *)m->y_slabs : nullptr;
         if (m->down_cols == 256) {
             // full-width items: one wave per SIMD (experts_up4_kernel, DOWN)
@@ -1203,11 +1203,7 @@ hipError_t launch_experts_bf16(const omega_moe *m, const void *x, int T, int whi
             hipLaunchKernelGGL(experts_bf16_kernel<MODE_DOWN>, dim3(m->n_wg), dim3(NWAVES * 64), SMEM_BYTES, s, (const bf16_t *)m->a,
                                (const bf16_t *)nullptr, (const bf16_t *)m->W2, (const bf16_t *)nullptr, (void *)m->y,
                                slabs, (void *)nullptr, m->wq_down, c.d, c.H);
-        if (slabs != nullptr) {
-            hipError_t e = hipGetLastError();
-            if (e != hipSuccess) return e;
-            return launch_down_slab_reduce(m, m->y, s);
-        }
+        m->y_partial = slabs != nullptr;
     }
     return hipGetLastError();
 }

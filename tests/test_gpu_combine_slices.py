@@ -1,0 +1,47 @@
+"""The k slices of a down product that the combine kernel adds: the bits of the kernel that adds them into y, every tile sliced, the
+last tiles only, none, with shared experts, and behind an output that only the element-wise combine can write."""
+import numpy as np
+import pytest
+
+from oracle import oracle_np as N
+from tests.synth import C, scaled
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("kw", [
+    dict(T=70, d=512, H=1024, E=4, K=2, Es=0),      # 4 slices of every tile
+    dict(T=90, d=768, H=4096, E=3, K=3, Es=2),      # 8 slices, shared experts
+    dict(T=300, d=1024, H=640, E=7, K=7, Es=1),     # 2 slices, two row tiles per expert
+    dict(T=4400, d=4096, H=4096, E=1, K=1, Es=0),   # the last tiles only: 18 x 16 tiles, 32 of them in 2 slices
+    dict(T=1100, d=256, H=256, E=4, K=1, Es=0),     # room for slices, and none made
+], ids=lambda k: "-".join(str(v) for v in k.values()))
+def test_combine_adds_the_k_slices(kw):
+    """The sums the combine kernel forms from y and the slices are those of the kernel that adds them into y: the same bits."""
+    from tests import gpu_util as G
+    cfg = scaled(C.CONFIGS["c4_finegrained"], **kw)
+    layer = G.P.MoELayer(cfg.d, cfg.H, cfg.E, cfg.K, renorm=cfg.renorm, nShared=cfg.Es, bias=False, ctx=G.ctx(), dtype="bf16")
+    layer.init_synthetic(13, C, cfg)
+    x = G.P.DeviceBuffer(G.ctx(), (cfg.T, cfg.d), "bf16")
+    x.fill_normal(13, C.STREAM_X, 1.0)
+    out = layer.forward(x).to_numpy()
+    y = layer.workspace("y", cfg.T)             # adds the slices into y
+    o = G.P.DeviceBuffer(G.ctx(), (cfg.T * cfg.d + 8,), "bf16")
+    layer.ctx.check(layer.lib.omega_moe_combine(layer.handle, cfg.T, o.ptr))
+    assert np.array_equal(o.to_numpy()[:cfg.T * cfg.d].reshape(cfg.T, cfg.d), out)
+    assert np.array_equal(layer.workspace("y", cfg.T), y)
+    # an output off the 16-byte boundary: the element-wise combine needs y whole
+    layer.ctx.check(layer.lib.omega_moe_forward(layer.handle, x.ptr, cfg.T, o.ptr.value + 2))
+    assert np.array_equal(o.to_numpy()[1:cfg.T * cfg.d + 1].reshape(cfg.T, cfg.d), out)
+    # rows by the definition, from the layer's own y
+    r = layer.routing()
+    t = np.arange(0, cfg.T, max(1, cfg.T // 16))
+    ref = np.zeros((len(t), cfg.d))
+    for j in range(cfg.K):
+        ref += r["w"][t, j, None].astype(np.float64) * y[r["dst"].reshape(cfg.T, cfg.K)[t, j]]
+    for s in range(cfg.Es):
+        ref += y[cfg.T * cfg.K + s * cfg.T + t]
+    assert N.rel_l2(out[t], ref) <= 4e-3        # one rounding to bf16: at most 2^-9 of an element
+    for b in (o, x):
+        b.free()
+    layer.close()
