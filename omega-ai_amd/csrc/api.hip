@@ -629,7 +629,7 @@ static int stage_router(omega_moe *m, const void *x, int T)
 static int ensure_y_whole(omega_moe *m)
 {
     if (!m->y_partial) return OMEGA_OK;
-    OMEGA_HIP_CHECK(m->ctx, launch_down_slab_reduce(m, m->y, m->ctx->stream));
+    OMEGA_HIP_CHECK(m->ctx, launch_experts_bf16(m, nullptr, 0, 2, m->ctx->stream, false));
     m->y_partial = false;
     return OMEGA_OK;
 }
@@ -709,6 +709,7 @@ static int stage_experts(omega_moe *m, const void *x, int T, int which)
         return OMEGA_OK;
     }
     m->y_valid = true;
+    m->y_partial = m->cfg.dtype == OMEGA_DTYPE_BF16 && (m->down_ks_max > 1 || m->down_tail_ks > 1);
     // (the backward pass behind a training forward reads y)
     return keeps_for_backward(m, T) ? ensure_y_whole(m) : OMEGA_OK;
 }

@@ -7,8 +7,6 @@
 // (J/engine/ad/op/gpu/OPKernel.cu:359-366).  No atomics: every output element has one writer.
 #include "common.h"
 
-#define MAXK 64
-
 // The slices of KU rows of y (SL below) added to what the lane holds of them, VEC columns from c0 on.  Lanes whose tile has fewer
 // slices than others' read a row again and drop it: no branch keeps the loads from being in flight together.
 template <int KU, int VEC>
@@ -200,13 +198,6 @@ __global__ __launch_bounds__(256) void combine_scalar_kernel(const float *__rest
         if (BF16) ((bf16_t *)out)[(size_t)t * d + c] = f32_to_bf16(acc);
         else ((float *)out)[(size_t)t * d + c] = acc;
     }
-}
-
-// 16-byte loads and stores (the only form that adds the k slices of a down product)
-bool combine_by_vectors(const omega_moe *m, const void *out, const void *resid)
-{
-    const int vec = m->cfg.dtype == OMEGA_DTYPE_BF16 ? 8 : 4;
-    return m->cfg.d % vec == 0 && (((uintptr_t)out | (uintptr_t)resid) % 16) == 0 && m->cfg.K <= MAXK;
 }
 
 hipError_t launch_combine(const omega_moe *m, int T, void *out, const void *resid, hipStream_t s)

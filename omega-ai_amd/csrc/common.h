@@ -168,6 +168,14 @@ struct omega_moe {
     size_t prof_used = 0;
 };
 
+// Whether the combine kernel takes 16-byte loads and stores (the only form that adds the k slices of a down product)
+#define COMBINE_MAXK 64
+static inline bool combine_by_vectors(const omega_moe *m, const void *out, const void *resid)
+{
+    const int vec = m->cfg.dtype == OMEGA_DTYPE_BF16 ? 8 : 4;
+    return m->cfg.d % vec == 0 && (((uintptr_t)out | (uintptr_t)resid) % 16) == 0 && m->cfg.K <= COMBINE_MAXK;
+}
+
 // Tokens per router workgroup = per row of tile_counts and per workgroup of the dispatch kernel: 16 for layers with at most
 // 16 experts and for exact bf16 layers with more while such tiles find a compute unit each, else 32 (router.hip).
 int router_tok_tile(const omega_moe *m, int T);
@@ -207,9 +215,9 @@ enum { F32_UP = 0, F32_DOWN, F32_RAW, F32_DA, F32_DXG, F32_WG2, F32_WG13 };
 // bw_h1 / bw_h3, as launch_experts_bf16 does)
 hipError_t launch_product_f32(const omega_moe *m, int op, const float *x, const float *dout, int T, hipStream_t s, bool gather = false,
                               bool keep = false);
-hipError_t launch_experts_bf16(omega_moe *m, const void *x, int T, int which, hipStream_t s, bool keep);
+// which: 0 up product, 1 down product, 2 the k slices the down product has left (y_partial) added into y
+hipError_t launch_experts_bf16(const omega_moe *m, const void *x, int T, int which, hipStream_t s, bool keep);
 // resid != nullptr: out = resid + layer output (one rounding of the fp32 sum)
-bool combine_by_vectors(const omega_moe *m, const void *out, const void *resid);
 hipError_t launch_combine(const omega_moe *m, int T, void *out, const void *resid, hipStream_t s);
 hipError_t launch_backward_f32(omega_moe *m, const void *x, const void *dout, int T, void *dx, hipStream_t s);
 hipError_t launch_backward_bf16(const omega_moe *m, const void *x, const void *dout, int T, void *dx, hipStream_t s);

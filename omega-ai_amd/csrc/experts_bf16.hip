@@ -1152,9 +1152,10 @@ hipError_t experts_bf16_init(void)
     return hipSuccess;
 }
 
-hipError_t launch_experts_bf16(omega_moe *m, const void *x, int T, int which, hipStream_t s, bool keep)
+hipError_t launch_experts_bf16(const omega_moe *m, const void *x, int T, int which, hipStream_t s, bool keep)
 {
     const omega_moe_config &c = m->cfg;
+    if (which == 2) return launch_down_slab_reduce(m, m->y, s);
     // the ring must be shorter than an item: K >= (NSTAGE + 1) * BK (guaranteed at creation: d, H >= 256)
     if ((which == 0 ? c.d : c.H) < (NSTAGE + 1) * BK) return hipErrorInvalidValue;
     // A batch with at most 64 rows per routed expert on average streams every weight tile once (one row tile per
@@ -1203,7 +1204,6 @@ hipError_t launch_experts_bf16(omega_moe *m, const void *x, int T, int which, hi
             hipLaunchKernelGGL(experts_bf16_kernel<MODE_DOWN>, dim3(m->n_wg), dim3(NWAVES * 64), SMEM_BYTES, s, (const bf16_t *)m->a,
                                (const bf16_t *)nullptr, (const bf16_t *)m->W2, (const bf16_t *)nullptr, (void *)m->y,
                                slabs, (void *)nullptr, m->wq_down, c.d, c.H);
-        m->y_partial = slabs != nullptr;
     }
     return hipGetLastError();
 }
