@@ -625,6 +625,15 @@ static int stage_router(omega_moe *m, const void *x, int T)
     m->routed_T = T;
     return OMEGA_OK;
 }
+// the work queues of the batch the dispatch stage last ran for (a backward pass), if its forward pass went without them: the same
+// launch from the same routing
+static int ensure_queues(omega_moe *m, int T)
+{
+    if (!m->few) return OMEGA_OK;
+    m->few = false;
+    OMEGA_HIP_CHECK(m->ctx, launch_dispatch_index(m, T, m->bm, m->ctx->stream, nullptr));
+    return OMEGA_OK;
+}
 // y with the k slices of its down product added, for whatever reads y other than the combine kernel
 static int ensure_y_whole(omega_moe *m)
 {
@@ -672,9 +681,11 @@ static int stage_dispatch(omega_moe *m, const void *x, int T, bool up_follows = 
     // (bf16 layers: the index launch copies the rows as well; fp32 layers gather in a launch of its own, or leave it to the
     // up product that follows, which fetches its rows from x and writes the gathered copy beside: a launch less, 4 of 35 us at
     // 256 tokens x 128 columns)
+    // (a few tokens, bf16: the products need neither queues nor, when they follow, a gathered copy; they leave it as fp32 layers' do)
     const bool bf = m->cfg.dtype == OMEGA_DTYPE_BF16;
-    OMEGA_HIP_CHECK(m->ctx, launch_dispatch_index(m, T, bm, m->ctx->stream, bf && !m->gather_on_load ? x : nullptr));
-    const bool up_gathers = !bf && up_follows && (double)T * m->cfg.d * 4.0 < 4.0e9;
+    m->few = up_follows && !m->training && experts_few_rows(m, T);
+    const bool up_gathers = up_follows && (m->few || (!bf && (double)T * m->cfg.d * 4.0 < 4.0e9));
+    OMEGA_HIP_CHECK(m->ctx, launch_dispatch_index(m, T, bm, m->ctx->stream, bf && !m->gather_on_load && !up_gathers ? x : nullptr));
     if (!bf && !up_gathers) OMEGA_HIP_CHECK(m->ctx, launch_dispatch_gather(m, x, T, m->ctx->stream));
     m->xg_valid = !m->gather_on_load && !up_gathers;
     m->dispatched_T = T;
@@ -697,8 +708,11 @@ static int stage_experts(omega_moe *m, const void *x, int T, int which)
     if (which == 0 && m->gather_on_load && !x) OMEGA_FAIL(m->ctx, OMEGA_ERR_INVALID_ARG, "experts: x is NULL");
     if (which == 1 && !m->a_valid) OMEGA_FAIL(m->ctx, OMEGA_ERR_INVALID_ARG, "experts_down: the up product has not run since `a` was overwritten");
     const bool keep = which == 0 && keeps_for_backward(m, T);
-    if (m->cfg.dtype == OMEGA_DTYPE_BF16) OMEGA_HIP_CHECK(m->ctx, launch_experts_bf16(m, x, T, which, m->ctx->stream, keep));
-    else if (which == 0) {
+    if (m->cfg.dtype == OMEGA_DTYPE_BF16) {
+        if (which == 0 && m->few && !m->xg_valid && !x) OMEGA_FAIL(m->ctx, OMEGA_ERR_INVALID_ARG, "experts: x is NULL");
+        OMEGA_HIP_CHECK(m->ctx, launch_experts_bf16(m, x, T, which, m->ctx->stream, keep));
+        if (which == 0 && m->few && !m->gather_on_load) m->xg_valid = true;
+    } else if (which == 0) {
         const bool gather = !m->xg_valid;
         if (gather && !x) OMEGA_FAIL(m->ctx, OMEGA_ERR_INVALID_ARG, "experts: x is NULL");
         OMEGA_HIP_CHECK(m->ctx, launch_product_f32(m, F32_UP, (const float *)x, nullptr, T, m->ctx->stream, gather, keep));
@@ -709,7 +723,7 @@ static int stage_experts(omega_moe *m, const void *x, int T, int which)
         return OMEGA_OK;
     }
     m->y_valid = true;
-    m->y_partial = m->cfg.dtype == OMEGA_DTYPE_BF16 && (m->down_ks_max > 1 || m->down_tail_ks > 1);
+    m->y_partial = m->cfg.dtype == OMEGA_DTYPE_BF16 && !m->few && (m->down_ks_max > 1 || m->down_tail_ks > 1);
     // (the backward pass behind a training forward reads y)
     return keeps_for_backward(m, T) ? ensure_y_whole(m) : OMEGA_OK;
 }
@@ -847,7 +861,10 @@ static int backward_impl(omega_moe *m, const void *x, const void *dout, int T, v
     // and meets the gradient of the residual branch
     const void *xin = block ? m->hbuf : x;
     void *dxl = block ? m->bw_dhx : dx;
-    if (bf) RUN(ensure_gathered(m, xin, T));
+    if (bf) {
+        RUN(ensure_gathered(m, xin, T));
+        RUN(ensure_queues(m, T));
+    }
     RUN(ensure_y_whole(m));
     OMEGA_HIP_CHECK(ctx, bf ? launch_backward_bf16(m, xin, dout, T, dxl, ctx->stream) : launch_backward_f32(m, xin, dout, T, dxl, ctx->stream));
     if (bf) {  // the pass wrote the states of the weight-gradient blocks into the other copy
@@ -880,7 +897,10 @@ int omega_moe_time_backward(omega_moe *m, const void *x, const void *dout, int T
     RUN(moe_reserve_backward(m, T));
     m->bw_started = m->bw_ran = true;
     const bool bf = m->cfg.dtype == OMEGA_DTYPE_BF16;
-    if (bf) RUN(ensure_gathered(m, x, T));
+    if (bf) {
+        RUN(ensure_gathered(m, x, T));
+        RUN(ensure_queues(m, T));
+    }
     RUN(ensure_y_whole(m));
     // A pass of an fp32 layer uses up what a training forward kept (the d(a) product overwrites h1 and h3): it is put back in
     // front of every further one, outside the time, so that each is the pass of a training step.

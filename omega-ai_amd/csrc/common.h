@@ -98,6 +98,9 @@ struct omega_moe {
     int down_cols = 256;
     int down_ks_max = 1;             // > 1: the down table of this batch may hold k slices of every tile (small batches)
     int down_tail_ks = 1;            // > 1: the last tiles of the down table may be cut into up to this many k slices
+    // the batch is one of a few tokens in a forward pass: its products run on experts_few.hip and its dispatch made no work queues
+    // (what needs them has them made first: ensure_queues)
+    bool few = false;
     // the down product of the batch in y has left k slices in y_slabs that are not in y: the combine kernel adds them on its
     // way (combine.hip), whatever else reads y has them added first (ensure_y_whole)
     bool y_partial = false;
@@ -176,6 +179,11 @@ static inline bool combine_by_vectors(const omega_moe *m, const void *out, const
     return m->cfg.d % vec == 0 && (((uintptr_t)out | (uintptr_t)resid) % 16) == 0 && m->cfg.K <= COMBINE_MAXK;
 }
 
+// Batches whose forward products run on experts_few.hip: up to 64 tokens, four units of 16 rows.  Beyond, the rows' fragments,
+// which every workgroup there reads for 16 or 32 columns only, weigh as much as the weights.  80 / 128 tokens x 4096 x 14336, 8 experts,
+// pass, us, tile kernels / there: 485 / 485, 514 / 560; 80 / 192 tokens x 2048 x 1408, 64 experts: 241 / 231, 253 / 257.
+static inline bool experts_few_rows(const omega_moe *m, int T) { return m->cfg.dtype == OMEGA_DTYPE_BF16 && T <= 64; }
+
 // Tokens per router workgroup = per row of tile_counts and per workgroup of the dispatch kernel: 16 for layers with at most
 // 16 experts and for exact bf16 layers with more while such tiles find a compute unit each, else 32 (router.hip).
 int router_tok_tile(const omega_moe *m, int T);
@@ -217,6 +225,7 @@ hipError_t launch_product_f32(const omega_moe *m, int op, const float *x, const 
                               bool keep = false);
 // which: 0 up product, 1 down product, 2 the k slices the down product has left (y_partial) added into y
 hipError_t launch_experts_bf16(const omega_moe *m, const void *x, int T, int which, hipStream_t s, bool keep);
+hipError_t launch_experts_few(const omega_moe *m, const void *x, int T, int which, hipStream_t s);
 // resid != nullptr: out = resid + layer output (one rounding of the fp32 sum)
 hipError_t launch_combine(const omega_moe *m, int T, void *out, const void *resid, hipStream_t s);
 hipError_t launch_backward_f32(omega_moe *m, const void *x, const void *dout, int T, void *dx, hipStream_t s);

@@ -666,11 +666,11 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8, 8))) vo
         if (tid == 0) tile_meta[0] = mt_s[G];
         for (int g = tid; g <= G; g += nthr) tile_meta[1 + g] = mt_s[g];
     }
-    // row-tile list: group g is written by workgroup g (mod grid), like the work-item tables below
-    for (int g = tile; g < G; g += gridDim.x) {
+    // row-tile list: eight lanes per group
+    for (int g = (tile * nthr + tid) >> 3; g < G; g += (n_tiles * nthr) >> 3) {
         const int rows = g < E ? off_s[g + 1] - off_s[g] : T;
         const int nm = mt_s[g + 1] - mt_s[g];
-        for (int mt = tid; mt < nm; mt += nthr) {
+        for (int mt = tid & 7; mt < nm; mt += 8) {
             omega_tile tl;
             tl.g = g;
             tl.row0 = (mt_s[g] + mt) * bm;
@@ -784,10 +784,11 @@ hipError_t launch_dispatch_index(const omega_moe *m, int T, int bm, hipStream_t 
     const int nt_stores = (size_t)T * c.K * c.d * 2 > OMEGA_LLC_BYTES / 2 ? 1 : 0;
     const int tok_tile = router_tok_tile(m, T);
     const int n_tiles = ceil_div(T, tok_tile);
-    const int n_sched = m->desc_up != nullptr ? SCHED_WGS : 0;  // bf16 layers
+    const bool queues = m->desc_up != nullptr && !m->few;  // bf16 layers, unless their products go without
+    const int n_sched = queues ? SCHED_WGS : 0;
     hipLaunchKernelGGL(dispatch_rank_kernel, dim3(n_tiles + n_sched), dim3(rows ? 1024 : 256), 0, s, m->ids, m->tile_counts, m->counts,
                        n_tiles, T, tok_tile, c.K, c.E, c.Es, bm, m->offsets, m->dst, m->dstp, m->src_row, m->tokp, m->tiles,
-                       m->tile_meta, m->desc_up, c.H / 128, 128, m->desc_down, c.d / m->down_cols, m->down_cols,
+                       m->tile_meta, queues ? m->desc_up : nullptr, c.H / 128, 128, queues ? m->desc_down : nullptr, c.d / m->down_cols, m->down_cols,
                        m->down_ks_max, c.H / 32, m->down_tail_ks, m->wq_up, m->wq_down, m->n_wg, (const unsigned char *)x, c.d,
                        (unsigned char *)(rows ? m->xg : nullptr), (unsigned char *)(rows ? m->xs : nullptr), nt_stores, n_sched,
                        m->down_ks_max > 1 || m->down_tail_ks > 1 ? m->slab_tab : nullptr);
