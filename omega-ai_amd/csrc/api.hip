@@ -563,6 +563,16 @@ int omega_moe_set_weights(omega_moe *m, int which, int expert, const void *src, 
     return OMEGA_OK;
 }
 
+// A weight or gradient into device memory of the caller, there when the call returns (R rows of a packed image, or bytes as they
+// are).  false: not for this kernel.
+static bool read_to_device(omega_moe *m, void *dst, const void *src, size_t bytes, int R, int Kd, hipError_t *e)
+{
+    if (launch_param_read == nullptr || (R == 0 && (((uintptr_t)dst | (uintptr_t)src) % 4 != 0 || bytes % 4 != 0))) return false;
+    *e = launch_param_read(dst, src, R, Kd, bytes / 4, m->ev1, m->ctx->stream);
+    if (*e == hipSuccess) *e = hipEventSynchronize(m->ev1);
+    return true;
+}
+
 int omega_moe_get_weights(omega_moe *m, int which, int expert, void *dst, int is_device)
 {
     if (!m) OMEGA_FAIL(nullptr, OMEGA_ERR_INVALID_ARG, "NULL layer");
@@ -571,15 +581,24 @@ int omega_moe_get_weights(omega_moe *m, int which, int expert, void *dst, int is
     void *p; size_t bytes;
     if (!dst || weight_slot(m, which, expert, &p, &bytes) != OMEGA_OK)
         OMEGA_FAIL(ctx, OMEGA_ERR_INVALID_ARG, "get_weights: bad kind, expert index or destination");
+    hipError_t e = hipSuccess;
     if (!weight_is_packed(m, which)) {
+        if (is_device && read_to_device(m, dst, p, bytes, 0, 0, &e)) {
+            OMEGA_HIP_CHECK(ctx, e);
+            return OMEGA_OK;
+        }
         OMEGA_HIP_CHECK(ctx, hipMemcpyAsync(dst, p, bytes, is_device ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost, ctx->stream));
         OMEGA_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
         return OMEGA_OK;
     }
     const int R = which == OMEGA_W_W2 ? m->cfg.d : m->cfg.H, Kd = which == OMEGA_W_W2 ? m->cfg.H : m->cfg.d;
+    if (is_device && read_to_device(m, dst, p, bytes, R, Kd, &e)) {
+        OMEGA_HIP_CHECK(ctx, e);
+        return OMEGA_OK;
+    }
     void *stage = nullptr;
     if (!is_device) OMEGA_HIP_CHECK(ctx, hipMalloc(&stage, bytes));
-    hipError_t e = launch_unpack_rows(is_device ? dst : stage, p, R, Kd, ctx->stream);
+    e = launch_unpack_rows(is_device ? dst : stage, p, R, Kd, ctx->stream);
     if (e == hipSuccess && !is_device) e = hipMemcpyAsync(dst, stage, bytes, hipMemcpyDeviceToHost, ctx->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
     if (stage) hipFree(stage);
@@ -958,6 +977,11 @@ int omega_moe_get_grad(omega_moe *m, int which, int expert, void *dst, int is_de
     float *p; size_t n;
     if (!dst || grad_slot(m, which, expert, &p, &n) != OMEGA_OK)
         OMEGA_FAIL(ctx, OMEGA_ERR_INVALID_ARG, "get_grad: bad kind, expert index or destination");
+    hipError_t e = hipSuccess;
+    if (is_device && read_to_device(m, dst, p, n * 4, 0, 0, &e)) {
+        OMEGA_HIP_CHECK(ctx, e);
+        return OMEGA_OK;
+    }
     OMEGA_HIP_CHECK(ctx, hipMemcpyAsync(dst, p, n * 4, is_device ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost, ctx->stream));
     OMEGA_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
     return OMEGA_OK;

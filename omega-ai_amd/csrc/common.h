@@ -259,6 +259,8 @@ struct omega_adamw {
 hipError_t launch_update_adamw(const omega_moe *m, float *master, float *mw, float *vw, const omega_adamw &p, hipStream_t s);
 hipError_t launch_pack_rows(void *dst_packed, const void *src_rowmajor, int R, int Kd, hipStream_t s);
 hipError_t launch_unpack_rows(void *dst_rowmajor, const void *src_packed, int R, int Kd, hipStream_t s);
+// (weak: where api.hip runs without the kernels behind it, it reads by the runtime's copies)
+hipError_t launch_param_read(void *dst, const void *src, int R, int Kd, size_t n, hipEvent_t done, hipStream_t s) __attribute__((weak));
 int experts_bf16_tile_m(const omega_moe *m, int T);
 bool wgrad_on_four_waves(const omega_moe *m, int T, int M, int N);  // which kernel takes the weight gradients of M x N per expert
 #define F32_TILE_M 128       // row-tile heights of fp32 layers: experts_f32_tile_m chooses one per batch
