@@ -1096,6 +1096,7 @@ int omega_moe_update_adamw(omega_moe *m, float lr, float beta1, float beta2, flo
         m->wT_valid = m->gate_img_valid = false;
     }
     OMEGA_HIP_CHECK(ctx, launch_update_adamw(m, m->master, m->adam_m, m->adam_v, p, ctx->stream));
+    m->wT_valid = m->W2T && m->W13T;  // (where they exist, the step writes the transposed copies too)
     stage_invalidates(m);  // the weights changed: a backward pass needs a new forward
     return OMEGA_OK;
 }

@@ -35,41 +35,69 @@ __global__ __launch_bounds__(256) void adamw_f32_kernel(float *__restrict__ w, s
     }
 }
 
-// bf16 expert weights: the step is taken on the fp32 master, the packed bf16 image is re-rounded from it.  A thread takes four
-// adjacent columns of a row of expert blockIdx.y, so that every load and store of a wave is one contiguous kilobyte (master,
-// gradient and moments share one layout; the image gets 8 bytes of a 16-byte chunk).  Bound: the 30 bytes per weight, which
-// pass the last-level cache by.  Two 16-byte halves of a chunk per thread and 64-bit indices -> now: 49 million weights 347
-// -> 269 us (5.5 TB/s), 470 million 3633 -> 3246 us (4.3 TB/s).  All of it with the blocks on cache lines: 64 bytes off the
-// line the new form took 293 us, 32 bytes off 3850.
+// bf16 expert weights: the step is taken on the fp32 master, the packed bf16 image is re-rounded from it, and with it the
+// transposed image that the next backward pass reads (T = true: it is there).  A workgroup takes 32 rows x 128 columns of expert
+// blockIdx.y: rows of 512 bytes of the four fp32 arrays, sixteen 16-byte loads in flight per thread; the bf16 tile goes through
+// LDS and out as whole 1 KiB blocks of either image (of the transposed one the 8 blocks of one k step of a row group: 8 KiB in
+// a row).  Bound: the 30 bytes per weight (32 with the transposed image, whose pass over the weights is saved: 4 bytes), which pass
+// the last-level cache by.  A thread per four columns, then this form (with the transposed image and the
+// blocks of 64 x 64 that made it in launches of their own): 3 x 49 million weights 3 x 269 + 3 x 37 -> 3 x 283 us, 1.41 billion 9.2 + 1.0 ->
+// 8.3 ms (5.4 TB/s).  The blocks have to start on cache lines: 32 bytes off the earlier form took 11.6 ms instead of 9.8.
 typedef __attribute__((ext_vector_type(4))) float adamw_f32x4;
+template <bool T>
 __global__ __launch_bounds__(256) void adamw_packed_kernel(float *__restrict__ master, const float *__restrict__ grad,
                                                            float *__restrict__ mw, float *__restrict__ vw, size_t stride,
-                                                           unsigned char *__restrict__ packed, size_t pstride, int R, int K,
-                                                           omega_adamw p)
+                                                           unsigned char *__restrict__ packed, size_t pstride, int K,
+                                                           unsigned char *__restrict__ tr, size_t tstride, int KTt, int kt0, omega_adamw p)
 {
-    const int g = blockIdx.y, KT = K >> 5;
-    const uint32_t nq = K >> 2, n = (uint32_t)R * nq;  // (an expert of 2^34 weights and its moments would not fit the memory)
-    adamw_f32x4 *w4 = (adamw_f32x4 *)(master + (size_t)g * stride), *m4 = (adamw_f32x4 *)(mw + (size_t)g * stride), *v4 = (adamw_f32x4 *)(vw + (size_t)g * stride);
-    const adamw_f32x4 *g4 = (const adamw_f32x4 *)(grad + (size_t)g * stride);
-    unsigned char *pg = packed + (size_t)g * pstride;
-    for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
-        const uint32_t r = i / nq, c4 = i % nq;
-        adamw_f32x4 wv = __builtin_nontemporal_load(w4 + i), mv = __builtin_nontemporal_load(m4 + i), vv = __builtin_nontemporal_load(v4 + i);
-        const adamw_f32x4 gv = __builtin_nontemporal_load(g4 + i);
+    constexpr int LDB = 136;  // LDS row of 128 columns: rows stay on 16 bytes and start 4 banks apart
+    __shared__ __attribute__((aligned(16))) bf16_t tile[32][LDB];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, KT = K >> 5, nct = K >> 7;
+    const int rt = blockIdx.x / nct, r0 = 32 * rt, c0 = 128 * (blockIdx.x - rt * nct);
+    const size_t at = (size_t)blockIdx.y * stride + (size_t)(r0 + (tid >> 5)) * K + c0 + 4 * (tid & 31);
+    adamw_f32x4 wv[4], mv[4], vv[4], gv[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const size_t o = at + (size_t)(8 * i) * K;
+        wv[i] = __builtin_nontemporal_load((const adamw_f32x4 *)(master + o));
+        mv[i] = __builtin_nontemporal_load((const adamw_f32x4 *)(mw + o));
+        vv[i] = __builtin_nontemporal_load((const adamw_f32x4 *)(vw + o));
+        gv[i] = __builtin_nontemporal_load((const adamw_f32x4 *)(grad + o));
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const size_t o = at + (size_t)(8 * i) * K;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            float mq = mv[q], vq = vv[q];
-            wv[q] = adamw_elem(wv[q], gv[q], mq, vq, p);
-            mv[q] = mq;
-            vv[q] = vq;
+            float mq = mv[i][q], vq = vv[i][q];
+            wv[i][q] = adamw_elem(wv[i][q], gv[i][q], mq, vq, p);
+            mv[i][q] = mq;
+            vv[i][q] = vq;
         }
-        __builtin_nontemporal_store(wv, w4 + i);
-        __builtin_nontemporal_store(mv, m4 + i);
-        __builtin_nontemporal_store(vv, v4 + i);
-        uint2 u;
-        u.x = (uint32_t)f32_to_bf16(wv[0]) | ((uint32_t)f32_to_bf16(wv[1]) << 16);
-        u.y = (uint32_t)f32_to_bf16(wv[2]) | ((uint32_t)f32_to_bf16(wv[3]) << 16);
-        *(uint2 *)(pg + pk_chunk_off(r, c4 >> 3, (c4 >> 1) & 3, KT) + (c4 & 1) * 8) = u;
+        __builtin_nontemporal_store(wv[i], (adamw_f32x4 *)(master + o));
+        __builtin_nontemporal_store(mv[i], (adamw_f32x4 *)(mw + o));
+        __builtin_nontemporal_store(vv[i], (adamw_f32x4 *)(vw + o));
+        const uint2 u = {(uint32_t)f32_to_bf16(wv[i][0]) | ((uint32_t)f32_to_bf16(wv[i][1]) << 16),
+                         (uint32_t)f32_to_bf16(wv[i][2]) | ((uint32_t)f32_to_bf16(wv[i][3]) << 16)};
+        *(uint2 *)&tile[8 * i + (tid >> 5)][4 * (tid & 31)] = u;
+    }
+    __syncthreads();
+    // lane: row lane / 4 of a block, chunk lane % 4 as stored
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int blk = 2 * wave + i, rb = blk >> 2, kb = blk & 3;  // block of 16 rows, k step
+        const int row = r0 + 16 * rb + (lane >> 2), c = (lane & 3) ^ pk_swz(row);
+        *(uint4 *)(packed + (size_t)blockIdx.y * pstride + pk_chunk_off(row, (c0 >> 5) + kb, c, KT)) = *(const uint4 *)&tile[16 * rb + (lane >> 2)][32 * kb + 8 * c];
+    }
+    if (T) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int col = 16 * (2 * wave + i) + (lane >> 2), c = (lane & 3) ^ pk_swz(c0 + col);  // 8 rows of a column
+            uint32_t u[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) u[q] = (uint32_t)tile[8 * c + 2 * q][col] | (uint32_t)tile[8 * c + 2 * q + 1][col] << 16;
+            *(uint4 *)(tr + (size_t)blockIdx.y * tstride + pk_chunk_off(c0 + col, kt0 + rt, c, KTt)) = make_uint4(u[0], u[1], u[2], u[3]);
+        }
     }
 }
 
@@ -114,13 +142,19 @@ hipError_t launch_update_adamw(const omega_moe *m, float *master, float *mw, flo
         hipLaunchKernelGGL(adamw_f32_kernel, dim3(grid_for(c.d, 1024)), dim3(256), 0, s, m->gamma, (size_t)0,
                            (const float *)m->dgamma, mw + o_gm, vw + o_gm, (size_t)0, (size_t)c.d, p);
     if (bf) {
-        const dim3 grid(512, m->G);
-        hipLaunchKernelGGL(adamw_packed_kernel, grid, dim3(256), 0, s, master + o13, (const float *)m->dW13, mw + o13, vw + o13,
-                           2 * HD, (unsigned char *)m->W1, HD * 2, c.H, c.d, p);
-        hipLaunchKernelGGL(adamw_packed_kernel, grid, dim3(256), 0, s, master + o13 + HD, (const float *)m->dW13 + HD,
-                           mw + o13 + HD, vw + o13 + HD, 2 * HD, (unsigned char *)m->W3, HD * 2, c.H, c.d, p);
-        hipLaunchKernelGGL(adamw_packed_kernel, grid, dim3(256), 0, s, master + o2, (const float *)m->dW2, mw + o2, vw + o2, HD,
-                           (unsigned char *)m->W2, HD * 2, c.d, c.H, p);
+        // (widths are multiples of 256 and 128; the images of m->W2T: [H,d] per expert, of m->W13T: [d, H | H])
+        auto step = [&](size_t o, size_t stride, void *w, int R, int K, void *tr, size_t tstride, int KTt, int kt0) {
+            const dim3 grid((unsigned)(R / 32) * (K / 128), m->G);
+            if (m->W2T && m->W13T)
+                hipLaunchKernelGGL(adamw_packed_kernel<true>, grid, dim3(256), 0, s, master + o, (const float *)m->grads + o, mw + o, vw + o, stride,
+                                   (unsigned char *)w, HD * 2, K, (unsigned char *)tr, tstride, KTt, kt0, p);
+            else
+                hipLaunchKernelGGL(adamw_packed_kernel<false>, grid, dim3(256), 0, s, master + o, (const float *)m->grads + o, mw + o, vw + o, stride,
+                                   (unsigned char *)w, HD * 2, K, (unsigned char *)nullptr, (size_t)0, 0, 0, p);
+        };
+        step(o13, 2 * HD, m->W1, c.H, c.d, m->W13T, 4 * HD, 2 * c.H / 32, 0);
+        step(o13 + HD, 2 * HD, m->W3, c.H, c.d, m->W13T, 4 * HD, 2 * c.H / 32, c.H / 32);
+        step(o2, HD, m->W2, c.d, c.H, m->W2T, 2 * HD, c.d / 32, 0);
     } else {
         const dim3 grid(grid_for(HD, 512), m->G);
         hipLaunchKernelGGL(adamw_f32_kernel, grid, dim3(256), 0, s, (float *)m->W1, HD, (const float *)m->dW13, mw + o13,
