@@ -500,12 +500,19 @@ hipError_t launch_sumsq_f32(const float *src, size_t n, double *part, hipStream_
 // dst *= coef, one rounding per element (TensorOP.mul(diffW, clip_coef, diffW), Network.java:416-431)
 __global__ __launch_bounds__(256) void bw_scale_kernel(float *__restrict__ dst, float coef, size_t n)
 {
+    // Bound: HBM.  Four 16-byte pieces in flight per thread, in and out past the last-level cache: 590 MB 244 -> 186 us (6.3 TB/s),
+    // 5.6 GB 2478 -> 2207; cached stores 203 and 2200.
+    typedef float v4f __attribute__((ext_vector_type(4)));
     const size_t n4 = n >> 2;
-    float4 *d4 = (float4 *)dst;
-    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n4; i += (size_t)gridDim.x * 256) {
-        float4 v = d4[i];
-        v.x *= coef; v.y *= coef; v.z *= coef; v.w *= coef;
-        d4[i] = v;
+    v4f *d4 = (v4f *)dst;
+    for (size_t i = (size_t)blockIdx.x * 1024 + threadIdx.x; i < n4; i += (size_t)gridDim.x * 1024) {
+        v4f v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (i + u * 256 < n4) v[u] = __builtin_nontemporal_load(d4 + i + u * 256);
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (i + u * 256 < n4) __builtin_nontemporal_store(v[u] * coef, d4 + i + u * 256);
     }
     if (blockIdx.x == 0 && threadIdx.x < (n & 3)) dst[(n4 << 2) + threadIdx.x] *= coef;
 }
@@ -513,7 +520,7 @@ __global__ __launch_bounds__(256) void bw_scale_kernel(float *__restrict__ dst, 
 hipError_t launch_scale_f32(float *dst, float coef, size_t n, hipStream_t s)
 {
     if (n == 0) return hipSuccess;
-    const int grid = (int)((n + 255) / 256 < 4096 ? (n + 255) / 256 : 4096);
+    const int grid = (int)((n + 4095) / 4096 < 16384 ? (n + 4095) / 4096 : 16384);
     hipLaunchKernelGGL(bw_scale_kernel, dim3(grid), dim3(256), 0, s, dst, coef, n);
     return hipGetLastError();
 }
