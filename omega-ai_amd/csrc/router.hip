@@ -22,6 +22,7 @@
 // run the chains (Mixtral shape: 4096 tokens 33 -> 29 us, 64 tokens 27 -> 22 us; of the 22, 11 are the chain itself at
 // 6.25 clocks a term and 6.5 are launch, the first loads and phases 2 and 3).
 #include "common.h"
+#include <type_traits>
 
 typedef __attribute__((ext_vector_type(8))) __bf16 rt_bf16x8;
 typedef __attribute__((ext_vector_type(16))) float rt_f32x16;
@@ -47,11 +48,14 @@ int router_tok_tile(const omega_moe *m, int T)
 // which halves the LDS reads per multiply-add) and NT tokens.
 // EP: experts padded to a power of two; KC: k per staged chunk (larger for few experts, where one chunk in
 // flight per workgroup would otherwise leave the kernel waiting on memory latency).
-// XBF: x and Wg are stored as bf16 (else fp32).  FAST_IO: rows are 16-byte aligned and d is a multiple of KC, so
+// XBF: x and Wg are stored as bf16 (else fp32).  IO_FULL: rows are 16-byte aligned and d is a multiple of KC, so
 // every load is a whole 16-byte vector; rows beyond T or E are redirected to the last valid row (their sums are
 // never used), which keeps the loads free of branches - and with that really asynchronous: a load issued inside
-// a divergent branch makes the compiler wait for all earlier ones first.
-template <int EP, int KC, bool EXACT, bool XBF, bool FAST_IO>
+// a divergent branch makes the compiler wait for all earlier ones first.  IO_VEC: rows are 16-byte aligned and whole 16-byte
+// vectors long; vectors behind the row's end read its last one and count as zeros.  (Router launch, us, against
+// element by element: 256 tokens x 128 columns, 8 experts 7.6 -> 5.4; 4096 x 1000 20.0 -> 14.7; bf16, 6000 x 1280 26.3 -> 13.9.)
+enum { IO_ANY = 0, IO_VEC, IO_FULL };
+template <int EP, int KC, bool EXACT, bool XBF, int IO>
 __device__ __forceinline__ void router_sums(const void *__restrict__ x, const void *__restrict__ Wg, int T, int d, int E,
                                             int t0, float (*xs)[KC + 4], float (*ws)[KC + 4],
                                             float (&acc)[ROUTER_TT(EP) * EP / ROUTER_NTHR(EP)])
@@ -78,7 +82,17 @@ __device__ __forceinline__ void router_sums(const void *__restrict__ x, const vo
     auto load8 = [&](const void *base, int row, int rows, int k, uint4 *out) {
         out[0] = make_uint4(0, 0, 0, 0);
         out[1] = make_uint4(0, 0, 0, 0);
-        if (FAST_IO) {
+        if (IO == IO_VEC) {
+            const size_t row_off = (size_t)min(row, rows - 1) * d;
+            constexpr int V = XBF ? 8 : 4;
+#pragma unroll
+            for (int h = 0; h < 8 / V; ++h) {
+                const uint4 v = XBF ? *(const uint4 *)((const bf16_t *)base + row_off + min(k, d - V))
+                                    : *(const uint4 *)((const float *)base + row_off + min(k + 4 * h, d - V));
+                const bool in = k + 4 * h < d;
+                out[h] = make_uint4(in ? v.x : 0, in ? v.y : 0, in ? v.z : 0, in ? v.w : 0);
+            }
+        } else if (IO == IO_FULL) {
             const size_t off = (size_t)min(row, rows - 1) * d + k;
             if (XBF) {
                 out[0] = *(const uint4 *)((const bf16_t *)base + off);
@@ -179,13 +193,15 @@ __device__ __forceinline__ void router_sums(const void *__restrict__ x, const vo
     } while (0)
         if (!wave_live) {
             // every token of this wave lies beyond T: it only stages and keeps the barriers
-        } else if (FAST_IO || kend == KC) {
+        } else if (IO == IO_FULL || kend == KC) {
             // whole chunk: no exit test inside, so the LDS reads of later steps are issued ahead of the sums
 #pragma unroll(NT * EPT >= 8 ? 4 : 16)
             for (int k4 = 0; k4 < KC / 4; ++k4) ROUTER_K4(k4);
         } else {
-            // last, partial chunk (zero-filled beyond d: a +0 product leaves every sum unchanged)
-            for (int k4 = 0; k4 * 4 < kend; ++k4) ROUTER_K4(k4);
+            // last, partial chunk (zero-filled beyond d: a +0 product leaves every sum unchanged - none is ever -0), 32 k at a time
+            for (int k32 = 0; k32 * 32 < kend; ++k32)
+#pragma unroll
+                for (int k4 = 0; k4 < 8; ++k4) ROUTER_K4(8 * k32 + k4);
         }
 #undef ROUTER_K4
         __syncthreads();
@@ -341,13 +357,15 @@ __global__ __launch_bounds__(ROUTER_NTHR(EP)) void router_kernel(const void *__r
 #pragma unroll
     for (int i = 0; i < NT * EPT; ++i) acc[i] = 0.0f;
 
-    const bool fast_io = (d % KC == 0) && (((uintptr_t)x | (uintptr_t)Wg) % 16 == 0);
-    if (EP <= 16 && dtype == OMEGA_DTYPE_BF16) {  // (bf16 layers with more experts run on the matrix cores)
-        if (fast_io) router_sums<EP, KC, EXACT, true, true>(x, Wg, T, d, E, t0, xs, ws, acc);
-        else router_sums<EP, KC, EXACT, true, false>(x, Wg, T, d, E, t0, xs, ws, acc);
+    const bool aligned = ((uintptr_t)x | (uintptr_t)Wg) % 16 == 0, full = aligned && d % KC == 0;
+    if (EP <= 16 && dtype == OMEGA_DTYPE_BF16) {  // (bf16 layers with more experts run on the matrix cores; d is a multiple of 256)
+        if (full) router_sums<EP, KC, EXACT, true, IO_FULL>(x, Wg, T, d, E, t0, xs, ws, acc);
+        else if (aligned) router_sums<EP, KC, EXACT, true, IO_VEC>(x, Wg, T, d, E, t0, xs, ws, acc);
+        else router_sums<EP, KC, EXACT, true, IO_ANY>(x, Wg, T, d, E, t0, xs, ws, acc);
     } else {
-        if (fast_io) router_sums<EP, KC, EXACT, false, true>(x, Wg, T, d, E, t0, xs, ws, acc);
-        else router_sums<EP, KC, EXACT, false, false>(x, Wg, T, d, E, t0, xs, ws, acc);
+        if (full) router_sums<EP, KC, EXACT, false, IO_FULL>(x, Wg, T, d, E, t0, xs, ws, acc);
+        else if (aligned && d % 4 == 0) router_sums<EP, KC, EXACT, false, IO_VEC>(x, Wg, T, d, E, t0, xs, ws, acc);
+        else router_sums<EP, KC, EXACT, false, IO_ANY>(x, Wg, T, d, E, t0, xs, ws, acc);
     }
 #pragma unroll
     for (int x_ = 0; x_ < EPT; ++x_) {
@@ -606,7 +624,8 @@ __global__ __launch_bounds__(64 * NW) void router_units_kernel(const bf16_t *__r
     router_select<EP, false, TT, NTHR>(lg, hist, t0, tile, T, E, K, renorm, ids, wout, tile_counts, probs_out);
 }
 
-// Batches of at most one 16-token tile per compute unit, bf16, at most 16 experts, d a multiple of 512: the whole
+// Batches of at most one 16-token tile per compute unit, bf16, at most 16 experts (d is a multiple of 256: the
+// last chunk may be half full; 90 tokens x 3328, 7 experts, on the kernel above 46 us, here 17; 777 x 2304, 16 experts 35 -> 16): the whole
 // kernel is as long as ONE chain of d dependent multiply-adds (about 6 clocks a term on a SIMD that has no second wave
 // to fill them), so everything else is taken out of the waves that run the chains.  The workgroup has two kinds of
 // waves: 16*EP/64 sum waves, one lane per (token, expert), that only read LDS and add; and two staging waves that
@@ -631,7 +650,7 @@ __global__ __launch_bounds__(16 * EP + RP_STAGERS) void router_pipe_kernel(
     __shared__ int hist[EP];
     const int tid = threadIdx.x, tile = blockIdx.x, t0 = tile * TT;
     if (tid < EP) hist[tid] = 0;
-    const int nch = d / KC;
+    const int nch = (d + KC - 1) / KC;  // (the last chunk of an odd multiple of 256 is half full)
     if (tid >= CT) {
         // staging wave: thread st carries 8 consecutive k (16 bytes of bf16) of one row per load
         const int st = tid - CT;
@@ -643,12 +662,12 @@ __global__ __launch_bounds__(16 * EP + RP_STAGERS) void router_pipe_kernel(
 #pragma unroll
             for (int c = 0; c < XCH; ++c) {
                 const int idx = st + c * ST;
-                xr[c] = *(const uint4 *)(x + (size_t)min(t0 + idx / (KC / 8), T - 1) * d + k0 + (idx % (KC / 8)) * 8);
+                xr[c] = *(const uint4 *)(x + (size_t)min(t0 + idx / (KC / 8), T - 1) * d + min(k0 + (idx % (KC / 8)) * 8, d - 8));
             }
 #pragma unroll
             for (int c = 0; c < WCH; ++c) {
                 const int idx = st + c * ST;
-                wr[c] = *(const uint4 *)(Wg + (size_t)min(idx / (KC / 8), E - 1) * d + k0 + (idx % (KC / 8)) * 8);
+                wr[c] = *(const uint4 *)(Wg + (size_t)min(idx / (KC / 8), E - 1) * d + min(k0 + (idx % (KC / 8)) * 8, d - 8));
             }
         };
         auto widen = [&](const uint4 &v, float *dst) {
@@ -699,19 +718,24 @@ __global__ __launch_bounds__(16 * EP + RP_STAGERS) void router_pipe_kernel(
     }
             // the LDS reads of the next 32 k are in flight while the terms of the current 32 are added (the fences
             // keep the reads where they are written: ahead of the other set's terms)
-            ROUTER_LD(wa, xa, 0)
-            for (int g = 0; g < KC / 32; g += 2) {
-                __builtin_amdgcn_sched_barrier(0);
-                ROUTER_LD(wb, xb, g + 1)
-                __builtin_amdgcn_sched_barrier(0);
-                ROUTER_FM(wa, xa)
-                __builtin_amdgcn_sched_barrier(0);
-                if (g + 2 < KC / 32) {
-                    ROUTER_LD(wa, xa, g + 2)
+            auto sum = [&](auto groups) {  // of 32 k (the number is known at compile time: the loop unrolls)
+                ROUTER_LD(wa, xa, 0)
+#pragma unroll
+                for (int g = 0; g < decltype(groups)::value; g += 2) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    ROUTER_LD(wb, xb, g + 1)
+                    __builtin_amdgcn_sched_barrier(0);
+                    ROUTER_FM(wa, xa)
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (g + 2 < decltype(groups)::value) {
+                        ROUTER_LD(wa, xa, g + 2)
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                    ROUTER_FM(wb, xb)
                 }
-                __builtin_amdgcn_sched_barrier(0);
-                ROUTER_FM(wb, xb)
-            }
+            };
+            if (d - c * KC >= KC) sum(std::integral_constant<int, KC / 32>());
+            else sum(std::integral_constant<int, KC / 64>());
 #undef ROUTER_LD
 #undef ROUTER_FM
         }
@@ -778,7 +802,7 @@ hipError_t launch_router(const omega_moe *m, const void *x, int T, float *logits
         return hipGetLastError();
     }
     // at most 16 experts, bf16, at most one tile per compute unit: chains fed by staging waves (either mode: same bits)
-    if (c.dtype == OMEGA_DTYPE_BF16 && c.E <= 16 && tiles <= m->ctx->num_cus && c.d % RP_KC == 0 &&
+    if (c.dtype == OMEGA_DTYPE_BF16 && c.E <= 16 && tiles <= m->ctx->num_cus &&
         (((uintptr_t)x | (uintptr_t)m->Wg) % 16) == 0) {
         if (c.E <= 8)
             hipLaunchKernelGGL(router_pipe_kernel<8>, dim3(tiles), dim3(16 * 8 + RP_STAGERS), router_pipe_smem_bytes(8), s,
