@@ -6,6 +6,7 @@
 // (J/engine/gpu/BaseKernel.cu:228-241) generalised to K terms; shared rows are added as add_kernel
 // (J/engine/ad/op/gpu/OPKernel.cu:359-366).  No atomics: every output element has one writer.
 #include "common.h"
+#include <algorithm>
 
 // The slices of KU rows of y (SL below) added to what the lane holds of them, VEC columns from c0 on.  Lanes whose tile has fewer
 // slices than others' read a row again and drop it: no branch keeps the loads from being in flight together.
@@ -77,15 +78,15 @@ __global__ __launch_bounds__(256) void combine_kernel(const float *__restrict__ 
                                                       const float *__restrict__ w, int T, int K, int d, int Es,
                                                       const int32_t *__restrict__ tile_meta, int E, int bm,
                                                       const void *__restrict__ resid, void *__restrict__ out, int split,
-                                                      const float *__restrict__ slabs, const int32_t *__restrict__ slab_tab)
+                                                      const float *__restrict__ slabs, const int32_t *__restrict__ slab_tab, int dc)
 {
-    // `split` waves share a token, each taking d / split consecutive columns (more waves, more loads in flight, when
-    // the batch has few tokens for the compute units there are)
+    // `split` waves share a token, each taking dc consecutive columns, the last one what is left (more waves, more loads in
+    // flight, when the batch has few tokens for the compute units there are)
     const int lane = threadIdx.x & 63;
     const int wv = blockIdx.x * 4 + (threadIdx.x >> 6);
     const int t = wv / split, part = wv - t * split;
     if (t >= T) return;
-    const int dc = d / split;
+    const int cend = min((part + 1) * dc, d);
     // lane j < K holds row index and weight of slot j, lane j < Es the row of shared expert j; handed out by lane reads
     int myrow = 0, shrow = 0;
     float myw = 0.0f;
@@ -97,8 +98,8 @@ __global__ __launch_bounds__(256) void combine_kernel(const float *__restrict__ 
     const bool sliced = SL && tile_meta[E + Es + 9] > 0;  // (the host knows bounds of the number of tiles only)
     const int n = K + Es;
     // (lanes past the row's end work on column 0 and store nothing)
-    for (int cb = part * dc; cb < (part + 1) * dc; cb += 64 * VEC) {
-        const bool on = cb + lane * VEC < (part + 1) * dc;
+    for (int cb = part * dc; cb < cend; cb += 64 * VEC) {
+        const bool on = cb + lane * VEC < cend;
         const int c0 = on ? cb + lane * VEC : 0;
         float acc[VEC];
 #pragma unroll
@@ -209,15 +210,18 @@ hipError_t launch_combine(const omega_moe *m, int T, void *out, const void *resi
         const bool nt = (size_t)T * (c.K + c.Es) * c.d * 4 > OMEGA_LLC_BYTES;
         // several waves per token, each with a share of the columns, until the launch has 256 waves per compute unit:
         // more loads in flight (4096 tokens x 4096 columns: 36.3 -> 30.6 us with 8 waves per token; 64 tokens:
-        // 12.0 -> 6.9 us; 8192 tokens x 2048 columns x 8 rows: 122.6 -> 113.8 us with 4; 16384 tokens: 228 -> 210 us)
-        int split = 1;
-        while (split < 8 && (long long)T * split < 256LL * m->ctx->num_cus && c.d % (64 * vec * split * 2) == 0) split *= 2;
+        // 12.0 -> 6.9 us; 8192 tokens x 2048 columns x 8 rows: 122.6 -> 113.8 us with 4; 16384 tokens: 228 -> 210 us;
+        // shares are whole trips of a wave, the last may be less: 90 tokens x 3328 columns, top 3, 7.3 -> 3.8 us with seven for one)
+        const int trips = ceil_div(c.d, 64 * vec);
+        int want = 1;
+        while (want < 8 && (long long)T * want < 256LL * m->ctx->num_cus) want *= 2;
+        const int dc = ceil_div(trips, std::min(want, trips)) * 64 * vec, split = ceil_div(c.d, dc);
         const bool sl = m->y_partial;
         const int n = c.K + c.Es, ku = ceil_div(n, ceil_div(n, 8));  // rows of a token in groups of one size, eight at most
         const int grid = ceil_div(T * split, 4);
 #define COMBINE_LAUNCH(VECV, BFV, KUV, NTV, SLV)                                                                                       \
     hipLaunchKernelGGL((combine_kernel<VECV, BFV, KUV, NTV, SLV>), dim3(grid), dim3(256), 0, s, m->y, m->dstp, m->w, T, c.K, c.d, c.Es, \
-                       m->tile_meta, c.E, m->bm, resid, out, split, m->y_slabs, m->slab_tab)
+                       m->tile_meta, c.E, m->bm, resid, out, split, m->y_slabs, m->slab_tab, dc)
 #define COMBINE_SLOTS(VECV, BFV, NTV, SLV)                  \
     do {                                                     \
         switch (ku) {                                        \
