@@ -50,7 +50,7 @@
 //   UP     tile 256 x (128 of Wa + 128 of Wb), silu(h1)*h3 -> packed bf16 a
 //   DOWN   tile 256 x 256, fp32 row-major output; an item may be a k slice of a tile (see make_ctx)
 //   UPRAW  as UP, but h1 and h3 are stored as they sit in the accumulators (Cout = h1, Aux1 = h3): one 4 KiB record
-//          per 32x32 MFMA block, [row block][column block][register 0..15][lane 0..63]
+//          per 32x32 MFMA block, [row block][column block][16 x 16 piece][lane 0..63][register 0..3]
 //   UPREC  UP and UPRAW in one: the forward pass of a layer in training mode (a -> Cout, h1 -> Aux1, h3 -> Aux2)
 //   DA     tile 256 x 256 of d(a) = dy . W2 (B = packed W2^T); the epilogue reads the h1/h3 records of its blocks
 //          (Aux1, Aux2), applies the SwiGLU backward and writes dh1 | dh3 as one packed bf16 image with 2N columns
@@ -489,11 +489,11 @@ __device__ __forceinline__ void run_tile(unsigned char *smem, const TileCtx ctx_
 #pragma unroll
         for (int i = 0; i < NBLK; ++i) {
             const size_t rb = (size_t)ctx.rec0 + 2 * i + wm;
-            float *o1 = r1 + (rb * ncb + cb) * 1024 + lane, *o3 = r3 + (rb * ncb + cb) * 1024 + lane;
+            f32x4_t *o1 = (f32x4_t *)(r1 + (rb * ncb + cb) * 1024) + lane, *o3 = (f32x4_t *)(r3 + (rb * ncb + cb) * 1024) + lane;
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                o1[r * 64] = acc[i][0][(r >> 3) & 1][(r >> 2) & 1][r & 3];
-                o3[r * 64] = acc[i][1][(r >> 3) & 1][(r >> 2) & 1][r & 3];
+            for (int q = 0; q < 4; ++q) {
+                o1[q * 64] = acc[i][0][q >> 1][q & 1];
+                o3[q * 64] = acc[i][1][q >> 1][q & 1];
             }
         }
     } else if (MODE == MODE_DA) {
@@ -501,39 +501,46 @@ __device__ __forceinline__ void run_tile(unsigned char *smem, const TileCtx ctx_
         // elements come from their records.  dh3 = da * silu(h1); dh1 = da*h3 * s*(1 + h1*(1-s)), s = sigmoid(h1)
         // (silu_backward, J/engine/nn/layer/active/gpu/activeFunction.cu:182-190).  Output: packed image with 2N
         // columns, dh1 in k steps 0..N/32-1, dh3 behind them.
+        // (the records of the next block are asked for before this one is worked on: with one block's in flight at a time, in 4-byte
+        // pieces, an item of 128 steps spent a quarter of its time here)
         const int ncb = N >> 5, KTa = 2 * ncb;
+        f32x4_t h1v[2][4], h3v[2][4];
+        auto ask = [&](int b) {
+            const size_t rb = (size_t)ctx.rec0 + 2 * (b >> 1) + wm;
+            const int cb = min((ctx.n0 >> 5) + wn * 2 + (b & 1), ncb - 1);
+            const f32x4_t *p1 = (const f32x4_t *)((const float *)Aux1 + (rb * ncb + cb) * 1024) + lane;
+            const f32x4_t *p3 = (const f32x4_t *)((const float *)Aux2 + (rb * ncb + cb) * 1024) + lane;
 #pragma unroll
-        for (int i = 0; i < NBLK; ++i) {
-            const size_t rb = (size_t)ctx.rec0 + 2 * i + wm;
+            for (int q = 0; q < 4; ++q) {
+                h1v[b & 1][q] = p1[q * 64];
+                h3v[b & 1][q] = p3[q * 64];
+            }
+        };
+        if (NBLK > 0) ask(0);
 #pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                const int cb = (ctx.n0 >> 5) + wn * 2 + j;
-                if (cb >= ncb) continue;  // last column tile of a width that is not a multiple of 256
-                const float *p1 = (const float *)Aux1 + (rb * ncb + cb) * 1024 + lane;
-                const float *p3 = (const float *)Aux2 + (rb * ncb + cb) * 1024 + lane;
+        for (int b = 0; b < 2 * NBLK; ++b) {
+            const int i = b >> 1, j = b & 1, cb = (ctx.n0 >> 5) + wn * 2 + j;
+            __builtin_amdgcn_sched_barrier(0);
+            if (b + 1 < 2 * NBLK) ask(b + 1);
+            __builtin_amdgcn_sched_barrier(0);
+            if (cb >= ncb) continue;  // last column tile of a width that is not a multiple of 256
 #pragma unroll
-                for (int rh = 0; rh < 2; ++rh) {
-                    const int row = (2 * i + wm) * 32 + 16 * rh + l16;
-                    const int prow = ctx.row0 + row;
+            for (int q = 0; q < 4; ++q) {
+                const int rh = q >> 1, ch = q & 1, row = (2 * i + wm) * 32 + 16 * rh + l16, prow = ctx.row0 + row;
+                float g1[4], g3[4];
 #pragma unroll
-                    for (int ch = 0; ch < 2; ++ch) {
-                        float g1[4], g3[4];
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) {
-                            const int rr = (rh * 2 + ch) * 4 + r;
-                            const float h1 = p1[rr * 64], h3 = p3[rr * 64], da = acc[i][j][rh][ch][r];
-                            const float sg = __builtin_amdgcn_rcpf(1.0f + __expf(-h1));
-                            g3[r] = da * (h1 * sg);
-                            g1[r] = (da * h3) * sg * (1.0f + h1 * (1.0f - sg));
-                        }
-                        if (row < ctx.rows) {
-                            const uint2 o1 = {pack_bf16x2(g1[0], g1[1]), pack_bf16x2(g1[2], g1[3])};
-                            const uint2 o3 = {pack_bf16x2(g3[0], g3[1]), pack_bf16x2(g3[2], g3[3])};
-                            const int t = 2 * ch + (lq >> 1);
-                            *(uint2 *)((unsigned char *)Cout + pk_chunk_off(prow, cb, t, KTa) + (lq & 1) * 8) = o1;
-                            *(uint2 *)((unsigned char *)Cout + pk_chunk_off(prow, ncb + cb, t, KTa) + (lq & 1) * 8) = o3;
-                        }
-                    }
+                for (int r = 0; r < 4; ++r) {
+                    const float h1 = h1v[b & 1][q][r], h3 = h3v[b & 1][q][r], da = acc[i][j][rh][ch][r];
+                    const float sg = __builtin_amdgcn_rcpf(1.0f + __expf(-h1));
+                    g3[r] = da * (h1 * sg);
+                    g1[r] = (da * h3) * sg * (1.0f + h1 * (1.0f - sg));
+                }
+                if (row < ctx.rows) {
+                    const uint2 o1 = {pack_bf16x2(g1[0], g1[1]), pack_bf16x2(g1[2], g1[3])};
+                    const uint2 o3 = {pack_bf16x2(g3[0], g3[1]), pack_bf16x2(g3[2], g3[3])};
+                    const int t = 2 * ch + (lq >> 1);
+                    *(uint2 *)((unsigned char *)Cout + pk_chunk_off(prow, cb, t, KTa) + (lq & 1) * 8) = o1;
+                    *(uint2 *)((unsigned char *)Cout + pk_chunk_off(prow, ncb + cb, t, KTa) + (lq & 1) * 8) = o3;
                 }
             }
         }
