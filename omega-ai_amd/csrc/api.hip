@@ -195,11 +195,11 @@ static void moe_free_backward_workspace(omega_moe *m)
 static void moe_free_workspace(omega_moe *m)
 {
     void *ptrs[] = {m->ids, m->w, m->tile_counts, m->dst, m->dstp, m->src_row, m->tiles, m->xg, m->xs, m->a, m->y,
-                    m->desc_up, m->desc_down, m->wq_up, m->wq_down, m->rms, m->hbuf, m->tokp, m->slab_tab};
+                    m->desc_up, m->desc_down, m->wq_up, m->wq_down, m->rms, m->hbuf, m->tokp, m->slab_tab, m->gate_logits};
     for (void *p : ptrs)
         if (p) hipFree(p);
     m->ids = nullptr; m->w = nullptr; m->tile_counts = nullptr; m->dst = nullptr; m->dstp = nullptr; m->src_row = nullptr; m->xs = nullptr; m->desc_up = nullptr; m->desc_down = nullptr; m->wq_up = nullptr; m->wq_down = nullptr; m->rms = nullptr; m->hbuf = nullptr;
-    m->tiles = nullptr; m->xg = nullptr; m->a = nullptr; m->y = nullptr; m->tokp = nullptr; m->slab_tab = nullptr;
+    m->tiles = nullptr; m->xg = nullptr; m->a = nullptr; m->y = nullptr; m->tokp = nullptr; m->slab_tab = nullptr; m->gate_logits = nullptr;
     m->xg_valid = m->y_partial = false;
     m->T_cap = 0;
     moe_free_backward_workspace(m);
@@ -390,6 +390,8 @@ static int moe_reserve(omega_moe *m, int T)
         OMEGA_HIP_CHECK(ctx, hipMemsetAsync(m->wq_up, 0, q_up * m->n_wg * sizeof(omega_tile_desc), ctx->stream));
         OMEGA_HIP_CHECK(ctx, hipMemsetAsync(m->wq_down, 0, q_down * m->n_wg * sizeof(omega_tile_desc), ctx->stream));
     }
+    if (c.dtype == OMEGA_DTYPE_BF16 && c.E > 16)  // (as many tokens as such a batch can have: router.hip)
+        OMEGA_HIP_CHECK(ctx, hipMalloc((void **)&m->gate_logits, (size_t)std::min(T, 16 * ctx->num_cus) * c.E * 4));
     if (c.dtype == OMEGA_DTYPE_BF16 && c.Es > 0) {
         const size_t xs_rows = (size_t)ceil_div(T, bm) * bm;
         OMEGA_HIP_CHECK(ctx, hipMalloc(&m->xs, xs_rows * c.d * m->esize));

@@ -59,6 +59,7 @@ struct omega_moe {
     float *bg = nullptr;  // [E]
     float *gate_img = nullptr;            // bf16 layers with more than 16 experts: fp32 image of Wg for the router (router.hip) ...
     mutable bool gate_img_valid = false;  // ... made by the next router launch after Wg has changed
+    float *gate_logits = nullptr;         // ... and the logits of a batch whose tiles the router splits by experts
     void *W1 = nullptr;   // [G,H,d]
     void *W3 = nullptr;   // [G,H,d]
     void *W2 = nullptr;   // [G,d,H]

@@ -635,21 +635,31 @@ __global__ __launch_bounds__(64 * NW) void router_units_kernel(const bf16_t *__r
 // fused multiply-adds: the same bits as the separate multiply and add of the sequential sum, in either router mode.
 #define RP_KC 512
 #define RP_LDW (RP_KC + 4)
+// SPLIT (more than 16 experts): `groups` workgroups per token tile take 16 experts each and leave the logits in logits_out, for
+// router_select_kernel: where those find a compute unit each, a chain of the vector units' and a launch more are shorter than one
+// of the matrix cores' in a workgroup that fetches the whole gate.  Router, us, matrix cores -> here: 1 token x 3328, 86 experts
+// 38.6 -> 19.5; 2 x 3072, 26 experts 22.2 -> 16.3; 48 x 2048, 64 experts 18.2 -> 15.7; 109 x 3328, 83 experts 39 -> 21.5; 500 x 2048, 128 experts 27.7 ->
+// 21.0; 1 x 2048, 250 experts 44 -> 17.7.
 #define RP_STAGERS 128
-template <int EP>
+template <int EP, bool SPLIT>
 __global__ __launch_bounds__(16 * EP + RP_STAGERS) void router_pipe_kernel(
-    const bf16_t *__restrict__ x, const bf16_t *__restrict__ Wg, const float *__restrict__ bg, int T, int d, int E, int K,
+    const bf16_t *__restrict__ x, const bf16_t *__restrict__ Wg, const float *__restrict__ bg, int T, int d, int E_all, int K,
     int renorm, int32_t *__restrict__ ids, float *__restrict__ wout, int32_t *__restrict__ tile_counts,
-    float *__restrict__ logits_out, float *__restrict__ probs_out)
+    float *__restrict__ logits_out, float *__restrict__ probs_out, int groups, int tpw)
 {
     constexpr int TT = 16, CT = 16 * EP, ST = RP_STAGERS, KC = RP_KC, LDW = RP_LDW;
+    const int tile = SPLIT ? blockIdx.x / groups : blockIdx.x, e0 = SPLIT ? (blockIdx.x - tile * groups) * EP : 0;
+    const int E = SPLIT ? min(EP, E_all - e0) : E_all;
+    Wg += (size_t)e0 * d;
+    if (bg != nullptr) bg += e0;
     extern __shared__ __attribute__((aligned(16))) float rp_smem[];
     float(*xs)[TT][LDW] = (float(*)[TT][LDW])rp_smem;                  // [2][TT][LDW]
     float(*ws)[EP][LDW] = (float(*)[EP][LDW])(rp_smem + 2 * TT * LDW);  // [2][EP][LDW]
     __shared__ float lg[TT][EP];
     __shared__ int hist[EP];
-    const int tid = threadIdx.x, tile = blockIdx.x, t0 = tile * TT;
-    if (tid < EP) hist[tid] = 0;
+    const int tid = threadIdx.x, t0 = tile * (SPLIT ? tpw : TT);
+    if (SPLIT) T = min(T, t0 + tpw);  // (tokens behind are another workgroup's)
+    if (!SPLIT && tid < EP) hist[tid] = 0;
     const int nch = (d + KC - 1) / KC;  // (the last chunk of an odd multiple of 256 is half full)
     if (tid >= CT) {
         // staging wave: thread st carries 8 consecutive k (16 bytes of bf16) of one row per load
@@ -740,9 +750,10 @@ __global__ __launch_bounds__(16 * EP + RP_STAGERS) void router_pipe_kernel(
 #undef ROUTER_FM
         }
         const float z = (bg != nullptr && e1 < E) ? a_ + bg[e1] : a_;
-        lg[tg][e1] = z;
-        if (logits_out != nullptr && t0 + tg < T && e1 < E) logits_out[(size_t)(t0 + tg) * E + e1] = z;
+        if (!SPLIT) lg[tg][e1] = z;
+        if ((SPLIT || logits_out != nullptr) && t0 + tg < T && e1 < E) logits_out[(size_t)(t0 + tg) * E_all + e0 + e1] = z;
     }
+    if (SPLIT) return;
     __syncthreads();
     if (tid < CT) {
         router_select<EP, false, TT, CT>(lg, hist, t0, tile, T, E, K, renorm, ids, wout, tile_counts, probs_out);
@@ -752,16 +763,35 @@ __global__ __launch_bounds__(16 * EP + RP_STAGERS) void router_pipe_kernel(
     }
 }
 
+// Selection from logits in memory, a workgroup per 16 tokens
+template <int EP>
+__global__ __launch_bounds__(256) void router_select_kernel(const float *__restrict__ logits, int T, int E, int K, int renorm,
+                                                            int32_t *__restrict__ ids, float *__restrict__ wout,
+                                                            int32_t *__restrict__ tile_counts, float *__restrict__ probs_out)
+{
+    __shared__ float lg[16][EP];
+    __shared__ int hist[EP];
+    const int tid = threadIdx.x, t0 = blockIdx.x * 16;
+    for (int i = tid; i < EP; i += 256) hist[i] = 0;
+    for (int i = tid; i < 16 * EP; i += 256) {
+        const int tt = i / EP, e = i % EP;
+        lg[tt][e] = e < E && t0 + tt < T ? logits[(size_t)(t0 + tt) * E + e] : 0.0f;
+    }
+    __syncthreads();
+    router_select<EP, false, 16, 256>(lg, hist, t0, blockIdx.x, T, E, K, renorm, ids, wout, tile_counts, probs_out);
+}
+
 int router_pipe_smem_bytes(int EP) { return 2 * (16 + EP) * RP_LDW * (int)sizeof(float); }
 
 hipError_t router_init(void)
 {
-    hipError_t e = hipFuncSetAttribute((const void *)router_pipe_kernel<8>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       router_pipe_smem_bytes(8));
-    if (e == hipSuccess)
-        e = hipFuncSetAttribute((const void *)router_pipe_kernel<16>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                router_pipe_smem_bytes(16));
-    return e;
+    const struct { const void *f; int ep; } fns[] = {{(const void *)router_pipe_kernel<8, false>, 8}, {(const void *)router_pipe_kernel<16, false>, 16},
+                                                     {(const void *)router_pipe_kernel<16, true>, 16}};
+    for (const auto &k : fns) {
+        hipError_t e = hipFuncSetAttribute(k.f, hipFuncAttributeMaxDynamicSharedMemorySize, router_pipe_smem_bytes(k.ep));
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 hipError_t launch_router(const omega_moe *m, const void *x, int T, float *logits_out, float *probs_out, hipStream_t s)
@@ -779,6 +809,28 @@ hipError_t launch_router(const omega_moe *m, const void *x, int T, float *logits
         else if (c.E <= 128) ROUTER_MFMA_LAUNCH(128);
         else ROUTER_MFMA_LAUNCH(256);
 #undef ROUTER_MFMA_LAUNCH
+        return hipGetLastError();
+    }
+    // (tokens per workgroup of the split form: the fewest that leave a workgroup a compute unit of its own, 4 are one wave of sums;
+    // short rows of few experts are as quick in one launch: 100 tokens x 1024, 20 experts 10.0 / 10.2 us, 16 x 1024, 64 experts 11.6 / 11.7)
+    const int groups = ceil_div(c.E, 16);
+    int tpw = 4;
+    while (tpw < 16 && ceil_div(T, tpw) * groups > m->ctx->num_cus) tpw *= 2;
+    if (router_on_mfma(m) && (logits_out != nullptr || m->gate_logits != nullptr) && router_tok_tile(m, T) == 16 &&
+        ceil_div(T, tpw) * groups <= m->ctx->num_cus && (c.E > 64 || (tpw < 16 && c.d > 1024)) && (((uintptr_t)x | (uintptr_t)m->Wg) % 16) == 0) {
+        float *lg = logits_out != nullptr ? logits_out : m->gate_logits;
+        hipLaunchKernelGGL((router_pipe_kernel<16, true>), dim3(ceil_div(T, tpw) * groups), dim3(16 * 16 + RP_STAGERS), router_pipe_smem_bytes(16),
+                           s, (const bf16_t *)x, (const bf16_t *)m->Wg, bg, T, c.d, c.E, c.K, c.renorm, m->ids, m->w, m->tile_counts, lg,
+                           (float *)nullptr, groups, tpw);
+        hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+#define ROUTER_SELECT(EPV) \
+    hipLaunchKernelGGL(router_select_kernel<EPV>, dim3(tiles), dim3(256), 0, s, (const float *)lg, T, c.E, c.K, c.renorm, m->ids, m->w, m->tile_counts, probs_out)
+        if (c.E <= 32) ROUTER_SELECT(32);
+        else if (c.E <= 64) ROUTER_SELECT(64);
+        else if (c.E <= 128) ROUTER_SELECT(128);
+        else ROUTER_SELECT(256);
+#undef ROUTER_SELECT
         return hipGetLastError();
     }
     if (router_on_mfma(m)) {
@@ -805,13 +857,13 @@ hipError_t launch_router(const omega_moe *m, const void *x, int T, float *logits
     if (c.dtype == OMEGA_DTYPE_BF16 && c.E <= 16 && tiles <= m->ctx->num_cus &&
         (((uintptr_t)x | (uintptr_t)m->Wg) % 16) == 0) {
         if (c.E <= 8)
-            hipLaunchKernelGGL(router_pipe_kernel<8>, dim3(tiles), dim3(16 * 8 + RP_STAGERS), router_pipe_smem_bytes(8), s,
+            hipLaunchKernelGGL((router_pipe_kernel<8, false>), dim3(tiles), dim3(16 * 8 + RP_STAGERS), router_pipe_smem_bytes(8), s,
                                (const bf16_t *)x, (const bf16_t *)m->Wg, bg, T, c.d, c.E, c.K, c.renorm, m->ids, m->w,
-                               m->tile_counts, logits_out, probs_out);
+                               m->tile_counts, logits_out, probs_out, 1, 16);
         else
-            hipLaunchKernelGGL(router_pipe_kernel<16>, dim3(tiles), dim3(16 * 16 + RP_STAGERS), router_pipe_smem_bytes(16), s,
+            hipLaunchKernelGGL((router_pipe_kernel<16, false>), dim3(tiles), dim3(16 * 16 + RP_STAGERS), router_pipe_smem_bytes(16), s,
                                (const bf16_t *)x, (const bf16_t *)m->Wg, bg, T, c.d, c.E, c.K, c.renorm, m->ids, m->w,
-                               m->tile_counts, logits_out, probs_out);
+                               m->tile_counts, logits_out, probs_out, 1, 16);
         return hipGetLastError();
     }
 #define ROUTER_LAUNCH(EPV, KCV)                                                                                    \

@@ -7,6 +7,7 @@ import pytest
 from oracle import oracle as O
 from oracle import oracle_np as N
 from tests.synth import C, scaled
+from tests.test_gpu_router_units import test_exact_logits_bit_for_bit as logits_bit_for_bit
 
 pytestmark = pytest.mark.gpu
 
@@ -29,3 +30,9 @@ def test_widths_between_chunks(name, kw):
     assert N.rel_l2(out, ref["out"]) <= (1e-2 if cfg.dtype == "bf16" else 1e-5)
     x.free()
     layer.close()
+
+
+# the sums split by experts: 4, 8 and 16 tokens per workgroup, a last group of one expert, of fifteen, ragged token groups
+@pytest.mark.parametrize("T,d,E,K", [(3, 1536, 17, 2), (5, 3328, 31, 3), (131, 1280, 64, 6), (500, 1280, 40, 2), (500, 512, 100, 4), (257, 256, 241, 8)])
+def test_sums_split_by_experts(T, d, E, K):
+    logits_bit_for_bit(T, d, E, K)
