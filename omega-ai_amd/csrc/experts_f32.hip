@@ -24,7 +24,8 @@
 // (up product, ragged tiles and the last round included: MFMA busy 0.80 and 125 TFLOP/s at k = 1024, 0.82 and 124 at k =
 // 8192).  No vector instruction but the address sums of the loads is spent per step.
 // The down and the input-gradient product, which have the fewest column tiles, take tiles of 128 x 64 (N = 1024, 8192
-// rows: 0.65 -> 0.55 and 1.26 -> 1.10 ms: 544 tiles of 128 x 128 leave the third round of two per compute unit nearly empty).
+// rows: 0.65 -> 0.55 and 1.26 -> 1.10 ms: 544 tiles of 128 x 128 leave the third round of two per compute unit nearly empty;
+// 0.49 and 0.99 since a nearly empty last round goes in parts).
 // A small batch leaves compute units idle and is as long as the chain of one wave: its tiles are 32 x 32 of four waves with
 // one block of v_mfma_f32_16x16x4 each (the same rate, four k in 32 cycles instead of two in 64) and steps of 64 k, so a wave's
 // chain is a quarter of that of the 64 x 64 tiles they replace.  Forward pass of 8 experts, top 2, us: 256 tokens x 128 x 256
@@ -37,8 +38,8 @@
 // it); what they bring meets a zero (k past the end) or is never stored.
 //
 // T = 4096, d = 1024, H = 3584, E = 8, K = 2 (8192 rows), ms, before (64 x 64 tiles for the forward products, FMA kernels
-// for the others) and now: up 1.14 -> 0.96 (125 TFLOP/s), down 0.63 -> 0.55 (109), h1 and h3 again 1.91 -> 0.97, d(a) 1.08 -> 0.58,
-// dxg 3.00 -> 1.10, dW2 0.99 -> 0.48, dW1 and dW3 2.01 -> 0.94.
+// for the others) and now: up 1.14 -> 0.96 (125 TFLOP/s), down 0.63 -> 0.49 (124), h1 and h3 again 1.91 -> 0.97, d(a) 1.08 -> 0.58,
+// dxg 3.00 -> 0.99, dW2 0.99 -> 0.48, dW1 and dW3 2.01 -> 0.94.
 #include "common.h"
 #include <algorithm>
 #include <cmath>
@@ -58,7 +59,8 @@ template <> struct f32_block<16> {
 
 // LDS row stride in floats of an operand kept [row][FBK]: 16 consecutive rows start in 16 different groups of four banks
 #define F32_LD_ROW (FBK + 4)
-#define F32_LDS_FLOATS(TX, KMAJ) ((KMAJ) ? FBK * ((TX) + 4) : (TX) * F32_LD_ROW)
+#define F32_FBK(TM) ((TM) == F32_TILE_M_SMALL ? 64 : 32)  // k places of a step
+constexpr int f32_lds_floats(int tx, bool kmaj, int fbk) { return kmaj ? fbk * (tx + 4) : tx * (fbk + 4); }
 
 // Pieces of one step of FBK k places that a thread carries: NV x 4 floats.  [row][k]: row r0 + (1024/FBK) u, 4 consecutive
 // k; [k][column]: k place k0 + (1024/TX) u, 4 consecutive columns.
@@ -120,10 +122,13 @@ struct f32_args {
     const int32_t *tile_meta, *counts;
     int N, Kd;               // row products: output columns and k; F32_WG*: columns and rows of one dW (k is the group's rows)
     int E, G, T, bm;
+    int slots, part_max;     // workgroups an XCD holds at a time; tiles of a last round that go in parts
 };
 
 #define F32_IS_WG(OP) ((OP) == F32_WG2 || (OP) == F32_WG13)
 #define F32_PAIR(OP) ((OP) == F32_UP || (OP) == F32_RAW)
+// parts of 32 rows x 32 output columns that a row product's tile of 128 rows may be cut into
+#define F32_PARTS(OP, TM) (F32_IS_WG(OP) || (TM) != F32_TILE_M ? 1 : (OP) == F32_DA ? 16 : 8)
 
 // Gathered rows of a launch whose product workgroups fetch theirs from the tokens (a wave per token, the row read once and
 // written to its K places): the backward pass reads them.  Beside the products instead of a launch in front of them.
@@ -152,47 +157,23 @@ __device__ __forceinline__ void copy_gathered(const f32_args &p, int wg, int lan
     }
 }
 
+// One tile: row tile mt from its row r0 on (row products) or from row mt * TM of gradient matrix mat, and columns n0 ..; as and bs
+// hold both operands of a row product twice.  (Weight gradients keep arrays of their own: read through pointers dW1 and dW3 of 4096
+// tokens x 1024 x 3584, 8 experts, took 936 us instead of 915.  For the same reason p is a copy.)
 template <int OP, int TM, int TN, bool VEC>
-__global__ __launch_bounds__(256, 2) void f32_product_kernel(f32_args p)
+__device__ __forceinline__ void f32_tile(const f32_args p, float *as, float *bs, int mt, int r0, int n0, int mat)
 {
     constexpr bool WG = F32_IS_WG(OP), PAIR = F32_PAIR(OP);
     constexpr bool AK = WG, BK_ = WG || OP == F32_DA || OP == F32_DXG;  // operand contiguous across k
-    constexpr int BS = TM == F32_TILE_M_SMALL ? 16 : 32, GK = 256 / BS, FBK = 4 * GK;  // blocks; k places of a group and of a step
+    constexpr int BS = TM == F32_TILE_M_SMALL ? 16 : 32, GK = 256 / BS, FBK = F32_FBK(TM);  // blocks; k places of a group
     constexpr int MB = TM / (2 * BS), NB = TN / (2 * BS), NVA = TM * FBK / 1024, NVB = TN * FBK / 1024, NR = BS * BS / 64;
     typedef typename f32_block<BS>::acc_t acc_t;
     constexpr int CT = PAIR ? TN / 2 : TN;                             // output columns per tile
-    __shared__ __attribute__((aligned(16))) float As[2][F32_LDS_FLOATS(TM, AK)];
-    __shared__ __attribute__((aligned(16))) float Bs[2][F32_LDS_FLOATS(TN, BK_)];
+    constexpr int LA = f32_lds_floats(TM, AK, FBK), LB = f32_lds_floats(TN, BK_, FBK);
+    __shared__ __attribute__((aligned(16))) float As[2][WG ? LA : 1];
+    __shared__ __attribute__((aligned(16))) float Bs[2][WG ? LB : 1];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lb = lane % BS, kh = lane / BS, wr = wave >> 1, wc = wave & 1;
-    if (OP == F32_UP && (int)blockIdx.x >= (int)gridDim.x - p.copy_wgs) {
-        copy_gathered<VEC>(p, blockIdx.x - (gridDim.x - p.copy_wgs), lane, wave);
-        return;
-    }
-
-    // Tile of this workgroup.  Consecutive workgroups go round the eight XCDs.  Row products: XCD x takes the x-th eighth of the tiles, and
-    // within it up to 8 row tiles walk the column tiles together, so that its workgroups share operand rows in its L2.  Weight
-    // gradients, whose length is the expert's rows: every XCD takes an eighth of every matrix, in the same order.  (An eighth of all
-    // tiles each left the other XCDs idle behind the one with the longest expert.  Backward pass, us: 3000 tokens x 512 x 1024, 16 experts,
-    // Zipf 911 -> 535; 4096 x 256 x 512, 6 experts and a shared one 375 -> 340; 4096 x 1024 x 3584, 8 even experts 3223 -> 3196.)
-    const int NT = (p.N + CT - 1) / CT;
-    const int MT = WG ? (p.Kd + TM - 1) / TM : p.tile_meta[0];  // row tiles (of one gradient matrix)
-    const int mats = OP == F32_WG13 ? 2 * p.G : OP == F32_WG2 ? p.G : 1;
-    const int total = MT * NT * mats, x = blockIdx.x & 7, j = blockIdx.x >> 3;
-    int t, mat = 0;
-    if (WG) {
-        const int c = max(1, (MT * NT) >> 3);
-        t = ((j / c) * 8 + x) * c + j % c;
-        if (t >= total) return;
-        mat = t / (MT * NT);
-        t -= mat * MT * NT;
-    } else {
-        const int per = (total + 7) >> 3;
-        t = x * per + j;
-        if (j >= per || t >= total) return;
-    }
-    const int rb = t / (8 * NT), nrb = min(8, MT - 8 * rb), ti = t - rb * 8 * NT;
-    const int mt = 8 * rb + ti % nrb, n0 = (ti / nrb) * CT;
 
     int g, rows, K1, row0 = 0, m0 = 0;
     const float *A0, *A1 = nullptr, *B0, *B1 = nullptr;
@@ -210,13 +191,14 @@ __global__ __launch_bounds__(256, 2) void f32_product_kernel(f32_args p)
     } else {
         const omega_tile tl = p.tiles[mt];
         g = tl.g;
-        rows = tl.rows;
-        row0 = tl.row0;
+        rows = min(TM, tl.rows - r0);
+        if (rows <= 0 || n0 >= p.N) return;  // (a part of a ragged tile)
+        row0 = tl.row0 + r0;
         K1 = p.Kd;
-        A0 = p.Atok && tl.xrow0 >= 0 ? p.Atok + (size_t)tl.xrow0 * p.Kd : p.A0 + (size_t)tl.row0 * p.Kd;
+        A0 = p.Atok && tl.xrow0 >= 0 ? p.Atok + (size_t)(tl.xrow0 + r0) * p.Kd : p.A0 + (size_t)row0 * p.Kd;
         fetch_rows = OP == F32_UP && p.tokp != nullptr && tl.xrow0 < 0;
         if (fetch_rows) A0 = p.Atok;
-        if (OP == F32_DXG) A1 = p.A1 + (size_t)tl.row0 * p.Kd;
+        if (OP == F32_DXG) A1 = p.A1 + (size_t)row0 * p.Kd;
         B0 = p.B0 + (size_t)g * p.N * p.Kd;
         if (PAIR || OP == F32_DXG) B1 = p.B1 + (size_t)g * p.N * p.Kd;
     }
@@ -274,8 +256,8 @@ __global__ __launch_bounds__(256, 2) void f32_product_kernel(f32_args p)
     auto fetch_b = [&](int u) {
         vb[u] = fetch_piece<BK_, VEC>(PAIR && u >= NVB / 2 ? b3_at : b_at, ob[u], f32_piece<TN, BK_, FBK>::x(tid, u), p.N - n0);
     };
-    auto put_a = [&](int c, int u) { *(float4 *)&As[c][f32_piece<TM, AK, FBK>::lds(tid, u)] = va[u]; };
-    auto put_b = [&](int c, int u) { *(float4 *)&Bs[c][f32_piece<TN, BK_, FBK>::lds(tid, u)] = vb[u]; };
+    auto put_a = [&](int c, int u) { *(float4 *)&(WG ? As[c] : as + c * LA)[f32_piece<TM, AK, FBK>::lds(tid, u)] = va[u]; };
+    auto put_b = [&](int c, int u) { *(float4 *)&(WG ? Bs[c] : bs + c * LB)[f32_piece<TN, BK_, FBK>::lds(tid, u)] = vb[u]; };
     // the load pointers move on to step s (which the next loads bring); behind the last one they stay
     auto advance = [&](int s) {
         if (s >= steps) return;
@@ -298,8 +280,8 @@ __global__ __launch_bounds__(256, 2) void f32_product_kernel(f32_args p)
         float4 fa[2][MBL > 0 ? MBL : 1], fb[2][NB];
         auto read = [&](int set, int c, int j, int r) {
             const int k = GK * j + 4 * kh;
-            if (r < MBL) fa[set][r < MBL ? r : 0] = frag<TM, AK, FBK>(As[c], xa + 2 * BS * r, k);
-            else if (r < NF) fb[set][r - MBL < NB ? r - MBL : 0] = frag<TN, BK_, FBK>(Bs[c], xb[r - MBL < NB ? r - MBL : 0], k);
+            if (r < MBL) fa[set][r < MBL ? r : 0] = frag<TM, AK, FBK>(WG ? As[c] : as + c * LA, xa + 2 * BS * r, k);
+            else if (r < NF) fb[set][r - MBL < NB ? r - MBL : 0] = frag<TN, BK_, FBK>(WG ? Bs[c] : bs + c * LB, xb[r - MBL < NB ? r - MBL : 0], k);
         };
         auto group = [&](auto cc, auto jj) {
             constexpr int c = decltype(cc)::value, j = decltype(jj)::value;
@@ -448,6 +430,65 @@ __global__ __launch_bounds__(256, 2) void f32_product_kernel(f32_args p)
     }
 }
 
+template <int OP, int TM, int TN, bool VEC>
+__global__ __launch_bounds__(256, 2) void f32_product_kernel(f32_args p)
+{
+    constexpr bool WG = F32_IS_WG(OP), PAIR = F32_PAIR(OP), PARTS = F32_PARTS(OP, TM) > 1;
+    constexpr int CT = PAIR ? TN / 2 : TN;                             // output columns per tile
+    constexpr bool BK_ = WG || OP == F32_DA || OP == F32_DXG;
+    constexpr int PN = PAIR ? 64 : 32;                                 // MFMA columns of a part
+    constexpr int LA = f32_lds_floats(TM, WG, F32_FBK(TM)), LB0 = f32_lds_floats(TN, BK_, F32_FBK(TM));
+    constexpr int LB = PARTS && f32_lds_floats(PN, BK_, F32_FBK(32)) > LB0 ? f32_lds_floats(PN, BK_, F32_FBK(32)) : LB0;
+    static_assert(!PARTS || f32_lds_floats(32, WG, F32_FBK(32)) <= LA, "a part's rows fit");
+    __shared__ __attribute__((aligned(16))) float as[WG ? 1 : 2 * LA], bs[WG ? 1 : 2 * LB];
+    if (OP == F32_UP && (int)blockIdx.x >= (int)gridDim.x - p.copy_wgs) {
+        copy_gathered<VEC>(p, blockIdx.x - (gridDim.x - p.copy_wgs), threadIdx.x & 63, threadIdx.x >> 6);
+        return;
+    }
+
+    // Tile of this workgroup.  Consecutive workgroups go round the eight XCDs.  Row products: XCD x takes the x-th eighth of the tiles, and
+    // within it up to 8 row tiles walk the column tiles together, so that its workgroups share operand rows in its L2.  Weight
+    // gradients, whose length is the expert's rows: every XCD takes an eighth of every matrix, in the same order.  (An eighth of all
+    // tiles each left the other XCDs idle behind the one with the longest expert.  Backward pass, us: 3000 tokens x 512 x 1024, 16 experts,
+    // Zipf 911 -> 535; 4096 x 256 x 512, 6 experts and a shared one 375 -> 340; 4096 x 1024 x 3584, 8 even experts 3223 -> 3196.)
+    const int NT = (p.N + CT - 1) / CT;
+    const int MT = WG ? (p.Kd + TM - 1) / TM : p.tile_meta[0];  // row tiles (of one gradient matrix)
+    const int mats = OP == F32_WG13 ? 2 * p.G : OP == F32_WG2 ? p.G : 1;
+    const int total = MT * NT * mats, x = blockIdx.x & 7, j = blockIdx.x >> 3;
+    int t, mat = 0, part = -1;
+    if (WG) {
+        const int c = max(1, (MT * NT) >> 3);
+        t = ((j / c) * 8 + x) * c + j % c;
+        if (t >= total) return;
+        mat = t / (MT * NT);
+        t -= mat * MT * NT;
+    } else {
+        // Tiles of 128 rows: where at least one whole round of p.slots workgroups is followed by a last one of a quarter or less of it
+        // (p.part_max), that last round's tiles go in parts of 32 rows x 32 columns: eight or sixteen workgroups share what one would
+        // work on while the rest of the XCD idles.  Down product of 8192 rows, k = 3584, N = 1024 (two rounds and 12 of 64 tiles) 540 -> 486
+        // us, dxg 1090 -> 986.  Parts cost more per element than a tile: k = 1536, rounds and rest, us in tiles / parts: 1 + 16
+        // 143 / 132, 1 + 24 145 / 149, 1 + 32 149 / 165, 2 + 8 236 / 210, 2 + 24 238 / 247.
+        const int per = (total + 7) >> 3, rest = per % p.slots;
+        int i = j;
+        if (PARTS && rest <= p.part_max && per >= p.slots && j >= per - rest) {
+            part = (j - (per - rest)) % F32_PARTS(OP, TM);
+            i = per - rest + (j - (per - rest)) / F32_PARTS(OP, TM);
+        }
+        t = x * per + i;
+        if (i >= per || t >= total) return;
+    }
+    const int rb = t / (8 * NT), nrb = min(8, MT - 8 * rb), ti = t - rb * 8 * NT;
+    const int mt = 8 * rb + ti % nrb, n0 = (ti / nrb) * CT;
+
+    if constexpr (PARTS) {
+        if (part >= 0) {
+            f32_tile<OP, 32, PN, VEC>(p, as, bs, mt, 32 * (part & 3), n0 + 32 * (part >> 2), mat);
+            return;
+        }
+    }
+    f32_tile<OP, TM, TN, VEC>(p, as, bs, mt, 0, n0, mat);
+}
+
 // The largest row-tile height that a batch of up to T tokens takes: with fewer than 128 rows per expert always 32 (160 shapes of
 // 1 to 4096 tokens, d = 64 .. 1024, H = 64 .. 3584, 2 to 16 experts: tiles of 64 took 0.97 to 1.90 times as long)
 int experts_f32_tile_m_max(const omega_moe *m, int T)
@@ -497,7 +538,8 @@ static hipError_t f32_launch(const f32_args &p, bool vec, int max_tiles, hipStre
     const size_t tiles = (size_t)ceil_div(p.N, CT) * (F32_IS_WG(OP) ? (size_t)ceil_div(p.Kd, TM) * p.G * (OP == F32_WG13 ? 2 : 1) : max_tiles);
     // (weight gradients: to eight parts of a matrix)
     const size_t c = F32_IS_WG(OP) ? std::max((size_t)1, (size_t)ceil_div(p.N, CT) * ceil_div(p.Kd, TM) / 8) : 1;
-    const unsigned grid = (unsigned)(F32_IS_WG(OP) ? (tiles + 8 * c - 1) / (8 * c) * (8 * c) : (tiles + 7) / 8 * 8) + p.copy_wgs;
+    const size_t parts = F32_PARTS(OP, TM) > 1 && (tiles + 7) / 8 >= (size_t)p.slots ? (size_t)8 * p.part_max * (F32_PARTS(OP, TM) - 1) : 0;
+    const unsigned grid = (unsigned)(F32_IS_WG(OP) ? (tiles + 8 * c - 1) / (8 * c) * (8 * c) : (tiles + 7) / 8 * 8 + parts) + p.copy_wgs;
     if (vec) hipLaunchKernelGGL((f32_product_kernel<OP, TM, TN, true>), dim3(grid), dim3(256), 0, s, p);
     else hipLaunchKernelGGL((f32_product_kernel<OP, TM, TN, false>), dim3(grid), dim3(256), 0, s, p);
     return hipGetLastError();
@@ -514,6 +556,8 @@ hipError_t launch_product_f32(const omega_moe *m, int op, const float *x, const 
     p.G = m->G;
     p.T = T;
     p.bm = m->bm;
+    p.slots = 2 * (m->ctx->num_cus / 8);  // (two of the large tiles' workgroups per compute unit)
+    p.part_max = p.slots / 4;
     const float *W1 = (const float *)m->W1, *W3 = (const float *)m->W3, *W2 = (const float *)m->W2;
     switch (op) {
         case F32_UP:

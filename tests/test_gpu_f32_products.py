@@ -204,3 +204,21 @@ def test_timed_backward_passes_leave_the_gradients_of_one():
     got = [dx.to_numpy(), layer.grad(L.W_GATE), layer.grad(L.W_W1, 1), layer.grad(L.W_W2, 3)]
     assert all(np.array_equal(a, b) for a, b in zip(got, want))
     layer.close()
+
+
+@pytest.mark.parametrize("T,d,H,E", [(5377, 195, 483, 3), (5662, 200, 412, 3), (5087, 76, 452, 2)])
+def test_last_round_of_tiles_in_parts(T, d, H, E):
+    """Tiles of 128 rows whose eighth is one round of 64, or two, and at most 16 more, which go in parts of 32 x 32: every product
+    without 16-byte loads, a single row in an expert's last tile and 35 columns in a product's; down, d(a) and input gradient with
+    16-byte loads; up with them."""
+    G, cfg, inp, dout, layer = _setup("c1_tiny_f32", dict(T=T, d=d, H=H, E=E, K=E), 85)
+    x = G.P.DeviceBuffer.from_numpy(G.ctx(), inp["x"], cfg.dtype)
+    g = G.P.DeviceBuffer.from_numpy(G.ctx(), dout, cfg.dtype)
+    out = layer.forward(x).to_numpy()
+    ref = G.oracle_forward(cfg, inp)["out"]
+    assert N.rel_l2(out, ref) < 1e-5 and N.rel_l2(out[-3:], ref[-3:]) < 1e-5
+    dx = layer.back(g).to_numpy()
+    ref = O.moe_backward(inp["x"], dout, inp["Wg"], inp["bg"], inp["W1"], inp["W3"], inp["W2"], cfg.K, cfg.renorm, cfg.Es)
+    assert N.rel_l2(dx, ref["dx"]) < 1e-5
+    _check_grads(layer, cfg, ref, 1e-5)
+    layer.close()
