@@ -127,8 +127,9 @@ struct f32_args {
 
 #define F32_IS_WG(OP) ((OP) == F32_WG2 || (OP) == F32_WG13)
 #define F32_PAIR(OP) ((OP) == F32_UP || (OP) == F32_RAW)
-// parts of 32 rows x 32 output columns that a row product's tile of 128 rows may be cut into
-#define F32_PARTS(OP, TM) (F32_IS_WG(OP) || (TM) != F32_TILE_M ? 1 : (OP) == F32_DA ? 16 : 8)
+// parts of 32 rows x 32 output columns that a row product's tile of 128 or 64 rows may be cut into (the input gradient's of 64 rows
+// without 16-byte loads is left whole: the second body alone made its tiles slower, 38 -> 41 us at 2180 x 290 x 225)
+#define F32_PARTS(OP, TM, TN, VEC) (F32_IS_WG(OP) || (TM) == F32_TILE_M_SMALL || ((OP) == F32_DXG && (TM) == F32_TILE_M_MID && !(VEC)) ? 1 : (TM) / 32 * ((TN) / (F32_PAIR(OP) ? 64 : 32)))
 
 // Gathered rows of a launch whose product workgroups fetch theirs from the tokens (a wave per token, the row read once and
 // written to its K places): the backward pass reads them.  Beside the products instead of a launch in front of them.
@@ -433,7 +434,7 @@ __device__ __forceinline__ void f32_tile(const f32_args p, float *as, float *bs,
 template <int OP, int TM, int TN, bool VEC>
 __global__ __launch_bounds__(256, 2) void f32_product_kernel(f32_args p)
 {
-    constexpr bool WG = F32_IS_WG(OP), PAIR = F32_PAIR(OP), PARTS = F32_PARTS(OP, TM) > 1;
+    constexpr bool WG = F32_IS_WG(OP), PAIR = F32_PAIR(OP), PARTS = F32_PARTS(OP, TM, TN, VEC) > 1;
     constexpr int CT = PAIR ? TN / 2 : TN;                             // output columns per tile
     constexpr bool BK_ = WG || OP == F32_DA || OP == F32_DXG;
     constexpr int PN = PAIR ? 64 : 32;                                 // MFMA columns of a part
@@ -463,16 +464,18 @@ __global__ __launch_bounds__(256, 2) void f32_product_kernel(f32_args p)
         mat = t / (MT * NT);
         t -= mat * MT * NT;
     } else {
-        // Tiles of 128 rows: where at least one whole round of p.slots workgroups is followed by a last one of a quarter or less of it
-        // (p.part_max), that last round's tiles go in parts of 32 rows x 32 columns: eight or sixteen workgroups share what one would
-        // work on while the rest of the XCD idles.  Down product of 8192 rows, k = 3584, N = 1024 (two rounds and 12 of 64 tiles) 540 -> 486
-        // us, dxg 1090 -> 986.  Parts cost more per element than a tile: k = 1536, rounds and rest, us in tiles / parts: 1 + 16
-        // 143 / 132, 1 + 24 145 / 149, 1 + 32 149 / 165, 2 + 8 236 / 210, 2 + 24 238 / 247.
+        // Where at least one whole round of p.slots workgroups is followed by a last one of a quarter or less of it (p.part_max), that
+        // last round's tiles go in parts of 32 rows x 32 columns: the workgroups that would idle share what one would work on.  us in
+        // tiles / parts, tiles of 128 rows: down product of 8192 rows, k = 3584, N = 1024 (two rounds and 12 of 64 tiles) 540 / 486,
+        // dxg 1090 / 986; of 64 rows: up product of 4024 tokens x 928 x 252, 12 experts, top 2 (one round and 1) 93 / 74, down product of
+        // 2036 x 680 x 1980, 3 experts, top 3 (one round and 4 of 128) 173 / 152.  Parts cost more per element than a tile: k = 1536,
+        // N = 1024, 128 rows, rounds + rest: 1 + 16 143 / 132, 1 + 24 145 / 149, 1 + 32 149 / 165, 2 + 8 236 / 210, 2 + 24 238 / 247; forward
+        // passes with 64 rows and up's rest at 3/8 63.0 / 65.4, at 1/2 141 / 149.
         const int per = (total + 7) >> 3, rest = per % p.slots;
         int i = j;
         if (PARTS && rest <= p.part_max && per >= p.slots && j >= per - rest) {
-            part = (j - (per - rest)) % F32_PARTS(OP, TM);
-            i = per - rest + (j - (per - rest)) / F32_PARTS(OP, TM);
+            part = (j - (per - rest)) % F32_PARTS(OP, TM, TN, VEC);
+            i = per - rest + (j - (per - rest)) / F32_PARTS(OP, TM, TN, VEC);
         }
         t = x * per + i;
         if (i >= per || t >= total) return;
@@ -482,7 +485,7 @@ __global__ __launch_bounds__(256, 2) void f32_product_kernel(f32_args p)
 
     if constexpr (PARTS) {
         if (part >= 0) {
-            f32_tile<OP, 32, PN, VEC>(p, as, bs, mt, 32 * (part & 3), n0 + 32 * (part >> 2), mat);
+            f32_tile<OP, 32, PN, VEC>(p, as, bs, mt, 32 * (part % (TM / 32)), n0 + 32 * (part / (TM / 32)), mat);
             return;
         }
     }
@@ -532,13 +535,15 @@ int experts_f32_tile_m(const omega_moe *m, int T)
 }
 
 template <int OP, int TM, int TN>
-static hipError_t f32_launch(const f32_args &p, bool vec, int max_tiles, hipStream_t s)
+static hipError_t f32_launch(f32_args p, bool vec, int max_tiles, hipStream_t s)
 {
     constexpr int CT = F32_PAIR(OP) ? TN / 2 : TN;
     const size_t tiles = (size_t)ceil_div(p.N, CT) * (F32_IS_WG(OP) ? (size_t)ceil_div(p.Kd, TM) * p.G * (OP == F32_WG13 ? 2 : 1) : max_tiles);
     // (weight gradients: to eight parts of a matrix)
     const size_t c = F32_IS_WG(OP) ? std::max((size_t)1, (size_t)ceil_div(p.N, CT) * ceil_div(p.Kd, TM) / 8) : 1;
-    const size_t parts = F32_PARTS(OP, TM) > 1 && (tiles + 7) / 8 >= (size_t)p.slots ? (size_t)8 * p.part_max * (F32_PARTS(OP, TM) - 1) : 0;
+    p.slots *= TM == F32_TILE_M || F32_PAIR(OP) ? 2 : 4;  // (what LDS holds of the workgroups of tiles of 128 and 64 rows)
+    p.part_max = p.slots / 4;
+    const size_t parts = F32_PARTS(OP, TM, TN, vec) > 1 && (tiles + 7) / 8 >= (size_t)p.slots ? (size_t)8 * p.part_max * (F32_PARTS(OP, TM, TN, vec) - 1) : 0;
     const unsigned grid = (unsigned)(F32_IS_WG(OP) ? (tiles + 8 * c - 1) / (8 * c) * (8 * c) : (tiles + 7) / 8 * 8 + parts) + p.copy_wgs;
     if (vec) hipLaunchKernelGGL((f32_product_kernel<OP, TM, TN, true>), dim3(grid), dim3(256), 0, s, p);
     else hipLaunchKernelGGL((f32_product_kernel<OP, TM, TN, false>), dim3(grid), dim3(256), 0, s, p);
@@ -556,8 +561,7 @@ hipError_t launch_product_f32(const omega_moe *m, int op, const float *x, const 
     p.G = m->G;
     p.T = T;
     p.bm = m->bm;
-    p.slots = 2 * (m->ctx->num_cus / 8);  // (two of the large tiles' workgroups per compute unit)
-    p.part_max = p.slots / 4;
+    p.slots = m->ctx->num_cus / 8;  // (f32_launch: times the workgroups of a compute unit)
     const float *W1 = (const float *)m->W1, *W3 = (const float *)m->W3, *W2 = (const float *)m->W2;
     switch (op) {
         case F32_UP:

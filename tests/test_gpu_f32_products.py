@@ -206,11 +206,11 @@ def test_timed_backward_passes_leave_the_gradients_of_one():
     layer.close()
 
 
-@pytest.mark.parametrize("T,d,H,E", [(5377, 195, 483, 3), (5662, 200, 412, 3), (5087, 76, 452, 2)])
+@pytest.mark.parametrize("T,d,H,E", [(5377, 195, 483, 3), (5662, 200, 412, 3), (5087, 76, 452, 2), (2111, 724, 324, 3), (2113, 723, 323, 3)])
 def test_last_round_of_tiles_in_parts(T, d, H, E):
-    """Tiles of 128 rows whose eighth is one round of 64, or two, and at most 16 more, which go in parts of 32 x 32: every product
-    without 16-byte loads, a single row in an expert's last tile and 35 columns in a product's; down, d(a) and input gradient with
-    16-byte loads; up with them."""
+    """An eighth of the tiles is one or two rounds of what an XCD holds (64; 128 of 64 x 64) and at most a quarter more, which goes in
+    parts of 32 x 32.  Tiles of 128 rows: every product without 16-byte loads, a single row in an expert's last tile and 35 columns in a
+    product's; down, d(a) and input gradient with 16-byte loads; up with them.  Of 64: up, down and input gradient."""
     G, cfg, inp, dout, layer = _setup("c1_tiny_f32", dict(T=T, d=d, H=H, E=E, K=E), 85)
     x = G.P.DeviceBuffer.from_numpy(G.ctx(), inp["x"], cfg.dtype)
     g = G.P.DeviceBuffer.from_numpy(G.ctx(), dout, cfg.dtype)
