@@ -569,7 +569,7 @@ int omega_moe_set_weights(omega_moe *m, int which, int expert, const void *src, 
 // are).  false: not for this kernel.
 static bool read_to_device(omega_moe *m, void *dst, const void *src, size_t bytes, int R, int Kd, hipError_t *e)
 {
-    if (launch_param_read == nullptr || (R == 0 && (((uintptr_t)dst | (uintptr_t)src) % 4 != 0 || bytes % 4 != 0))) return false;
+    if (R == 0 && (((uintptr_t)dst | (uintptr_t)src) % 4 != 0 || bytes % 4 != 0)) return false;
     *e = launch_param_read(dst, src, R, Kd, bytes / 4, m->ev1, m->ctx->stream);
     if (*e == hipSuccess) *e = hipEventSynchronize(m->ev1);
     return true;
@@ -659,7 +659,7 @@ static int ensure_queues(omega_moe *m, int T)
 static int ensure_y_whole(omega_moe *m)
 {
     if (!m->y_partial) return OMEGA_OK;
-    OMEGA_HIP_CHECK(m->ctx, launch_experts_bf16(m, nullptr, 0, 2, m->ctx->stream, false));
+    OMEGA_HIP_CHECK(m->ctx, launch_down_slab_reduce(m, m->y, m->ctx->stream));
     m->y_partial = false;
     return OMEGA_OK;
 }

@@ -224,7 +224,7 @@ enum { F32_UP = 0, F32_DOWN, F32_RAW, F32_DA, F32_DXG, F32_WG2, F32_WG13 };
 // bw_h1 / bw_h3, as launch_experts_bf16 does)
 hipError_t launch_product_f32(const omega_moe *m, int op, const float *x, const float *dout, int T, hipStream_t s, bool gather = false,
                               bool keep = false);
-// which: 0 up product, 1 down product, 2 the k slices the down product has left (y_partial) added into y
+// which: 0 up product, 1 down product
 hipError_t launch_experts_bf16(const omega_moe *m, const void *x, int T, int which, hipStream_t s, bool keep);
 hipError_t launch_experts_few(const omega_moe *m, const void *x, int T, int which, hipStream_t s);
 // resid != nullptr: out = resid + layer output (one rounding of the fp32 sum)
@@ -260,8 +260,7 @@ struct omega_adamw {
 hipError_t launch_update_adamw(const omega_moe *m, float *master, float *mw, float *vw, const omega_adamw &p, hipStream_t s);
 hipError_t launch_pack_rows(void *dst_packed, const void *src_rowmajor, int R, int Kd, hipStream_t s);
 hipError_t launch_unpack_rows(void *dst_rowmajor, const void *src_packed, int R, int Kd, hipStream_t s);
-// (weak: where api.hip runs without the kernels behind it, it reads by the runtime's copies)
-hipError_t launch_param_read(void *dst, const void *src, int R, int Kd, size_t n, hipEvent_t done, hipStream_t s) __attribute__((weak));
+hipError_t launch_param_read(void *dst, const void *src, int R, int Kd, size_t n, hipEvent_t done, hipStream_t s);
 int experts_bf16_tile_m(const omega_moe *m, int T);
 bool wgrad_on_four_waves(const omega_moe *m, int T, int M, int N);  // which kernel takes the weight gradients of M x N per expert
 #define F32_TILE_M 128       // row-tile heights of fp32 layers: experts_f32_tile_m chooses one per batch
@@ -270,7 +269,7 @@ bool wgrad_on_four_waves(const omega_moe *m, int T, int M, int N);  // which ker
 int experts_f32_tile_m(const omega_moe *m, int T);
 int experts_f32_tile_m_max(const omega_moe *m, int T);  // no batch of up to T tokens takes a larger one
 hipError_t experts_bf16_init(void);
-hipError_t launch_down_slab_reduce(const omega_moe *m, float *y, hipStream_t s);  // y += partial results of k-sliced items
+hipError_t launch_down_slab_reduce(const omega_moe *m, float *y, hipStream_t s);  // y += partial results of k-sliced items (y_partial)
 hipError_t router_init(void);  // kernel attributes of the router (LDS beyond 64 KiB), once per device
 
 // ---- device helpers ----

@@ -1162,7 +1162,6 @@ hipError_t experts_bf16_init(void)
 hipError_t launch_experts_bf16(const omega_moe *m, const void *x, int T, int which, hipStream_t s, bool keep)
 {
     const omega_moe_config &c = m->cfg;
-    if (which == 2) return launch_down_slab_reduce(m, m->y, s);
     if (m->few) return launch_experts_few(m, x, T, which, s);
     // the ring must be shorter than an item: K >= (NSTAGE + 1) * BK (guaranteed at creation: d, H >= 256)
     if ((which == 0 ? c.d : c.H) < (NSTAGE + 1) * BK) return hipErrorInvalidValue;

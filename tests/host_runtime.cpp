@@ -113,6 +113,7 @@ hipError_t launch_experts_bf16(const omega_moe *m, const void *, int, int which,
     if (keep && (!m->bw_h1 || !m->bw_h3)) return line("experts_bf16 without room for h1 and h3");
     return line("experts_bf16 which=%d keep=%d", which, keep);
 }
+hipError_t launch_down_slab_reduce(const omega_moe *, float *, hipStream_t) { return line("slab_reduce"); }
 hipError_t launch_combine(const omega_moe *, int, void *, const void *, hipStream_t) { return line("combine"); }
 hipError_t launch_backward_f32(omega_moe *m, const void *, const void *, int, void *, hipStream_t)
 {
@@ -145,3 +146,4 @@ hipError_t launch_sumsq_f32(const float *, size_t, double *, hipStream_t) { retu
 hipError_t launch_scale_f32(float *, float, size_t, hipStream_t) { return line("scale"); }
 hipError_t launch_pack_rows(void *, const void *, int, int, hipStream_t) { return line("pack"); }
 hipError_t launch_unpack_rows(void *, const void *, int, int, hipStream_t) { return line("unpack"); }
+hipError_t launch_param_read(void *, const void *, int R, int, size_t, hipEvent_t, hipStream_t) { return line(R > 0 ? "param_read of a packed image" : "param_read"); }

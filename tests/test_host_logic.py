@@ -193,3 +193,20 @@ def test_expert_blocks_of_the_optimiser_start_on_a_cache_line(lib, dtype, d, E):
         assert m.forward(8) == 0 and m.back(8) == 0
     m.close()
     assert lib.host_live_count() == 0
+
+
+def test_reads_into_device_memory_go_through_the_kernel(lib):
+    """The library does not load without it: there is no other way that a build which lost it could fall back to."""
+    import numpy as np
+    m = Layer(lib, "bf16")
+    assert m.forward(8) == 0 and m.back(8) == 0
+    p = C.c_void_p()
+    assert lib.omega_hip_malloc(m.ctx, 256 * 256 * 4, C.byref(p)) == 0
+    for get, which, line in ((lib.omega_moe_get_weights, L.W_W1, "param_read of a packed image"), (lib.omega_moe_get_weights, L.W_GATE, "param_read"),
+                             (lib.omega_moe_get_grad, L.W_W1, "param_read")):
+        m.log()
+        assert get(m.h, which, 0, p, 1) == 0 and m.log() == [line]
+        host = np.empty(256 * 256, np.float32)
+        assert get(m.h, which, 0, host.ctypes.data, 0) == 0 and line not in m.log()
+    assert lib.omega_hip_free(m.ctx, p) == 0
+    m.close()
