@@ -565,11 +565,25 @@ int omega_moe_set_weights(omega_moe *m, int which, int expert, const void *src, 
     return OMEGA_OK;
 }
 
+// Whether the n bytes at p are memory of the context's own device: what a kernel may store to.  Another device's, managed or host
+// memory, and a pointer or an end that the runtime does not know, are the runtime's to copy or to refuse.  (0.1 to 0.3 us of a read of 9 to 11.)
+static bool own_device_memory(const omega_ctx *ctx, const void *p, size_t n)
+{
+    hipPointerAttribute_t at;
+    hipDeviceptr_t base = nullptr;
+    size_t size = 0;
+    const bool known = hipPointerGetAttributes(&at, p) == hipSuccess && at.type == hipMemoryTypeDevice && at.device == ctx->device &&
+                       hipMemGetAddressRange(&base, &size, (hipDeviceptr_t)p) == hipSuccess;
+    if (!known) (void)hipGetLastError();  // (the next launch would report it)
+    return known && n <= size - (size_t)((const char *)p - (const char *)base);
+}
+
 // A weight or gradient into device memory of the caller, there when the call returns (R rows of a packed image, or bytes as they
 // are).  false: not for this kernel.
 static bool read_to_device(omega_moe *m, void *dst, const void *src, size_t bytes, int R, int Kd, hipError_t *e)
 {
     if (R == 0 && (((uintptr_t)dst | (uintptr_t)src) % 4 != 0 || bytes % 4 != 0)) return false;
+    if (!own_device_memory(m->ctx, dst, bytes)) return false;
     *e = launch_param_read(dst, src, R, Kd, bytes / 4, m->ev1, m->ctx->stream);
     if (*e == hipSuccess) *e = hipEventSynchronize(m->ev1);
     return true;
@@ -599,11 +613,11 @@ int omega_moe_get_weights(omega_moe *m, int which, int expert, void *dst, int is
         return OMEGA_OK;
     }
     void *stage = nullptr;
-    if (!is_device) OMEGA_HIP_CHECK(ctx, hipMalloc(&stage, bytes));
-    e = launch_unpack_rows(is_device ? dst : stage, p, R, Kd, ctx->stream);
-    if (e == hipSuccess && !is_device) e = hipMemcpyAsync(dst, stage, bytes, hipMemcpyDeviceToHost, ctx->stream);
+    OMEGA_HIP_CHECK(ctx, hipMalloc(&stage, bytes));
+    e = launch_unpack_rows(stage, p, R, Kd, ctx->stream);
+    if (e == hipSuccess) e = hipMemcpyAsync(dst, stage, bytes, is_device ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost, ctx->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-    if (stage) hipFree(stage);
+    hipFree(stage);
     OMEGA_HIP_CHECK(ctx, e);
     return OMEGA_OK;
 }

@@ -12,6 +12,7 @@
 #include "common.h"
 
 static std::map<void *, size_t> g_live;
+static std::map<void *, int> g_device;  // blocks of another device than 0
 static size_t g_bytes;
 static int g_fail_in;  // > 0: the allocation with this number from now on fails
 static hipError_t g_last = hipSuccess;
@@ -34,6 +35,7 @@ static hipError_t line(const char *fmt, ...)
 extern "C" {
 
 void host_fail_allocation(int n) { g_fail_in = n; }
+void host_move_to_device(void *p, int device) { g_device[p] = device; }
 size_t host_live_bytes(void) { return g_bytes; }
 int host_live_count(void) { return (int)g_live.size(); }
 const char *host_take_log(void)
@@ -61,11 +63,43 @@ hipError_t hipFree(void *p)
     if (it == g_live.end()) abort();  // freed twice, or never allocated
     g_bytes -= it->second;
     g_live.erase(it);
+    g_device.erase(p);
     free(p);
     return hipSuccess;
 }
 hipError_t hipMemsetAsync(void *p, int v, size_t n, hipStream_t) { memset(p, v, n); return hipSuccess; }
-hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t) { memcpy(d, s, n); return hipSuccess; }
+// the allocation that p points into
+static std::map<void *, size_t>::iterator live_at(const void *p)
+{
+    auto it = g_live.upper_bound((void *)p);
+    if (it == g_live.begin() || (char *)p >= (char *)(--it)->first + it->second) return g_live.end();
+    return it;
+}
+hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind kind, hipStream_t)
+{
+    auto it = live_at(d);
+    if (it != g_live.end() && (char *)d + n > (char *)it->first + it->second) return g_last = hipErrorInvalidValue;
+    g_log += kind == hipMemcpyDeviceToDevice ? "copy\n" : "";
+    memcpy(d, s, n);
+    return hipSuccess;
+}
+hipError_t hipPointerGetAttributes(hipPointerAttribute_t *a, const void *p)
+{
+    auto it = live_at(p);
+    if (it == g_live.end()) return g_last = hipErrorInvalidValue;
+    memset(a, 0, sizeof *a);
+    a->type = hipMemoryTypeDevice;
+    a->device = g_device.count(it->first) ? g_device[it->first] : 0;
+    return hipSuccess;
+}
+hipError_t hipMemGetAddressRange(hipDeviceptr_t *base, size_t *size, hipDeviceptr_t p)
+{
+    auto it = live_at(p);
+    if (it == g_live.end()) return g_last = hipErrorInvalidValue;
+    *base = it->first;
+    *size = it->second;
+    return hipSuccess;
+}
 hipError_t hipGetLastError(void) { hipError_t e = g_last; g_last = hipSuccess; return e; }
 const char *hipGetErrorString(hipError_t e) { return e == hipErrorOutOfMemory ? "out of memory" : "error"; }
 hipError_t hipGetDeviceCount(int *n) { *n = 1; return hipSuccess; }

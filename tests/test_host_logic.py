@@ -210,3 +210,38 @@ def test_reads_into_device_memory_go_through_the_kernel(lib):
         assert get(m.h, which, 0, host.ctypes.data, 0) == 0 and line not in m.log()
     assert lib.omega_hip_free(m.ctx, p) == 0
     m.close()
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_the_kernel_stores_to_memory_of_its_own_device_only(lib, dtype):
+    """Where the caller's buffer is host memory, another device's, unknown or too short, the runtime copies - or refuses - as it
+    always did, and leaves no error behind."""
+    import numpy as np
+    m = Layer(lib, dtype)
+    n = 256 * 256 * 4
+    assert m.forward(8) == 0 and m.back(8) == 0
+    p = C.c_void_p()
+    assert lib.omega_hip_malloc(m.ctx, n, C.byref(p)) == 0
+    lib.host_move_to_device.argtypes = [C.c_void_p, C.c_int]
+    reads = [(lib.omega_moe_get_weights, L.W_W1, n // (2 if dtype == "bf16" else 1)), (lib.omega_moe_get_weights, L.W_GATE_BIAS, 16), (lib.omega_moe_get_grad, L.W_W2, n)]
+    host = np.empty(n, np.uint8)
+
+    def read(get, which, dst):
+        m.log()
+        st = get(m.h, which, 0, dst, 1)
+        return st, [s for s in m.log() if s != "unpack"]
+
+    for get, which, size in reads:
+        st, log = read(get, which, p.value + n - size)              # to the last byte
+        assert st == 0 and len(log) == 1 and log[0].startswith("param_read")
+        assert read(get, which, host.ctypes.data) == (0, ["copy"])
+        assert read(get, which, p.value + n - size + 4) == (3, [])  # past the end: OMEGA_ERR_HIP
+        lib.host_move_to_device(p, 1)
+        assert read(get, which, p.value) == (0, ["copy"])
+        lib.host_move_to_device(p, 0)
+        assert m.forward(8) == 0
+    live = lib.host_live_count()
+    read(lib.omega_moe_get_weights, L.W_W1, host.ctypes.data)
+    assert lib.host_live_count() == live
+    assert lib.omega_hip_free(m.ctx, p) == 0
+    m.close()
