@@ -666,7 +666,9 @@ static int ensure_queues(omega_moe *m, int T)
 {
     if (!m->few) return OMEGA_OK;
     m->few = false;
-    OMEGA_HIP_CHECK(m->ctx, launch_dispatch_index(m, T, m->bm, m->ctx->stream, nullptr));
+    const hipError_t e = launch_dispatch_index(m, T, m->bm, m->ctx->stream, nullptr);
+    m->few = e != hipSuccess;  // (the next to ask tries again: the queues are still an earlier batch's)
+    OMEGA_HIP_CHECK(m->ctx, e);
     return OMEGA_OK;
 }
 // y with the k slices of its down product added, for whatever reads y other than the combine kernel

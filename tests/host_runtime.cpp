@@ -16,6 +16,7 @@ static std::map<void *, int> g_device;  // blocks of another device than 0
 static size_t g_bytes;
 static int g_fail_in;  // > 0: the allocation with this number from now on fails
 static hipError_t g_last = hipSuccess;
+static std::string g_fail_launch;  // the next launch of this name fails
 static float g_clock;  // advanced by every launch: what the events read
 static std::string g_log;
 
@@ -26,6 +27,10 @@ static hipError_t line(const char *fmt, ...)
     va_start(ap, fmt);
     vsnprintf(buf, sizeof buf, fmt, ap);
     va_end(ap);
+    if (g_fail_launch == buf) {
+        g_fail_launch.clear();
+        return hipErrorLaunchFailure;
+    }
     g_log += buf;
     g_log += '\n';
     g_clock += 1.0f;
@@ -35,6 +40,7 @@ static hipError_t line(const char *fmt, ...)
 extern "C" {
 
 void host_fail_allocation(int n) { g_fail_in = n; }
+void host_fail_launch(const char *name) { g_fail_launch = name; }
 void host_move_to_device(void *p, int device) { g_device[p] = device; }
 size_t host_live_bytes(void) { return g_bytes; }
 int host_live_count(void) { return (int)g_live.size(); }

@@ -245,3 +245,20 @@ def test_the_kernel_stores_to_memory_of_its_own_device_only(lib, dtype):
     assert lib.host_live_count() == live
     assert lib.omega_hip_free(m.ctx, p) == 0
     m.close()
+
+
+def test_queues_that_could_not_be_made_are_made_by_the_next_pass(lib):
+    """A forward pass of a few tokens leaves the tile kernels' queues to the backward pass; where their launch fails they are still
+    those of an earlier batch, and no product may run on them."""
+    m = Layer(lib, "bf16")
+    ms = C.c_float()
+    for back in (m.back, lambda T: lib.omega_moe_time_backward(m.h, m.x, m.g, T, m.out, 0, 1, C.byref(ms))):
+        assert m.forward(64) == 0 and m.back(64) == 0 and m.forward(8) == 0
+        m.log()
+        lib.host_fail_launch(b"index")
+        assert back(8) == 3 and not any(s.startswith("backward") for s in m.log())      # OMEGA_ERR_HIP
+        assert back(8) == 0
+        log = m.log()
+        assert log.index("index") < log.index("backward_bf16 kept=0")
+        assert back(8) == 0 and "index" not in m.log()
+    m.close()
