@@ -272,7 +272,9 @@ int omega_moe_fill_workspace(omega_moe *moe, int which, int byte_value);
  * context's stream: runs `iters` back-to-back repetitions of the stage (0 router, 1 dispatch,
  * 2 experts_up, 3 experts_down, 4 combine, 5 whole forward, 6 dispatch index kernels only, 7 dispatch
  * row gather only, 8 whole forward_block, 9 the pre-norm kernel of the block form only) after `warmup` untimed ones.
- * x_dev/out_dev as for forward; the stages before `stage` must have been run for this T. */
+ * x_dev/out_dev as for forward; the stages before `stage` must have been run for this T.  5 and 8 are omega_moe_forward
+ * and omega_moe_forward_block themselves, and leave what those leave.  Partial results of a down product that cut k into
+ * slices are added by 4, in training mode by 3. */
 int omega_moe_time_stage(omega_moe *moe, int stage, const void *x_dev, int T, void *out_dev, int warmup, int iters,
                          float *ms_avg);
 

@@ -1374,13 +1374,7 @@ int omega_moe_time_stage(omega_moe *m, int stage, const void *x, int T, void *ou
             case 9:
                 OMEGA_HIP_CHECK(ctx, launch_rmsnorm(m, x, T, m->hbuf, ctx->stream));
                 return OMEGA_OK;
-            default:
-                m->y_partial = false;  // (y is written again below)
-                RUN(stage_router(m, x, T));
-                RUN(stage_dispatch(m, x, T));
-                RUN(stage_experts(m, x, T, 0));
-                RUN(stage_experts(m, x, T, 1));
-                return stage_combine(m, T, out, nullptr);
+            default: return forward_impl(m, x, T, out, 0);
         }
     };
     for (int i = 0; i < warmup; ++i) RUN(once());

@@ -262,3 +262,19 @@ def test_queues_that_could_not_be_made_are_made_by_the_next_pass(lib):
         assert log.index("index") < log.index("backward_bf16 kept=0")
         assert back(8) == 0 and "index" not in m.log()
     m.close()
+
+
+@pytest.mark.parametrize("dtype,T,training", [("f32", 8, 0), ("bf16", 8, 0), ("bf16", 64, 0), ("bf16", 65, 0), ("bf16", 8, 1)])
+def test_a_timed_forward_pass_is_one(lib, dtype, T, training):
+    """Stage 5 of time_stage makes the launches of omega_moe_forward, and leaves what it leaves."""
+    m = Layer(lib, dtype)
+    assert lib.omega_moe_set_training(m.h, training) == 0
+    for _ in range(2):
+        m.log()
+        assert m.forward(T) == 0
+        want = m.log()
+    ms = C.c_float()
+    assert lib.omega_moe_time_stage(m.h, 5, m.x, T, m.out, 1, 2, C.byref(ms)) == 0
+    assert m.log() == 3 * want and ms.value == len(want)
+    assert m.back(T) == 0
+    m.close()
