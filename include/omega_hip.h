@@ -166,8 +166,10 @@ int omega_moe_backward_block(omega_moe *moe, const void *x_dev, const void *dout
 /* Training mode (off at creation).  The reference's layers keep their outputs for back() (LlamaMLPLayer.diff reads
  * active.getOutput() and getLinear3().getOutput(), J/engine/nn/layer/llama/LlamaMLPLayer.java:148-152); with training
  * on, omega_moe_forward likewise stores h1 and h3 (fp32, from the accumulators of its up product) and
- * omega_moe_backward reads them instead of recomputing them.  Same results either way; the forward pass writes
- * 8*H bytes more per expert row and allocates what the backward pass works on. */
+ * omega_moe_backward reads them instead of recomputing them; the forward pass writes 8*H bytes more per expert row and
+ * allocates what the backward pass works on.  Same results either way, bit for bit but for bf16 batches of up to 64
+ * tokens: outside training these run on kernels that add the fp32 sums over d and H in another order, so that an element
+ * of `a` or of the output may round to the neighbouring bf16 value. */
 int omega_moe_set_training(omega_moe *moe, int on);
 /* How the rows of x reach the experts of a bf16 layer.  The reference has no dispatch (its row gathers, e.g.
  * img_token_drop, J/engine/nn/layer/dit/kernel/TokenDropKernel.cu:147-160, always write the gathered copy).
@@ -222,8 +224,8 @@ int omega_moe_update(omega_moe *moe, float lr);
  * (AdamWKernel.java:25-26), weight_decay 1e-4 (AdamW.java:27). */
 int omega_moe_update_adamw(omega_moe *moe, float lr, float beta1, float beta2, float weight_decay, int train_time);
 
-/* The four stages of forward, callable one at a time (per-stage timing and tests); they use the
- * same kernels and workspace as omega_moe_forward and must be called in this order for one T:
+/* The four stages of forward, callable one at a time (per-stage timing and tests); they use the same product kernels and
+ * workspace as omega_moe_forward, with the same results bit for bit, and must be called in this order for one T:
  *   router   x -> ids, weights, per-tile expert histogram      (gate: FullyLayer.output, FullyLayer.java:218-243;
  *                                                               softmax: J/engine/gpu/SoftmaxKernel.cu:4-24)
  *   dispatch histogram -> counts, offsets, dst, src_row, tile list; gather x rows into the

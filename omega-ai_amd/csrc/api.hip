@@ -664,10 +664,10 @@ static int stage_router(omega_moe *m, const void *x, int T)
 // launch from the same routing
 static int ensure_queues(omega_moe *m, int T)
 {
-    if (!m->few) return OMEGA_OK;
-    m->few = false;
+    if (m->queued) return OMEGA_OK;
+    m->queued = true;
     const hipError_t e = launch_dispatch_index(m, T, m->bm, m->ctx->stream, nullptr);
-    m->few = e != hipSuccess;  // (the next to ask tries again: the queues are still an earlier batch's)
+    m->queued = e == hipSuccess;  // (the next to ask tries again: the queues are still an earlier batch's)
     OMEGA_HIP_CHECK(m->ctx, e);
     return OMEGA_OK;
 }
@@ -718,9 +718,11 @@ static int stage_dispatch(omega_moe *m, const void *x, int T, bool up_follows = 
     // (bf16 layers: the index launch copies the rows as well; fp32 layers gather in a launch of its own, or leave it to the
     // up product that follows, which fetches its rows from x and writes the gathered copy beside: a launch less, 4 of 35 us at
     // 256 tokens x 128 columns)
-    // (a few tokens, bf16: the products need neither queues nor, when they follow, a gathered copy; they leave it as fp32 layers' do)
+    // (a few tokens, bf16: the products need neither queues nor, when they follow, a gathered copy; they leave it as fp32 layers' do.
+    // Stages called one by one run on the same kernels: what they return and how long they take is what a forward pass does.)
     const bool bf = m->cfg.dtype == OMEGA_DTYPE_BF16;
-    m->few = up_follows && !m->training && experts_few_rows(m, T);
+    m->few = !m->training && experts_few_rows(m, T);
+    m->queued = !m->few;
     const bool up_gathers = up_follows && (m->few || (!bf && (double)T * m->cfg.d * 4.0 < 4.0e9));
     OMEGA_HIP_CHECK(m->ctx, launch_dispatch_index(m, T, bm, m->ctx->stream, bf && !m->gather_on_load && !up_gathers ? x : nullptr));
     if (!bf && !up_gathers) OMEGA_HIP_CHECK(m->ctx, launch_dispatch_gather(m, x, T, m->ctx->stream));

@@ -99,9 +99,9 @@ struct omega_moe {
     int down_cols = 256;
     int down_ks_max = 1;             // > 1: the down table of this batch may hold k slices of every tile (small batches)
     int down_tail_ks = 1;            // > 1: the last tiles of the down table may be cut into up to this many k slices
-    // the batch is one of a few tokens in a forward pass: its products run on experts_few.hip and its dispatch made no work queues
+    // the batch is one of a few tokens outside training: its products run on experts_few.hip and its dispatch made no work queues
     // (what needs them has them made first: ensure_queues)
-    bool few = false;
+    bool few = false, queued = true;
     // the down product of the batch in y has left k slices in y_slabs that are not in y: the combine kernel adds them on its
     // way (combine.hip), whatever else reads y has them added first (ensure_y_whole)
     bool y_partial = false;

@@ -786,7 +786,7 @@ hipError_t launch_dispatch_index(const omega_moe *m, int T, int bm, hipStream_t 
     const int nt_stores = (size_t)T * c.K * c.d * 2 > OMEGA_LLC_BYTES / 2 ? 1 : 0;
     const int tok_tile = router_tok_tile(m, T);
     const int n_tiles = ceil_div(T, tok_tile);
-    const bool queues = m->desc_up != nullptr && !m->few;  // bf16 layers, unless their products go without
+    const bool queues = m->desc_up != nullptr && m->queued;  // bf16 layers, unless their products go without
     const int n_sched = queues ? SCHED_WGS : 0;
     hipLaunchKernelGGL(dispatch_rank_kernel, dim3(n_tiles + n_sched), dim3(rows ? 1024 : 256), 0, s, m->ids, m->tile_counts, m->counts,
                        n_tiles, T, tok_tile, c.K, c.E, c.Es, bm, m->offsets, m->dst, m->dstp, m->src_row, m->tokp, m->tiles,

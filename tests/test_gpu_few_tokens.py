@@ -78,3 +78,30 @@ def test_backward_behind_a_forward_of_few_tokens(T):
             assert N.rel_l2(layer.grad(which, g), bw[name][g]) <= 1e-2, (g, name)
     x.free()
     layer.close()
+
+
+@pytest.mark.parametrize("mode", [1, 2])
+@pytest.mark.parametrize("kw", [dict(FINE, T=1), dict(FINE, T=17), dict(FINE, T=64), dict(T=33, d=256, H=384, E=5, K=2, Es=0)],
+                         ids=lambda k: "-".join(str(v) for v in k.values()))
+def test_stages_of_a_few_tokens_are_those_of_a_forward_pass(kw, mode):
+    """Called one by one they run on the same kernels, from the rows the dispatch stage has copied or left: the same bits."""
+    G, cfg, inp, layer, x = _layer(kw, 13, mode)
+    out = layer.forward(x).to_numpy()
+    y, a = layer.workspace("y", cfg.T), layer.workspace("a", cfg.T)
+    for w in ("a", "y"):
+        layer.fill_workspace(w, 0xFF)
+    o = G.P.DeviceBuffer(G.ctx(), (cfg.T, cfg.d), cfg.dtype)
+    for s in ("router", "dispatch", "experts"):
+        layer.stage(s, x)
+    layer.stage("combine", out=o)
+    assert np.array_equal(o.to_numpy(), out)
+    assert np.array_equal(layer.workspace("a", cfg.T), a) and np.array_equal(layer.workspace("y", cfg.T), y)
+    assert np.array_equal(layer.workspace("xg", cfg.T), inp["x"][layer.routing()["src_row"]])
+    # ... and still are behind a backward pass, which has the tile kernels' queues made
+    assert np.array_equal(layer.forward(x).to_numpy(), out)
+    layer.back(x)
+    layer.stage("experts", x)
+    assert np.array_equal(layer.workspace("y", cfg.T), y)
+    for b in (o, x):
+        b.free()
+    layer.close()
