@@ -1,6 +1,6 @@
 // Combine: out[t,:] = sum_j w[t,j] * y[row of pair t*K+j,:] in slot order, then + the shared experts' rows
 // (rows are the physical rows the dispatch stage assigned; shared expert s owns rows first_tile[E+s]*bm + t).
-// One wave per token; each lane owns 4 (fp32 out) or 8 (bf16 out) consecutive columns, read from the
+// One to eight waves per token, each with a share of the columns; each lane owns 4 (fp32 out) or 8 (bf16 out) consecutive columns, read from the
 // fp32 rows of y with 16-byte loads; products and sums are separate fp32 operations in slot order
 // (this file is compiled with -ffp-contract=off), the weighted sum of add_mul_kernel
 // (J/engine/gpu/BaseKernel.cu:228-241) generalised to K terms; shared rows are added as add_kernel
@@ -22,7 +22,7 @@ __device__ __forceinline__ void add_slices(float4 (&v)[KU][VEC / 4], const int (
     for (int u = 0; u < KU; ++u) most = max(most, (ent[u] >> 9) & 15);
     if (__ballot(most > 1) == 0) return;
     const bool more = __ballot(most > 5) != 0;
-    constexpr int SB = KU <= 4 ? KU : (KU + 1) / 2;  // rows whose slices are in flight together
+    constexpr int SB = KU < 2 ? KU : 2;  // rows whose slices are in flight together
 #pragma unroll
     for (int u0 = 0; u0 < KU; u0 += SB) {
         for (int s0 = 1; s0 < (more ? 8 : 4); s0 += 4) {
@@ -70,9 +70,13 @@ __device__ __forceinline__ void add_slices(float4 (&v)[KU][VEC / 4], const int (
 // the buffer][column tile] = first slice's place | slices << 9 | block within the tile << 13, 0 for a tile that is whole in y.
 // They are added here, to the row of y and in slice order - the sums down_slab_reduce_kernel forms -, while the rows are in
 // registers anyway: a launch and a round trip of y less.  (That kernel is left to what reads y itself: training, backward
-// passes, omega_moe_get_workspace.)  Whole passes, reduce and combine -> combine, d = 4096, H = 14336, 8 experts, top 2, us: 1 token
-// 144.6 -> 142.5, 64 tokens 488 -> 484, 777 tokens (block form; 2 slices of every tile) 639 -> 625, 4096 tokens (4 of the last 64)
-// 2240 -> 2230.
+// passes, omega_moe_get_workspace.)  Whole passes, reduce and combine / combine, us: 777 tokens x 4096 x 14336, 8 experts, top 2 (2
+// slices of every tile) 630 / 624, 256 x 4096 x 7168 302 / 293, 4096 x 4096 x 14336 (4 slices of the last 64 tiles) 2208-2224 / 2210-2215.
+// Rows in groups of four, two rows' slices in flight: 148 registers, three waves per SIMD; eight rows at a time, as
+// without slices, and half of them in flight took 256, one wave, and lost where the table has few slices or none (the host knows bounds of
+// the tiles only).  Combine, us, eight at a time / now: 1100 tokens x 4096, 8 experts of 4096, top 8 60.6 / 41.1 (pass 763 / 751, with the
+// reduce launch 753); 300 x 2048, 64 experts, 6 + 2 rows, no slices 10.5 / 8.7; 200 x 1024, 6 + 2 rows, 6 slices of every tile 15.2 /
+// 15.8 (one row's slices in flight 17.8, registers capped at 128 22.0); 4 rows: 300 x 2048 7.1 / 7.4, 200 x 1024 11.4 / 11.2, 1100 x 4096 26.8 / 25.4.
 template <int VEC, bool BF16, int KU, bool NT, bool SL>
 __global__ __launch_bounds__(256) void combine_kernel(const float *__restrict__ y, const int32_t *__restrict__ dst,
                                                       const float *__restrict__ w, int T, int K, int d, int Es,
@@ -217,30 +221,40 @@ hipError_t launch_combine(const omega_moe *m, int T, void *out, const void *resi
         while (want < 8 && (long long)T * want < 256LL * m->ctx->num_cus) want *= 2;
         const int dc = ceil_div(trips, std::min(want, trips)) * 64 * vec, split = ceil_div(c.d, dc);
         const bool sl = m->y_partial;
-        const int n = c.K + c.Es, ku = ceil_div(n, ceil_div(n, 8));  // rows of a token in groups of one size, eight at most
+        const int n = c.K + c.Es, ku = ceil_div(n, ceil_div(n, sl ? 4 : 8));  // rows of a token in groups of one size, eight at most
         const int grid = ceil_div(T * split, 4);
 #define COMBINE_LAUNCH(VECV, BFV, KUV, NTV, SLV)                                                                                       \
     hipLaunchKernelGGL((combine_kernel<VECV, BFV, KUV, NTV, SLV>), dim3(grid), dim3(256), 0, s, m->y, m->dstp, m->w, T, c.K, c.d, c.Es, \
                        m->tile_meta, c.E, m->bm, resid, out, split, m->y_slabs, m->slab_tab, dc)
-#define COMBINE_SLOTS(VECV, BFV, NTV, SLV)                  \
-    do {                                                     \
-        switch (ku) {                                        \
-        case 1: COMBINE_LAUNCH(VECV, BFV, 1, NTV, SLV); break; \
-        case 2: COMBINE_LAUNCH(VECV, BFV, 2, NTV, SLV); break; \
-        case 3: COMBINE_LAUNCH(VECV, BFV, 3, NTV, SLV); break; \
-        case 4: COMBINE_LAUNCH(VECV, BFV, 4, NTV, SLV); break; \
-        case 5: COMBINE_LAUNCH(VECV, BFV, 5, NTV, SLV); break; \
-        case 6: COMBINE_LAUNCH(VECV, BFV, 6, NTV, SLV); break; \
-        case 7: COMBINE_LAUNCH(VECV, BFV, 7, NTV, SLV); break; \
-        default: COMBINE_LAUNCH(VECV, BFV, 8, NTV, SLV);      \
-        }                                                    \
+#define COMBINE_SLOTS(VECV, BFV, NTV)                           \
+    do {                                                         \
+        switch (ku) {                                            \
+        case 1: COMBINE_LAUNCH(VECV, BFV, 1, NTV, false); break; \
+        case 2: COMBINE_LAUNCH(VECV, BFV, 2, NTV, false); break; \
+        case 3: COMBINE_LAUNCH(VECV, BFV, 3, NTV, false); break; \
+        case 4: COMBINE_LAUNCH(VECV, BFV, 4, NTV, false); break; \
+        case 5: COMBINE_LAUNCH(VECV, BFV, 5, NTV, false); break; \
+        case 6: COMBINE_LAUNCH(VECV, BFV, 6, NTV, false); break; \
+        case 7: COMBINE_LAUNCH(VECV, BFV, 7, NTV, false); break; \
+        default: COMBINE_LAUNCH(VECV, BFV, 8, NTV, false);       \
+        }                                                        \
     } while (0)
-        if (sl && nt) COMBINE_SLOTS(8, true, true, true);
-        else if (sl) COMBINE_SLOTS(8, true, false, true);
-        else if (bf && nt) COMBINE_SLOTS(8, true, true, false);
-        else if (bf) COMBINE_SLOTS(8, true, false, false);
-        else if (nt) COMBINE_SLOTS(4, false, true, false);
-        else COMBINE_SLOTS(4, false, false, false);
+#define COMBINE_SLICED(NTV)                              \
+    do {                                                  \
+        switch (ku) {                                     \
+        case 1: COMBINE_LAUNCH(8, true, 1, NTV, true); break; \
+        case 2: COMBINE_LAUNCH(8, true, 2, NTV, true); break; \
+        case 3: COMBINE_LAUNCH(8, true, 3, NTV, true); break; \
+        default: COMBINE_LAUNCH(8, true, 4, NTV, true);       \
+        }                                                 \
+    } while (0)
+        if (sl && nt) COMBINE_SLICED(true);
+        else if (sl) COMBINE_SLICED(false);
+        else if (bf && nt) COMBINE_SLOTS(8, true, true);
+        else if (bf) COMBINE_SLOTS(8, true, false);
+        else if (nt) COMBINE_SLOTS(4, false, true);
+        else COMBINE_SLOTS(4, false, false);
+#undef COMBINE_SLICED
 #undef COMBINE_SLOTS
 #undef COMBINE_LAUNCH
     } else {

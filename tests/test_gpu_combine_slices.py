@@ -13,6 +13,9 @@ pytestmark = pytest.mark.gpu
     dict(T=70, d=512, H=1024, E=4, K=2, Es=0),      # 4 slices of every tile
     dict(T=90, d=768, H=4096, E=3, K=3, Es=2),      # 8 slices, shared experts
     dict(T=300, d=1024, H=640, E=7, K=7, Es=1),     # 2 slices, two row tiles per expert
+    dict(T=200, d=1024, H=2048, E=8, K=6, Es=2),    # 6 slices, eight rows in two groups
+    dict(T=130, d=512, H=1024, E=5, K=4, Es=1),     # five rows in groups of three
+    dict(T=300, d=2048, H=1408, E=64, K=6, Es=2),   # room for slices, and none made: too many tiles
     dict(T=4400, d=4096, H=4096, E=1, K=1, Es=0),   # the last tiles only: 18 x 16 tiles, 32 of them in 2 slices
     dict(T=1100, d=256, H=256, E=4, K=1, Es=0),     # room for slices, and none made
 ], ids=lambda k: "-".join(str(v) for v in k.values()))
