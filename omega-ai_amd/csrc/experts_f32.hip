@@ -438,10 +438,14 @@ __global__ __launch_bounds__(256, 2) void f32_product_kernel(f32_args p)
     constexpr int CT = PAIR ? TN / 2 : TN;                             // output columns per tile
     constexpr bool BK_ = WG || OP == F32_DA || OP == F32_DXG;
     constexpr int PN = PAIR ? 64 : 32;                                 // MFMA columns of a part
-    constexpr int LA = f32_lds_floats(TM, WG, F32_FBK(TM)), LB0 = f32_lds_floats(TN, BK_, F32_FBK(TM));
-    constexpr int LB = PARTS && f32_lds_floats(PN, BK_, F32_FBK(32)) > LB0 ? f32_lds_floats(PN, BK_, F32_FBK(32)) : LB0;
-    static_assert(!PARTS || f32_lds_floats(32, WG, F32_FBK(32)) <= LA, "a part's rows fit");
-    __shared__ __attribute__((aligned(16))) float as[WG ? 1 : 2 * LA], bs[WG ? 1 : 2 * LB];
+    constexpr int LA = f32_lds_floats(TM, WG, F32_FBK(TM)), LB = f32_lds_floats(TN, BK_, F32_FBK(TM));
+    // A part works in the room of its tile.  The input gradient's of 128 rows, whose B is wider in a part than in the tile, keeps both
+    // operands in one array, behind one another from its start on: 54272 bytes, three workgroups per compute unit, where 55296 would
+    // leave two (backward pass, us: 4096 tokens x 1024 x 3584, 8 experts 2982 / 2972, 3333 x 333 x 1111, 6 experts 755-761 / 750).
+    constexpr int LAP = f32_lds_floats(32, WG, F32_FBK(32)), LBP = f32_lds_floats(PN, BK_, F32_FBK(32));
+    constexpr bool ONE = OP == F32_DXG && TM == F32_TILE_M;
+    static_assert(!PARTS || (ONE ? LAP + LBP <= LA + LB : LAP <= LA), "a part's operands fit");
+    __shared__ __attribute__((aligned(16))) float as[WG ? 1 : ONE ? 2 * (LA + LB) : 2 * LA], bs[WG || ONE ? 1 : 2 * (PARTS && LBP > LB ? LBP : LB)];
     if (OP == F32_UP && (int)blockIdx.x >= (int)gridDim.x - p.copy_wgs) {
         copy_gathered<VEC>(p, blockIdx.x - (gridDim.x - p.copy_wgs), threadIdx.x & 63, threadIdx.x >> 6);
         return;
@@ -485,11 +489,11 @@ __global__ __launch_bounds__(256, 2) void f32_product_kernel(f32_args p)
 
     if constexpr (PARTS) {
         if (part >= 0) {
-            f32_tile<OP, 32, PN, VEC>(p, as, bs, mt, 32 * (part % (TM / 32)), n0 + 32 * (part / (TM / 32)), mat);
+            f32_tile<OP, 32, PN, VEC>(p, as, ONE ? as + 2 * LAP : bs, mt, 32 * (part % (TM / 32)), n0 + 32 * (part / (TM / 32)), mat);
             return;
         }
     }
-    f32_tile<OP, TM, TN, VEC>(p, as, bs, mt, 0, n0, mat);
+    f32_tile<OP, TM, TN, VEC>(p, as, ONE ? as + 2 * LA : bs, mt, 0, n0, mat);
 }
 
 // The largest row-tile height that a batch of up to T tokens takes: with fewer than 128 rows per expert always 32 (160 shapes of
@@ -541,7 +545,9 @@ static hipError_t f32_launch(f32_args p, bool vec, int max_tiles, hipStream_t s)
     const size_t tiles = (size_t)ceil_div(p.N, CT) * (F32_IS_WG(OP) ? (size_t)ceil_div(p.Kd, TM) * p.G * (OP == F32_WG13 ? 2 : 1) : max_tiles);
     // (weight gradients: to eight parts of a matrix)
     const size_t c = F32_IS_WG(OP) ? std::max((size_t)1, (size_t)ceil_div(p.N, CT) * ceil_div(p.Kd, TM) / 8) : 1;
-    p.slots *= TM == F32_TILE_M || F32_PAIR(OP) ? 2 : 4;  // (what LDS holds of the workgroups of tiles of 128 and 64 rows)
+    // (what LDS holds of the workgroups of tiles of 128 and 64 rows; a third one of the input gradient's comes and goes between the others:
+    // with rounds of three 2972 -> 3088 and 795 -> 868 us at 4096 tokens x 1024 x 3584, 8 experts and x 512 x 1536, 4 experts)
+    p.slots *= TM == F32_TILE_M || F32_PAIR(OP) ? 2 : 4;
     p.part_max = p.slots / 4;
     const size_t parts = F32_PARTS(OP, TM, TN, vec) > 1 && (tiles + 7) / 8 >= (size_t)p.slots ? (size_t)8 * p.part_max * (F32_PARTS(OP, TM, TN, vec) - 1) : 0;
     const unsigned grid = (unsigned)(F32_IS_WG(OP) ? (tiles + 8 * c - 1) / (8 * c) * (8 * c) : (tiles + 7) / 8 * 8 + parts) + p.copy_wgs;
