@@ -263,6 +263,42 @@ hipError_t launch_unpack_rows(void *dst_rowmajor, const void *src_packed, int R,
 hipError_t launch_param_read(void *dst, const void *src, int R, int Kd, size_t n, hipEvent_t done, hipStream_t s);
 int experts_bf16_tile_m(const omega_moe *m, int T);
 bool wgrad_on_four_waves(const omega_moe *m, int T, int M, int N);  // which kernel takes the weight gradients of M x N per expert
+// Tile (of all matrices, one after the other) of the j-th workgroup of XCD x in a launch over `mats` gradient matrices of n tiles, -1: none.
+// Every XCD takes a run of n / 8 tiles of every matrix, in the same order of matrices, and what n leaves over is dealt out one by one:
+// extra tile e of the launch to XCD e % 8.  (An eighth of all tiles each left the other XCDs idle behind the one with the longest expert.
+// Backward pass, us: 3000 tokens x 512 x 1024, 16 experts, Zipf 911 -> 535; 4096 x 256 x 512, 6 experts and a shared one 375 -> 340.  Runs dealt in
+// turn, without the one by one, gave some XCDs more tiles than compute units.  dW1 and dW3, an eighth of all / in turn / now: 474 x 325 x
+// 588, 2 experts, top 1 13.2 / 21.2 / 13.3, 881 x 933 x 290, 5 experts, top 3 59 / 73 / 61.)
+// Matrices of few tiles go together, four or eight as one: a run of one or two tiles fetches its operands for nobody else (2867 tokens x 68 x
+// 357, 11 experts, top 7 and a shared one, 12 tiles each, dW1 and dW3: 137 in fours, 112 in eights; 2081 x 632 x 672, 7 experts, top 7, 30 tiles,
+// backward pass 893 in twos, 876 in fours).
+static inline int wgrad_together(int n) { return n >= 32 ? 1 : n >= 16 ? 4 : 8; }
+struct wgrad_deal {
+    int n, groups, rest, together;  // tiles of a whole group of `together` matrices, their number, tiles of the group of what is left
+};
+static inline wgrad_deal wgrad_deal_of(int n, int mats)
+{
+    const int together = wgrad_together(n);
+    return {n * together, mats / together, n * (mats % together), together};
+}
+__host__ __device__ static inline int wgrad_tile(const wgrad_deal &w, int x, int j)
+{
+    int n = w.n, first = 0, g = 0, own = w.groups * (n >> 3) + ((w.groups * (n & 7) + 7 - x) >> 3);  // tiles of XCD x in the whole groups
+    if (j >= own) {
+        j -= own;
+        first = w.groups * n;
+        n = w.rest;
+        if (j >= (n >> 3) + (((n & 7) + 7 - x) >> 3)) return -1;
+    } else {
+        g = 8 * j / n;
+    }
+    const int q = n >> 3, r = n & 7;
+    auto before = [&](int k) { return k * q + ((k * r + 7 - x) >> 3); };  // tiles of XCD x in groups 0 .. k - 1
+    while (g > 0 && before(g) > j) --g;
+    while (before(g + 1) <= j) ++g;
+    const int s = (g * r) & 7, e = s + r;  // the group's extra tiles go to XCDs s .. e - 1, modulo 8
+    return first + g * n + x * q + (x < e ? x : e) - (x < s ? x : s) + (x < e - 8 ? x : e > 8 ? e - 8 : 0) + j - before(g);
+}
 #define F32_TILE_M 128       // row-tile heights of fp32 layers: experts_f32_tile_m chooses one per batch
 #define F32_TILE_M_MID 64
 #define F32_TILE_M_SMALL 32

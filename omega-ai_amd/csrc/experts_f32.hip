@@ -122,6 +122,7 @@ struct f32_args {
     const int32_t *tile_meta, *counts;
     int N, Kd;               // row products: output columns and k; F32_WG*: columns and rows of one dW (k is the group's rows)
     int E, G, T, bm;
+    wgrad_deal deal;         // F32_WG*: how the tiles go to the XCDs
     int slots, part_max;     // workgroups an XCD holds at a time; tiles of a last round that go in parts
 };
 
@@ -453,18 +454,14 @@ __global__ __launch_bounds__(256, 2) void f32_product_kernel(f32_args p)
 
     // Tile of this workgroup.  Consecutive workgroups go round the eight XCDs.  Row products: XCD x takes the x-th eighth of the tiles, and
     // within it up to 8 row tiles walk the column tiles together, so that its workgroups share operand rows in its L2.  Weight
-    // gradients, whose length is the expert's rows: every XCD takes an eighth of every matrix, in the same order.  (An eighth of all
-    // tiles each left the other XCDs idle behind the one with the longest expert.  Backward pass, us: 3000 tokens x 512 x 1024, 16 experts,
-    // Zipf 911 -> 535; 4096 x 256 x 512, 6 experts and a shared one 375 -> 340; 4096 x 1024 x 3584, 8 even experts 3223 -> 3196.)
+    // gradients, whose length is the expert's rows: every XCD takes an eighth of every matrix (wgrad_tile).
     const int NT = (p.N + CT - 1) / CT;
     const int MT = WG ? (p.Kd + TM - 1) / TM : p.tile_meta[0];  // row tiles (of one gradient matrix)
-    const int mats = OP == F32_WG13 ? 2 * p.G : OP == F32_WG2 ? p.G : 1;
-    const int total = MT * NT * mats, x = blockIdx.x & 7, j = blockIdx.x >> 3;
+    const int x = blockIdx.x & 7, j = blockIdx.x >> 3;
     int t, mat = 0, part = -1;
     if (WG) {
-        const int c = max(1, (MT * NT) >> 3);
-        t = ((j / c) * 8 + x) * c + j % c;
-        if (t >= total) return;
+        t = wgrad_tile(p.deal, x, j);
+        if (t < 0) return;
         mat = t / (MT * NT);
         t -= mat * MT * NT;
     } else {
@@ -475,7 +472,7 @@ __global__ __launch_bounds__(256, 2) void f32_product_kernel(f32_args p)
         // 2036 x 680 x 1980, 3 experts, top 3 (one round and 4 of 128) 173 / 152.  Parts cost more per element than a tile: k = 1536,
         // N = 1024, 128 rows, rounds + rest: 1 + 16 143 / 132, 1 + 24 145 / 149, 1 + 32 149 / 165, 2 + 8 236 / 210, 2 + 24 238 / 247; forward
         // passes with 64 rows and up's rest at 3/8 63.0 / 65.4, at 1/2 141 / 149.
-        const int per = (total + 7) >> 3, rest = per % p.slots;
+        const int total = MT * NT, per = (total + 7) >> 3, rest = per % p.slots;
         int i = j;
         if (PARTS && rest <= p.part_max && per >= p.slots && j >= per - rest) {
             part = (j - (per - rest)) % F32_PARTS(OP, TM, TN, VEC);
@@ -543,14 +540,14 @@ static hipError_t f32_launch(f32_args p, bool vec, int max_tiles, hipStream_t s)
 {
     constexpr int CT = F32_PAIR(OP) ? TN / 2 : TN;
     const size_t tiles = (size_t)ceil_div(p.N, CT) * (F32_IS_WG(OP) ? (size_t)ceil_div(p.Kd, TM) * p.G * (OP == F32_WG13 ? 2 : 1) : max_tiles);
-    // (weight gradients: to eight parts of a matrix)
-    const size_t c = F32_IS_WG(OP) ? std::max((size_t)1, (size_t)ceil_div(p.N, CT) * ceil_div(p.Kd, TM) / 8) : 1;
     // (what LDS holds of the workgroups of tiles of 128 and 64 rows; a third one of the input gradient's comes and goes between the others:
     // with rounds of three 2972 -> 3088 and 795 -> 868 us at 4096 tokens x 1024 x 3584, 8 experts and x 512 x 1536, 4 experts)
     p.slots *= TM == F32_TILE_M || F32_PAIR(OP) ? 2 : 4;
     p.part_max = p.slots / 4;
     const size_t parts = F32_PARTS(OP, TM, TN, vec) > 1 && (tiles + 7) / 8 >= (size_t)p.slots ? (size_t)8 * p.part_max * (F32_PARTS(OP, TM, TN, vec) - 1) : 0;
-    const unsigned grid = (unsigned)(F32_IS_WG(OP) ? (tiles + 8 * c - 1) / (8 * c) * (8 * c) : (tiles + 7) / 8 * 8 + parts) + p.copy_wgs;
+    if (F32_IS_WG(OP)) p.deal = wgrad_deal_of(ceil_div(p.N, CT) * ceil_div(p.Kd, TM), p.G * (OP == F32_WG13 ? 2 : 1));
+    // (weight gradients: whole groups of matrices and one of what is left over, each to eight XCDs)
+    const unsigned grid = (unsigned)(F32_IS_WG(OP) ? (tiles + 7) / 8 * 8 + (p.deal.rest > 0 ? 8 : 0) : (tiles + 7) / 8 * 8 + parts) + p.copy_wgs;
     if (vec) hipLaunchKernelGGL((f32_product_kernel<OP, TM, TN, true>), dim3(grid), dim3(256), 0, s, p);
     else hipLaunchKernelGGL((f32_product_kernel<OP, TM, TN, false>), dim3(grid), dim3(256), 0, s, p);
     return hipGetLastError();

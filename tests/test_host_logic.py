@@ -278,3 +278,24 @@ def test_a_timed_forward_pass_is_one(lib, dtype, T, training):
     assert m.log() == 3 * want and ms.value == len(want)
     assert m.back(T) == 0
     m.close()
+
+
+@pytest.mark.parametrize("n", [1, 2, 7, 8, 9, 12, 15, 16, 31, 33, 54, 60, 64, 127])
+@pytest.mark.parametrize("mats", [1, 2, 5, 8, 17, 24])
+def test_tiles_of_weight_gradients_are_dealt_evenly(lib, n, mats):
+    """Every tile of every matrix to one workgroup, the XCDs' totals next to alike, and each one's share a run in rising order; of a
+    matrix of 32 tiles or more an eighth, rounded up or down."""
+    seen, totals = set(), []
+    per = -(-n * mats // 8) + (1 if n < 32 else 0)      # the launch's workgroups per XCD
+    for x in range(8):
+        got = [lib.host_wgrad_tile(n, mats, x, j) for j in range(per + 3)]
+        assert set(got[per:]) == {-1}
+        got = [t for t in got if t >= 0]
+        assert got == sorted(got) and not seen & set(got)
+        seen |= set(got)
+        totals.append(len(got))
+        if n >= 32:
+            for m in range(mats):
+                run = [t for t in got if t // n == m]
+                assert len(run) in (n // 8, -(-n // 8)) and run == list(range(run[0], run[0] + len(run)))
+    assert seen == set(range(n * mats)) and max(totals) - min(totals) <= (1 if n >= 32 else 2)
