@@ -263,7 +263,8 @@ hipError_t launch_unpack_rows(void *dst_rowmajor, const void *src_packed, int R,
 hipError_t launch_param_read(void *dst, const void *src, int R, int Kd, size_t n, hipEvent_t done, hipStream_t s);
 int experts_bf16_tile_m(const omega_moe *m, int T);
 bool wgrad_on_four_waves(const omega_moe *m, int T, int M, int N);  // which kernel takes the weight gradients of M x N per expert
-// Tile (of all matrices, one after the other) of the j-th workgroup of XCD x in a launch over `mats` gradient matrices of n tiles, -1: none.
+// Tile of the j-th workgroup of XCD x in a launch over `mats` gradient matrices of n tiles, counted from the first tile of matrix *mat (the first
+// of its group) on, -1: none.
 // Every XCD takes a run of n / 8 tiles of every matrix, in the same order of matrices, and what n leaves over is dealt out one by one:
 // extra tile e of the launch to XCD e % 8.  (An eighth of all tiles each left the other XCDs idle behind the one with the longest expert.
 // Backward pass, us: 3000 tokens x 512 x 1024, 16 experts, Zipf 911 -> 535; 4096 x 256 x 512, 6 experts and a shared one 375 -> 340.  Runs dealt in
@@ -275,29 +276,32 @@ bool wgrad_on_four_waves(const omega_moe *m, int T, int M, int N);  // which ker
 static inline int wgrad_together(int n) { return n >= 32 ? 1 : n >= 16 ? 4 : 8; }
 struct wgrad_deal {
     int n, groups, rest, together;  // tiles of a whole group of `together` matrices, their number, tiles of the group of what is left
+    float recip;                    // 1 / n
 };
 static inline wgrad_deal wgrad_deal_of(int n, int mats)
 {
     const int together = wgrad_together(n);
-    return {n * together, mats / together, n * (mats % together), together};
+    return {n * together, mats / together, n * (mats % together), together, 1.0f / (n * together)};
 }
-__host__ __device__ static inline int wgrad_tile(const wgrad_deal &w, int x, int j)
+__host__ __device__ static inline int wgrad_tile(const wgrad_deal &w, int x, int j, int *mat)
 {
-    int n = w.n, first = 0, g = 0, own = w.groups * (n >> 3) + ((w.groups * (n & 7) + 7 - x) >> 3);  // tiles of XCD x in the whole groups
+    int n = w.n, g = 0, own = w.groups * (n >> 3) + ((w.groups * (n & 7) + 7 - x) >> 3);  // tiles of XCD x in the whole groups
     if (j >= own) {
         j -= own;
-        first = w.groups * n;
+        *mat = w.groups * w.together;
         n = w.rest;
         if (j >= (n >> 3) + (((n & 7) + 7 - x) >> 3)) return -1;
     } else {
-        g = 8 * j / n;
+        *mat = 0;
+        g = (int)(8.0f * j * w.recip);  // off by one at most; a division of integers costs 0.3 us
     }
     const int q = n >> 3, r = n & 7;
     auto before = [&](int k) { return k * q + ((k * r + 7 - x) >> 3); };  // tiles of XCD x in groups 0 .. k - 1
     while (g > 0 && before(g) > j) --g;
     while (before(g + 1) <= j) ++g;
     const int s = (g * r) & 7, e = s + r;  // the group's extra tiles go to XCDs s .. e - 1, modulo 8
-    return first + g * n + x * q + (x < e ? x : e) - (x < s ? x : s) + (x < e - 8 ? x : e > 8 ? e - 8 : 0) + j - before(g);
+    *mat += g * w.together;
+    return x * q + (x < e ? x : e) - (x < s ? x : s) + (x < e - 8 ? x : e > 8 ? e - 8 : 0) + j - before(g);
 }
 #define F32_TILE_M 128       // row-tile heights of fp32 layers: experts_f32_tile_m chooses one per batch
 #define F32_TILE_M_MID 64

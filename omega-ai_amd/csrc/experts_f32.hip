@@ -460,10 +460,9 @@ __global__ __launch_bounds__(256, 2) void f32_product_kernel(f32_args p)
     const int x = blockIdx.x & 7, j = blockIdx.x >> 3;
     int t, mat = 0, part = -1;
     if (WG) {
-        t = wgrad_tile(p.deal, x, j);
+        t = wgrad_tile(p.deal, x, j, &mat);
         if (t < 0) return;
-        mat = t / (MT * NT);
-        t -= mat * MT * NT;
+        for (; p.deal.together > 1 && t >= MT * NT; t -= MT * NT) ++mat;
     } else {
         // Where at least one whole round of p.slots workgroups is followed by a last one of a quarter or less of it (p.part_max), that
         // last round's tiles go in parts of 32 rows x 32 columns: the workgroups that would idle share what one would work on.  us in

@@ -41,7 +41,12 @@ extern "C" {
 
 void host_fail_allocation(int n) { g_fail_in = n; }
 void host_fail_launch(const char *name) { g_fail_launch = name; }
-int host_wgrad_tile(int n, int mats, int x, int j) { return wgrad_tile(wgrad_deal_of(n, mats), x, j); }
+int host_wgrad_tile(int n, int mats, int x, int j)  // of all matrices, one after the other
+{
+    int mat = 0;
+    const int t = wgrad_tile(wgrad_deal_of(n, mats), x, j, &mat);
+    return t < 0 ? -1 : mat * n + t;
+}
 void host_move_to_device(void *p, int device) { g_device[p] = device; }
 size_t host_live_bytes(void) { return g_bytes; }
 int host_live_count(void) { return (int)g_live.size(); }
