@@ -502,31 +502,35 @@ int experts_f32_tile_m_max(const omega_moe *m, int T)
 // From there on the height whose forward products are the shortest by this estimate.  A tile takes its k places in whole steps, a
 // fixed number more and, for a last partial step, `rest` more, at a rate that falls a little with its size (`a`: time per
 // column of k); a product takes rounds of one tile per compute unit, its last, partial round `part` of one and that share of the
-// rest, all of them `least` rounds or more; an expert has `pad` tiles more than its rows.  The numbers are fitted to 540 forward
-// passes of the range above at all three heights, of which the estimate takes the best or one within 5 % (0.4 % in the mean).
-// Forward pass, us, at 32 / 64 / 128 rows: 2048 tokens x 1024 x 1024, 16 experts, top 2 272 / 281 / 361, 1001 tokens x 124 x 1676, 6 experts,
-// top 5 and 2 shared 196 / 143 / 160, 3496 tokens x 120 x 452, 9 experts, top 7 192 / 148 / 144, 4096 tokens x 1024 x 3584, 8 experts, top 2
-// 1654 / 1547 / 1535.  (The 64 x 64 tiles of an earlier kernel: 330, 143, 142, 1715.)
+// rest, or `cut` of its share where it goes in parts (f32_product_kernel), all of them `least` rounds or more; an expert has `pad` tiles
+// more than its rows.  The numbers are fitted to 720 forward passes of the range above at all three heights, of which the estimate takes
+// the best or one within 5 % (14 within 13 %; 0.4 % in the mean).  The fit to the kernels without parts charged a nearly empty last round four
+// or five tenths of one: 0.8 % in the mean, 36 passes more than 5 % off, one of them 44 %.  Within 2 % the tallest is taken, for the backward
+// pass: 4096 tokens x 1024 x 3584, 8 experts, top 2 at 64 / 128 rows forward 1526 / 1523, step of training 5255 / 5091; over 160 steps the estimate
+// is 0.5 % off in the mean, the earlier one 0.8.  Forward pass, us, at 32 / 64 / 128 rows: 2073 tokens x 296 x 264, 4 experts, top 3 72 / 65 / 95,
+// 1001 x 124 x 1676, 6 experts, top 5 and 2 shared 190 / 136 / 152, 3496 x 120 x 452, 9 experts, top 7 189 / 146 / 139, 2048 x 1024 x 1024, 16 experts,
+// top 2 283 / 284 / 367.
 int experts_f32_tile_m(const omega_moe *m, int T)
 {
     if (experts_f32_tile_m_max(m, T) == F32_TILE_M_SMALL) return F32_TILE_M_SMALL;
     const omega_moe_config &c = m->cfg;
-    static const struct { int bm, step, cols; double a, more, rest, pad, least, part; } form[] = {
-        {F32_TILE_M_SMALL, 64, 32, 1.0, 104, 64, 1.0, 0.6, 0.15},
-        {F32_TILE_M_MID, 32, 64, 4.0, 60, 42, 0.55, 0.95, 0.4},
-        {F32_TILE_M, 32, 64, 7.3, 64, 52, 0.65, 0.8, 0.5}};
+    static const struct { int bm, step, cols; double a, more, rest, pad, least, part, cut; } form[] = {
+        {F32_TILE_M_SMALL, 64, 32, 1.0, 104, 74, 0.925, 1.26, 0.216, 1.0},
+        {F32_TILE_M_MID, 32, 64, 4.0, 60, 43, 0.57, 0.79, 0.395, 1.65},
+        {F32_TILE_M, 32, 64, 7.2, 65, 39, 0.8, 0.9, 0.865, 2.1}};
     int best = F32_TILE_M_SMALL;
     double least_time = 0.0;
     for (const auto &f : form) {
         const double tiles_m = (double)T * c.K / f.bm + f.pad * c.E + (double)c.Es * ceil_div(T, f.bm);
-        auto product = [&](int k, int n) {
-            const double all = tiles_m * ceil_div(n, f.cols) / m->ctx->num_cus, whole = std::floor(all);
-            const double rounds = all < f.least ? f.least : whole + (all > whole ? f.part + (1.0 - f.part) * (all - whole) : 0.0);
+        auto product = [&](int k, int n, int slots) {  // (workgroups of a compute unit: a round of f32_product_kernel)
+            const double all = tiles_m * ceil_div(n, f.cols) / m->ctx->num_cus, whole = std::floor(all), full = std::floor(all / slots) * slots;
+            double rounds = all < f.least ? f.least : whole + (all > whole ? f.part + (1.0 - f.part) * (all - whole) : 0.0);
+            if (f.bm != F32_TILE_M_SMALL && full > 0.0 && all - full <= 0.25 * slots) rounds = std::min(rounds, full + f.cut * (all - full));
             return rounds * (ceil_div(k, f.step) * f.step + f.more + (k % f.step != 0 ? f.rest : 0.0));
         };
         // (the up product's tiles hold two columns of weights for each of their own)
-        const double time = f.a * (product(c.d, c.H) + 0.56 * product(c.H, c.d));
-        if (f.bm == F32_TILE_M_SMALL || time < least_time) {
+        const double time = f.a * (product(c.d, c.H, 2) + 0.58 * product(c.H, c.d, f.bm == F32_TILE_M_MID ? 4 : 2));
+        if (f.bm == F32_TILE_M_SMALL || time < (f.bm == F32_TILE_M ? 1.02 : 1.0) * least_time) {
             best = f.bm;
             least_time = time;
         }
