@@ -125,3 +125,41 @@ def test_adamw_training_reduces_a_regression_loss_bf16():
         g.free()
     assert losses[-1] < 0.8 * losses[0] and all(np.isfinite(losses)), losses
     layer.close()
+
+
+@pytest.mark.parametrize("training", [False, True])
+@pytest.mark.parametrize("d,H", [(256, 384), (512, 256), (768, 640)])
+def test_adamw_step_writes_the_transposed_images_of_the_next_backward(training, d, H):
+    """The step leaves W1, W3 and W2 transposed for the backward pass that follows: the gradients are, bit for bit, those of a layer that is
+    given the same rounded weights and transposes them itself.  Widths of one column group more than whole tiles, a shared expert."""
+    from tests import gpu_util as G
+    cfg = scaled(C.CONFIGS["c2_mixtral"], T=90, d=d, H=H, E=3, K=2, Es=1)
+    inp = make_inputs(cfg, 41)
+    x = G.P.DeviceBuffer.from_numpy(G.ctx(), inp["x"], cfg.dtype)
+    g = G.P.DeviceBuffer.from_numpy(G.ctx(), O.round_bf16(O.fill_normal(cfg.T * d, 41, 901, 1.0).reshape(cfg.T, d)), cfg.dtype)
+    layer = G.build_layer(cfg, inp)
+    layer.set_training(training)
+    for t in (1, 2):
+        layer.forward(x)
+        layer.back(g)
+        layer.updateAdamW(2e-2, t)             # (every weight moves by several of its roundings)
+    now = dict(inp, Wg=layer._download_weight(L.W_GATE, 0, (cfg.E, d)), bg=None if inp["bg"] is None else layer._download_weight(L.W_GATE_BIAS, 0, (cfg.E,)))
+    for k, w, s in (("W1", L.W_W1, (H, d)), ("W3", L.W_W3, (H, d)), ("W2", L.W_W2, (d, H))):
+        now[k] = np.stack([layer._download_weight(w, e, s) for e in range(cfg.E + cfg.Es)])
+        assert (now[k] != inp[k]).mean() > 0.9
+    fresh = G.build_layer(cfg, now)
+    fresh.set_training(training)
+
+    def step(m):
+        out = m.forward(x).to_numpy()
+        return [out, m.back(g).to_numpy(), m.grad(L.W_GATE)] + [m.grad(w, e) for e in range(cfg.E + cfg.Es) for w in (L.W_W1, L.W_W3, L.W_W2)]
+
+    for i, (a, b) in enumerate(zip(step(layer), step(fresh))):
+        assert np.array_equal(a, b), i
+    layer.set_expert(1, inp["W1"][1], inp["W3"][1], inp["W2"][1])      # weights set behind a step: transposed again
+    fresh.set_expert(1, inp["W1"][1], inp["W3"][1], inp["W2"][1])
+    assert all(np.array_equal(a, b) for a, b in zip(step(layer), step(fresh)))
+    for m in (layer, fresh):
+        m.close()
+    for b in (x, g):
+        b.free()
