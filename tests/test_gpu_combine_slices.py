@@ -3,6 +3,7 @@ last tiles only, none, with shared experts, and behind an output that only the e
 import numpy as np
 import pytest
 
+from oracle import oracle as O
 from oracle import oracle_np as N
 from tests.synth import C, scaled
 
@@ -17,7 +18,7 @@ pytestmark = pytest.mark.gpu
     dict(T=130, d=512, H=1024, E=5, K=4, Es=1),     # five rows in groups of three
     dict(T=300, d=2048, H=1408, E=64, K=6, Es=2),   # room for slices, and none made: too many tiles
     dict(T=4400, d=4096, H=4096, E=1, K=1, Es=0),   # the last tiles only: 18 x 16 tiles, 32 of them in 2 slices
-    dict(T=1100, d=256, H=256, E=4, K=1, Es=0),     # room for slices, and none made
+    dict(T=1100, d=256, H=256, E=4, K=1, Es=0),     # items of 128 columns, no slices
 ], ids=lambda k: "-".join(str(v) for v in k.values()))
 def test_combine_adds_the_k_slices(kw):
     """The sums the combine kernel forms from y and the slices are those of the kernel that adds them into y: the same bits."""
@@ -47,4 +48,32 @@ def test_combine_adds_the_k_slices(kw):
     assert N.rel_l2(out[t], ref) <= 4e-3        # one rounding to bf16: at most 2^-9 of an element
     for b in (o, x):
         b.free()
+    layer.close()
+
+
+def test_a_batch_without_slices_behind_one_with_them():
+    """4400 tokens leave a last round of 32 tiles, in 2 slices each; 4096 are one whole round: room for slices, and none made, but y_slabs
+    and the table of the batch before are still there.  Then the first again."""
+    from tests import gpu_util as G
+    cfg = scaled(C.CONFIGS["c4_finegrained"], T=4400, d=4096, H=4096, E=1, K=1, Es=0)
+
+    def build():
+        layer = G.P.MoELayer(cfg.d, cfg.H, cfg.E, cfg.K, renorm=cfg.renorm, nShared=cfg.Es, bias=False, ctx=G.ctx(), dtype="bf16")
+        layer.init_synthetic(17, C, cfg)
+        return layer
+
+    layer = build()
+    x = G.P.DeviceBuffer(G.ctx(), (cfg.T, cfg.d), "bf16")
+    x.fill_normal(17, C.STREAM_X, 1.0)
+    bits = x.to_numpy()
+    for T in (4400, 4096, 4400):
+        xt = G.P.DeviceBuffer.from_numpy(G.ctx(), bits[:T], "bf16")
+        out = layer.forward(xt).to_numpy()
+        y = layer.workspace("y", T)                     # one expert, combine weight 1: the output is y
+        assert np.array_equal(out, O.round_bf16(y)), T
+        alone = build()
+        assert np.array_equal(alone.forward(xt).to_numpy(), out), T
+        alone.close()
+        xt.free()
+    x.free()
     layer.close()
