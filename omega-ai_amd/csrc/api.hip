@@ -694,7 +694,8 @@ static int stage_dispatch(omega_moe *m, const void *x, int T, bool up_follows = 
         // A batch whose down product has output tiles for at most half of the compute units is bound by the weight
         // bytes each workgroup keeps in flight.  With H >= 512 the table builder then cuts every tile's k range into
         // up to 8 slices (as many as fill the compute units; it knows how many experts have rows), which write partial
-        // results that a small kernel adds up; narrower layers get 128-column items instead.
+        // results that the combine adds as it reads y, or down_slab_reduce_kernel where y itself is read; narrower layers
+        // get 128-column items instead.
         // (The host knows only bounds of the number of row tiles: slicing is switched on when the fewest tiles this
         //  batch can have would qualify, and the table builder decides by the tiles there are.)
         const omega_moe_config &c = m->cfg;

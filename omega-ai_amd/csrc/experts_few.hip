@@ -51,7 +51,8 @@ __device__ __forceinline__ void few_copy(const few_args &p, int wg, int lane, in
     }
 }
 
-// k steps in flight per wave: what 128 registers, four waves per SIMD, leave
+// k steps in flight per wave: what 128 registers, four waves per SIMD, leave.  (Tiles of four units with four blocks have room for one step
+// and spill three registers, one in the down product: stored once in front of the k loop and read once behind it.)
 constexpr int few_depth(int U, int NB)
 {
     const int d = (104 - 4 * U * NB) / (4 * (U + NB));
