@@ -22,6 +22,7 @@
 // run the chains (Mixtral shape: 4096 tokens 33 -> 29 us, 64 tokens 27 -> 22 us; of the 22, 11 are the chain itself at
 // 6.25 clocks a term and 6.5 are launch, the first loads and phases 2 and 3).
 #include "common.h"
+#include <limits.h>
 #include <type_traits>
 
 typedef __attribute__((ext_vector_type(8))) __bf16 rt_bf16x8;
@@ -811,13 +812,17 @@ hipError_t launch_router(const omega_moe *m, const void *x, int T, float *logits
 #undef ROUTER_MFMA_LAUNCH
         return hipGetLastError();
     }
-    // (tokens per workgroup of the split form: the fewest that leave a workgroup a compute unit of its own, 4 are one wave of sums;
-    // short rows of few experts are as quick in one launch: 100 tokens x 1024, 20 experts 10.0 / 10.2 us, 16 x 1024, 64 experts 11.6 / 11.7)
+    // (tokens per workgroup of the split form: the fewest that leave a workgroup a compute unit of its own, 4 are one wave of sums.
+    // Rows have to be long enough to pay for the second launch, and the longer the fewer experts share a workgroup's chain on the matrix
+    // cores.  One launch / two, us, around each line: 500 tokens x 1280, 20 experts 12.2 / 12.1, 640 x 1280 12.2 / 12.6, 1000 x 1536 13.9 / 13.7; 64
+    // experts, 64 x 1280 12.8 / 12.7, 64 x 1536 14.6 / 13.4, 33 experts, 500 x 1536 14.0 / 14.4, 500 x 2048 16.9 / 16.4; 100 experts, 200 x 512 11.9 / 13.1,
+    // 200 x 768 14.8 / 14.2, 500 x 768 14.9 / 15.6, 500 x 1024 17.5 / 16.5; 200 experts, 60 x 256 13.6 / 16.5, 60 x 512 18.2 / 16.0.)
     const int groups = ceil_div(c.E, 16);
     int tpw = 4;
     while (tpw < 16 && ceil_div(T, tpw) * groups > m->ctx->num_cus) tpw *= 2;
+    const int split_d = c.E > 128 ? 512 : c.E > 64 ? (tpw < 16 ? 768 : 1024) : tpw == 16 ? INT_MAX : c.E > 32 ? (tpw < 8 ? 1536 : 2048) : (tpw < 8 ? 1280 : 1536);
     if (router_on_mfma(m) && (logits_out != nullptr || m->gate_logits != nullptr) && router_tok_tile(m, T) == 16 &&
-        ceil_div(T, tpw) * groups <= m->ctx->num_cus && (c.E > 64 || (tpw < 16 && c.d > 1024)) && (((uintptr_t)x | (uintptr_t)m->Wg) % 16) == 0) {
+        ceil_div(T, tpw) * groups <= m->ctx->num_cus && c.d >= split_d && (((uintptr_t)x | (uintptr_t)m->Wg) % 16) == 0) {
         float *lg = logits_out != nullptr ? logits_out : m->gate_logits;
         hipLaunchKernelGGL((router_pipe_kernel<16, true>), dim3(ceil_div(T, tpw) * groups), dim3(16 * 16 + RP_STAGERS), router_pipe_smem_bytes(16),
                            s, (const bf16_t *)x, (const bf16_t *)m->Wg, bg, T, c.d, c.E, c.K, c.renorm, m->ids, m->w, m->tile_counts, lg,

@@ -33,6 +33,7 @@ def test_widths_between_chunks(name, kw):
 
 
 # the sums split by experts: 4, 8 and 16 tokens per workgroup, a last group of one expert, of fifteen, ragged token groups
-@pytest.mark.parametrize("T,d,E,K", [(3, 1536, 17, 2), (5, 3328, 31, 3), (131, 1280, 64, 6), (500, 1280, 40, 2), (500, 512, 100, 4), (257, 256, 241, 8)])
+@pytest.mark.parametrize("T,d,E,K", [(3, 1536, 17, 2), (5, 3328, 31, 3), (131, 1280, 64, 6), (500, 1280, 40, 2), (500, 512, 100, 4), (257, 256, 241, 8),
+                                     (131, 1536, 64, 6), (500, 2048, 40, 2), (500, 1024, 100, 4), (230, 512, 241, 8), (9, 768, 65, 3)])
 def test_sums_split_by_experts(T, d, E, K):
     logits_bit_for_bit(T, d, E, K)
