@@ -6,7 +6,7 @@
 //
 // Bound: HBM, 3 d H weights of two bytes per expert used.  The tile kernels keep five k steps of a 256-column item in flight
 // per compute unit, in LDS, and a launch has few items: 6 experts of H = 768 are 36 for 256 compute units, 66 of d = 2048 are
-// 2.06 rounds of 256-column items in the down product.  Here a workgroup takes 16 columns of W1 and of W3 (down: 32 of W2)
+// 2.06 rounds of 256-column items in the down product.  Here a workgroup takes 16 or 32 columns of W1 and of W3 (down: 32 or 64 of W2)
 // of one expert, its waves share k, and each wave streams its blocks of the packed image straight into registers: a 1 KiB
 // block is one MFMA fragment (16 rows x 32 k, lane l row l % 16, chunk l / 16), one coalesced 16-byte load per lane, past the
 // last-level cache since nobody reads it again.  PF steps of loads are in flight per wave and 16 waves per compute unit.  The
