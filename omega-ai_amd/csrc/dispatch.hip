@@ -668,8 +668,8 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8, 8))) vo
         if (tid == 0) tile_meta[0] = mt_s[G];
         for (int g = tid; g <= G; g += nthr) tile_meta[1 + g] = mt_s[g];
     }
-    // row-tile list: eight lanes per group
-    for (int g = (tile * nthr + tid) >> 3; g < G; g += (n_tiles * nthr) >> 3) {
+    // row-tile list, for the kernels that go without queues: eight lanes per group
+    for (int g = n_sched > 0 ? G : (tile * nthr + tid) >> 3; g < G; g += (n_tiles * nthr) >> 3) {
         const int rows = g < E ? off_s[g + 1] - off_s[g] : T;
         const int nm = mt_s[g + 1] - mt_s[g];
         for (int mt = tid & 7; mt < nm; mt += 8) {
