@@ -725,7 +725,9 @@ static int stage_dispatch(omega_moe *m, const void *x, int T, bool up_follows = 
     m->few = !m->training && experts_few_rows(m, T);
     m->queued = !m->few;
     const bool up_gathers = up_follows && (m->few || (!bf && (double)T * m->cfg.d * 4.0 < 4.0e9));
-    OMEGA_HIP_CHECK(m->ctx, launch_dispatch_index(m, T, bm, m->ctx->stream, bf && !m->gather_on_load && !up_gathers ? x : nullptr));
+    // (a few tokens: their up product makes the index itself)
+    m->index_in_up = up_follows && m->few && experts_few_index(m, T);
+    if (!m->index_in_up) OMEGA_HIP_CHECK(m->ctx, launch_dispatch_index(m, T, bm, m->ctx->stream, bf && !m->gather_on_load && !up_gathers ? x : nullptr));
     if (!bf && !up_gathers) OMEGA_HIP_CHECK(m->ctx, launch_dispatch_gather(m, x, T, m->ctx->stream));
     m->xg_valid = !m->gather_on_load && !up_gathers;
     m->dispatched_T = T;
@@ -750,7 +752,13 @@ static int stage_experts(omega_moe *m, const void *x, int T, int which)
     const bool keep = which == 0 && keeps_for_backward(m, T);
     if (m->cfg.dtype == OMEGA_DTYPE_BF16) {
         if (which == 0 && m->few && !m->xg_valid && !x) OMEGA_FAIL(m->ctx, OMEGA_ERR_INVALID_ARG, "experts: x is NULL");
-        OMEGA_HIP_CHECK(m->ctx, launch_experts_bf16(m, x, T, which, m->ctx->stream, keep));
+        const bool index = which == 0 && m->index_in_up;
+        if (index) {
+            m->index_in_up = false;
+            m->dispatched_T = -1;  // (until the launch that makes it is under way)
+        }
+        OMEGA_HIP_CHECK(m->ctx, launch_experts_bf16(m, x, T, which, m->ctx->stream, keep, index));
+        if (index) m->dispatched_T = T;
         if (which == 0 && m->few && !m->gather_on_load) m->xg_valid = true;
     } else if (which == 0) {
         const bool gather = !m->xg_valid;

@@ -102,6 +102,7 @@ struct omega_moe {
     // the batch is one of a few tokens outside training: its products run on experts_few.hip and its dispatch made no work queues
     // (what needs them has them made first: ensure_queues)
     bool few = false, queued = true;
+    bool index_in_up = false;        // ... and its up product, not launched yet, makes the dispatch index
     // the down product of the batch in y has left k slices in y_slabs that are not in y: the combine kernel adds them on its
     // way (combine.hip), whatever else reads y has them added first (ensure_y_whole)
     bool y_partial = false;
@@ -225,8 +226,10 @@ enum { F32_UP = 0, F32_DOWN, F32_RAW, F32_DA, F32_DXG, F32_WG2, F32_WG13 };
 hipError_t launch_product_f32(const omega_moe *m, int op, const float *x, const float *dout, int T, hipStream_t s, bool gather = false,
                               bool keep = false);
 // which: 0 up product, 1 down product
-hipError_t launch_experts_bf16(const omega_moe *m, const void *x, int T, int which, hipStream_t s, bool keep);
-hipError_t launch_experts_few(const omega_moe *m, const void *x, int T, int which, hipStream_t s);
+hipError_t launch_experts_bf16(const omega_moe *m, const void *x, int T, int which, hipStream_t s, bool keep, bool index);
+// index: the up launch makes the dispatch index as well (experts_few_index says whether it can)
+hipError_t launch_experts_few(const omega_moe *m, const void *x, int T, int which, hipStream_t s, bool index);
+bool experts_few_index(const omega_moe *m, int T);
 // resid != nullptr: out = resid + layer output (one rounding of the fp32 sum)
 hipError_t launch_combine(const omega_moe *m, int T, void *out, const void *resid, hipStream_t s);
 hipError_t launch_backward_f32(omega_moe *m, const void *x, const void *dout, int T, void *dx, hipStream_t s);

@@ -31,20 +31,174 @@ struct few_args {
     const unsigned char *B0, *B1;  // W1, W3; down: W2, unused
     unsigned char *a;           // up: output
     float *y;                   // down: output
-    const omega_tile *tiles;
-    const int32_t *tile_meta, *tokp, *dstp;
-    unsigned char *xg, *xs;     // up: the gathered copy, written by the launch's last copy_wgs workgroups
+    omega_tile *tiles;
+    int32_t *tile_meta, *tokp, *dstp;
+    const int32_t *ids;         // up: the launch makes the dispatch index itself from the router's choices (or null: it is there)
+    int32_t *counts, *offsets, *dst, *src_row;
+    int E, Es;
+    unsigned char *xg, *xs;     // up: the gathered copy, written by the launch's first copy_wgs workgroups (behind the one of the index)
     int copy_wgs, T, K;
     int N, Kd;                  // output columns and k
 };
 
+// The dispatch index within the up launch.  A batch's pairs are so few that a workgroup finds its expert and rows from the router's choices in the
+// time that reading them out of the index takes (three dependent loads), so nothing has to run in front of the product but the router;
+// the index itself - what dispatch_rank_kernel leaves - is made by a workgroup of its own beside the products, the launch's last: the products'
+// workgroups keep their XCDs, four that share the lines of a row group on XCDs 0-3 or 4-7 (moved on by one, two or three, 64 tokens x 4096 x 14336, 8
+// experts, up product 278 -> 307, 327, 307 us).  Forward pass, us, with a launch for the index / without: 1 and 64 tokens x 4096 x 14336, 8 experts,
+// top 2 132.1 -> 127.2, 454.5 -> 449; 48 tokens x 2048 x 1408, 64 experts, top 6, 2 shared 202 -> 195.6
+#define FEW_PAIRS_MAX 1024
+#define FEW_BM 256         // rows of a tile: every expert that is used has one
+struct few_shared {
+    uint8_t flag[256];      // experts that have rows
+    uint8_t id[FEW_PAIRS_MAX];
+    uint8_t tok[64];        // tokens of the workgroup's rows
+};
+struct few_used { unsigned long long m[4]; };  // the flags as bits, uniform
+
+// The choices of all pairs, and who is chosen at all
+__device__ __forceinline__ few_used few_choices(const few_args &p, few_shared &sh, int lane, int wave, int waves)
+{
+    const int P = p.T * p.K;
+    if (wave == 0) ((uint32_t *)sh.flag)[lane] = 0u;
+    __syncthreads();
+    for (int i0 = 64 * wave; i0 < P; i0 += 64 * waves) {
+        const int e = i0 + lane < P ? p.ids[i0 + lane] : 0;
+        if (i0 + lane < P) {
+            sh.id[i0 + lane] = (uint8_t)e;
+            sh.flag[e] = 1;
+        }
+    }
+    __syncthreads();
+    few_used u;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) u.m[q] = __ballot(sh.flag[64 * q + lane] != 0);
+    return u;
+}
+// experts below e that have rows: e's row tile
+__device__ __forceinline__ int few_tile(const few_used &us, int e)
+{
+    int n = 0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) n += __popcll(64 * q + 64 <= e ? us.m[q] : 64 * q < e ? us.m[q] & ((1ull << (e & 63)) - 1ull) : 0ull);
+    return n;
+}
+// pairs before pair u (uniform over the wave) with its expert: its rank among that expert's rows
+__device__ __forceinline__ int few_rank(const few_shared &sh, int u, int lane)
+{
+    const int e = sh.id[u];
+    int n = 0;
+    for (int c = 0; c < u; c += 64) n += __popcll(__ballot(c + lane < u && sh.id[c + lane] == e));
+    return n;
+}
+// Row tile `mt` of the batch (the used experts in rising order, then the shared ones) and the tokens of its rows; every wave by itself
+__device__ __forceinline__ omega_tile few_find(const few_args &p, few_shared &sh, const few_used &us, int mt, int n_used, int lane)
+{
+    omega_tile tl;
+    tl.row0 = mt * FEW_BM;
+    if (mt >= n_used) {
+        tl.g = p.E + mt - n_used;
+        tl.rows = p.T;
+        tl.xrow0 = 0;
+        return tl;
+    }
+    tl.xrow0 = -1;
+    tl.g = 0;
+    int k = mt;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int c = __popcll(us.m[q]);
+        if (k >= 0 && k < c) tl.g = 64 * q + __ffsll(__ballot((us.m[q] >> lane & 1ull) && __popcll(us.m[q] & ((1ull << lane) - 1ull)) == k)) - 1;
+        k -= c;
+    }
+    const int P = p.T * p.K;
+    int n = 0;
+    for (int c = 0; c < P; c += 64) {
+        const bool mine = c + lane < P && sh.id[c + lane] == tl.g;
+        const unsigned long long m = __ballot(mine);
+        if (mine) sh.tok[n + __popcll(m & ((1ull << lane) - 1ull))] = (uint8_t)((c + lane) / p.K);  // (each wave the same)
+        n += __popcll(m);
+    }
+    tl.rows = n;
+    return tl;
+}
+// The index, by one workgroup: counts, offsets, the pairs' places, the row -> token table and the row-tile list
+__device__ __forceinline__ void few_index(const few_args &p, const few_shared &sh, const few_used &us, int *run, int *off, int n_used, int lane, int wave, int nthr)
+{
+    const int P = p.T * p.K, tid = threadIdx.x;
+    for (int e = tid; e < p.E; e += nthr) run[e] = 0;
+    __syncthreads();
+    for (int i = tid; i < P; i += nthr) atomicAdd(&run[sh.id[i]], 1);
+    __syncthreads();
+    if (wave > 0) return;
+    // exclusive scan of the counts, four experts per lane; run[e] becomes the rows of e that have their place
+    int c[4], sum = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int e = 4 * lane + i;
+        c[i] = e < p.E ? run[e] : 0;
+        sum += c[i];
+    }
+    int incl = sum;
+#pragma unroll
+    for (int m = 1; m < 64; m <<= 1) {
+        const int o = __shfl_up(incl, m, 64);
+        if (lane >= m) incl += o;
+    }
+    int at = incl - sum;
+    if (lane == 63) p.offsets[p.E] = incl;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int e = 4 * lane + i;
+        if (e >= p.E) continue;
+        const int mt = few_tile(us, e);
+        p.counts[e] = c[i];
+        p.offsets[e] = at;
+        p.tile_meta[1 + e] = mt;
+        if (c[i] > 0) p.tiles[mt] = {e, mt * FEW_BM, c[i], -1};
+        run[e] = 0;
+        off[e] = at;
+        at += c[i];
+    }
+    for (int s = lane; s <= p.Es; s += 64) {
+        p.tile_meta[1 + p.E + s] = n_used + s;
+        if (s < p.Es) p.tiles[n_used + s] = {p.E + s, (n_used + s) * FEW_BM, p.T, 0};
+    }
+    if (lane == 0) p.tile_meta[0] = n_used + p.Es;
+    // stable ranks, 64 pairs at a time: the lanes with one expert find each other by ballot, run[e] moves on by their number
+    for (int c0 = 0; c0 < P; c0 += 64) {
+        const int i = c0 + lane;
+        const bool valid = i < P;
+        const int e = valid ? sh.id[i] : -1;
+        unsigned long long todo = __ballot(valid), mine = 0;
+        while (todo) {
+            const int le = __builtin_amdgcn_readlane(e, __ffsll((long long)todo) - 1);
+            const unsigned long long m = __ballot(e == le);
+            if (e == le) mine = m;
+            todo &= ~m;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        const unsigned long long below = mine & ((1ull << lane) - 1ull);
+        if (valid) {
+            const int rank = run[e] + __popcll(below), r = off[e] + rank, prow = few_tile(us, e) * FEW_BM + rank, t = i / p.K;
+            p.dst[i] = r;
+            p.dstp[i] = prow;
+            p.src_row[r] = t;
+            p.tokp[prow] = t;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        if (valid && below == 0) run[e] += __popcll(mine);
+    }
+}
+
 // Wave per row of the copy (a pair's row of xg, then the token rows of xs): what the dispatch launch does for larger batches,
 // beside the products instead of in front of them
-__device__ __forceinline__ void few_copy(const few_args &p, int wg, int lane, int wave, int waves)
+__device__ __forceinline__ void few_copy(const few_args &p, const few_shared &sh, const few_used &us, int wg, int lane, int wave, int waves)
 {
     const int KT = p.Kd >> 5, P = p.T * p.K, n = P + (p.xs != nullptr ? p.T : 0);
     for (int u = wg * waves + wave; u < n; u += waves * p.copy_wgs) {
-        const int t = u < P ? u / p.K : u - P, row = u < P ? p.dstp[u] : t;
+        const int t = u < P ? u / p.K : u - P;
+        const int row = u >= P ? t : p.ids != nullptr ? few_tile(us, sh.id[u]) * FEW_BM + few_rank(sh, u, lane) : p.dstp[u];
         const unsigned char *src = p.x + (size_t)t * p.Kd * 2;
         unsigned char *dst = u < P ? p.xg : p.xs;
         for (int c = lane; c < 4 * KT; c += 64) *(uint4 *)(dst + pk_chunk_off(row, c >> 2, c & 3, KT)) = *(const uint4 *)(src + (size_t)c * 16);
@@ -110,19 +264,37 @@ template <bool UP, int UM, int NW, int NB>
 __global__ __launch_bounds__(64 * NW, 4) void few_rows_kernel(few_args p)
 {
     __shared__ few_f32x4 part[UM > 1 ? 2 : 1][NW][NB][64];
+    __shared__ few_shared sh;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int l16 = lane & 15, lq = lane >> 4;
     constexpr int NC = UP ? NB / 2 : NB;  // 16-column blocks of the output per workgroup
     const int nc = p.N / (16 * NC);
-    if (UP && (int)blockIdx.x >= (int)gridDim.x - p.copy_wgs) {
-        few_copy(p, blockIdx.x - (gridDim.x - p.copy_wgs), lane, wave, NW);
+    const bool self = UP && p.ids != nullptr;
+    const int blk = blockIdx.x;
+    int n_used = 0;
+    few_used us = {};
+    if (self) {
+        us = few_choices(p, sh, lane, wave, NW);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) n_used += __popcll(us.m[q]);
+        if (blk == (int)gridDim.x - 1) {
+            static_assert(sizeof(part) >= 2 * 256 * sizeof(int), "room for the index");
+            few_index(p, sh, us, (int *)part, (int *)part + 256, n_used, lane, wave, 64 * NW);
+            return;
+        }
+    }
+    const int copy0 = (int)gridDim.x - (self ? 1 : 0) - p.copy_wgs;
+    if (UP && blk >= copy0) {
+        few_copy(p, sh, us, blk - copy0, lane, wave, NW);
         return;
     }
     // the row tiles in falling order, which takes the shared experts - all T rows - first
-    const int wt = blockIdx.x / nc, n0 = (blockIdx.x - wt * nc) * (16 * NC);
-    const int mt = p.tile_meta[0] - 1 - wt;
+    const int wt = blk / nc, n0 = (blk - wt * nc) * (16 * NC);
+    const int mt = (self ? n_used + p.Es : p.tile_meta[0]) - 1 - wt;
     if (mt < 0) return;
-    const omega_tile tl = p.tiles[mt];
+    omega_tile tl = self ? few_find(p, sh, us, mt, n_used, lane) : p.tiles[mt];
+    tl = {__builtin_amdgcn_readfirstlane(tl.g), __builtin_amdgcn_readfirstlane(tl.row0), __builtin_amdgcn_readfirstlane(tl.rows),
+          __builtin_amdgcn_readfirstlane(tl.xrow0)};
     const int KT = p.Kd >> 5, units = (tl.rows + 15) >> 4;
     const int s0 = wave * KT / NW, n = (wave + 1) * KT / NW - s0;
     // uniform: k step s0 of the workgroup's 16-row blocks of the weights; lane: its chunk of a block (the swizzle depends on the
@@ -152,7 +324,7 @@ __global__ __launch_bounds__(64 * NW, 4) void few_rows_kernel(few_args p)
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const int r = 16 * u + l16 < tl.rows ? 16 * u + l16 : 0;
-            a_off[u] = gather ? (uint32_t)(tl.xrow0 >= 0 ? tl.xrow0 + r : p.tokp[tl.row0 + r]) * (uint32_t)(p.Kd * 2) + lq * 16
+            a_off[u] = gather ? (uint32_t)(tl.xrow0 >= 0 ? tl.xrow0 + r : self ? (int)sh.tok[r] : p.tokp[tl.row0 + r]) * (uint32_t)(p.Kd * 2) + lq * 16
                               : (uint32_t)((r >> 4) * 1024 + (r & 15) * 64 + ((lq ^ pk_swz(r)) << 4));
         }
         few_f32x4 acc[U][NB];
@@ -198,8 +370,10 @@ __global__ __launch_bounds__(64 * NW, 4) void few_rows_kernel(few_args p)
     else run(std::integral_constant<int, UM>());
 }
 
+bool experts_few_index(const omega_moe *m, int T) { return T * m->cfg.K <= FEW_PAIRS_MAX; }
+
 // which: 0 up - the rows come from x unless there is a gathered copy, and one is left beside if the layer keeps one -, 1 down
-hipError_t launch_experts_few(const omega_moe *m, const void *x, int T, int which, hipStream_t s)
+hipError_t launch_experts_few(const omega_moe *m, const void *x, int T, int which, hipStream_t s, bool index)
 {
     const omega_moe_config &c = m->cfg;
     const bool gather = !m->xg_valid, copy = gather && !m->gather_on_load;
@@ -220,13 +394,22 @@ hipError_t launch_experts_few(const omega_moe *m, const void *x, int T, int whic
         p.a = (unsigned char *)m->a;
         p.N = c.H;
         p.Kd = c.d;
+        if (index) {
+            p.ids = m->ids;
+            p.counts = m->counts;
+            p.offsets = m->offsets;
+            p.dst = m->dst;
+            p.src_row = m->src_row;
+            p.E = c.E;
+            p.Es = c.Es;
+        }
         if (copy) {
             p.xg = (unsigned char *)m->xg;
             p.xs = (unsigned char *)m->xs;
             p.copy_wgs = std::min(ceil_div(T * (c.K + (c.Es > 0 ? 1 : 0)), 4), m->ctx->num_cus);
         }
 #define FEW_LAUNCH(UPV, UMV, NWV, NBV)                                                                                              \
-    hipLaunchKernelGGL((few_rows_kernel<UPV, UMV, NWV, NBV>), dim3(tiles * (p.N / (UPV ? 8 * NBV : 16 * NBV)) + p.copy_wgs), dim3(64 * NWV), 0, s, p)
+    hipLaunchKernelGGL((few_rows_kernel<UPV, UMV, NWV, NBV>), dim3(tiles * (p.N / (UPV ? 8 * NBV : 16 * NBV)) + (p.ids != nullptr ? 1 : 0) + p.copy_wgs), dim3(64 * NWV), 0, s, p)
         // Four blocks of weights per step from 17 tokens on (two units of rows: 64 tokens x 4096 x 14336, 8 experts, up product 326 ->
         // 294 us), two below (1 token 71 against 73, 1 token x 3328 x 896, 86 experts 12.0 against 15.9).  Two waves where four would
         // have 8 k steps each or fewer, which is all start-up (64 tokens x 1024 x 768, 128 experts: pass 133 -> 128.5; d = 1536 169
