@@ -725,8 +725,8 @@ static int stage_dispatch(omega_moe *m, const void *x, int T, bool up_follows = 
     m->few = !m->training && experts_few_rows(m, T);
     m->queued = !m->few;
     const bool up_gathers = up_follows && (m->few || (!bf && (double)T * m->cfg.d * 4.0 < 4.0e9));
-    // (a few tokens: their up product makes the index itself)
-    m->index_in_up = up_follows && m->few && experts_few_index(m, T);
+    // (a few tokens, or pairs of an fp32 layer: their up product makes the index itself)
+    m->index_in_up = up_gathers && (bf ? experts_few_index(m, T) : product_f32_index(m, T));
     if (!m->index_in_up) OMEGA_HIP_CHECK(m->ctx, launch_dispatch_index(m, T, bm, m->ctx->stream, bf && !m->gather_on_load && !up_gathers ? x : nullptr));
     if (!bf && !up_gathers) OMEGA_HIP_CHECK(m->ctx, launch_dispatch_gather(m, x, T, m->ctx->stream));
     m->xg_valid = !m->gather_on_load && !up_gathers;
@@ -749,23 +749,22 @@ static int stage_experts(omega_moe *m, const void *x, int T, int which)
         OMEGA_FAIL(m->ctx, OMEGA_ERR_INVALID_ARG, "experts: dispatch has not run for this T");
     if (which == 0 && m->gather_on_load && !x) OMEGA_FAIL(m->ctx, OMEGA_ERR_INVALID_ARG, "experts: x is NULL");
     if (which == 1 && !m->a_valid) OMEGA_FAIL(m->ctx, OMEGA_ERR_INVALID_ARG, "experts_down: the up product has not run since `a` was overwritten");
-    const bool keep = which == 0 && keeps_for_backward(m, T);
+    const bool keep = which == 0 && keeps_for_backward(m, T), index = which == 0 && m->index_in_up;
+    if (index) {
+        m->index_in_up = false;
+        m->dispatched_T = -1;  // (until the launch that makes it is under way)
+    }
     if (m->cfg.dtype == OMEGA_DTYPE_BF16) {
         if (which == 0 && m->few && !m->xg_valid && !x) OMEGA_FAIL(m->ctx, OMEGA_ERR_INVALID_ARG, "experts: x is NULL");
-        const bool index = which == 0 && m->index_in_up;
-        if (index) {
-            m->index_in_up = false;
-            m->dispatched_T = -1;  // (until the launch that makes it is under way)
-        }
         OMEGA_HIP_CHECK(m->ctx, launch_experts_bf16(m, x, T, which, m->ctx->stream, keep, index));
-        if (index) m->dispatched_T = T;
         if (which == 0 && m->few && !m->gather_on_load) m->xg_valid = true;
     } else if (which == 0) {
         const bool gather = !m->xg_valid;
         if (gather && !x) OMEGA_FAIL(m->ctx, OMEGA_ERR_INVALID_ARG, "experts: x is NULL");
-        OMEGA_HIP_CHECK(m->ctx, launch_product_f32(m, F32_UP, (const float *)x, nullptr, T, m->ctx->stream, gather, keep));
+        OMEGA_HIP_CHECK(m->ctx, launch_product_f32(m, F32_UP, (const float *)x, nullptr, T, m->ctx->stream, gather, keep, index));
         m->xg_valid = true;
     } else OMEGA_HIP_CHECK(m->ctx, launch_product_f32(m, F32_DOWN, nullptr, nullptr, T, m->ctx->stream));
+    if (index) m->dispatched_T = T;
     if (which == 0) {
         m->a_valid = true;
         return OMEGA_OK;

@@ -224,7 +224,8 @@ enum { F32_UP = 0, F32_DOWN, F32_RAW, F32_DA, F32_DXG, F32_WG2, F32_WG13 };
 // (gather: F32_UP fetches the routed rows from x and leaves the gathered copy beside it; keep: it leaves h1 and h3 in
 // bw_h1 / bw_h3, as launch_experts_bf16 does)
 hipError_t launch_product_f32(const omega_moe *m, int op, const float *x, const float *dout, int T, hipStream_t s, bool gather = false,
-                              bool keep = false);
+                              bool keep = false, bool index = false);
+bool product_f32_index(const omega_moe *m, int T);  // whether F32_UP, with `gather`, can make the dispatch index as well (`index`)
 // which: 0 up product, 1 down product
 hipError_t launch_experts_bf16(const omega_moe *m, const void *x, int T, int which, hipStream_t s, bool keep, bool index);
 // index: the up launch makes the dispatch index as well (experts_few_index says whether it can)

@@ -38,6 +38,30 @@
 // parts of 32 rows x 32 output columns that a row product's tile of 64 rows may be cut into
 #define F32_PARTS(OP, TM, TN) (F32_IS_WG(OP) || (TM) == F32_TILE_M_SMALL ? 1 : (TM) / 32 * ((TN) / (F32_PAIR(OP) ? 64 : 32)))
 
+// The up product of a few pairs finds its rows from the router's choices and leaves the dispatch index, made by the launch's last workgroup, to the
+// launches behind: a launch less in front of it.  First column of this workgroup's tile (tl, tokens of its rows in tok), or -1: nothing to do.
+// Forward pass of 256 tokens x 128 x 256, 8 experts, top 2: 23.5 -> 19.8 us (with loops over the chunks that branch 22.8, with the index made in LDS by
+// small_index 21.9).
+template <int NC, bool VEC>
+__device__ __forceinline__ int f32_self(const f32_args &p, uint16_t *tok, omega_tile &tl)
+{
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), last = gridDim.x - 1;
+    f32_choices<NC> ch;
+    ch.read(p, lane);
+    if ((int)blockIdx.x >= last - p.copy_wgs) {
+        if ((int)blockIdx.x == last) ch.leave(p.index, lane, wave);
+        else copy_gathered<VEC, true>(p, blockIdx.x - (last - p.copy_wgs), lane, wave, ch);
+        return -1;
+    }
+    // (the tile as f32_product_kernel finds it)
+    const int NT = (p.N + 31) / 32, MT = ch.tiles + (p.G - p.E) * ((p.T + F32_TILE_M_SMALL - 1) / F32_TILE_M_SMALL), total = MT * NT, per = (total + 7) >> 3;
+    const int i = blockIdx.x >> 3, t = (blockIdx.x & 7) * per + i;
+    if (i >= per || t >= total) return -1;
+    const int rb = t / (8 * NT), nrb = min(8, MT - 8 * rb), ti = t - rb * 8 * NT;
+    tl = ch.find(p, 8 * rb + ti % nrb, lane, tok);
+    return (ti / nrb) * 32;
+}
+
 template <int OP, int TM, int TN, bool VEC>
 __global__ __launch_bounds__(256, 2) void f32_product_kernel(f32_args p)
 {
@@ -50,8 +74,18 @@ __global__ __launch_bounds__(256, 2) void f32_product_kernel(f32_args p)
     constexpr int LAP = f32_lds_floats(32, WG, F32_FBK(32)), LBP = f32_lds_floats(PN, BK_, F32_FBK(32));
     static_assert(!PARTS || LAP <= LA, "a part's operands fit");
     __shared__ __attribute__((aligned(16))) float as[WG ? 1 : 2 * LA], bs[WG ? 1 : 2 * (PARTS && LBP > LB ? LBP : LB)];
+    if constexpr (OP == F32_UP && TM == F32_TILE_M_SMALL) {
+        if (p.index.ids != nullptr) {
+            __shared__ uint16_t tok[F32_TILE_M_SMALL];
+            omega_tile tl;
+            const int P = p.T * p.K;
+            const int n0 = P <= 256 ? f32_self<4, VEC>(p, tok, tl) : P <= 512 ? f32_self<8, VEC>(p, tok, tl) : f32_self<F32_SELF_CHUNKS, VEC>(p, tok, tl);
+            if (n0 >= 0) f32_tile<OP, TM, TN, VEC>(p, as, bs, 0, tl, 0, n0, 0, tok);
+            return;
+        }
+    }
     if (OP == F32_UP && (int)blockIdx.x >= (int)gridDim.x - p.copy_wgs) {
-        copy_gathered<VEC>(p, blockIdx.x - (gridDim.x - p.copy_wgs), threadIdx.x & 63, threadIdx.x >> 6);
+        copy_gathered<VEC, false>(p, blockIdx.x - (gridDim.x - p.copy_wgs), threadIdx.x & 63, threadIdx.x >> 6, 0);
         return;
     }
 
@@ -81,11 +115,11 @@ __global__ __launch_bounds__(256, 2) void f32_product_kernel(f32_args p)
 
     if constexpr (PARTS) {
         if (part >= 0) {
-            f32_tile<OP, 32, PN, VEC>(p, as, bs, mt, 32 * (part % (TM / 32)), n0 + 32 * (part / (TM / 32)), mat);
+            f32_tile<OP, 32, PN, VEC>(p, as, bs, mt, p.tiles[mt], 32 * (part % (TM / 32)), n0 + 32 * (part / (TM / 32)), mat);
             return;
         }
     }
-    f32_tile<OP, TM, TN, VEC>(p, as, bs, mt, 0, n0, mat);
+    f32_tile<OP, TM, TN, VEC>(p, as, bs, mt, WG ? omega_tile{} : p.tiles[mt], 0, n0, mat);
 }
 
 // The largest row-tile height that a batch of up to T tokens takes: with fewer than 128 rows per expert always 32 (160 shapes of
@@ -144,13 +178,19 @@ static hipError_t f32_launch(f32_args p, bool vec, int max_tiles, hipStream_t s)
     p.part_max = p.slots / 4;
     if (F32_IS_WG(OP)) p.deal = wgrad_deal_of(ceil_div(p.N, CT) * ceil_div(p.Kd, TM), p.G * (OP == F32_WG13 ? 2 : 1));
     // (weight gradients: whole groups of matrices and one of what is left over, each to eight XCDs)
-    const unsigned grid = (F32_IS_WG(OP) ? (unsigned)((tiles + 7) / 8 * 8 + (p.deal.rest > 0 ? 8 : 0)) : f32_grid(p, tiles, F32_PARTS(OP, TM, TN))) + p.copy_wgs;
+    const unsigned grid = (F32_IS_WG(OP) ? (unsigned)((tiles + 7) / 8 * 8 + (p.deal.rest > 0 ? 8 : 0)) : f32_grid(p, tiles, F32_PARTS(OP, TM, TN))) + p.copy_wgs + (p.index.ids != nullptr ? 1 : 0);
     if (vec) hipLaunchKernelGGL((f32_product_kernel<OP, TM, TN, true>), dim3(grid), dim3(256), 0, s, p);
     else hipLaunchKernelGGL((f32_product_kernel<OP, TM, TN, false>), dim3(grid), dim3(256), 0, s, p);
     return hipGetLastError();
 }
 
-hipError_t launch_product_f32(const omega_moe *m, int op, const float *x, const float *dout, int T, hipStream_t s, bool gather, bool keep)
+// Up launches that make the index themselves: tiles of 32 rows, what f32_choices holds
+bool product_f32_index(const omega_moe *m, int T)
+{
+    return m->bm == F32_TILE_M_SMALL && m->cfg.E <= F32_SELF_EXPERTS && (long long)T * m->cfg.K <= 64 * F32_SELF_CHUNKS;
+}
+
+hipError_t launch_product_f32(const omega_moe *m, int op, const float *x, const float *dout, int T, hipStream_t s, bool gather, bool keep, bool index)
 {
     const omega_moe_config &c = m->cfg;
     f32_args p = {};
@@ -175,6 +215,7 @@ hipError_t launch_product_f32(const omega_moe *m, int op, const float *x, const 
                 // turn behind the last product; 4096 tokens x 64 x 64, 64 experts, top 6, forward pass: 48.0 -> 46.4 us)
                 p.copy_wgs = std::min(ceil_div(T, 4), 4 * m->ctx->num_cus);
             }
+            if (index) p.index = index_args_of(m, T);
             if (op == F32_RAW || keep) { p.H1 = m->bw_h1; p.H3 = m->bw_h3; }
             break;
         case F32_DOWN:

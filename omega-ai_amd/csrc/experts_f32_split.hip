@@ -103,7 +103,7 @@ __global__ __launch_bounds__(256, SP_WAVES(NB)) void f32_split_kernel(f32_args p
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l16 = lane & 15, lq = lane >> 4, wr = wave / WC, wc = wave % WC;
     if (OP == F32_UP && (int)blockIdx.x >= (int)gridDim.x - p.copy_wgs) {
-        copy_gathered<VEC>(p, blockIdx.x - (gridDim.x - p.copy_wgs), lane, wave);
+        copy_gathered<VEC, false>(p, blockIdx.x - (gridDim.x - p.copy_wgs), lane, wave, 0);
         return;
     }
     const int NT = (p.N + CT - 1) / CT;
@@ -129,7 +129,7 @@ __global__ __launch_bounds__(256, SP_WAVES(NB)) void f32_split_kernel(f32_args p
     if constexpr (!WG) {
         if (part >= 0) {
             constexpr int PN = PAIR ? 64 : 32, LAP = f32_lds_floats(32, false, F32_FBK(32));
-            f32_tile<OP, 32, PN, VEC>(p, (float *)sp_lds, (float *)sp_lds + 2 * LAP, mt, 32 * (part % (TM / 32)), n0 + 32 * (part / (TM / 32)), mat);
+            f32_tile<OP, 32, PN, VEC>(p, (float *)sp_lds, (float *)sp_lds + 2 * LAP, mt, p.tiles[mt], 32 * (part % (TM / 32)), n0 + 32 * (part / (TM / 32)), mat);
             return;
         }
     }

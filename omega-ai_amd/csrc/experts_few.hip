@@ -14,7 +14,7 @@
 // Forward pass, us, tile kernels -> here: 1 / 16 / 64 tokens, d = 4096, H = 14336, 8 experts, top 2: 144 -> 132, 482 -> 452, 470 -> 458
 // (up product 6.6 TB/s of weights, 6.4 at 64 tokens); 16 / 48 tokens, d = 2048, H = 1408, 64 experts, top 6, 2 shared: 193 -> 163,
 // 226 -> 209; 2 tokens, d = 3072, H = 768, 4 experts, 2 shared: 86 -> 48; 4 tokens, d = 1024, H = 1024, 64 experts, top 4: 53 -> 37.
-#include "common.h"
+#include "index_small.h"
 #include "pack.h"
 #include <algorithm>
 #include <type_traits>
@@ -31,11 +31,9 @@ struct few_args {
     const unsigned char *B0, *B1;  // W1, W3; down: W2, unused
     unsigned char *a;           // up: output
     float *y;                   // down: output
-    omega_tile *tiles;
-    int32_t *tile_meta, *tokp, *dstp;
-    const int32_t *ids;         // up: the launch makes the dispatch index itself from the router's choices (or null: it is there)
-    int32_t *counts, *offsets, *dst, *src_row;
-    int E, Es;
+    const omega_tile *tiles;
+    const int32_t *tile_meta, *tokp, *dstp;
+    index_args index;           // up: the launch makes the dispatch index itself from index.ids, the router's choices (or null: it is there)
     unsigned char *xg, *xs;     // up: the gathered copy, written by the launch's first copy_wgs workgroups (behind the one of the index)
     int copy_wgs, T, K;
     int N, Kd;                  // output columns and k
@@ -63,7 +61,7 @@ __device__ __forceinline__ few_used few_choices(const few_args &p, few_shared &s
     if (wave == 0) ((uint32_t *)sh.flag)[lane] = 0u;
     __syncthreads();
     for (int i0 = 64 * wave; i0 < P; i0 += 64 * waves) {
-        const int e = i0 + lane < P ? p.ids[i0 + lane] : 0;
+        const int e = i0 + lane < P ? p.index.ids[i0 + lane] : 0;
         if (i0 + lane < P) {
             sh.id[i0 + lane] = (uint8_t)e;
             sh.flag[e] = 1;
@@ -97,7 +95,7 @@ __device__ __forceinline__ omega_tile few_find(const few_args &p, few_shared &sh
     omega_tile tl;
     tl.row0 = mt * FEW_BM;
     if (mt >= n_used) {
-        tl.g = p.E + mt - n_used;
+        tl.g = p.index.E + mt - n_used;
         tl.rows = p.T;
         tl.xrow0 = 0;
         return tl;
@@ -122,75 +120,6 @@ __device__ __forceinline__ omega_tile few_find(const few_args &p, few_shared &sh
     tl.rows = n;
     return tl;
 }
-// The index, by one workgroup: counts, offsets, the pairs' places, the row -> token table and the row-tile list
-__device__ __forceinline__ void few_index(const few_args &p, const few_shared &sh, const few_used &us, int *run, int *off, int n_used, int lane, int wave, int nthr)
-{
-    const int P = p.T * p.K, tid = threadIdx.x;
-    for (int e = tid; e < p.E; e += nthr) run[e] = 0;
-    __syncthreads();
-    for (int i = tid; i < P; i += nthr) atomicAdd(&run[sh.id[i]], 1);
-    __syncthreads();
-    if (wave > 0) return;
-    // exclusive scan of the counts, four experts per lane; run[e] becomes the rows of e that have their place
-    int c[4], sum = 0;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int e = 4 * lane + i;
-        c[i] = e < p.E ? run[e] : 0;
-        sum += c[i];
-    }
-    int incl = sum;
-#pragma unroll
-    for (int m = 1; m < 64; m <<= 1) {
-        const int o = __shfl_up(incl, m, 64);
-        if (lane >= m) incl += o;
-    }
-    int at = incl - sum;
-    if (lane == 63) p.offsets[p.E] = incl;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int e = 4 * lane + i;
-        if (e >= p.E) continue;
-        const int mt = few_tile(us, e);
-        p.counts[e] = c[i];
-        p.offsets[e] = at;
-        p.tile_meta[1 + e] = mt;
-        if (c[i] > 0) p.tiles[mt] = {e, mt * FEW_BM, c[i], -1};
-        run[e] = 0;
-        off[e] = at;
-        at += c[i];
-    }
-    for (int s = lane; s <= p.Es; s += 64) {
-        p.tile_meta[1 + p.E + s] = n_used + s;
-        if (s < p.Es) p.tiles[n_used + s] = {p.E + s, (n_used + s) * FEW_BM, p.T, 0};
-    }
-    if (lane == 0) p.tile_meta[0] = n_used + p.Es;
-    // stable ranks, 64 pairs at a time: the lanes with one expert find each other by ballot, run[e] moves on by their number
-    for (int c0 = 0; c0 < P; c0 += 64) {
-        const int i = c0 + lane;
-        const bool valid = i < P;
-        const int e = valid ? sh.id[i] : -1;
-        unsigned long long todo = __ballot(valid), mine = 0;
-        while (todo) {
-            const int le = __builtin_amdgcn_readlane(e, __ffsll((long long)todo) - 1);
-            const unsigned long long m = __ballot(e == le);
-            if (e == le) mine = m;
-            todo &= ~m;
-        }
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-        const unsigned long long below = mine & ((1ull << lane) - 1ull);
-        if (valid) {
-            const int rank = run[e] + __popcll(below), r = off[e] + rank, prow = few_tile(us, e) * FEW_BM + rank, t = i / p.K;
-            p.dst[i] = r;
-            p.dstp[i] = prow;
-            p.src_row[r] = t;
-            p.tokp[prow] = t;
-        }
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-        if (valid && below == 0) run[e] += __popcll(mine);
-    }
-}
-
 // Wave per row of the copy (a pair's row of xg, then the token rows of xs): what the dispatch launch does for larger batches,
 // beside the products instead of in front of them
 __device__ __forceinline__ void few_copy(const few_args &p, const few_shared &sh, const few_used &us, int wg, int lane, int wave, int waves)
@@ -198,7 +127,7 @@ __device__ __forceinline__ void few_copy(const few_args &p, const few_shared &sh
     const int KT = p.Kd >> 5, P = p.T * p.K, n = P + (p.xs != nullptr ? p.T : 0);
     for (int u = wg * waves + wave; u < n; u += waves * p.copy_wgs) {
         const int t = u < P ? u / p.K : u - P;
-        const int row = u >= P ? t : p.ids != nullptr ? few_tile(us, sh.id[u]) * FEW_BM + few_rank(sh, u, lane) : p.dstp[u];
+        const int row = u >= P ? t : p.index.ids != nullptr ? few_tile(us, sh.id[u]) * FEW_BM + few_rank(sh, u, lane) : p.dstp[u];
         const unsigned char *src = p.x + (size_t)t * p.Kd * 2;
         unsigned char *dst = u < P ? p.xg : p.xs;
         for (int c = lane; c < 4 * KT; c += 64) *(uint4 *)(dst + pk_chunk_off(row, c >> 2, c & 3, KT)) = *(const uint4 *)(src + (size_t)c * 16);
@@ -269,7 +198,7 @@ __global__ __launch_bounds__(64 * NW, 4) void few_rows_kernel(few_args p)
     const int l16 = lane & 15, lq = lane >> 4;
     constexpr int NC = UP ? NB / 2 : NB;  // 16-column blocks of the output per workgroup
     const int nc = p.N / (16 * NC);
-    const bool self = UP && p.ids != nullptr;
+    const bool self = UP && p.index.ids != nullptr;
     const int blk = blockIdx.x;
     int n_used = 0;
     few_used us = {};
@@ -278,8 +207,8 @@ __global__ __launch_bounds__(64 * NW, 4) void few_rows_kernel(few_args p)
 #pragma unroll
         for (int q = 0; q < 4; ++q) n_used += __popcll(us.m[q]);
         if (blk == (int)gridDim.x - 1) {
-            static_assert(sizeof(part) >= 2 * 256 * sizeof(int), "room for the index");
-            few_index(p, sh, us, (int *)part, (int *)part + 256, n_used, lane, wave, 64 * NW);
+            static_assert(sizeof(part) >= 3 * 256 * sizeof(int), "room for the index");
+            small_index(p.index, sh.id, (int *)part, FEW_BM, 64 * NW);
             return;
         }
     }
@@ -290,7 +219,7 @@ __global__ __launch_bounds__(64 * NW, 4) void few_rows_kernel(few_args p)
     }
     // the row tiles in falling order, which takes the shared experts - all T rows - first
     const int wt = blk / nc, n0 = (blk - wt * nc) * (16 * NC);
-    const int mt = (self ? n_used + p.Es : p.tile_meta[0]) - 1 - wt;
+    const int mt = (self ? n_used + p.index.Es : p.tile_meta[0]) - 1 - wt;
     if (mt < 0) return;
     omega_tile tl = self ? few_find(p, sh, us, mt, n_used, lane) : p.tiles[mt];
     tl = {__builtin_amdgcn_readfirstlane(tl.g), __builtin_amdgcn_readfirstlane(tl.row0), __builtin_amdgcn_readfirstlane(tl.rows),
@@ -394,22 +323,14 @@ hipError_t launch_experts_few(const omega_moe *m, const void *x, int T, int whic
         p.a = (unsigned char *)m->a;
         p.N = c.H;
         p.Kd = c.d;
-        if (index) {
-            p.ids = m->ids;
-            p.counts = m->counts;
-            p.offsets = m->offsets;
-            p.dst = m->dst;
-            p.src_row = m->src_row;
-            p.E = c.E;
-            p.Es = c.Es;
-        }
+        if (index) p.index = index_args_of(m, T);
         if (copy) {
             p.xg = (unsigned char *)m->xg;
             p.xs = (unsigned char *)m->xs;
             p.copy_wgs = std::min(ceil_div(T * (c.K + (c.Es > 0 ? 1 : 0)), 4), m->ctx->num_cus);
         }
 #define FEW_LAUNCH(UPV, UMV, NWV, NBV)                                                                                              \
-    hipLaunchKernelGGL((few_rows_kernel<UPV, UMV, NWV, NBV>), dim3(tiles * (p.N / (UPV ? 8 * NBV : 16 * NBV)) + (p.ids != nullptr ? 1 : 0) + p.copy_wgs), dim3(64 * NWV), 0, s, p)
+    hipLaunchKernelGGL((few_rows_kernel<UPV, UMV, NWV, NBV>), dim3(tiles * (p.N / (UPV ? 8 * NBV : 16 * NBV)) + (p.index.ids != nullptr ? 1 : 0) + p.copy_wgs), dim3(64 * NWV), 0, s, p)
         // Four blocks of weights per step from 17 tokens on (two units of rows: 64 tokens x 4096 x 14336, 8 experts, up product 326 ->
         // 294 us), two below (1 token 71 against 73, 1 token x 3328 x 896, 86 experts 12.0 against 15.9).  Two waves where four would
         // have 8 k steps each or fewer, which is all start-up (64 tokens x 1024 x 768, 128 experts: pass 133 -> 128.5; d = 1536 169

@@ -1,6 +1,6 @@
 // What the two kernels of the fp32 products (experts_f32.hip, experts_f32_split.hip) share: arguments, gathered copy.
 #pragma once
-#include "common.h"
+#include "index_small.h"
 #include <algorithm>
 #include <type_traits>
 
@@ -10,6 +10,7 @@ struct f32_args {
     const int32_t *tokp;     // F32_UP: routed rows come from Atok through this row -> token table (or null: from A0) ...
     float *xg;               // ... and the launch's last `copy_wgs` workgroups leave the gathered rows here
     const int32_t *dstp;     // pair -> row
+    index_args index;        // F32_UP, tiles of 32 rows: the launch makes the dispatch index itself (index.ids not null)
     int copy_wgs, K;
     const float *B0, *B1;    // weights (F32_UP, F32_RAW: W1 and W3; F32_DXG: second pair), F32_WG*: the layer input rows
     const float *Btok;       // F32_WG*: as Atok
@@ -25,14 +26,133 @@ struct f32_args {
 #define F32_IS_WG(OP) ((OP) == F32_WG2 || (OP) == F32_WG13)
 #define F32_PAIR(OP) ((OP) == F32_UP || (OP) == F32_RAW)
 
+// The choices of a batch of few pairs in every wave's registers, for an up product that makes its own index
+#define F32_SELF_CHUNKS 16  // 64 pairs each, at most
+#define F32_SELF_EXPERTS 16
+template <int NC>
+struct f32_choices {
+    int id[NC];                // choice of pair 64 c + lane, -1 behind the last (every loop over the chunks is straight: its branches cost more than its sums)
+    int first, tiles;          // first: lane e < E: the experts' first row tile; tiles: those of the routed experts
+    int count;                 // lane e < E: pairs of expert e
+    __device__ __forceinline__ void read(const f32_args &p, int lane)
+    {
+        const int P = p.T * p.K;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) id[c] = p.index.ids[min(64 * c + lane, P - 1)];
+#pragma unroll
+        for (int c = 0; c < NC; ++c) id[c] = 64 * c + lane < P ? id[c] : -1;
+        first = count = tiles = 0;
+        for (int e = 0; e < p.E; ++e) {
+            int n = 0;
+#pragma unroll
+            for (int c = 0; c < NC; ++c)
+                n += __popcll(__ballot(id[c] == e));
+            first = lane == e ? tiles : first;
+            count = lane == e ? n : count;
+            tiles += (n + F32_TILE_M_SMALL - 1) / F32_TILE_M_SMALL;
+        }
+    }
+    // row tile mt, and the tokens of its rows, to LDS; every wave by itself
+    __device__ __forceinline__ omega_tile find(const f32_args &p, int mt, int lane, uint16_t *tok) const
+    {
+        omega_tile tl;
+        tl.row0 = mt * F32_TILE_M_SMALL;
+        if (mt >= tiles) {
+            const int per = (p.T + F32_TILE_M_SMALL - 1) / F32_TILE_M_SMALL, s = (mt - tiles) / per;
+            tl.g = p.E + s;
+            tl.xrow0 = (mt - tiles - s * per) * F32_TILE_M_SMALL;
+            tl.rows = min(F32_TILE_M_SMALL, p.T - tl.xrow0);
+            return tl;
+        }
+        const int nt = (count + F32_TILE_M_SMALL - 1) / F32_TILE_M_SMALL;
+        tl.g = __ffsll(__ballot(lane < p.E && first <= mt && mt < first + nt)) - 1;
+        tl.xrow0 = -1;
+        const int r0 = (mt - __builtin_amdgcn_readlane(first, tl.g)) * F32_TILE_M_SMALL;
+        tl.rows = min(F32_TILE_M_SMALL, __builtin_amdgcn_readlane(count, tl.g) - r0);
+        int n = -r0;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            const unsigned long long m = __ballot(id[c] == tl.g);
+            const int rank = n + __popcll(m & ((1ull << lane) - 1ull));
+            if (id[c] == tl.g && rank >= 0 && rank < F32_TILE_M_SMALL) tok[rank] = (uint16_t)((64 * c + lane) / p.K);
+            n += __popcll(m);
+        }
+        return tl;
+    }
+    // The index, by the four waves of a workgroup, every fourth chunk of pairs each: what small_index leaves, from registers (its LDS
+    // atomics and one wave's chain of ranks would outlast the products of such a batch)
+    __device__ __forceinline__ void leave(const index_args &p, int lane, int wave) const
+    {
+        const int per = (p.T + F32_TILE_M_SMALL - 1) / F32_TILE_M_SMALL;
+        int r[NC] = {}, row[NC] = {}, off = 0, at = 0;
+        for (int e = 0; e < p.E; ++e) {
+            const int row0 = __builtin_amdgcn_readlane(first, e) * F32_TILE_M_SMALL;
+            int n = 0;
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                const unsigned long long m = __ballot(id[c] == e);
+                const int rank = n + __popcll(m & ((1ull << lane) - 1ull));
+                r[c] = id[c] == e ? off + rank : r[c];
+                row[c] = id[c] == e ? row0 + rank : row[c];
+                n += __popcll(m);
+            }
+            at = lane == e ? off : at;
+            off += n;
+        }
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            if ((c & 3) != wave || id[c] < 0) continue;
+            const int i = 64 * c + lane, t = i / p.K;
+            p.dst[i] = r[c];
+            p.dstp[i] = row[c];
+            p.src_row[r[c]] = t;
+            p.tokp[row[c]] = t;
+        }
+        if (wave > 0) return;
+        if (lane < p.E) {
+            p.counts[lane] = count;
+            p.offsets[lane] = at;
+            p.tile_meta[1 + lane] = first;
+            for (int q = 0; q < count; q += F32_TILE_M_SMALL)
+                p.tiles[first + q / F32_TILE_M_SMALL] = {lane, first * F32_TILE_M_SMALL + q, min(F32_TILE_M_SMALL, count - q), -1};
+        }
+        for (int s = lane; s <= p.Es; s += 64) p.tile_meta[1 + p.E + s] = tiles + s * per;
+        for (int q = lane; q < p.Es * per; q += 64) {
+            const int s = q / per, x = (q - s * per) * F32_TILE_M_SMALL;
+            p.tiles[tiles + q] = {p.E + s, (tiles + q) * F32_TILE_M_SMALL, min(F32_TILE_M_SMALL, p.T - x), x};
+        }
+        if (lane == 0) {
+            p.offsets[p.E] = off;
+            p.tile_meta[0] = tiles + p.Es * per;
+        }
+    }
+    // row of pair u (uniform over the wave)
+    __device__ __forceinline__ int row(const f32_args &p, int u, int lane) const
+    {
+        const int e = p.index.ids[u];
+        int n = 0;
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+            n += __popcll(__ballot(id[c] == e && 64 * c + lane < u));
+        return __builtin_amdgcn_readlane(first, e) * F32_TILE_M_SMALL + n;
+    }
+};
+
 // Gathered rows of a launch whose product workgroups fetch theirs from the tokens (a wave per token, the row read once and
 // written to its K places): the backward pass reads them.  Beside the products instead of a launch in front of them.
-template <bool VEC>
-__device__ __forceinline__ void copy_gathered(const f32_args &p, int wg, int lane, int wave)
+// OWN: the places are found from the choices
+template <bool VEC, bool OWN, class Choices>
+__device__ __forceinline__ void copy_gathered(const f32_args &p, int wg, int lane, int wave, const Choices &own)
 {
     const int d = p.Kd;
     for (int t = 4 * wg + wave; t < p.T; t += 4 * p.copy_wgs) {
-        const int row = lane < p.K ? p.dstp[(size_t)t * p.K + lane] : 0;
+        int row = 0;
+        if constexpr (OWN) {
+            for (int j = 0; j < p.K; ++j) {
+                const int r = own.row(p, t * p.K + j, lane);
+                row = lane == j ? r : row;
+            }
+        } else if (lane < p.K) row = p.dstp[(size_t)t * p.K + lane];
         const float *src = p.Atok + (size_t)t * d;
         for (int c0 = 0; c0 < d; c0 += VEC ? 256 : 64) {  // (every lane makes every trip: the cross-lane reads need them all)
             const int c = c0 + (VEC ? 4 : 1) * lane;
@@ -115,11 +235,11 @@ __device__ __forceinline__ float4 frag(const float *S, int x, int k)
     return make_float4(S[k * (TX + 4) + x], S[(k + 1) * (TX + 4) + x], S[(k + 2) * (TX + 4) + x], S[(k + 3) * (TX + 4) + x]);
 }
 
-// One tile: row tile mt from its row r0 on (row products) or from row mt * TM of gradient matrix mat, and columns n0 ..; as and bs
+// One tile: row tile mt (tl) from its row r0 on (row products) or from row mt * TM of gradient matrix mat, and columns n0 ..; as and bs
 // hold both operands of a row product twice.  (Weight gradients keep arrays of their own: read through pointers dW1 and dW3 of 4096
 // tokens x 1024 x 3584, 8 experts, took 936 us instead of 915.  For the same reason p is a copy.)
 template <int OP, int TM, int TN, bool VEC>
-__device__ __forceinline__ void f32_tile(const f32_args p, float *as, float *bs, int mt, int r0, int n0, int mat)
+__device__ __forceinline__ void f32_tile(const f32_args p, float *as, float *bs, int mt, const omega_tile tl, int r0, int n0, int mat, const uint16_t *tok = nullptr)
 {
     constexpr bool WG = F32_IS_WG(OP), PAIR = F32_PAIR(OP);
     constexpr bool AK = WG, BK_ = WG || OP == F32_DA || OP == F32_DXG;  // operand contiguous across k
@@ -147,14 +267,13 @@ __device__ __forceinline__ void f32_tile(const f32_args p, float *as, float *bs,
         A0 = shared && p.Atok ? p.Atok : Ad + (size_t)row0 * p.Kd;
         B0 = shared && p.Btok ? p.Btok : p.B0 + (size_t)row0 * p.N;
     } else {
-        const omega_tile tl = p.tiles[mt];
         g = tl.g;
         rows = min(TM, tl.rows - r0);
         if (rows <= 0 || n0 >= p.N) return;  // (a part of a ragged tile)
         row0 = tl.row0 + r0;
         K1 = p.Kd;
         A0 = p.Atok && tl.xrow0 >= 0 ? p.Atok + (size_t)(tl.xrow0 + r0) * p.Kd : p.A0 + (size_t)row0 * p.Kd;
-        fetch_rows = OP == F32_UP && p.tokp != nullptr && tl.xrow0 < 0;
+        fetch_rows = OP == F32_UP && p.tokp != nullptr && tl.xrow0 < 0;  // (up: through tokp, or tok)
         if (fetch_rows) A0 = p.Atok;
         if (OP == F32_DXG) A1 = p.A1 + (size_t)row0 * p.Kd;
         B0 = p.B0 + (size_t)g * p.N * p.Kd;
@@ -167,7 +286,7 @@ __device__ __forceinline__ void f32_tile(const f32_args p, float *as, float *bs,
 #pragma unroll
     for (int u = 0; u < NVA; ++u) {
         const int x = f32_piece<TM, AK, FBK>::x(tid, u), k = f32_piece<TM, AK, FBK>::k(tid, u);
-        oa[u] = 4u * (AK ? (uint32_t)k * p.Kd + min(x, p.Kd - m0 - (VEC ? 4 : 1)) : (uint32_t)(fetch_rows ? p.tokp[row0 + min(x, rows - 1)] : min(x, rows - 1)) * K1 + k);
+        oa[u] = 4u * (AK ? (uint32_t)k * p.Kd + min(x, p.Kd - m0 - (VEC ? 4 : 1)) : (uint32_t)(!fetch_rows ? min(x, rows - 1) : tok != nullptr ? (int)tok[min(x, rows - 1)] : p.tokp[row0 + min(x, rows - 1)]) * K1 + k);
     }
 #pragma unroll
     for (int u = 0; u < NVB; ++u) {
