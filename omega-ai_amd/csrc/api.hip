@@ -666,6 +666,7 @@ static int ensure_queues(omega_moe *m, int T)
 {
     if (m->queued) return OMEGA_OK;
     m->queued = true;
+    m->index_in_up = false;
     const hipError_t e = launch_dispatch_index(m, T, m->bm, m->ctx->stream, nullptr);
     m->queued = e == hipSuccess;  // (the next to ask tries again: the queues are still an earlier batch's)
     OMEGA_HIP_CHECK(m->ctx, e);
@@ -726,8 +727,8 @@ static int stage_dispatch(omega_moe *m, const void *x, int T, bool up_follows = 
     m->queued = !m->few;
     const bool up_gathers = up_follows && (m->few || (!bf && (double)T * m->cfg.d * 4.0 < 4.0e9));
     // (a few tokens, or pairs of an fp32 layer: their up product makes the index itself)
-    m->index_in_up = up_gathers && (bf ? experts_few_index(m, T) : product_f32_index(m, T));
-    if (!m->index_in_up) OMEGA_HIP_CHECK(m->ctx, launch_dispatch_index(m, T, bm, m->ctx->stream, bf && !m->gather_on_load && !up_gathers ? x : nullptr));
+    m->index_in_up = up_gathers && makes_index_in_up(m, T);
+    OMEGA_HIP_CHECK(m->ctx, launch_dispatch_index(m, T, bm, m->ctx->stream, bf && !m->gather_on_load && !up_gathers ? x : nullptr));
     if (!bf && !up_gathers) OMEGA_HIP_CHECK(m->ctx, launch_dispatch_gather(m, x, T, m->ctx->stream));
     m->xg_valid = !m->gather_on_load && !up_gathers;
     m->dispatched_T = T;
@@ -750,21 +751,21 @@ static int stage_experts(omega_moe *m, const void *x, int T, int which)
     if (which == 0 && m->gather_on_load && !x) OMEGA_FAIL(m->ctx, OMEGA_ERR_INVALID_ARG, "experts: x is NULL");
     if (which == 1 && !m->a_valid) OMEGA_FAIL(m->ctx, OMEGA_ERR_INVALID_ARG, "experts_down: the up product has not run since `a` was overwritten");
     const bool keep = which == 0 && keeps_for_backward(m, T), index = which == 0 && m->index_in_up;
-    if (index) {
-        m->index_in_up = false;
-        m->dispatched_T = -1;  // (until the launch that makes it is under way)
-    }
+    if (index) m->dispatched_T = -1;  // (until the launch that makes it is under way)
     if (m->cfg.dtype == OMEGA_DTYPE_BF16) {
         if (which == 0 && m->few && !m->xg_valid && !x) OMEGA_FAIL(m->ctx, OMEGA_ERR_INVALID_ARG, "experts: x is NULL");
-        OMEGA_HIP_CHECK(m->ctx, launch_experts_bf16(m, x, T, which, m->ctx->stream, keep, index));
+        OMEGA_HIP_CHECK(m->ctx, launch_experts_bf16(m, x, T, which, m->ctx->stream, keep));
         if (which == 0 && m->few && !m->gather_on_load) m->xg_valid = true;
     } else if (which == 0) {
         const bool gather = !m->xg_valid;
         if (gather && !x) OMEGA_FAIL(m->ctx, OMEGA_ERR_INVALID_ARG, "experts: x is NULL");
-        OMEGA_HIP_CHECK(m->ctx, launch_product_f32(m, F32_UP, (const float *)x, nullptr, T, m->ctx->stream, gather, keep, index));
+        OMEGA_HIP_CHECK(m->ctx, launch_product_f32(m, F32_UP, (const float *)x, nullptr, T, m->ctx->stream, gather, keep));
         m->xg_valid = true;
     } else OMEGA_HIP_CHECK(m->ctx, launch_product_f32(m, F32_DOWN, nullptr, nullptr, T, m->ctx->stream));
-    if (index) m->dispatched_T = T;
+    if (index) {
+        m->index_in_up = false;
+        m->dispatched_T = T;
+    }
     if (which == 0) {
         m->a_valid = true;
         return OMEGA_OK;
@@ -1377,6 +1378,7 @@ int omega_moe_time_stage(omega_moe *m, int stage, const void *x, int T, void *ou
             case 7:
                 // parts of a dispatch that has already run for this T (same buffers, same result)
                 if (m->dispatched_T != T) OMEGA_FAIL(ctx, OMEGA_ERR_INVALID_ARG, "time_stage: dispatch has not run for this T");
+                m->index_in_up = false;
                 if (stage == 6) OMEGA_HIP_CHECK(ctx, launch_dispatch_index(m, T, m->bm, ctx->stream));
                 else OMEGA_HIP_CHECK(ctx, launch_dispatch_gather(m, x, T, ctx->stream));
                 return OMEGA_OK;

@@ -102,7 +102,8 @@ struct omega_moe {
     // the batch is one of a few tokens outside training: its products run on experts_few.hip and its dispatch made no work queues
     // (what needs them has them made first: ensure_queues)
     bool few = false, queued = true;
-    bool index_in_up = false;        // ... and its up product, not launched yet, makes the dispatch index
+    // the up product that is launched next makes the dispatch index of its batch: launch_dispatch_index leaves it to it
+    bool index_in_up = false;
     // the down product of the batch in y has left k slices in y_slabs that are not in y: the combine kernel adds them on its
     // way (combine.hip), whatever else reads y has them added first (ensure_y_whole)
     bool y_partial = false;
@@ -186,6 +187,16 @@ static inline bool combine_by_vectors(const omega_moe *m, const void *out, const
 // pass, us, tile kernels / there: 485 / 485, 514 / 560; 80 / 192 tokens x 2048 x 1408, 64 experts: 241 / 231, 253 / 257.
 static inline bool experts_few_rows(const omega_moe *m, int T) { return m->cfg.dtype == OMEGA_DTYPE_BF16 && T <= 64; }
 
+// Forward passes whose up product makes the dispatch index itself (omega_moe::index_in_up): bf16 batches of a few tokens, fp32 ones in tiles of 32 rows,
+// with no more pairs (and experts) than their workgroups hold
+#define INDEX_IN_UP_PAIRS 1024
+#define INDEX_IN_UP_EXPERTS_F32 16
+static inline bool makes_index_in_up(const omega_moe *m, int T)
+{
+    const bool fits = m->cfg.dtype == OMEGA_DTYPE_BF16 ? m->few : m->bm == 32 && m->cfg.E <= INDEX_IN_UP_EXPERTS_F32;
+    return fits && (long long)T * m->cfg.K <= INDEX_IN_UP_PAIRS;
+}
+
 // Tokens per router workgroup = per row of tile_counts and per workgroup of the dispatch kernel: 16 for layers with at most
 // 16 experts and for exact bf16 layers with more while such tiles find a compute unit each, else 32 (router.hip).
 int router_tok_tile(const omega_moe *m, int T);
@@ -224,13 +235,10 @@ enum { F32_UP = 0, F32_DOWN, F32_RAW, F32_DA, F32_DXG, F32_WG2, F32_WG13 };
 // (gather: F32_UP fetches the routed rows from x and leaves the gathered copy beside it; keep: it leaves h1 and h3 in
 // bw_h1 / bw_h3, as launch_experts_bf16 does)
 hipError_t launch_product_f32(const omega_moe *m, int op, const float *x, const float *dout, int T, hipStream_t s, bool gather = false,
-                              bool keep = false, bool index = false);
-bool product_f32_index(const omega_moe *m, int T);  // whether F32_UP, with `gather`, can make the dispatch index as well (`index`)
+                              bool keep = false);
 // which: 0 up product, 1 down product
-hipError_t launch_experts_bf16(const omega_moe *m, const void *x, int T, int which, hipStream_t s, bool keep, bool index);
-// index: the up launch makes the dispatch index as well (experts_few_index says whether it can)
-hipError_t launch_experts_few(const omega_moe *m, const void *x, int T, int which, hipStream_t s, bool index);
-bool experts_few_index(const omega_moe *m, int T);
+hipError_t launch_experts_bf16(const omega_moe *m, const void *x, int T, int which, hipStream_t s, bool keep);
+hipError_t launch_experts_few(const omega_moe *m, const void *x, int T, int which, hipStream_t s);
 // resid != nullptr: out = resid + layer output (one rounding of the fp32 sum)
 hipError_t launch_combine(const omega_moe *m, int T, void *out, const void *resid, hipStream_t s);
 hipError_t launch_backward_f32(omega_moe *m, const void *x, const void *dout, int T, void *dx, hipStream_t s);

@@ -1159,10 +1159,10 @@ hipError_t experts_bf16_init(void)
     return hipSuccess;
 }
 
-hipError_t launch_experts_bf16(const omega_moe *m, const void *x, int T, int which, hipStream_t s, bool keep, bool index)
+hipError_t launch_experts_bf16(const omega_moe *m, const void *x, int T, int which, hipStream_t s, bool keep)
 {
     const omega_moe_config &c = m->cfg;
-    if (m->few) return launch_experts_few(m, x, T, which, s, index);
+    if (m->few) return launch_experts_few(m, x, T, which, s);
     // the ring must be shorter than an item: K >= (NSTAGE + 1) * BK (guaranteed at creation: d, H >= 256)
     if ((which == 0 ? c.d : c.H) < (NSTAGE + 1) * BK) return hipErrorInvalidValue;
     // A batch with at most 64 rows per routed expert on average streams every weight tile once (one row tile per

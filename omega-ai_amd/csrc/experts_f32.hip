@@ -184,13 +184,7 @@ static hipError_t f32_launch(f32_args p, bool vec, int max_tiles, hipStream_t s)
     return hipGetLastError();
 }
 
-// Up launches that make the index themselves: tiles of 32 rows, what f32_choices holds
-bool product_f32_index(const omega_moe *m, int T)
-{
-    return m->bm == F32_TILE_M_SMALL && m->cfg.E <= F32_SELF_EXPERTS && (long long)T * m->cfg.K <= 64 * F32_SELF_CHUNKS;
-}
-
-hipError_t launch_product_f32(const omega_moe *m, int op, const float *x, const float *dout, int T, hipStream_t s, bool gather, bool keep, bool index)
+hipError_t launch_product_f32(const omega_moe *m, int op, const float *x, const float *dout, int T, hipStream_t s, bool gather, bool keep)
 {
     const omega_moe_config &c = m->cfg;
     f32_args p = {};
@@ -215,7 +209,7 @@ hipError_t launch_product_f32(const omega_moe *m, int op, const float *x, const 
                 // turn behind the last product; 4096 tokens x 64 x 64, 64 experts, top 6, forward pass: 48.0 -> 46.4 us)
                 p.copy_wgs = std::min(ceil_div(T, 4), 4 * m->ctx->num_cus);
             }
-            if (index) p.index = index_args_of(m, T);
+            if (op == F32_UP && gather && m->index_in_up) p.index = index_args_of(m, T);
             if (op == F32_RAW || keep) { p.H1 = m->bw_h1; p.H3 = m->bw_h3; }
             break;
         case F32_DOWN:

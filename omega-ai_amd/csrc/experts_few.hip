@@ -45,11 +45,10 @@ struct few_args {
 // workgroups keep their XCDs, four that share the lines of a row group on XCDs 0-3 or 4-7 (moved on by one, two or three, 64 tokens x 4096 x 14336, 8
 // experts, up product 278 -> 307, 327, 307 us).  Forward pass, us, with a launch for the index / without: 1 and 64 tokens x 4096 x 14336, 8 experts,
 // top 2 132.1 -> 127.2, 454.5 -> 449; 48 tokens x 2048 x 1408, 64 experts, top 6, 2 shared 202 -> 195.6
-#define FEW_PAIRS_MAX 1024
 #define FEW_BM 256         // rows of a tile: every expert that is used has one
 struct few_shared {
     uint8_t flag[256];      // experts that have rows
-    uint8_t id[FEW_PAIRS_MAX];
+    uint8_t id[INDEX_IN_UP_PAIRS];
     uint8_t tok[64];        // tokens of the workgroup's rows
 };
 struct few_used { unsigned long long m[4]; };  // the flags as bits, uniform
@@ -299,10 +298,8 @@ __global__ __launch_bounds__(64 * NW, 4) void few_rows_kernel(few_args p)
     else run(std::integral_constant<int, UM>());
 }
 
-bool experts_few_index(const omega_moe *m, int T) { return T * m->cfg.K <= FEW_PAIRS_MAX; }
-
 // which: 0 up - the rows come from x unless there is a gathered copy, and one is left beside if the layer keeps one -, 1 down
-hipError_t launch_experts_few(const omega_moe *m, const void *x, int T, int which, hipStream_t s, bool index)
+hipError_t launch_experts_few(const omega_moe *m, const void *x, int T, int which, hipStream_t s)
 {
     const omega_moe_config &c = m->cfg;
     const bool gather = !m->xg_valid, copy = gather && !m->gather_on_load;
@@ -323,7 +320,7 @@ hipError_t launch_experts_few(const omega_moe *m, const void *x, int T, int whic
         p.a = (unsigned char *)m->a;
         p.N = c.H;
         p.Kd = c.d;
-        if (index) p.index = index_args_of(m, T);
+        if (m->index_in_up) p.index = index_args_of(m, T);
         if (copy) {
             p.xg = (unsigned char *)m->xg;
             p.xs = (unsigned char *)m->xs;

@@ -27,8 +27,7 @@ struct f32_args {
 #define F32_PAIR(OP) ((OP) == F32_UP || (OP) == F32_RAW)
 
 // The choices of a batch of few pairs in every wave's registers, for an up product that makes its own index
-#define F32_SELF_CHUNKS 16  // 64 pairs each, at most
-#define F32_SELF_EXPERTS 16
+#define F32_SELF_CHUNKS (INDEX_IN_UP_PAIRS / 64)
 template <int NC>
 struct f32_choices {
     int id[NC];                // choice of pair 64 c + lane, -1 behind the last (every loop over the chunks is straight: its branches cost more than its sums)
