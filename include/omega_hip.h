@@ -294,6 +294,9 @@ int omega_moe_time_backward(omega_moe *moe, const void *x_dev, const void *dout_
  * cudaDeviceSynchronize + System.nanoTime prints of J/engine/nn/network/Llama3.java:140-156. */
 int omega_moe_set_profiling(omega_moe *moe, int on);
 int omega_moe_get_profile(omega_moe *moe, float stage_ms_sum[5], int *n_calls);
+/* Tiles that the products of an fp32 layer take for a batch of T tokens: tiles[0] = rows of a row tile (32, 64 or 128), tiles[1] and
+ * tiles[2] = edge of a tile of dW2 and of dW1 | dW3 (64 or 128).  For tests, which have to know which kernel they check. */
+int omega_moe_get_f32_tiles(omega_moe *moe, int T, int32_t tiles[3]);
 
 #ifdef __cplusplus
 }

@@ -76,6 +76,7 @@ SIGNATURES = {
                                        C.POINTER(C.c_float)]),
     "omega_moe_set_profiling": (C.c_int, [C.c_void_p, C.c_int]),
     "omega_moe_get_profile": (C.c_int, [C.c_void_p, C.POINTER(C.c_float), C.POINTER(C.c_int)]),
+    "omega_moe_get_f32_tiles": (C.c_int, [C.c_void_p, C.c_int, C.POINTER(C.c_int32)]),
 }
 
 _lib = None

@@ -1165,6 +1165,16 @@ int omega_moe_get_profile(omega_moe *m, float *stage_ms_sum, int *n_calls)
     return OMEGA_OK;
 }
 
+int omega_moe_get_f32_tiles(omega_moe *m, int T, int32_t *tiles)
+{
+    MOE_ENTER(m);
+    if (!tiles || T <= 0 || m->cfg.dtype != OMEGA_DTYPE_F32) OMEGA_FAIL(ctx, OMEGA_ERR_INVALID_ARG, "get_f32_tiles: NULL argument, T <= 0 or no fp32 layer");
+    tiles[0] = moe_tile_m(m, T);
+    tiles[1] = f32_wgrad_wide(m, T, m->G) ? 128 : 64;
+    tiles[2] = f32_wgrad_wide(m, T, 2 * m->G) ? 128 : 64;
+    return OMEGA_OK;
+}
+
 int omega_moe_router(omega_moe *m, const void *x, int T)
 {
     MOE_ENTER(m);

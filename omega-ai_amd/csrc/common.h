@@ -209,6 +209,15 @@ __host__ __device__ static inline int ceil_div(int a, int b) { return (a + b - 1
 
 int omega_set_error(omega_ctx *ctx, int status, const char *what, hipError_t herr, const char *file, int line);
 
+// Weight gradients of fp32 layers (`mats` matrices), whose tiles do not depend on the row tiles: on the bf16 matrix cores (experts_f32_split.hip), in tiles of
+// 128 x 128, from 128 rows per expert on, once there are five for four compute units.  Training step, us, 64 x 64 of experts_f32.hip / there: 2272 tokens x
+// 339 x 2671, 4 experts, top 2 1213 / 988, 3300 x 780 x 2924, 6 experts, top 4 4945 / 4150, 2373 x 840 x 1100, 12 experts 1684 / 1580; with 0.8 tiles per
+// compute unit 447 / 473 and 1151 / 1221, with 70 to 90 rows per expert 516 / 533, 663 / 607, 643 / 645.
+static inline bool f32_wgrad_wide(const omega_moe *m, int T, int mats)
+{
+    return (long long)T * m->cfg.K >= 128LL * m->cfg.E && 4LL * ceil_div(m->cfg.d, 128) * ceil_div(m->cfg.H, 128) * mats >= 5LL * m->ctx->num_cus;
+}
+
 #define OMEGA_FAIL(ctx, status, what) return omega_set_error((ctx), (status), (what), hipSuccess, __FILE__, __LINE__)
 #define OMEGA_HIP_CHECK(ctx, expr)                                                             \
     do {                                                                                       \

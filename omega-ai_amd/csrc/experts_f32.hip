@@ -235,17 +235,11 @@ hipError_t launch_product_f32(const omega_moe *m, int op, const float *x, const 
     // of 4096 tokens, 8 experts, top 2, us, both widths asked of every product and now: d = 1024, H = 2731 1238 -> 1214; d = 512, H = 1001 305 -> 299.)
     const bool d4 = c.d % 4 == 0, H4 = c.H % 4 == 0;
     const bool vec = (op == F32_DOWN || d4) && (op == F32_UP || op == F32_RAW || H4) && (((uintptr_t)p.Atok | (uintptr_t)p.Btok) % 16) == 0;
-    // Weight gradients, whose tiles do not depend on the row tiles: split (experts_f32_split.hip), in tiles of 128 x 128, from 128 rows per
-    // expert on, once there are five for four compute units.  Training step, us, 64 x 64 here / there: 2272 tokens x 339 x 2671, 4 experts, top 2
-    // 1213 / 988, 3300 x 780 x 2924, 6 experts, top 4 4945 / 4150, 2373 x 840 x 1100, 12 experts 1684 / 1580; with 0.8 tiles per compute unit 447 / 473 and
-    // 1151 / 1221, with 70 to 90 rows per expert 516 / 533, 663 / 607, 643 / 645.
-    const long long rows = (long long)T * c.K;
-    auto wide = [&](int mats) { return rows >= 128LL * c.E && 4LL * ceil_div(c.d, 128) * ceil_div(c.H, 128) * mats >= 5LL * m->ctx->num_cus; };
     // Row products: tiles of 128 rows are split ones, those of 64 where they read H columns of weights (the others have fewer columns
     // and a longer k).  Up product of 64 rows, split / fp32 MFMAs in 64 x 128: from one tile per compute unit on 0.60 - 0.97, below, where most
     // launches go in parts of 32 x 32, 1.03 - 1.14.
     const bool mid = m->bm == F32_TILE_M_MID && op != F32_DOWN && op != F32_DXG;
-    if (op == F32_WG2 || op == F32_WG13 ? wide(op == F32_WG13 ? 2 * m->G : m->G) : m->bm == F32_TILE_M || mid)
+    if (op == F32_WG2 || op == F32_WG13 ? f32_wgrad_wide(m, T, op == F32_WG13 ? 2 * m->G : m->G) : m->bm == F32_TILE_M || mid)
         return launch_product_f32_split(p, op, vec, m->max_m_tiles, s);
 #define F32_ROWS(OP)                                                                           \
     (m->bm == F32_TILE_M_MID ? f32_launch<OP, F32_TILE_M_MID, 64>(p, vec, m->max_m_tiles, s) \

@@ -360,6 +360,12 @@ class MoELayer:
         names = ("router", "dispatch", "experts_up", "experts_down", "combine")
         return {k: ms[i] / max(n.value, 1) for i, k in enumerate(names)}, n.value
 
+    def f32_tiles(self, T):
+        """(rows of a row tile, edge of a tile of dW2, of dW1 | dW3) of an fp32 layer's products for T tokens."""
+        t = (C.c_int32 * 3)()
+        self.ctx.check(self.lib.omega_moe_get_f32_tiles(self.handle, int(T), t))
+        return tuple(t)
+
     def routing(self, T=None):
         T = self.number if T is None else T
         K, E = self.topK, self.nExperts
