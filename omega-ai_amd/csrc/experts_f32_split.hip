@@ -81,6 +81,22 @@ __device__ __forceinline__ void sp_fetch_partial(float (&v)[sp_unit<KMAJ>], cons
     }
 }
 
+// places k .. k + 3 of a row or column (ld: distance of two places of a column), zero from K1 on
+template <bool KMAJ, bool VEC>
+__device__ __forceinline__ void sp_four(float (&v)[4], const float *x, int k, int K1, int ld)
+{
+    if constexpr (!KMAJ && VEC) {  // (K1 % 4 == 0)
+        const float4 q = *(const float4 *)(x + min(k, K1 - 4));
+        v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = x[(size_t)min(k + i, K1 - 1) * (KMAJ ? ld : 1)];
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        if (k + i >= K1) v[i] = 0.0f;
+}
+
 // Chunk swizzle of the planes (rows of 64 bytes).  LDS serves a ds_read_b128 in four passes of 16 lanes - 0-3, 12-15 and 20-27; 4-11, 16-19 and
 // 28-31; the same of the upper half - over 64 banks: a fragment's pass takes rows 0-3 and 12-15 of one chunk and 4-11 of its neighbour, and rows r,
 // r + 12 (chunk c), r + 4 and r + 8 (c ^ 1), which share four places, are kept apart by 0, 3, 2, 1 (4.7 cycles a read; 8 with pk_swz)
@@ -336,6 +352,15 @@ __global__ __launch_bounds__(256, SP_WAVES(NB)) void f32_split_kernel(f32_args p
             for (int n = 0; n < NB; ++n) acc[i][n] = sp_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
         for (int seg = 0; seg < (OP == F32_DXG ? 2 : 1); ++seg) {
             const float *A = seg ? A1 : A0, *B = OP == F32_DXG && seg ? B1 : B0;
+            if (seg) {  // (the second pair's own sum, as in f32_tile)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int n = 0; n < NB; ++n) {
+                        low[i][n] = acc[i][n];
+                        acc[i][n] = sp_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                    }
+            }
             size_t xa[4], xo[NB];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
@@ -347,23 +372,25 @@ __global__ __launch_bounds__(256, SP_WAVES(NB)) void f32_split_kernel(f32_args p
                 const int x = min(PAIR && n >= NB / 2 ? xb[n] - CT : xb[n], p.N - 1 - n0);
                 xo[n] = BKM ? (size_t)x : (size_t)x * K1;
             }
-            for (int k0 = 0; k0 < K1; k0 += 4) {
-                const int k = min(k0 + lq, K1 - 1);
-                const bool in = k0 + lq < K1;
-                float b[NB];
+            for (int k0 = 0; k0 < K1; k0 += 16) {  // (lane quarter q: places 4 q .. 4 q + 3 of 16)
+                const int k = k0 + 4 * lq;
+                float a[4][4], b[NB][4];
 #pragma unroll
-                for (int n = 0; n < NB; ++n) {
-                    const float *q = PAIR && n >= NB / 2 ? B1 : B;
-                    b[n] = BKM ? q[(size_t)k * p.N + xo[n]] : q[xo[n] + k];
-                    if (!in) b[n] = 0.0f;
-                }
+                for (int n = 0; n < NB; ++n) sp_four<BKM, VEC>(b[n], (PAIR && n >= NB / 2 ? B1 : B) + xo[n], k, K1, p.N);
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    float a = AK ? A[(size_t)k * p.Kd + xa[i]] : A[xa[i] + k];
-                    if (!in) a = 0.0f;
+                for (int i = 0; i < 4; ++i) sp_four<AK, VEC>(a[i], A + xa[i], k, K1, p.Kd);
 #pragma unroll
-                    for (int n = 0; n < NB; ++n) acc[i][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b[n], acc[i][n], 0, 0, 0);
-                }
+                for (int u = 0; u < 4; ++u)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+#pragma unroll
+                        for (int n = 0; n < NB; ++n) acc[i][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i][u], b[n][u], acc[i][n], 0, 0, 0);
+            }
+            if (seg) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int n = 0; n < NB; ++n) acc[i][n] += low[i][n];
             }
         }
     }

@@ -65,3 +65,29 @@ def test_gradients_of_tiny_deltas(kw):
     for a, b in zip(*got):
         assert N.rel_l2(b.astype(np.float64) / float(s), a) < 1e-5
     layer.close()
+
+
+def test_tiles_computed_again_add_two_sums():
+    """Weights that make a few columns of the input gradient smaller than what three bf16 parts carry: the columns beside them, computed again, are
+    still the sum of two sums (test_input_gradient_adds_two_sums has the bound), and the few are as close."""
+    T, d, H = 8192, 1024, 3584
+    G, cfg, inp, dout, layer = _setup("c1_tiny_f32", dict(T=T, d=d, H=H, E=1, K=1), 94)
+    layer.close()
+    few = np.arange(5, d, 64)
+    for w in ("W1", "W3"):
+        inp[w][0][:, few] *= np.float32(2.0 ** -100)
+    layer = G.build_layer(cfg, inp)
+    assert layer.f32_tiles(T)[0] == 128
+    layer.forward(G.P.DeviceBuffer.from_numpy(G.ctx(), inp["x"], cfg.dtype))
+    dx = layer.back(G.P.DeviceBuffer.from_numpy(G.ctx(), dout, cfg.dtype)).to_numpy()
+    rows = np.linspace(0, T - 1, 64).astype(int)
+    x, g, W1, W3, W2 = (a.astype(np.float64) for a in (inp["x"][rows], dout[rows], inp["W1"][0], inp["W3"][0], inp["W2"][0]))
+    h1, h3, da = x @ W1.T, x @ W3.T, g @ W2
+    s = 1.0 / (1.0 + np.exp(-h1))
+    dh1, dh3 = da * h3 * s * (1.0 + h1 * (1.0 - s)), da * h1 * s
+    exact = dh1 @ W1 + dh3 @ W3
+    two = _chain(dh1.astype(np.float32), inp["W1"][0]) + _chain(dh3.astype(np.float32), inp["W3"][0])
+    dx = dx[rows].astype(np.float64)
+    for cols in (few, np.setdiff1d(np.arange(d), few)):
+        assert N.rel_l2(dx[:, cols], exact[:, cols]) < 1.2 * N.rel_l2(two[:, cols].astype(np.float64), exact[:, cols])
+    layer.close()
