@@ -7,7 +7,13 @@
 // sum of its own, the five small ones another, and the two are added once: a sum of K terms is rounded K / 32 times where a chain of
 // fp32 fused multiply-adds is rounded K times.  Error against float64, 2-norm, chain -> here: normal factors, K = 32 1.0e-7 -> 3.9e-8, 256 2.9e-7 ->
 // 9.1e-8, 1024 5.7e-7 -> 1.9e-7, 3584 1.06e-6 -> 3.7e-7; positive ones, 3584 9.1e-7 -> 3.3e-7 (with one sum for all six parts 9.2e-7 and 5.7e-7).
-// A wave whose sums are infinite, no numbers or below 2^-80 - parts may have been lost - computes its part of the tile again on fp32 MFMAs.
+// A wave whose sums are infinite, no numbers or below 2^-100 - partial products round to multiples of 2^-149, as denormal factors and results do on
+// these matrix cores, and 2^20 of them are then below 2^-27 of the sum - computes its part of the tile again on fp32 MFMAs.  A factor below 2^-110
+// other than zero, whose last part would need bits below those of a bf16 denormal, loses up to 2^-134 of itself: where there is one, a tile's sums are held to
+// 2^-106 of the largest factor times the number of terms, so that what is lost is below 2^-26 of them.
+// The look at every factor costs 2.7 - 3.5 % of these launches (one v_min3_f32 per two of them, and a branch for the zeros).  Where there is a tiny one the
+// largest is found by fetching all of them once more (input gradient below 700 -> 950 us), and a launch all of whose waves compute again takes 2.7 times as
+// long (dW1 and dW3 below 675 -> 1810: a unit in 64 that is saturated, h1 = -64, for every token).
 //
 // Bound: bf16 MFMA at a sixth of its rate, 417 TFLOP/s nominal, 240 under the power cap where fp32 MFMA has 154.  One workgroup = four waves of 64 rows
 // x 64 columns (64 x 128 tiles: 64 x 32), two (three) workgroups per compute unit, one writing its parts to LDS while the other multiplies:
@@ -15,8 +21,8 @@
 // between leaves the matrix cores busy half of the time at 1.9 - 2.0 GHz.  Tried on the way (up product of 8192 rows, d = 1024, H = 3584, us): eight
 // waves of 64 x 32 in one workgroup, two LDS buffers, the split between the MFMAs 745; the order of that pinned 727 - 740; four waves as here, 64-bit
 // addresses per unit in registers, which spilled 917; as here 660.  Wave priorities, loads two steps ahead: no gain.
-// T = 4096, d = 1024, H = 3584, E = 8, K = 2 (8192 rows), us, fp32 MFMAs -> here: up 1018 -> 660, down 515 -> 323, d(a) 604 -> 446, dxg 1040 -> 714, dW2
-// 494 -> 360, dW1 and dW3 980 -> 700.
+// T = 4096, d = 1024, H = 3584, E = 8, K = 2 (8192 rows), us, fp32 MFMAs -> here: up 1018 -> 690, down 515 -> 335, d(a) 604 -> 440, dxg 1040 -> 705, dW2
+// 494 -> 350, dW1 and dW3 980 -> 675.
 #include "f32_product.h"
 #include "pack.h"
 #include <algorithm>
@@ -43,6 +49,12 @@ __device__ __forceinline__ void sp_split(float a, float b, uint32_t &h, uint32_t
     const float ra = a - __uint_as_float(h << 16), rb = b - __uint_as_float(h & 0xffff0000u);
     m = sp_pack(ra, rb);
     l = sp_pack(ra - __uint_as_float(m << 16), rb - __uint_as_float(m & 0xffff0000u));
+}
+
+// smallest magnitude so far (no number: left out)
+__device__ __forceinline__ void sp_least(float &least, float a, float b)
+{
+    asm("v_min3_f32 %0, %0, |%1|, |%2|" : "+v"(least) : "v"(a), "v"(b));
 }
 
 // A thread's unit of one step: U = 4 k places of a row of an operand contiguous in k (a line of a row per 8 lanes), 8 of a column of one
@@ -106,6 +118,8 @@ __device__ __forceinline__ int sp_swz(int row) { return ((row >> 2) & 1) | (((ro
 #define SP_PARTS(OP, TM, CT) (F32_IS_WG(OP) ? 1 : (TM) / 32 * ((CT) / 32))
 // waves per SIMD, that is workgroups per compute unit, that the registers leave room for
 #define SP_WAVES(NB) ((NB) == 2 ? 3 : 2)
+#define SP_FACTOR_MIN 0x1p-110f
+#define SP_SUM_MIN 0x1p-100f
 // One tile of 64 WR rows x 16 NB WC MFMA columns (up: half of them W1's, half W3's): WR x WC = 4 waves of 4 x NB blocks of 16 x 16.
 template <int OP, int WR, int WC, int NB, bool VEC>
 __global__ __launch_bounds__(256, SP_WAVES(NB)) void f32_split_kernel(f32_args p)
@@ -220,6 +234,16 @@ __global__ __launch_bounds__(256, SP_WAVES(NB)) void f32_split_kernel(f32_args p
             b_at = B1;
         }
     };
+    const int kleft = K1 - S1 * 32;
+    auto fetch_rest = [&](int seg) {  // the places behind the whole steps
+        const float *at = (seg ? A1 : A0) + (AK ? (size_t)S1 * 32 * p.Kd : S1 * 32);
+        const float *bt = (OP == F32_DXG && seg ? B1 : B0) + (BKM ? (size_t)S1 * 32 * p.N : S1 * 32);
+        const float *b3t = PAIR ? B1 + S1 * 32 : bt;
+#pragma unroll
+        for (int u = 0; u < NUA; ++u) sp_fetch_partial<AK>(va[u], at, oa[u], unit_k(AK, TM, u), kleft, p.Kd);
+#pragma unroll
+        for (int u = 0; u < NUB; ++u) sp_fetch_partial<BKM>(vb[u], of_w3(u) ? b3t : bt, ob[u], unit_k(BKM, TN, u), kleft, p.N);
+    };
     // Splitting: pair q of the thread's places (A's units, then B's) into w, which goes to LDS with the last pair of a unit
     constexpr int QA = NUA * UA / 2, QB = NUB * UB / 2;
     struct parts { uint32_t h[4], m[4], l[4]; };
@@ -238,6 +262,8 @@ __global__ __launch_bounds__(256, SP_WAVES(NB)) void f32_split_kernel(f32_args p
         store(at + (a ? PA : PB), w.m, U == 8);
         store(at + 2 * (a ? PA : PB), w.l, U == 8);
     };
+
+    uint32_t smallest = 0xffffffffu;  // of this lane's factors other than zero, where there are small ones: the bits but the sign, less one
 
     // row units of 16: unit WR i + wr; columns: block n of the wave
     const int live = max(0, min(4, ((rows + 15) / 16 + WR - 1 - wr) / WR));
@@ -279,8 +305,24 @@ __global__ __launch_bounds__(256, SP_WAVES(NB)) void f32_split_kernel(f32_args p
         };
         auto stage = [&]() {
             parts w;
+            float least = 1.0f;
 #pragma unroll
-            for (int q = 0; q < QA + QB; ++q) split(w, q);
+            for (int q = 0; q < QA + QB; ++q) {
+                const int qq = q < QA ? q : q - QA;
+                if (q < QA) sp_least(least, va[qq / (UA / 2)][2 * (qq % (UA / 2))], va[qq / (UA / 2)][2 * (qq % (UA / 2)) + 1]);
+                else sp_least(least, vb[qq / (UB / 2)][2 * (qq % (UB / 2))], vb[qq / (UB / 2)][2 * (qq % (UB / 2)) + 1]);
+                split(w, q);
+            }
+            if (__any(least < SP_FACTOR_MIN)) {  // (zeros, as a rule: they wrap)
+#pragma unroll
+                for (int u = 0; u < NUA; ++u)
+#pragma unroll
+                    for (int i = 0; i < UA; ++i) smallest = min(smallest, (__float_as_uint(va[u][i]) << 1) - 1u);
+#pragma unroll
+                for (int u = 0; u < NUB; ++u)
+#pragma unroll
+                    for (int i = 0; i < UB; ++i) smallest = min(smallest, (__float_as_uint(vb[u][i]) << 1) - 1u);
+            }
         };
         auto multiply = [&]() {
             read_a(0);
@@ -308,15 +350,8 @@ __global__ __launch_bounds__(256, SP_WAVES(NB)) void f32_split_kernel(f32_args p
                 __syncthreads();
             }
         }
-        const int kleft = K1 - S1 * 32;
         for (int seg = 0; kleft > 0 && seg < (OP == F32_DXG ? 2 : 1); ++seg) {
-            const float *at = (seg ? A1 : A0) + (AK ? (size_t)S1 * 32 * p.Kd : S1 * 32);
-            const float *bt = (OP == F32_DXG && seg ? B1 : B0) + (BKM ? (size_t)S1 * 32 * p.N : S1 * 32);
-            const float *b3t = PAIR ? B1 + S1 * 32 : bt;
-#pragma unroll
-            for (int u = 0; u < NUA; ++u) sp_fetch_partial<AK>(va[u], at, oa[u], unit_k(AK, TM, u), kleft, p.Kd);
-#pragma unroll
-            for (int u = 0; u < NUB; ++u) sp_fetch_partial<BKM>(vb[u], of_w3(u) ? b3t : bt, ob[u], unit_k(BKM, TN, u), kleft, p.N);
+            fetch_rest(seg);
             stage();
             __syncthreads();
             multiply();
@@ -331,8 +366,49 @@ __global__ __launch_bounds__(256, SP_WAVES(NB)) void f32_split_kernel(f32_args p
         default: run(std::integral_constant<int, 0>()); break;
     }
 
-    // Sums that the three parts cannot carry: infinite or no number (an infinite h times a part that is zero, and what rounds to an
-    // infinite h), or so small that parts of their factors may have been lost.  Fragments straight from memory: as slow as it is rare.
+    // What the three parts cannot carry: sums that are infinite or no number (an infinite h times a part that is zero, and what rounds to an
+    // infinite h), or so small that what factors and partial products have lost counts.  Their wave computes its part of the tile again: fragments
+    // straight from memory, 16 k places at a time.
+    float limit = SP_SUM_MIN;
+    uint32_t *word = (uint32_t *)sp_lds + wave;  // (every wave's last reads of the planes are behind it)
+    auto words = [&](uint32_t v) {               // one of each wave
+        if (lane == 0) *word = v;
+        __syncthreads();
+        const sp_u32x4 w = *(const sp_u32x4 *)sp_lds;
+        __syncthreads();
+        return w;
+    };
+    const sp_u32x4 w = words(__any(smallest < 2u * __float_as_uint(SP_FACTOR_MIN) - 1u));
+    const bool tiny = __builtin_amdgcn_readfirstlane(w[0] | w[1] | w[2] | w[3]) != 0;
+    if (tiny) {  // the largest factor, from all of them once more
+        float most = 0.0f;
+        auto all = [&]() {
+#pragma unroll
+            for (int u = 0; u < NUA; ++u)
+#pragma unroll
+                for (int i = 0; i < UA; ++i) most = fmaxf(most, fabsf(va[u][i]));
+#pragma unroll
+            for (int u = 0; u < NUB; ++u)
+#pragma unroll
+                for (int i = 0; i < UB; ++i) most = fmaxf(most, fabsf(vb[u][i]));
+        };
+        a_at = A0;
+        b_at = B0;
+        b3_at = B1;
+        for (int s = 0; s < steps; ++s) {
+            fetch();
+            advance(s + 1);
+            all();
+        }
+        for (int seg = 0; kleft > 0 && seg < (OP == F32_DXG ? 2 : 1); ++seg) {
+            fetch_rest(seg);
+            all();
+        }
+#pragma unroll
+        for (int q = 1; q < 64; q <<= 1) most = fmaxf(most, __shfl_xor(most, q, 64));
+        const sp_u32x4 m = words(__float_as_uint(most));
+        limit = fmaxf(limit, __uint_as_float(max(max(m[0], m[1]), max(m[2], m[3]))) * K1 * 0x1p-106f);
+    }
     bool odd = false;
 #pragma unroll
     for (int i = 0; i < 4; ++i)
@@ -341,8 +417,8 @@ __global__ __launch_bounds__(256, SP_WAVES(NB)) void f32_split_kernel(f32_args p
             acc[i][n] += low[i][n];
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const uint32_t v = __float_as_uint(acc[i][n][r]) & 0x7fffffffu;
-                odd |= v >= 0x7f800000u || v - 1u < 0x17800000u;  // 0x17800000: 2^-80
+                const float v = fabsf(acc[i][n][r]);
+                odd |= i < live && (!(v < INFINITY) || (v < limit && (v != 0.0f || tiny)));
             }
         }
     if (__any(odd && live > 0)) {

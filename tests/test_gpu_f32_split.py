@@ -91,3 +91,38 @@ def test_tiles_computed_again_add_two_sums():
     for cols in (few, np.setdiff1d(np.arange(d), few)):
         assert N.rel_l2(dx[:, cols], exact[:, cols]) < 1.2 * N.rel_l2(two[:, cols].astype(np.float64), exact[:, cols])
     layer.close()
+
+
+WIDE_TALL = dict(T=1500, d=1284, H=772, E=5, K=2, Es=1)   # split weight gradients; row tiles of 128 ...
+WIDE_MID = dict(T=900, d=1284, H=1028, E=5, K=2, Es=1)    # ... and of 64
+
+# powers of two on x (the gate's weights and W1 take the opposite), W3, W2 and dout that leave the results what they are but for a power of two: a
+# factor of 2^-120 meets one of 2^120 in (a) up, (b) d(a), (c) d(a) and, with dh, the input gradient, (d) down and input gradient, (e) dW2
+SCALES = dict(up=(-120, 120, 0, 0), da=(0, 0, 120, -120), dxg=(-120, 120, 0, -120), down=(0, -120, 120, 0), wg2=(0, 120, 0, -120))
+
+
+@pytest.mark.parametrize("kw,rows", [(WIDE_TALL, 128), (WIDE_MID, 64), (dict(WIDE_TALL, d=1285, H=771), 128)])
+def test_tiny_factors_with_large_ones(kw, rows):
+    """Scaling by powers of two is exact in fp32 as long as nothing under- or overflows: the same results but for that power, to the error of fp32
+    sums in another order (K = 1285: 2e-6; factors of 2^-120 in three bf16 parts have 2e-5 and more)."""
+    G, cfg, inp, dout, _ = _setup("c1_tiny_f32", kw, 96)
+
+    def step(ex, e3, e2, eo):
+        two = [np.float32(2.0 ** e) for e in (ex, e3, e2, eo, -ex)]
+        p = dict(inp, x=inp["x"] * two[0], Wg=inp["Wg"] * two[4], W1=[w * two[4] for w in inp["W1"]], W3=[w * two[1] for w in inp["W3"]],
+                 W2=[w * two[2] for w in inp["W2"]])
+        layer = G.build_layer(cfg, p)
+        assert layer.f32_tiles(cfg.T) == (rows, 128, 128)
+        r = [layer.forward(G.P.DeviceBuffer.from_numpy(G.ctx(), p["x"], cfg.dtype)).to_numpy(),
+             layer.back(G.P.DeviceBuffer.from_numpy(G.ctx(), dout * two[3], cfg.dtype)).to_numpy()]
+        r += [layer.grad(w, g) for g in (0, cfg.E) for w in (L.W_W1, L.W_W3, L.W_W2)]
+        layer.close()
+        return r
+
+    want = step(0, 0, 0, 0)
+    for name, (ex, e3, e2, eo) in SCALES.items():
+        a, h = ex + e3, eo + e2                                 # of a, and of d(a)
+        power = [a + e2, h + e3] + 2 * [h + e3 + 2 * ex, h + ex, eo + a]
+        for got, ref, e in zip(step(ex, e3, e2, eo), want, power):
+            if -100 < e < 126:
+                assert N.rel_l2(got.astype(np.float64) * 2.0 ** -e, ref) < 2e-6, (name, e)
