@@ -139,8 +139,8 @@ int experts_f32_tile_m_max(const omega_moe *m, int T)
 // 114 / 85 / 102, 1376 x 223 x 3135, 15 experts, top 6 455 / 351 / 378, 4096 x 1024 x 3584, 8 experts, top 2 1690 / 1420 / 980. 
 int experts_f32_tile_m(const omega_moe *m, int T)
 {
-    if (experts_f32_tile_m_max(m, T) == F32_TILE_M_SMALL) return F32_TILE_M_SMALL;
     const omega_moe_config &c = m->cfg;
+    if (experts_f32_tile_m_max(m, T) == F32_TILE_M_SMALL || c.d < SP_TERMS_MIN || c.H < SP_TERMS_MIN) return F32_TILE_M_SMALL;
     struct product { int step, cols, slots; double a, more, rest, pad, least, part, cut, few, base; };
     static const struct { int bm; product up, down; } form[] = {
         {F32_TILE_M_SMALL, {64, 32, 2, 9.5, 66, 58, 0.45, 1.02, 0.93, 1, 0, 3.1}, {64, 32, 2, 5.2, 37, 67, 0.51, 1.01, 1, 1, 0, 3.1}},

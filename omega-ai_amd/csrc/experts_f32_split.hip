@@ -215,7 +215,10 @@ __global__ __launch_bounds__(256, SP_WAVES(NB)) void f32_split_kernel(f32_args p
     }
     auto of_w3 = [](int u) { return PAIR && THR / 8 * u >= CT; };
 
-    const int S1 = K1 / 32, steps = OP == F32_DXG ? 2 * S1 : S1;
+    // (weight gradients of a few rows: of one product the sum of its six parts is rounded several times.  Largest error against float64, chain / here, of
+    // one term 5.96e-8 / 1.03e-7 of it, of four 1.9e-7 / 1.6e-7)
+    const bool few = WG && K1 < SP_TERMS_MIN;
+    const int S1 = few ? 0 : K1 / 32, steps = OP == F32_DXG ? 2 * S1 : S1;
     const float *a_at = A0, *b_at = B0, *b3_at = B1;
     float va[NUA][UA], vb[NUB][UB];
     auto fetch = [&]() {
@@ -234,7 +237,7 @@ __global__ __launch_bounds__(256, SP_WAVES(NB)) void f32_split_kernel(f32_args p
             b_at = B1;
         }
     };
-    const int kleft = K1 - S1 * 32;
+    const int kleft = few ? 0 : K1 - S1 * 32;
     auto fetch_rest = [&](int seg) {  // the places behind the whole steps
         const float *at = (seg ? A1 : A0) + (AK ? (size_t)S1 * 32 * p.Kd : S1 * 32);
         const float *bt = (OP == F32_DXG && seg ? B1 : B0) + (BKM ? (size_t)S1 * 32 * p.N : S1 * 32);
@@ -409,7 +412,7 @@ __global__ __launch_bounds__(256, SP_WAVES(NB)) void f32_split_kernel(f32_args p
         const sp_u32x4 m = words(__float_as_uint(most));
         limit = fmaxf(limit, __uint_as_float(max(max(m[0], m[1]), max(m[2], m[3]))) * K1 * 0x1p-106f);
     }
-    bool odd = false;
+    bool odd = few;
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll

@@ -523,4 +523,5 @@ static inline unsigned f32_grid(const f32_args &p, size_t tiles, int parts)
     return (unsigned)(8 * (per + cut * (parts - 1)));
 }
 
+#define SP_TERMS_MIN 4  // sums of fewer terms are not split
 hipError_t launch_product_f32_split(const f32_args &p, int op, bool vec, int max_tiles, hipStream_t s);  // experts_f32_split.hip

@@ -126,3 +126,21 @@ def test_tiny_factors_with_large_ones(kw, rows):
         for got, ref, e in zip(step(ex, e3, e2, eo), want, power):
             if -100 < e < 126:
                 assert N.rel_l2(got.astype(np.float64) * 2.0 ** -e, ref) < 2e-6, (name, e)
+
+
+def test_weight_gradient_of_a_single_row_is_rounded_once():
+    """An expert with one row in a batch whose weight gradients are split: every element is one product, rounded once."""
+    G, cfg, inp, dout, layer = _setup("c1_tiny_f32", dict(T=512, d=1664, H=1664, E=2, K=1), 97)
+    layer.close()
+    t = 7
+    inp["x"][:, 0], inp["x"][t, 0] = -1.0, 1.0
+    inp["Wg"][:] = 0.0
+    inp["Wg"][1, 0] = 1.0
+    layer = G.build_layer(cfg, inp)
+    assert layer.f32_tiles(cfg.T)[1:] == (128, 128)
+    layer.forward(G.P.DeviceBuffer.from_numpy(G.ctx(), inp["x"], cfg.dtype))
+    assert layer.routing()["counts"].tolist() == [511, 1]
+    a = layer.workspace("a", cfg.T)[-1]
+    layer.back(G.P.DeviceBuffer.from_numpy(G.ctx(), dout, cfg.dtype))
+    assert np.array_equal(layer.grad(L.W_W2, 1), dout[t][:, None] * a[None, :])
+    layer.close()
