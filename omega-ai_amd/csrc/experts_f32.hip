@@ -62,7 +62,9 @@ __device__ __forceinline__ int f32_self(const f32_args &p, uint16_t *tok, omega_
     return (ti / nrb) * 32;
 }
 
-template <int OP, int TM, int TN, bool VEC>
+// SELF: the launch makes the dispatch index (a kernel of its own: in one with the others its registers, 105 for 84, and its scalar spills cost them up
+// to 6 %: forward pass, us, 2373 tokens x 142 x 88, 5 experts, top 1 30.7 -> 29.1, 566 x 192 x 109, 10 experts, top 3, one shared 30.5 -> 29.0)
+template <int OP, int TM, int TN, bool VEC, bool SELF>
 __global__ __launch_bounds__(256, 2) void f32_product_kernel(f32_args p)
 {
     constexpr bool WG = F32_IS_WG(OP), PAIR = F32_PAIR(OP), PARTS = F32_PARTS(OP, TM, TN) > 1;
@@ -74,15 +76,13 @@ __global__ __launch_bounds__(256, 2) void f32_product_kernel(f32_args p)
     constexpr int LAP = f32_lds_floats(32, WG, F32_FBK(32)), LBP = f32_lds_floats(PN, BK_, F32_FBK(32));
     static_assert(!PARTS || LAP <= LA, "a part's operands fit");
     __shared__ __attribute__((aligned(16))) float as[WG ? 1 : 2 * LA], bs[WG ? 1 : 2 * (PARTS && LBP > LB ? LBP : LB)];
-    if constexpr (OP == F32_UP && TM == F32_TILE_M_SMALL) {
-        if (p.index.ids != nullptr) {
-            __shared__ uint16_t tok[F32_TILE_M_SMALL];
-            omega_tile tl;
-            const int P = p.T * p.K;
-            const int n0 = P <= 256 ? f32_self<4, VEC>(p, tok, tl) : P <= 512 ? f32_self<8, VEC>(p, tok, tl) : f32_self<F32_SELF_CHUNKS, VEC>(p, tok, tl);
-            if (n0 >= 0) f32_tile<OP, TM, TN, VEC>(p, as, bs, 0, tl, 0, n0, 0, tok);
-            return;
-        }
+    if constexpr (SELF) {
+        __shared__ uint16_t tok[F32_TILE_M_SMALL];
+        omega_tile tl;
+        const int P = p.T * p.K;
+        const int n0 = P <= 256 ? f32_self<4, VEC>(p, tok, tl) : P <= 512 ? f32_self<8, VEC>(p, tok, tl) : f32_self<F32_SELF_CHUNKS, VEC>(p, tok, tl);
+        if (n0 >= 0) f32_tile<OP, TM, TN, VEC>(p, as, bs, 0, tl, 0, n0, 0, tok);
+        return;
     }
     if (OP == F32_UP && (int)blockIdx.x >= (int)gridDim.x - p.copy_wgs) {
         copy_gathered<VEC, false>(p, blockIdx.x - (gridDim.x - p.copy_wgs), threadIdx.x & 63, threadIdx.x >> 6, 0);
@@ -179,9 +179,14 @@ static hipError_t f32_launch(f32_args p, bool vec, int max_tiles, hipStream_t s)
     if (F32_IS_WG(OP)) p.deal = wgrad_deal_of(ceil_div(p.N, CT) * ceil_div(p.Kd, TM), p.G * (OP == F32_WG13 ? 2 : 1));
     // (weight gradients: whole groups of matrices and one of what is left over, each to eight XCDs)
     const unsigned grid = (F32_IS_WG(OP) ? (unsigned)((tiles + 7) / 8 * 8 + (p.deal.rest > 0 ? 8 : 0)) : f32_grid(p, tiles, F32_PARTS(OP, TM, TN))) + p.copy_wgs + (p.index.ids != nullptr ? 1 : 0);
-    if (vec) hipLaunchKernelGGL((f32_product_kernel<OP, TM, TN, true>), dim3(grid), dim3(256), 0, s, p);
-    else hipLaunchKernelGGL((f32_product_kernel<OP, TM, TN, false>), dim3(grid), dim3(256), 0, s, p);
-    return hipGetLastError();
+    auto launch = [&](auto self) {
+        if (vec) hipLaunchKernelGGL((f32_product_kernel<OP, TM, TN, true, decltype(self)::value>), dim3(grid), dim3(256), 0, s, p);
+        else hipLaunchKernelGGL((f32_product_kernel<OP, TM, TN, false, decltype(self)::value>), dim3(grid), dim3(256), 0, s, p);
+        return hipGetLastError();
+    };
+    if constexpr (OP == F32_UP && TM == F32_TILE_M_SMALL)
+        if (p.index.ids != nullptr) return launch(std::true_type());
+    return launch(std::false_type());
 }
 
 hipError_t launch_product_f32(const omega_moe *m, int op, const float *x, const float *dout, int T, hipStream_t s, bool gather, bool keep)
