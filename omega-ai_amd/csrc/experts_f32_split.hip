@@ -11,8 +11,8 @@
 // these matrix cores, and 2^20 of them are then below 2^-27 of the sum - computes its part of the tile again on fp32 MFMAs.  A factor below 2^-110
 // other than zero, whose last part would need bits below those of a bf16 denormal, loses up to 2^-134 of itself: where there is one, a tile's sums are held to
 // 2^-106 of the largest factor times the number of terms, so that what is lost is below 2^-26 of them.
-// The look at every factor costs 2.7 - 3.5 % of these launches (one v_min3_f32 per two of them, and a branch for the zeros).  Where there is a tiny one the
-// largest is found by fetching all of them once more (input gradient below 700 -> 950 us), and a launch all of whose waves compute again takes 2.7 times as
+// The look at every factor is one v_min3_f32 for two of them; from a wave's first step with a zero on - a second copy of its loop, which costs every launch less
+// than the branch in the first one - small ones are told from zeros.  Batches with zeros in every eighth row 1 % longer.  Where there is a tiny one the largest is found by fetching all of them once more (input gradient below 700 -> 950 us), and a launch all of whose waves compute again takes 2.7 times as
 // long (dW1 and dW3 below 675 -> 1810: a unit in 64 that is saturated, h1 = -64, for every token).
 //
 // Bound: bf16 MFMA at a sixth of its rate, 417 TFLOP/s nominal, 240 under the power cap where fp32 MFMA has 154.  One workgroup = four waves of 64 rows
@@ -21,8 +21,8 @@
 // between leaves the matrix cores busy half of the time at 1.9 - 2.0 GHz.  Tried on the way (up product of 8192 rows, d = 1024, H = 3584, us): eight
 // waves of 64 x 32 in one workgroup, two LDS buffers, the split between the MFMAs 745; the order of that pinned 727 - 740; four waves as here, 64-bit
 // addresses per unit in registers, which spilled 917; as here 660.  Wave priorities, loads two steps ahead: no gain.
-// T = 4096, d = 1024, H = 3584, E = 8, K = 2 (8192 rows), us, fp32 MFMAs -> here: up 1018 -> 690, down 515 -> 335, d(a) 604 -> 440, dxg 1040 -> 705, dW2
-// 494 -> 350, dW1 and dW3 980 -> 675.
+// T = 4096, d = 1024, H = 3584, E = 8, K = 2 (8192 rows), us, fp32 MFMAs -> here: up 1018 -> 660, down 515 -> 340, d(a) 604 -> 436, dxg 1040 -> 720, dW2
+// 494 -> 352, dW1 and dW3 980 -> 678.
 #include "f32_product.h"
 #include "pack.h"
 #include <algorithm>
@@ -266,7 +266,19 @@ __global__ __launch_bounds__(256, SP_WAVES(NB)) void f32_split_kernel(f32_args p
         store(at + 2 * (a ? PA : PB), w.l, U == 8);
     };
 
-    uint32_t smallest = 0xffffffffu;  // of this lane's factors other than zero, where there are small ones: the bits but the sign, less one
+    float least = 1.0f;               // smallest magnitude among this lane's factors of the steps before the first with a small one ...
+    int small_step = -1;              // ... and that step
+    uint32_t smallest = 0xffffffffu;  // of its factors other than zero, from there on: the bits but the sign, less one (zeros wrap)
+    auto note_small = [&]() {
+#pragma unroll
+        for (int u = 0; u < NUA; ++u)
+#pragma unroll
+            for (int i = 0; i < UA; ++i) smallest = min(smallest, (__float_as_uint(va[u][i]) << 1) - 1u);
+#pragma unroll
+        for (int u = 0; u < NUB; ++u)
+#pragma unroll
+            for (int i = 0; i < UB; ++i) smallest = min(smallest, (__float_as_uint(vb[u][i]) << 1) - 1u);
+    };
 
     // row units of 16: unit WR i + wr; columns: block n of the wave
     const int live = max(0, min(4, ((rows + 15) / 16 + WR - 1 - wr) / WR));
@@ -306,26 +318,17 @@ __global__ __launch_bounds__(256, SP_WAVES(NB)) void f32_split_kernel(f32_args p
             sp_f32x4 &d = m == 1 ? acc[i][n] : low[i][n];
             d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[i & 1][pa[m]], fb[n][pb[m]], d, 0, 0, 0);
         };
-        auto stage = [&]() {
+        auto stage = [&](auto careful) {
             parts w;
-            float least = 1.0f;
+            float now = 1.0f, &low_end = decltype(careful)::value ? now : least;
 #pragma unroll
             for (int q = 0; q < QA + QB; ++q) {
                 const int qq = q < QA ? q : q - QA;
-                if (q < QA) sp_least(least, va[qq / (UA / 2)][2 * (qq % (UA / 2))], va[qq / (UA / 2)][2 * (qq % (UA / 2)) + 1]);
-                else sp_least(least, vb[qq / (UB / 2)][2 * (qq % (UB / 2))], vb[qq / (UB / 2)][2 * (qq % (UB / 2)) + 1]);
+                if (q < QA) sp_least(low_end, va[qq / (UA / 2)][2 * (qq % (UA / 2))], va[qq / (UA / 2)][2 * (qq % (UA / 2)) + 1]);
+                else sp_least(low_end, vb[qq / (UB / 2)][2 * (qq % (UB / 2))], vb[qq / (UB / 2)][2 * (qq % (UB / 2)) + 1]);
                 split(w, q);
             }
-            if (__any(least < SP_FACTOR_MIN)) {  // (zeros, as a rule: they wrap)
-#pragma unroll
-                for (int u = 0; u < NUA; ++u)
-#pragma unroll
-                    for (int i = 0; i < UA; ++i) smallest = min(smallest, (__float_as_uint(va[u][i]) << 1) - 1u);
-#pragma unroll
-                for (int u = 0; u < NUB; ++u)
-#pragma unroll
-                    for (int i = 0; i < UB; ++i) smallest = min(smallest, (__float_as_uint(vb[u][i]) << 1) - 1u);
-            }
+            if (decltype(careful)::value && __any(now < SP_FACTOR_MIN)) note_small();
         };
         auto multiply = [&]() {
             read_a(0);
@@ -342,20 +345,30 @@ __global__ __launch_bounds__(256, SP_WAVES(NB)) void f32_split_kernel(f32_args p
                 __builtin_amdgcn_sched_barrier(0);
             }
         };
-        if (steps > 0) {
-            fetch();
-            for (int s = 0; s < steps; ++s) {
-                stage();
+        // from step s on; not careful: up to the first one with a zero or less than SP_FACTOR_MIN
+        auto steps_from = [&](auto careful, int s) {
+            for (bool small = false; s < steps && !small; ++s) {
+                stage(careful);
                 advance(s + 1);
                 fetch();
+                if (!decltype(careful)::value) small = __any(least < SP_FACTOR_MIN);
                 __syncthreads();
                 multiply();
                 __syncthreads();
             }
+            return s;
+        };
+        if (steps > 0) {
+            fetch();
+            const int s = steps_from(std::false_type(), 0);
+            if (__any(least < SP_FACTOR_MIN)) {
+                small_step = s - 1;
+                steps_from(std::true_type(), s);
+            }
         }
         for (int seg = 0; kleft > 0 && seg < (OP == F32_DXG ? 2 : 1); ++seg) {
             fetch_rest(seg);
-            stage();
+            stage(std::true_type());
             __syncthreads();
             multiply();
             __syncthreads();
@@ -373,15 +386,20 @@ __global__ __launch_bounds__(256, SP_WAVES(NB)) void f32_split_kernel(f32_args p
     // infinite h), or so small that what factors and partial products have lost counts.  Their wave computes its part of the tile again: fragments
     // straight from memory, 16 k places at a time.
     float limit = SP_SUM_MIN;
-    uint32_t *word = (uint32_t *)sp_lds + wave;  // (every wave's last reads of the planes are behind it)
-    auto words = [&](uint32_t v) {               // one of each wave
-        if (lane == 0) *word = v;
+    auto words = [&](int at, uint32_t v) {  // one of each wave (every wave's last reads of the planes are behind it)
+        if (lane == 0) ((uint32_t *)sp_lds)[at + wave] = v;
         __syncthreads();
-        const sp_u32x4 w = *(const sp_u32x4 *)sp_lds;
-        __syncthreads();
-        return w;
+        return *(const sp_u32x4 *)(sp_lds + 4 * at);
     };
-    const sp_u32x4 w = words(__any(smallest < 2u * __float_as_uint(SP_FACTOR_MIN) - 1u));
+    if (small_step >= 0) {  // (its factors were on their way out when it was seen)
+        const int s = OP == F32_DXG && small_step >= S1 ? small_step - S1 : small_step;
+        a_at = (s != small_step ? A1 : A0) + (AK ? (size_t)32 * s * p.Kd : 32 * s);
+        b_at = (s != small_step ? B1 : B0) + (BKM ? (size_t)32 * s * p.N : 32 * s);
+        b3_at = PAIR ? B1 + 32 * s : nullptr;
+        fetch();
+        note_small();
+    }
+    const sp_u32x4 w = words(0, __any(smallest < 2u * __float_as_uint(SP_FACTOR_MIN) - 1u));
     const bool tiny = __builtin_amdgcn_readfirstlane(w[0] | w[1] | w[2] | w[3]) != 0;
     if (tiny) {  // the largest factor, from all of them once more
         float most = 0.0f;
@@ -409,10 +427,12 @@ __global__ __launch_bounds__(256, SP_WAVES(NB)) void f32_split_kernel(f32_args p
         }
 #pragma unroll
         for (int q = 1; q < 64; q <<= 1) most = fmaxf(most, __shfl_xor(most, q, 64));
-        const sp_u32x4 m = words(__float_as_uint(most));
+        const sp_u32x4 m = words(4, __float_as_uint(most));
         limit = fmaxf(limit, __uint_as_float(max(max(m[0], m[1]), max(m[2], m[3]))) * K1 * 0x1p-106f);
     }
-    bool odd = few;
+    // (infinities and no numbers show in the sum of all, the smallest one other than zero in its bits; units behind the tile's rows are zero)
+    float all = 0.0f;
+    uint32_t low_end = 0xffffffffu;
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -420,10 +440,19 @@ __global__ __launch_bounds__(256, SP_WAVES(NB)) void f32_split_kernel(f32_args p
             acc[i][n] += low[i][n];
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const float v = fabsf(acc[i][n][r]);
-                odd |= i < live && (!(v < INFINITY) || (v < limit && (v != 0.0f || tiny)));
+                all += acc[i][n][r];
+                low_end = min(low_end, (__float_as_uint(acc[i][n][r]) << 1) - 1u);
             }
         }
+    bool odd = few || !(fabsf(all) < INFINITY) || low_end < 2u * __float_as_uint(limit) - 1u;
+    if (tiny) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int n = 0; n < NB; ++n)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) odd |= i < live && acc[i][n][r] == 0.0f;
+    }
     if (__any(odd && live > 0)) {
 #pragma unroll
         for (int i = 0; i < 4; ++i)
