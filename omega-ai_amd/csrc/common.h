@@ -213,9 +213,14 @@ int omega_set_error(omega_ctx *ctx, int status, const char *what, hipError_t her
 // 128 x 128, from 128 rows per expert on, once there are five for four compute units.  Training step, us, 64 x 64 of experts_f32.hip / there: 2272 tokens x
 // 339 x 2671, 4 experts, top 2 1213 / 988, 3300 x 780 x 2924, 6 experts, top 4 4945 / 4150, 2373 x 840 x 1100, 12 experts 1684 / 1580; with 0.8 tiles per
 // compute unit 447 / 473 and 1151 / 1221, with 70 to 90 rows per expert 516 / 533, 663 / 607, 643 / 645.
+// Tiles of shared experts have the k of all T rows and come last: with fewer than one for each compute unit, counted K + Es times over - less than half of
+// the launch's work in such a tile's time -, they hold it up.  Backward pass: 3156 x 300 x 656, 22 experts, top 2, one shared 483 / 630, 2365 x 176 x 1140, 9
+// experts, top 1, one shared 254 / 408, 3574 x 148 x 2600, 6 experts, top 1, two shared 844 / 1036.
 static inline bool f32_wgrad_wide(const omega_moe *m, int T, int mats)
 {
-    return (long long)T * m->cfg.K >= 128LL * m->cfg.E && 4LL * ceil_div(m->cfg.d, 128) * ceil_div(m->cfg.H, 128) * mats >= 5LL * m->ctx->num_cus;
+    const omega_moe_config &c = m->cfg;
+    const long long tiles = (long long)ceil_div(c.d, 128) * ceil_div(c.H, 128);  // of a matrix
+    return (long long)T * c.K >= 128LL * c.E && 4 * tiles * mats >= 5LL * m->ctx->num_cus && (c.Es == 0 || tiles * (mats / m->G) * (c.K + c.Es) >= m->ctx->num_cus);
 }
 
 #define OMEGA_FAIL(ctx, status, what) return omega_set_error((ctx), (status), (what), hipSuccess, __FILE__, __LINE__)
