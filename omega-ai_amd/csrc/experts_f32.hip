@@ -133,19 +133,21 @@ int experts_f32_tile_m_max(const omega_moe *m, int T)
 // places in whole steps, a fixed number more and, for a last partial step, `rest` more, at `a` ns per k; a product takes rounds of
 // one tile per compute unit, its last, partial round `part` of one and that share of the rest, or `cut` of its share where it goes in
 // parts (up to `few` of the workgroups that are there at a time), all of them `least` rounds or more; an expert has `pad` tiles more than its
-// rows.  The numbers are fitted to the stage times of 900 forward passes (64 to 6000 tokens, d = 64 .. 1536, H = 64 .. 3584, 1 to 16 experts) at all three
-// heights; of these passes the estimate takes the best or one within 5 % (41 are further off, one 23 %; 0.6 % in the mean).  Forward products, us, at 32 /
+// rows.  A product that goes in parts altogether takes `parts` times what tiles of 32 rows do.  Of two heights within 2 % the lower one is taken.  The
+// numbers are fitted to the stage times of 900 forward passes (64 to 8192 tokens, d = 64 .. 1024, H = 64 .. 3584, 1 to 24 experts) at all three heights; of
+// these passes the estimate takes the best or one within 5 % (40 are further off, one 23 %; 0.6 % in the mean), of the passes with a backward
+// pass behind them 22 are further off (one 18 %; 0.5 %).  (The earlier fit, to kernels that looked at no factors: 77 and 66, one 29 %.)  Forward products, us, at 32 /
 // 64 / 128 rows: 622 tokens x 130 x 420, one expert 13.9 / 22.2 / 46.9, 1982 x 512 x 1144, 4 experts, top 1 85.9 / 69.2 / 113.7, 2842 x 65 x 922, 4 experts, top 4
-// 114 / 85 / 102, 1376 x 223 x 3135, 15 experts, top 6 455 / 351 / 378, 4096 x 1024 x 3584, 8 experts, top 2 1690 / 1420 / 980. 
+// 114 / 85 / 102, 1376 x 223 x 3135, 15 experts, top 6 455 / 351 / 378, 4096 x 1024 x 3584, 8 experts, top 2 1690 / 1420 / 1000.
 int experts_f32_tile_m(const omega_moe *m, int T)
 {
     const omega_moe_config &c = m->cfg;
     if (experts_f32_tile_m_max(m, T) == F32_TILE_M_SMALL || c.d < SP_TERMS_MIN || c.H < SP_TERMS_MIN) return F32_TILE_M_SMALL;
-    struct product { int step, cols, slots; double a, more, rest, pad, least, part, cut, few, base; };
+    struct product { int step, cols, slots; double a, more, rest, pad, least, part, cut, few, base, parts; };
     static const struct { int bm; product up, down; } form[] = {
-        {F32_TILE_M_SMALL, {64, 32, 2, 9.5, 66, 58, 0.45, 1.02, 0.93, 1, 0, 3.1}, {64, 32, 2, 5.2, 37, 67, 0.51, 1.01, 1, 1, 0, 3.1}},
-        {F32_TILE_M_MID, {32, 64, 3, 25, 35, 19, 0.57, 1.08, 0.7, 1.56, 0.375, 5.9}, {32, 64, 4, 18.4, 28, 34, 0.48, 0.89, 0.8, 1.65, 0.25, 3.2}},
-        {F32_TILE_M, {32, 64, 2, 44, 55, 24, 0.6, 1.08, 0.54, 1.56, 0.375, 7.1}, {32, 128, 2, 46.1, 50, 26, 0.7, 1.07, 0.39, 1.27, 0.375, 4.7}}};
+        {F32_TILE_M_SMALL, {64, 32, 2, 8.35, 92.6, 58.9, 0.462, 0.97, 1.1, 1, 0, 3.62, 1}, {64, 32, 2, 4.81, 42, 63.6, 0.459, 1.02, 1.04, 1, 0, 3.21, 1}},
+        {F32_TILE_M_MID, {32, 64, 3, 23.1, 58.4, 30.2, 0.483, 1.01, 0.596, 1.48, 0.375, 6.48, 1}, {32, 64, 4, 18.5, 26.4, 21.9, 0.402, 0.326, 0.782, 2.65, 0.25, 3.18, 1.02}},
+        {F32_TILE_M, {32, 64, 2, 40.5, 78.8, 38.4, 0.465, 1.06, 0.412, 1.56, 0.375, 7.52, 1.09}, {32, 128, 2, 45.4, 25.8, 21.4, 0.659, 1.07, 0.439, 1.36, 0.375, 7.31, 1.24}}};
     int best = F32_TILE_M_SMALL;
     double least_time = 0.0;
     for (const auto &f : form) {
@@ -154,14 +156,15 @@ int experts_f32_tile_m(const omega_moe *m, int T)
         };
         auto time = [&](product q, const product &parts, int k, int n) {
             double all = rounds_of(q, f.bm, n);
+            const double slower = all <= 0.75 ? q.parts : 1.0;
             if (all <= 0.75) all = rounds_of(q = parts, F32_TILE_M_SMALL, n);  // (f32_part)
             const double whole = std::floor(all), full = std::floor(all / q.slots) * q.slots;
             double rounds = all < q.least ? q.least : whole + (all > whole ? q.part + (1.0 - q.part) * (all - whole) : 0.0);
             if (full > 0.0 && all - full <= q.few * q.slots) rounds = std::min(rounds, full + q.cut * (all - full));
-            return q.base + 1e-3 * q.a * rounds * (ceil_div(k, q.step) * q.step + q.more + (k % q.step != 0 ? q.rest : 0.0));
+            return slower * (q.base + 1e-3 * q.a * rounds * (ceil_div(k, q.step) * q.step + q.more + (k % q.step != 0 ? q.rest : 0.0)));
         };
         const double t = time(f.up, form[0].up, c.d, c.H) + time(f.down, form[0].down, c.H, c.d);
-        if (f.bm == F32_TILE_M_SMALL || t < least_time) {
+        if (f.bm == F32_TILE_M_SMALL || 1.02 * t < least_time) {
             best = f.bm;
             least_time = t;
         }
