@@ -63,17 +63,18 @@ __device__ __forceinline__ void small_index(const index_args &p, const uint8_t *
         p.offsets[p.E] = P;
         p.tile_meta[0] = tiles + p.Es * per_shared;
     }
-    // stable ranks, 64 pairs at a time: the lanes with one expert find each other by ballot, run[e] moves on by their number
+    // Stable ranks, 64 pairs at a time: the lanes with one expert find each other by one ballot per bit of its number, run[e] moves on by their
+    // number.  (This wave's chain ends the launch.  With a ballot per expert of the 64 pairs, forward pass of 26 tokens x 1024 x 384, 172 experts, top 38 153
+    // us, 130 with a launch for the index.)
+    const int bits = 32 - __clz(p.E - 1 | 1);
     for (int c0 = 0; c0 < P; c0 += 64) {
         const int i = c0 + lane;
         const bool valid = i < P;
         const int e = valid ? id[i] : -1;
-        unsigned long long todo = __ballot(valid), mine = 0;
-        while (todo) {
-            const int le = __builtin_amdgcn_readlane(e, __ffsll((long long)todo) - 1);
-            const unsigned long long m = __ballot(e == le);
-            if (e == le) mine = m;
-            todo &= ~m;
+        unsigned long long mine = __ballot(valid);
+        for (int b = 0; b < bits; ++b) {
+            const unsigned long long m = __ballot(e >> b & 1);
+            mine &= e >> b & 1 ? m : ~m;
         }
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         const unsigned long long below = mine & ((1ull << lane) - 1ull);
