@@ -666,7 +666,6 @@ static int ensure_queues(omega_moe *m, int T)
 {
     if (m->queued) return OMEGA_OK;
     m->queued = true;
-    m->index_in_up = false;
     const hipError_t e = launch_dispatch_index(m, T, m->bm, m->ctx->stream, nullptr);
     m->queued = e == hipSuccess;  // (the next to ask tries again: the queues are still an earlier batch's)
     OMEGA_HIP_CHECK(m->ctx, e);
@@ -728,7 +727,7 @@ static int stage_dispatch(omega_moe *m, const void *x, int T, bool up_follows = 
     const bool up_gathers = up_follows && (m->few || (!bf && (double)T * m->cfg.d * 4.0 < 4.0e9));
     // (a few tokens, or pairs of an fp32 layer: their up product makes the index itself)
     m->index_in_up = up_gathers && makes_index_in_up(m, T);
-    OMEGA_HIP_CHECK(m->ctx, launch_dispatch_index(m, T, bm, m->ctx->stream, bf && !m->gather_on_load && !up_gathers ? x : nullptr));
+    if (!m->index_in_up) OMEGA_HIP_CHECK(m->ctx, launch_dispatch_index(m, T, bm, m->ctx->stream, bf && !m->gather_on_load && !up_gathers ? x : nullptr));
     if (!bf && !up_gathers) OMEGA_HIP_CHECK(m->ctx, launch_dispatch_gather(m, x, T, m->ctx->stream));
     m->xg_valid = !m->gather_on_load && !up_gathers;
     m->dispatched_T = T;
@@ -1388,7 +1387,6 @@ int omega_moe_time_stage(omega_moe *m, int stage, const void *x, int T, void *ou
             case 7:
                 // parts of a dispatch that has already run for this T (same buffers, same result)
                 if (m->dispatched_T != T) OMEGA_FAIL(ctx, OMEGA_ERR_INVALID_ARG, "time_stage: dispatch has not run for this T");
-                m->index_in_up = false;
                 if (stage == 6) OMEGA_HIP_CHECK(ctx, launch_dispatch_index(m, T, m->bm, ctx->stream));
                 else OMEGA_HIP_CHECK(ctx, launch_dispatch_gather(m, x, T, ctx->stream));
                 return OMEGA_OK;

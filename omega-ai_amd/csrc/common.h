@@ -102,7 +102,7 @@ struct omega_moe {
     // the batch is one of a few tokens outside training: its products run on experts_few.hip and its dispatch made no work queues
     // (what needs them has them made first: ensure_queues)
     bool few = false, queued = true;
-    // the up product that is launched next makes the dispatch index of its batch: launch_dispatch_index leaves it to it
+    // the up product that is launched next makes the dispatch index of its batch (between the dispatch and the up stage of a forward pass)
     bool index_in_up = false;
     // the down product of the batch in y has left k slices in y_slabs that are not in y: the combine kernel adds them on its
     // way (combine.hip), whatever else reads y has them added first (ensure_y_whole)

@@ -780,7 +780,6 @@ __global__ __launch_bounds__(256) void dispatch_gather_bytes_kernel(const unsign
 // x != nullptr (bf16 layers): the workgroups also copy the rows of their token tiles into xg (and xs)
 hipError_t launch_dispatch_index(const omega_moe *m, int T, int bm, hipStream_t s, const void *x)
 {
-    if (m->index_in_up) return hipSuccess;
     const omega_moe_config &c = m->cfg;
     const bool rows = x != nullptr && c.dtype == OMEGA_DTYPE_BF16;
     // from half the last-level cache of gathered rows on, the rows are written around it

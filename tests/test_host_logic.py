@@ -299,3 +299,18 @@ def test_tiles_of_weight_gradients_are_dealt_evenly(lib, n, mats):
                 run = [t for t in got if t // n == m]
                 assert len(run) in (n // 8, -(-n // 8)) and run == list(range(run[0], run[0] + len(run)))
     assert seen == set(range(n * mats)) and max(totals) - min(totals) <= (1 if n >= 32 else 2)
+
+
+@pytest.mark.parametrize("dtype,up", [("bf16", "experts_bf16 which=0 keep=0"), ("f32", "product_f32 op=0 gather=1 keep=0")])
+def test_the_index_is_launched_unless_the_up_product_makes_it(lib, dtype, up):
+    """A forward pass of a few tokens leaves the dispatch index to its up product; whoever else asks for the index gets its launch, and a pass whose up
+    product was not launched leaves no index."""
+    m = Layer(lib, dtype)
+    assert m.forward(8) == 0 and "index" not in m.log()
+    assert m.back(8) == 0 and m.log().count("index") == (1 if dtype == "bf16" else 0)     # (the work queues of the backward pass)
+    assert m.stages(8) == [0, 0, 0] and m.log().count("index") == 1
+    assert m.forward(600) == 0 and m.log().count("index") == 1
+    lib.host_fail_launch(up.encode())
+    assert m.forward(8) != 0 and m.lib.omega_moe_experts_up(m.h, m.x, 8) != 0 and m.lib.omega_moe_experts_down(m.h, 8) != 0
+    assert m.forward(8) == 0
+    m.close()
