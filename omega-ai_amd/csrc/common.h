@@ -187,14 +187,31 @@ static inline bool combine_by_vectors(const omega_moe *m, const void *out, const
 // pass, us, tile kernels / there: 485 / 485, 514 / 560; 80 / 192 tokens x 2048 x 1408, 64 experts: 241 / 231, 253 / 257.
 static inline bool experts_few_rows(const omega_moe *m, int T) { return m->cfg.dtype == OMEGA_DTYPE_BF16 && T <= 64; }
 
+__host__ __device__ static inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
+
 // Forward passes whose up product makes the dispatch index itself (omega_moe::index_in_up): bf16 batches of a few tokens, fp32 ones in tiles of 32 rows,
-// with no more pairs (and experts) than their workgroups hold
+// with no more pairs than their workgroups hold.
+// bf16: every workgroup of the launch looks at all pairs, which outweighs a launch of 6 us once there are many of both.  Forward pass, us, with a launch for the
+// index / without, in million pairs x workgroups: 15 tokens x 256 x 2560, 49 experts, top 18 (2.1) 83.2 / 82.6, 30 x 256 x 2176, 108 experts, top 16 (3.5)
+// 84.7 / 84.3, 3 x 512 x 2432, 193 experts, top 49 (3.3) 191 / 195, 13 x 1024 x 3584, 43 experts, top 38 (4.8) 191 / 198, 12 x 256 x 3584, 91 experts, top 48 (11.7) 194 / 212.
+// fp32: expert by expert and 64 pairs at a time; in workgroups x experts x chunks: 179 tokens x 95 x 1956, 5 experts, top 2 (40000) 44.8 / 42.8, 77 x 169 x 1605, 8
+// experts, top 7, two shared (190000) 57.0 / 58.2, 177 x 49 x 2789, 14 experts, top 2, one shared (305000) 57.1 / 63.9; and 256 x 128 x 256, 32 experts, top
+// 2 27.7 / 32.0, 64 experts, top 4 34.7 / 79.1.
 #define INDEX_IN_UP_PAIRS 1024
+#define INDEX_IN_UP_WORK 2500000
+#define INDEX_IN_UP_WORK_F32 120000
 #define INDEX_IN_UP_EXPERTS_F32 16
+#define INDEX_IN_UP_CHUNKS_F32(pairs) ((pairs) <= 256 ? 4 : (pairs) <= 512 ? 8 : INDEX_IN_UP_PAIRS / 64)  // of 64 pairs, in registers
+static inline int few_up_cols(int T) { return T > 16 ? 32 : 16; }  // columns of a workgroup of the few-token up product (experts_few.hip)
 static inline bool makes_index_in_up(const omega_moe *m, int T)
 {
-    const bool fits = m->cfg.dtype == OMEGA_DTYPE_BF16 ? m->few : m->bm == 32 && m->cfg.E <= INDEX_IN_UP_EXPERTS_F32;
-    return fits && (long long)T * m->cfg.K <= INDEX_IN_UP_PAIRS;
+    const omega_moe_config &c = m->cfg;
+    const long long pairs = (long long)T * c.K;
+    if (pairs > INDEX_IN_UP_PAIRS) return false;
+    if (c.dtype != OMEGA_DTYPE_BF16)
+        return m->bm == 32 && c.E <= INDEX_IN_UP_EXPERTS_F32 &&
+               (long long)m->max_m_tiles * ceil_div(c.H, 32) * c.E * INDEX_IN_UP_CHUNKS_F32(pairs) <= INDEX_IN_UP_WORK_F32;
+    return m->few && pairs * ((pairs < c.E ? pairs : c.E) + c.Es) * (c.H / few_up_cols(T)) <= INDEX_IN_UP_WORK;
 }
 
 // Tokens per router workgroup = per row of tile_counts and per workgroup of the dispatch kernel: 16 for layers with at most
@@ -204,8 +221,6 @@ int router_tok_tile(const omega_moe *m, int T);
 
 // Size of the last-level (memory-side) cache of the device: streams larger than this are written / read around it.
 #define OMEGA_LLC_BYTES ((size_t)256 << 20)
-
-__host__ __device__ static inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
 
 int omega_set_error(omega_ctx *ctx, int status, const char *what, hipError_t herr, const char *file, int line);
 

@@ -80,7 +80,8 @@ __global__ __launch_bounds__(256, 2) void f32_product_kernel(f32_args p)
         __shared__ uint16_t tok[F32_TILE_M_SMALL];
         omega_tile tl;
         const int P = p.T * p.K;
-        const int n0 = P <= 256 ? f32_self<4, VEC>(p, tok, tl) : P <= 512 ? f32_self<8, VEC>(p, tok, tl) : f32_self<F32_SELF_CHUNKS, VEC>(p, tok, tl);
+        const int chunks = INDEX_IN_UP_CHUNKS_F32(P);
+        const int n0 = chunks == 4 ? f32_self<4, VEC>(p, tok, tl) : chunks == 8 ? f32_self<8, VEC>(p, tok, tl) : f32_self<F32_SELF_CHUNKS, VEC>(p, tok, tl);
         if (n0 >= 0) f32_tile<OP, TM, TN, VEC>(p, as, bs, 0, tl, 0, n0, 0, tok);
         return;
     }

@@ -35,3 +35,16 @@ def test_index_of_the_up_launch(kw):
     x.free()
     o.free()
     layer.close()
+
+
+@pytest.mark.parametrize("kw", [dict(T=4, E=161, K=32, H=1664, Es=1), dict(T=15, E=163, K=20, H=1792, Es=0)])
+def test_both_sides_of_the_work_limit(kw):
+    """1.7 and 5.5 million pairs x workgroups: an index by the up launch, and by a launch of its own (makes_index_in_up)."""
+    G, cfg, inp, layer, x = _layer(dict(kw, d=256), 16, 1)
+    out = layer.forward(x).to_numpy()
+    got = layer.routing()
+    ref = G.oracle_forward(cfg, inp)
+    G.assert_routing_bit_exact(got, ref)
+    assert N.rel_l2(out, ref["out"]) <= 1e-2
+    x.free()
+    layer.close()
