@@ -121,12 +121,13 @@ __device__ __forceinline__ omega_tile few_find(const few_args &p, few_shared &sh
 }
 // Wave per row of the copy (a pair's row of xg, then the token rows of xs): what the dispatch launch does for larger batches,
 // beside the products instead of in front of them
+template <bool SELF>
 __device__ __forceinline__ void few_copy(const few_args &p, const few_shared &sh, const few_used &us, int wg, int lane, int wave, int waves)
 {
     const int KT = p.Kd >> 5, P = p.T * p.K, n = P + (p.xs != nullptr ? p.T : 0);
     for (int u = wg * waves + wave; u < n; u += waves * p.copy_wgs) {
         const int t = u < P ? u / p.K : u - P;
-        const int row = u >= P ? t : p.index.ids != nullptr ? few_tile(us, sh.id[u]) * FEW_BM + few_rank(sh, u, lane) : p.dstp[u];
+        const int row = u >= P ? t : SELF && p.index.ids != nullptr ? few_tile(us, sh.id[u]) * FEW_BM + few_rank(sh, u, lane) : p.dstp[u];
         const unsigned char *src = p.x + (size_t)t * p.Kd * 2;
         unsigned char *dst = u < P ? p.xg : p.xs;
         for (int c = lane; c < 4 * KT; c += 64) *(uint4 *)(dst + pk_chunk_off(row, c >> 2, c & 3, KT)) = *(const uint4 *)(src + (size_t)c * 16);
@@ -188,7 +189,8 @@ __device__ __forceinline__ void few_sums(few_ptr A, const uint32_t (&a_off)[U], 
 }
 
 // UM: units of 16 rows a tile may have; NW: waves per workgroup; NB: 16-row blocks of weights per step (up: half W1's, half W3's)
-template <bool UP, int UM, int NW, int NB>
+// (SELF: the up product makes the dispatch index)
+template <bool UP, int UM, int NW, int NB, bool SELF>
 __global__ __launch_bounds__(64 * NW, 4) void few_rows_kernel(few_args p)
 {
     __shared__ few_f32x4 part[UM > 1 ? 2 : 1][NW][NB][64];
@@ -197,7 +199,8 @@ __global__ __launch_bounds__(64 * NW, 4) void few_rows_kernel(few_args p)
     const int l16 = lane & 15, lq = lane >> 4;
     constexpr int NC = UP ? NB / 2 : NB;  // 16-column blocks of the output per workgroup
     const int nc = p.N / (16 * NC);
-    const bool self = UP && p.index.ids != nullptr;
+    const bool self = SELF && p.index.ids != nullptr;  // (asked of the arguments in a SELF kernel too: known to be so, four units of rows spill 14 registers, not 3, and 64
+    // tokens x 4096 x 14336, 8 experts, take 473 us, not 451)
     const int blk = blockIdx.x;
     int n_used = 0;
     few_used us = {};
@@ -213,7 +216,7 @@ __global__ __launch_bounds__(64 * NW, 4) void few_rows_kernel(few_args p)
     }
     const int copy0 = (int)gridDim.x - (self ? 1 : 0) - p.copy_wgs;
     if (UP && blk >= copy0) {
-        few_copy(p, sh, us, blk - copy0, lane, wave, NW);
+        few_copy<SELF>(p, sh, us, blk - copy0, lane, wave, NW);
         return;
     }
     // the row tiles in falling order, which takes the shared experts - all T rows - first
@@ -327,7 +330,11 @@ hipError_t launch_experts_few(const omega_moe *m, const void *x, int T, int whic
             p.copy_wgs = std::min(ceil_div(T * (c.K + (c.Es > 0 ? 1 : 0)), 4), m->ctx->num_cus);
         }
 #define FEW_LAUNCH(UPV, UMV, NWV, NBV)                                                                                              \
-    hipLaunchKernelGGL((few_rows_kernel<UPV, UMV, NWV, NBV>), dim3(tiles * (p.N / (UPV ? 8 * NBV : 16 * NBV)) + (p.index.ids != nullptr ? 1 : 0) + p.copy_wgs), dim3(64 * NWV), 0, s, p)
+    do {                                                                                                                            \
+        const dim3 grid(tiles * (p.N / (UPV ? 8 * NBV : 16 * NBV)) + (p.index.ids != nullptr ? 1 : 0) + p.copy_wgs);                 \
+        if (UPV && p.index.ids != nullptr) hipLaunchKernelGGL((few_rows_kernel<UPV, UMV, NWV, NBV, UPV>), grid, dim3(64 * NWV), 0, s, p); \
+        else hipLaunchKernelGGL((few_rows_kernel<UPV, UMV, NWV, NBV, false>), grid, dim3(64 * NWV), 0, s, p);                       \
+    } while (0)
         // Four blocks of weights per step from 17 tokens on (two units of rows: 64 tokens x 4096 x 14336, 8 experts, up product 326 ->
         // 294 us), two below (1 token 71 against 73, 1 token x 3328 x 896, 86 experts 12.0 against 15.9).  Two waves where four would
         // have 8 k steps each or fewer, which is all start-up (64 tokens x 1024 x 768, 128 experts: pass 133 -> 128.5; d = 1536 169
