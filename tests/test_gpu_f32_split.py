@@ -6,22 +6,24 @@ import pytest
 
 from oracle import oracle as O
 from oracle import oracle_np as N
-from tests.test_gpu_backward import _setup
+from tests.test_gpu_backward import _check_grads, _setup
 from tests.test_gpu_f32_products import _chain
 
 pytestmark = pytest.mark.gpu
 L = importlib.import_module("omega-ai_amd._lib")
 
-TALL = dict(T=2600, d=516, H=452, E=2, K=2)            # tiles of 128 rows, ragged in rows, columns and k
-MID = dict(T=1450, d=644, H=996, E=5, K=2)             # of 64 (up product and d(a))
-ODD = dict(T=2601, d=515, H=451, E=2, K=2, Es=1)       # without 16-byte loads
+TALL = dict(T=3300, d=516, H=700, E=2, K=2)            # tiles of 128 rows, ragged in rows, columns and k
+MID = dict(T=1200, d=644, H=996, E=5, K=2)             # of 64 (up product and d(a)); split dW1 and dW3
+ODD = dict(T=2601, d=515, H=451, E=2, K=2, Es=1)       # 128 rows without 16-byte loads
+ROWS = [(TALL, 128), (MID, 64), (ODD, 128)]
 
 
-@pytest.mark.parametrize("T,d,H", [(8192, 128, 3584), (8192, 1024, 1100), (8190, 131, 33)])
+@pytest.mark.parametrize("T,d,H", [(8192, 128, 3584), (8192, 1024, 1100), (32766, 515, 33)])
 def test_error_against_float64_is_that_of_a_chain_at_most(T, d, H):
     """y of the down product, on the layer's own `a`: no further from float64 than a chain of fp32 fused multiply-adds (1.05: 64 rows
     scatter by a few percent)."""
     G, cfg, inp, _, layer = _setup("c1_tiny_f32", dict(T=T, d=d, H=H, E=1, K=1), 91)
+    assert layer.f32_tiles(T)[0] == 128
     layer.forward(G.P.DeviceBuffer.from_numpy(G.ctx(), inp["x"], cfg.dtype))
     rows = np.linspace(0, T - 1, 64).astype(int)
     a, y = layer.workspace("a", T)[rows], layer.workspace("y", T)[rows]
@@ -31,13 +33,14 @@ def test_error_against_float64_is_that_of_a_chain_at_most(T, d, H):
     layer.close()
 
 
-@pytest.mark.parametrize("kw", [TALL, MID, ODD])
+@pytest.mark.parametrize("kw,rows", ROWS)
 @pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan, 3.4e38])
-def test_infinite_and_largest_weights(kw, value):
+def test_infinite_and_largest_weights(kw, rows, value):
     """One element of W1: what the oracle makes infinite or no number is that here, and nothing else (3.4e38 rounds to an infinite bf16)."""
     G, cfg, inp, _, _ = _setup("c1_tiny_f32", kw, 92)
     inp["W1"][0][7, 3] = value
     layer = G.build_layer(cfg, inp)
+    assert layer.f32_tiles(cfg.T)[0] == rows
     out = layer.forward(G.P.DeviceBuffer.from_numpy(G.ctx(), inp["x"], cfg.dtype)).to_numpy()
     with np.errstate(all="ignore"):
         ref = G.oracle_forward(cfg, inp)["out"]
@@ -45,16 +48,17 @@ def test_infinite_and_largest_weights(kw, value):
         assert np.array_equal(f(out), f(ref))
     out, ref = out.astype(np.float64), ref.astype(np.float64)
     finite, large = np.isfinite(ref).all(axis=1), np.abs(ref).max(axis=1) > 1e6
-    for rows in (finite & large, finite & ~large):      # (the large weight's rows outweigh the others by far)
-        assert not rows.any() or N.rel_l2(out[rows], ref[rows]) < 1e-5
+    for some in (finite & large, finite & ~large):      # (the large weight's rows outweigh the others by far)
+        assert not some.any() or N.rel_l2(out[some], ref[some]) < 1e-5
     layer.close()
 
 
-@pytest.mark.parametrize("kw", [TALL, MID, ODD])
-def test_gradients_of_tiny_deltas(kw):
+@pytest.mark.parametrize("kw,rows", ROWS)
+def test_gradients_of_tiny_deltas(kw, rows):
     """The gradients are linear in dout: with dout times 2^-100, whose products' factors lie below what three bf16 parts hold, they are
     those of dout times 2^-100 (no fp32 denormals there: gradients of 1e-4 and more)."""
     G, cfg, inp, dout, layer = _setup("c1_tiny_f32", kw, 93)
+    assert layer.f32_tiles(cfg.T)[0] == rows
     x = G.P.DeviceBuffer.from_numpy(G.ctx(), inp["x"], cfg.dtype)
     s = np.float32(2.0 ** -100)
     got = []
@@ -143,4 +147,52 @@ def test_weight_gradient_of_a_single_row_is_rounded_once():
     a = layer.workspace("a", cfg.T)[-1]
     layer.back(G.P.DeviceBuffer.from_numpy(G.ctx(), dout, cfg.dtype))
     assert np.array_equal(layer.grad(L.W_W2, 1), dout[t][:, None] * a[None, :])
+    layer.close()
+
+
+@pytest.mark.parametrize("kw,rows", ROWS)
+@pytest.mark.parametrize("place,zeros", [(0, False), (0, True), (41, False), (41, True), (-1, True)])
+def test_tiny_factors_among_zeros(kw, rows, place, zeros):
+    """A column of x times 2^-120 that meets one of W1 and W3 times 2^120, in the first k step, a later one and the last, partial one, in a batch that has
+    zeros from its first step on and in one that has none: the same results (as test_tiny_factors_with_large_ones)."""
+    G, cfg, inp, dout, _ = _setup("c1_tiny_f32", kw, 98)
+    if zeros:
+        inp["x"][::8], dout[3::8] = 0.0, 0.0
+    inp["Wg"][:, place] = 0.0
+
+    def step(e):
+        two, inv = np.float32(2.0 ** e), np.float32(2.0 ** -e)
+        p = dict(inp, x=inp["x"].copy(), W1=[w.copy() for w in inp["W1"]], W3=[w.copy() for w in inp["W3"]])
+        p["x"][:, place] *= two
+        for w in p["W1"] + p["W3"]:
+            w[:, place] *= inv
+        layer = G.build_layer(cfg, p)
+        assert layer.f32_tiles(cfg.T)[0] == rows
+        out = layer.forward(G.P.DeviceBuffer.from_numpy(G.ctx(), p["x"], cfg.dtype)).to_numpy()
+        dx = layer.back(G.P.DeviceBuffer.from_numpy(G.ctx(), dout, cfg.dtype)).to_numpy().astype(np.float64)
+        dx[:, place] *= 2.0 ** e
+        r = [out, dx, layer.grad(L.W_W2, 0), np.delete(layer.grad(L.W_W1, 1), place, 1)]
+        layer.close()
+        return r
+
+    for got, ref in zip(step(-120), step(0)):
+        assert N.rel_l2(got, ref) < 2e-6
+
+
+@pytest.mark.parametrize("d,H,Es", [(900, 1300, 1), (899, 1301, 1), (900, 1300, 0)])
+def test_split_weight_gradients_match_oracle(d, H, Es):
+    """Every expert's gradients: all rows, all but ten of them, ten and none; a shared expert, whose rows are the tokens."""
+    G, cfg, inp, dout, layer = _setup("c1_tiny_f32", dict(T=300, d=d, H=H, E=4, K=2, Es=Es), 99)
+    layer.close()
+    inp["Wg"][:], inp["x"][:, 0], inp["x"][:, 1] = 0.0, 1.0, 0.0
+    inp["Wg"][:, 0], inp["Wg"][2, 1] = (3.0, 2.0, 0.0, -9.0), 2.5
+    inp["x"][17:187:17, 1] = 1.0
+    layer = G.build_layer(cfg, inp)
+    assert layer.f32_tiles(cfg.T)[1:] == (128, 128)
+    layer.forward(G.P.DeviceBuffer.from_numpy(G.ctx(), inp["x"], cfg.dtype))
+    assert layer.routing()["counts"].tolist() == [300, 290, 10, 0]
+    dx = layer.back(G.P.DeviceBuffer.from_numpy(G.ctx(), dout, cfg.dtype)).to_numpy()
+    ref = O.moe_backward(inp["x"], dout, inp["Wg"], inp["bg"], inp["W1"], inp["W3"], inp["W2"], cfg.K, cfg.renorm, cfg.Es)
+    assert N.rel_l2(dx, ref["dx"]) < 1e-5
+    _check_grads(layer, cfg, ref, 1e-5)
     layer.close()
