@@ -112,7 +112,11 @@ def main():
     rows = cfg.P + cfg.Es * cfg.T
     up_flops = 4.0 * cfg.d * cfg.H * rows
     down_flops = 2.0 * cfg.d * cfg.H * rows
-    peak = PEAK_BF16_TFLOPS if cfg.dtype == "bf16" else PEAK_F32_TFLOPS
+    # (fp32 products in tiles of 64 rows - the down product of 128 - and more: six bf16 products for one, experts_f32_split.hip)
+    tile = layer.f32_tiles(cfg.T)[0] if cfg.dtype != "bf16" else 0
+    peak = PEAK_BF16_TFLOPS if cfg.dtype == "bf16" else PEAK_BF16_TFLOPS / 6 if tile > 32 else PEAK_F32_TFLOPS
+    peak_down = PEAK_F32_TFLOPS if tile == 64 else peak
+    up_kernel = ("few_rows_kernel" if cfg.T <= 64 else "experts_up4_kernel") if cfg.dtype == "bf16" else "f32_split_kernel<0>" if tile > 32 else "f32_product_kernel<0>"
     up_tflops = up_flops / (stage_ms["experts_up"] * 1e-3) / 1e12
     down_tflops = down_flops / (stage_ms["experts_down"] * 1e-3) / 1e12
     # algorithmic bytes of the bandwidth-bound stages
@@ -122,9 +126,11 @@ def main():
     # bytes these kernels cannot avoid moving as the path is specified (not the algorithmic figures above): the gather
     # reads every token row once and writes it K times (+ once per batch for the shared experts' packed copy); the
     # combine reads the expert outputs as the fp32 rows the composition keeps them in
-    # (bf16 layers whose up product fetches the rows of x itself write no gathered copy: the dispatch stage then moves
-    #  index data only, and its byte fractions say nothing - they are left out)
-    on_load = layer.gather_on_load()
+    # (where the up product fetches the rows of x itself, and either no copy is gathered or it is written beside the products - fp32 layers, up to
+    #  64 tokens of bf16 ones -, the dispatch stage moves index data at most, and nothing at all where the up product makes the index too: its byte
+    #  fractions say nothing and are left out)
+    copy_beside = cfg.dtype != "bf16" or cfg.T <= 64
+    on_load = layer.gather_on_load() or copy_beside
     dispatch_real = cfg.T * cfg.d * b + cfg.P * cfg.d * b + (cfg.T * cfg.d * b if cfg.Es else 0) + cfg.P * 12
     combine_real = rows * cfg.d * 4 + cfg.T * cfg.d * b + cfg.P * 8
     # block form (out = x + layer(rmsnorm(x)), the widening next to the path): whole call and its pre-norm kernel
@@ -198,7 +204,7 @@ def main():
         "config": {"workload": f"{cfg.name}: T={cfg.T} ({cfg.batch}x{cfg.seq}) d={cfg.d} E={cfg.E} K={cfg.K} H={cfg.H} "
                                f"Es={cfg.Es} renorm={int(cfg.renorm)} {cfg.dtype}, fp32 accumulate",
                    "router_mode": a.router, "seed": a.seed},
-        "roofline": {"bound": "mfma", "kernel": ("f32_product_kernel<0>" if cfg.dtype != "bf16" else "few_rows_kernel" if cfg.T <= 64 else "experts_up4_kernel") + " (up product): a = silu(xg W1^T) * (xg W3^T)",
+        "roofline": {"bound": "mfma", "kernel": up_kernel + " (up product): a = silu(xg W1^T) * (xg W3^T)",
                      "achieved": up_tflops, "peak": peak, "unit": "TFLOP/s", "frac": up_tflops / peak,
                      "algorithmic_flops_per_launch": up_flops, "avg_launch_ms": stage_ms["experts_up"],
                      "traffic": traffic, "traffic_source": traffic_src,
@@ -208,10 +214,10 @@ def main():
         "backward": backward,
         "stages": {
             "avg_ms": stage_ms, "profiled_forwards": n_prof,
-            "experts_down": {"TFLOP/s": down_tflops, "frac_mfma": down_tflops / peak},
+            "experts_down": {"TFLOP/s": down_tflops, "frac_mfma": down_tflops / peak_down},
             "experts_total_frac_mfma": (up_flops + down_flops) / ((stage_ms["experts_up"] + stage_ms["experts_down"]) * 1e-3) / 1e12 / peak,
             "router": {"GB/s": router_bytes / (stage_ms["router"] * 1e-3) / 1e9, "frac_hbm": router_bytes / (stage_ms["router"] * 1e-3) / 1e9 / PEAK_HBM_GBPS},
-            "dispatch": {"rows": "fetched from x by the loads of the up product (no gathered copy)" if on_load
+            "dispatch": {"rows": "fetched from x by the loads of the up product" + ("; a gathered copy is written beside it" if copy_beside else " (no gathered copy)") if on_load
                                  else "gathered copy written by the dispatch launch",
                          "GB/s": None if on_load else dispatch_bytes / (stage_ms["dispatch"] * 1e-3) / 1e9,
                          "frac_hbm": None if on_load else dispatch_bytes / (stage_ms["dispatch"] * 1e-3) / 1e9 / PEAK_HBM_GBPS,

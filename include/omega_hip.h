@@ -286,6 +286,8 @@ int omega_moe_time_stage(omega_moe *moe, int stage, const void *x_dev, int T, vo
 int omega_moe_time_backward(omega_moe *moe, const void *x_dev, const void *dout_dev, int T, void *dx_dev, int warmup,
                             int iters, float *ms_avg);
 
+/* (Batches of a few pairs make the dispatch index within the up product's launch: in a forward pass their dispatch stage is empty, and its work is
+ * part of experts_up here; a dispatch stage called by itself runs a launch of its own.) */
 /* Per-stage timing of omega_moe_forward itself: while profiling is on, every forward records events
  * on the context's stream around its five stages (router, dispatch, experts_up, experts_down,
  * combine).  get_profile waits for the stream, returns the summed duration of each stage in
