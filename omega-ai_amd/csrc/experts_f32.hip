@@ -17,8 +17,7 @@
 // 32 x 32 (up: 32 x 64, half of the columns W1's, half W3's, so a wave holds h1 and h3 of the same elements; four waves with one block of
 // v_mfma_f32_16x16x4 each - the same rate, four k in 32 cycles instead of two in 64 - and steps of 64 k, so a wave's chain is a quarter of that
 // of 64 x 64).  Forward pass of 8 experts, top 2, us, 64 x 64 -> 32 x 32: 256 tokens x 128 x 256 33 -> 26, 1 token x 1024 x 3584 109 -> 56, 256
-// tokens 206 -> 164; forward + backward of 64 tokens x 256 x 1024 137 -> 101.  A wave's row blocks alternate with the other row half's, so a ragged tile
-// leaves both the same work.
+// tokens 206 -> 164; forward + backward of 64 tokens x 256 x 1024 137 -> 101.
 // A step left to the compiler's order (barrier, LDS writes, loads, fragment reads, MFMAs) loses half of its MFMA time again, and a second
 // workgroup on the compute unit does not hide it: both run in step.  So the order of a step is pinned: the fragments of the next 8 k are
 // read, the next step's pieces written to the other LDS buffer and the pieces of the step behind it asked for between the MFMAs, a few at
@@ -35,8 +34,8 @@
 #include <cmath>
 #include <type_traits>
 
-// parts of 32 rows x 32 output columns that a row product's tile of 64 rows may be cut into
-#define F32_PARTS(OP, TM, TN) (F32_IS_WG(OP) || (TM) == F32_TILE_M_SMALL ? 1 : (TM) / 32 * ((TN) / (F32_PAIR(OP) ? 64 : 32)))
+// parts of 32 rows x 32 columns that a row product's tile of 64 rows may be cut into (up products here have tiles of 32)
+#define F32_PARTS(OP, TM, TN) (F32_IS_WG(OP) || (TM) == F32_TILE_M_SMALL ? 1 : (TM) / 32 * ((TN) / 32))
 
 // The up product of a few pairs finds its rows from the router's choices and leaves the dispatch index, made by the launch's last workgroup, to the
 // launches behind: a launch less in front of it.  First column of this workgroup's tile (tl, tokens of its rows in tok), or -1: nothing to do.
@@ -70,10 +69,9 @@ __global__ __launch_bounds__(256, 2) void f32_product_kernel(f32_args p)
     constexpr bool WG = F32_IS_WG(OP), PAIR = F32_PAIR(OP), PARTS = F32_PARTS(OP, TM, TN) > 1;
     constexpr int CT = PAIR ? TN / 2 : TN;                             // output columns per tile
     constexpr bool BK_ = WG || OP == F32_DA || OP == F32_DXG;
-    constexpr int PN = PAIR ? 64 : 32;                                 // MFMA columns of a part
     constexpr int LA = f32_lds_floats(TM, WG, F32_FBK(TM)), LB = f32_lds_floats(TN, BK_, F32_FBK(TM));
     // (a part works in the room of its tile)
-    constexpr int LAP = f32_lds_floats(32, WG, F32_FBK(32)), LBP = f32_lds_floats(PN, BK_, F32_FBK(32));
+    constexpr int LAP = f32_lds_floats(32, WG, F32_FBK(32)), LBP = f32_lds_floats(32, BK_, F32_FBK(32));
     static_assert(!PARTS || LAP <= LA, "a part's operands fit");
     __shared__ __attribute__((aligned(16))) float as[WG ? 1 : 2 * LA], bs[WG ? 1 : 2 * (PARTS && LBP > LB ? LBP : LB)];
     if constexpr (SELF) {
@@ -116,7 +114,7 @@ __global__ __launch_bounds__(256, 2) void f32_product_kernel(f32_args p)
 
     if constexpr (PARTS) {
         if (part >= 0) {
-            f32_tile<OP, 32, PN, VEC>(p, as, bs, mt, p.tiles[mt], 32 * (part % (TM / 32)), n0 + 32 * (part / (TM / 32)), mat);
+            f32_tile<OP, 32, 32, VEC>(p, as, bs, mt, p.tiles[mt], 32 * (part % (TM / 32)), n0 + 32 * (part / (TM / 32)), mat);
             return;
         }
     }

@@ -3,7 +3,7 @@
 //
 // Every operand is split into three bf16 parts, each the rounding of what the parts before it leave: h + m + l = x exactly (24 bits in three times
 // 8, unless l falls below the bf16 denormals, |x| < 2^-110).  A product of two numbers is the six partial products hh, hm, mh, mm, hl and
-// lh - what is left out is below 2^-25 of it -, each exact in fp32, and v_mfma_f32_16x16x32_bf16 adds 32 of one kind to an fp32 sum.  hh has a
+// lh - what is left out, ml, lm and ll, is at most 2^-24.01 of it (|m| <= 2^-8, |l| <= 2^-17) -, each exact in fp32, and v_mfma_f32_16x16x32_bf16 adds 32 of one kind to an fp32 sum.  hh has a
 // sum of its own, the five small ones another, and the two are added once: a sum of K terms is rounded K / 32 times where a chain of
 // fp32 fused multiply-adds is rounded K times.  Error against float64, 2-norm, chain -> here: normal factors, K = 32 1.0e-7 -> 3.9e-8, 256 2.9e-7 ->
 // 9.1e-8, 1024 5.7e-7 -> 1.9e-7, 3584 1.06e-6 -> 3.7e-7; positive ones, 3584 9.1e-7 -> 3.3e-7 (with one sum for all six parts 9.2e-7 and 5.7e-7).
@@ -294,10 +294,9 @@ __global__ __launch_bounds__(256, SP_WAVES(NB)) void f32_split_kernel(f32_args p
 #pragma unroll
         for (int n = 0; n < NB; ++n) acc[i][n] = low[i][n] = sp_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
-    // All steps for a wave with MBL live row units.  A step is four groups of twelve MFMAs - two row units, one column block -, each in
-    // four quarters of three with a pair of the next step's places split between them; the barrier lies in front of the last group, whose
-    // fragment reads are the next step's first.  (Everything between two barriers reads buffer c and writes buffer 1 - c, except that last
-    // group's reads of 1 - c, which every wave has finished writing.)
+    // All steps for a wave with MBL live row units.  A step: the places in registers are split into the planes, the next step's are asked for, a barrier - the
+    // planes are whole -, the products, row unit by row unit, 6 NB MFMAs each with the next unit's fragments read before them, and a barrier: the planes,
+    // of which there is one set, have been read and may be written again.
     auto run = [&](auto mbl) {
         constexpr int MBL = decltype(mbl)::value;
         sp_bf16x8 fa[2][3], fb[NB][3];
@@ -513,7 +512,7 @@ __global__ __launch_bounds__(256, SP_WAVES(NB)) void f32_split_kernel(f32_args p
 #pragma unroll
         for (int n = 0; n < (PAIR ? NB / 2 : NB); ++n) {
             const int col = n0 + xb[n], rbase = 16 * (WR * i + wr) + 4 * lq;
-            if (col >= p.N ) continue;
+            if (col >= p.N) continue;
             const size_t o = (size_t)(WG ? m0 : row0) * p.N + col;
             float h1[4], h3[4];
             if (OP == F32_DA) {
@@ -532,15 +531,13 @@ __global__ __launch_bounds__(256, SP_WAVES(NB)) void f32_split_kernel(f32_args p
                 const float v = acc[i][n][r];
                 if (PAIR) {
                     const float u = acc[i][PAIR ? n + NB / 2 : 0][r];
-                    if (OP == F32_UP) C[at] = (v / (1.0f + expf(-v))) * u;
+                    if (OP == F32_UP) C[at] = f32_swiglu(v, u);
                     if (OP == F32_RAW || p.H1 != nullptr) {
                         p.H1[at] = v;
                         p.H3[at] = u;
                     }
                 } else if (OP == F32_DA) {
-                    const float sg = 1.0f / (1.0f + expf(-h1[r]));
-                    p.H3[at] = v * (h1[r] * sg);
-                    p.H1[at] = (v * h3[r]) * sg * (1.0f + h1[r] * (1.0f - sg));
+                    f32_swiglu_backward(v, h1[r], h3[r], p.H1[at], p.H3[at]);
                 } else {
                     C[at] = v;
                 }

@@ -34,7 +34,7 @@ struct few_args {
     const omega_tile *tiles;
     const int32_t *tile_meta, *tokp, *dstp;
     index_args index;           // up: the launch makes the dispatch index itself from index.ids, the router's choices (or null: it is there)
-    unsigned char *xg, *xs;     // up: the gathered copy, written by the launch's first copy_wgs workgroups (behind the one of the index)
+    unsigned char *xg, *xs;     // up: the gathered copy, written by copy_wgs workgroups behind the products'; the one that leaves the index is the last
     int copy_wgs, T, K;
     int N, Kd;                  // output columns and k
 };

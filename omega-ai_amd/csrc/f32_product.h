@@ -1,4 +1,5 @@
-// What the two kernels of the fp32 products (experts_f32.hip, experts_f32_split.hip) share: arguments, gathered copy.
+// What the two kernels of the fp32 products (experts_f32.hip, experts_f32_split.hip) share: arguments, the choices of a few pairs, the gathered copy, a
+// tile on fp32 MFMAs, and which tiles go in parts.
 #pragma once
 #include "index_small.h"
 #include <algorithm>
@@ -234,16 +235,26 @@ __device__ __forceinline__ float4 frag(const float *S, int x, int k)
     return make_float4(S[k * (TX + 4) + x], S[(k + 1) * (TX + 4) + x], S[(k + 2) * (TX + 4) + x], S[(k + 3) * (TX + 4) + x]);
 }
 
+// a of h1 and h3; dh1 and dh3 of d(a)
+__device__ __forceinline__ float f32_swiglu(float h1, float h3) { return (h1 / (1.0f + expf(-h1))) * h3; }
+__device__ __forceinline__ void f32_swiglu_backward(float da, float h1, float h3, float &dh1, float &dh3)
+{
+    const float sg = 1.0f / (1.0f + expf(-h1));
+    dh3 = da * (h1 * sg);
+    dh1 = (da * h3) * sg * (1.0f + h1 * (1.0f - sg));
+}
+
 // One tile: row tile mt (tl) from its row r0 on (row products) or from row mt * TM of gradient matrix mat, and columns n0 ..; as and bs
-// hold both operands of a row product twice.  (Weight gradients keep arrays of their own: read through pointers dW1 and dW3 of 4096
-// tokens x 1024 x 3584, 8 experts, took 936 us instead of 915.  For the same reason p is a copy.)
+// hold both operands of a row product twice.  (Weight gradients keep arrays of their own, and p is a copy: through pointers dW1 and dW3 of 4096 tokens x 1024
+// x 3584, 8 experts, took 936 us instead of 915, in the tiles of 128 x 128 that such batches then had here.)
 template <int OP, int TM, int TN, bool VEC>
 __device__ __forceinline__ void f32_tile(const f32_args p, float *as, float *bs, int mt, const omega_tile tl, int r0, int n0, int mat, const uint16_t *tok = nullptr)
 {
     constexpr bool WG = F32_IS_WG(OP), PAIR = F32_PAIR(OP);
     constexpr bool AK = WG, BK_ = WG || OP == F32_DA || OP == F32_DXG;  // operand contiguous across k
     constexpr int BS = TM == F32_TILE_M_SMALL ? 16 : 32, GK = 256 / BS, FBK = F32_FBK(TM);  // blocks; k places of a group
-    constexpr int MB = TM / (2 * BS), NB = TN / (2 * BS), NVA = TM * FBK / 1024, NVB = TN * FBK / 1024, NR = BS * BS / 64;
+    static_assert(TM == 2 * BS, "a wave has one block of rows");
+    constexpr int NB = TN / (2 * BS), NVA = TM * FBK / 1024, NVB = TN * FBK / 1024, NR = BS * BS / 64;
     typedef typename f32_block<BS>::acc_t acc_t;
     constexpr int CT = PAIR ? TN / 2 : TN;                             // output columns per tile
     constexpr int LA = f32_lds_floats(TM, AK, FBK), LB = f32_lds_floats(TN, BK_, FBK);
@@ -295,31 +306,26 @@ __device__ __forceinline__ void f32_tile(const f32_args p, float *as, float *bs,
 
     // (first: F32_DXG's sum over the first pair.  One chain over both would carry 1.4 times the rounding error of two that are
     // added once: H = 3584, relative to float64, 1.57e-6 against 1.09e-6)
-    acc_t acc[MB][NB], first[OP == F32_DXG ? MB : 1][OP == F32_DXG ? NB : 1];
+    acc_t acc[NB], first[OP == F32_DXG ? NB : 1];
 #pragma unroll
-    for (int i = 0; i < MB; ++i)
+    for (int n = 0; n < NB; ++n)
 #pragma unroll
-        for (int n = 0; n < NB; ++n)
-#pragma unroll
-            for (int r = 0; r < NR; ++r) {
-                acc[i][n][r] = 0.0f;
-                if (OP == F32_DXG) first[i][n][r] = 0.0f;
-            }
+        for (int r = 0; r < NR; ++r) {
+            acc[n][r] = 0.0f;
+            if (OP == F32_DXG) first[n][r] = 0.0f;
+        }
     auto swap_first = [&]() {
         if constexpr (OP == F32_DXG) {
 #pragma unroll
-            for (int i = 0; i < MB; ++i)
-#pragma unroll
-                for (int n = 0; n < NB; ++n) {
-                    const acc_t v = acc[i][n];
-                    acc[i][n] = first[i][n];
-                    first[i][n] = v;
-                }
+            for (int n = 0; n < NB; ++n) {
+                const acc_t v = acc[n];
+                acc[n] = first[n];
+                first[n] = v;
+            }
         }
     };
 
-    // this wave's row blocks: rows BS (2 i + wr) ..; columns: TN/2 wc + BS n (up: W1 columns BS wc, and the same of W3)
-    const int live = max(0, min(MB, ((rows + BS - 1) / BS + 1 - wr) / 2));
+    // this wave's block: rows BS wr ..; columns: TN/2 wc + BS n (up: W1 columns BS wc, and the same of W3)
     const int xa = BS * wr + lb;
     int xb[NB];
 #pragma unroll
@@ -345,19 +351,20 @@ __device__ __forceinline__ void f32_tile(const f32_args p, float *as, float *bs,
             b_at = B1 + n0;
         }
     };
-    // All steps for a wave with MBL live row blocks.  One group = GK k of the step in buffer c: its MFMAs on the fragments
+    // All steps for a wave whose block has rows (LIVE) or none.  One group = GK k of the step in buffer c: its MFMAs on the fragments
     // read during the group before, and spread between them (pinned, a quarter of the group at a time) the reads of the
     // next group's fragments and the group's share of the step's other work: group 0 writes the next step's pieces to the
     // other buffer, group 1 asks for those of the step behind it; the barrier lies in front of the last group, whose
     // fragment reads are the next step's first.  (Everything between two barriers of a step reads buffer c and writes
     // buffer 1 - c, except that last group's reads of 1 - c, which every wave has finished writing.)
-    auto run = [&](auto mbl) {
-        constexpr int MBL = decltype(mbl)::value, NF = MBL > 0 ? MBL + NB : 0;
-        float4 fa[2][MBL > 0 ? MBL : 1], fb[2][NB];
+    auto run = [&](auto live) {
+        constexpr bool LIVE = decltype(live)::value;
+        constexpr int NF = LIVE ? 1 + NB : 0;
+        float4 fa[2], fb[2][NB];
         auto read = [&](int set, int c, int j, int r) {
             const int k = GK * j + 4 * kh;
-            if (r < MBL) fa[set][r < MBL ? r : 0] = frag<TM, AK, FBK>(WG ? As[c] : as + c * LA, xa + 2 * BS * r, k);
-            else if (r < NF) fb[set][r - MBL < NB ? r - MBL : 0] = frag<TN, BK_, FBK>(WG ? Bs[c] : bs + c * LB, xb[r - MBL < NB ? r - MBL : 0], k);
+            if (r == 0) fa[set] = frag<TM, AK, FBK>(WG ? As[c] : as + c * LA, xa, k);
+            else if (r < NF) fb[set][r - 1 < NB ? r - 1 : 0] = frag<TN, BK_, FBK>(WG ? Bs[c] : bs + c * LB, xb[r - 1 < NB ? r - 1 : 0], k);
         };
         auto group = [&](auto cc, auto jj) {
             constexpr int c = decltype(cc)::value, j = decltype(jj)::value;
@@ -376,10 +383,7 @@ __device__ __forceinline__ void f32_tile(const f32_args p, float *as, float *bs,
                     for (int u = q; u < NVB; u += 4) fetch_b(u);
                 }
 #pragma unroll
-                for (int i = 0; i < MBL; ++i)
-#pragma unroll
-                    for (int n = 0; n < NB; ++n)
-                        acc[i][n] = f32_block<BS>::mfma(((const float *)&fa[j & 1][i])[q], ((const float *)&fb[j & 1][n])[q], acc[i][n]);
+                for (int n = 0; n < (LIVE ? NB : 0); ++n) acc[n] = f32_block<BS>::mfma(((const float *)&fa[j & 1])[q], ((const float *)&fb[j & 1][n])[q], acc[n]);
                 __builtin_amdgcn_sched_barrier(0);
             }
         };
@@ -449,58 +453,48 @@ __device__ __forceinline__ void f32_tile(const f32_args p, float *as, float *bs,
 #pragma unroll
                 for (int q = 0; q < 4; ++q)
 #pragma unroll
-                    for (int i = 0; i < MBL; ++i)
-#pragma unroll
-                        for (int n = 0; n < NB; ++n)
-                            acc[i][n] = f32_block<BS>::mfma(((const float *)&fa[0][i])[q], ((const float *)&fb[0][n])[q], acc[i][n]);
+                    for (int n = 0; n < (LIVE ? NB : 0); ++n) acc[n] = f32_block<BS>::mfma(((const float *)&fa[0])[q], ((const float *)&fb[0][n])[q], acc[n]);
             }
         }
     };
-    if (live == MB) run(std::integral_constant<int, MB>());
-    else if (MB > 1 && live == 1) run(std::integral_constant<int, 1>());
-    else run(std::integral_constant<int, 0>());
+    if (rows > BS * wr) run(std::true_type());
+    else run(std::false_type());
 
     // lane: column lb of a block; register r -> row 8*(r/4) + 4*kh + r%4
     float *C = p.C;
     if (OP == F32_WG2) C += (size_t)g * p.N * p.Kd;
     if (OP == F32_WG13) C += (size_t)mat * p.N * p.Kd;
 #pragma unroll
-    for (int i = 0; i < MB; ++i) {
-        if (i >= live) continue;
-#pragma unroll
-        for (int n = 0; n < (PAIR ? 1 : NB); ++n) {
-            const int col = n0 + xb[n], rbase = BS * (2 * i + wr) + 4 * kh;
-            if (col >= p.N) continue;
-            const size_t o = (size_t)(WG ? m0 : row0) * p.N + col;
-            float h1[NR], h3[NR];
-            if (OP == F32_DA) {  // all of the block's h1 and h3 are asked for before any is used (clamped rows: no branches)
-#pragma unroll
-                for (int r = 0; r < NR; ++r) {
-                    const size_t at = o + (size_t)min(rbase + 8 * (r >> 2) + (r & 3), rows - 1) * p.N;
-                    h1[r] = p.H1[at];
-                    h3[r] = p.H3[at];
-                }
-            }
+    for (int n = 0; n < (PAIR ? 1 : NB); ++n) {
+        const int col = n0 + xb[n], rbase = BS * wr + 4 * kh;
+        if (col >= p.N) continue;
+        const size_t o = (size_t)(WG ? m0 : row0) * p.N + col;
+        float h1[NR], h3[NR];
+        if (OP == F32_DA) {  // all of the block's h1 and h3 are asked for before any is used (clamped rows: no branches)
 #pragma unroll
             for (int r = 0; r < NR; ++r) {
-                const int row = rbase + 8 * (r >> 2) + (r & 3);
-                if (row >= rows) continue;
-                const size_t at = o + (size_t)row * p.N;
-                const float v = OP == F32_DXG ? first[OP == F32_DXG ? i : 0][OP == F32_DXG ? n : 0][r] + acc[i][n][r] : acc[i][n][r];
-                if (PAIR) {
-                    const float u = acc[i][NB - 1][r];
-                    if (OP == F32_UP) C[at] = (v / (1.0f + expf(-v))) * u;
-                    if (OP == F32_RAW || p.H1 != nullptr) {
-                        p.H1[at] = v;
-                        p.H3[at] = u;
-                    }
-                } else if (OP == F32_DA) {
-                    const float sg = 1.0f / (1.0f + expf(-h1[r]));
-                    p.H3[at] = v * (h1[r] * sg);
-                    p.H1[at] = (v * h3[r]) * sg * (1.0f + h1[r] * (1.0f - sg));
-                } else {
-                    C[at] = v;
+                const size_t at = o + (size_t)min(rbase + 8 * (r >> 2) + (r & 3), rows - 1) * p.N;
+                h1[r] = p.H1[at];
+                h3[r] = p.H3[at];
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+            const int row = rbase + 8 * (r >> 2) + (r & 3);
+            if (row >= rows) continue;
+            const size_t at = o + (size_t)row * p.N;
+            const float v = OP == F32_DXG ? first[OP == F32_DXG ? n : 0][r] + acc[n][r] : acc[n][r];
+            if (PAIR) {
+                const float u = acc[NB - 1][r];
+                if (OP == F32_UP) C[at] = f32_swiglu(v, u);
+                if (OP == F32_RAW || p.H1 != nullptr) {
+                    p.H1[at] = v;
+                    p.H3[at] = u;
                 }
+            } else if (OP == F32_DA) {
+                f32_swiglu_backward(v, h1[r], h3[r], p.H1[at], p.H3[at]);
+            } else {
+                C[at] = v;
             }
         }
     }
