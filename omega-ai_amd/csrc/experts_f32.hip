@@ -13,7 +13,7 @@
 // Row tiles come from the tile list written by the dispatch stage: a tile never straddles two experts.
 //
 // Bound: fp32 MFMA, 157.3 TFLOP/s (256 FLOP per clock and compute unit; 154 measured with nothing else going on), and for small batches the
-// chain of one wave.  One workgroup = four waves = one tile: 64 x 64 (v_mfma_f32_32x32x2, steps of 32 k; down, input gradient, weight gradients) or
+// chain of one wave.  One workgroup = four waves = one tile: 64 x 64 (v_mfma_f32_32x32x2, steps of 32 k; down, d(a), input gradient, weight gradients) or
 // 32 x 32 (up: 32 x 64, half of the columns W1's, half W3's, so a wave holds h1 and h3 of the same elements; four waves with one block of
 // v_mfma_f32_16x16x4 each - the same rate, four k in 32 cycles instead of two in 64 - and steps of 64 k, so a wave's chain is a quarter of that
 // of 64 x 64).  Forward pass of 8 experts, top 2, us, 64 x 64 -> 32 x 32: 256 tokens x 128 x 256 33 -> 26, 1 token x 1024 x 3584 109 -> 56, 256
@@ -245,7 +245,11 @@ hipError_t launch_product_f32(const omega_moe *m, int op, const float *x, const 
     // Row products: tiles of 128 rows are split ones, those of 64 where they read H columns of weights (the others have fewer columns
     // and a longer k).  Up product of 64 rows, split / fp32 MFMAs in 64 x 128: from one tile per compute unit on 0.60 - 0.97, below, where most
     // launches go in parts of 32 x 32, 1.03 - 1.14.
-    const bool mid = m->bm == F32_TILE_M_MID && op != F32_DOWN && op != F32_DXG;
+    // d(a) of 64 rows: tiles of 64 x 128 from three for two compute units on, for a short k from six for one, else 64 x 64 on fp32 MFMAs.  Backward pass, split / fp32, by
+    // tiles of 64 x 128 per compute unit, means of 10 to 30 shapes: 0.2 - 0.5 1.01 - 1.04, 0.75 - 1 1.06, 1 - 1.5 1.03, from 1.5 on with d >= 256 0.99 - 0.96, with
+    // d < 256 1.5 - 6 1.01, beyond 0.99.  (1240 tokens x 624 x 352, 4 experts, top 2, the launch alone 29.8 / 20.9.)
+    const double da_tiles = (double)m->max_m_tiles * ceil_div(c.H, 128) / m->ctx->num_cus;
+    const bool mid = m->bm == F32_TILE_M_MID && (op == F32_UP || op == F32_RAW || (op == F32_DA && da_tiles >= (c.d < 256 ? 6.0 : 1.5)));
     if (op == F32_WG2 || op == F32_WG13 ? f32_wgrad_wide(m, T, op == F32_WG13 ? 2 * m->G : m->G) : m->bm == F32_TILE_M || mid)
         return launch_product_f32_split(p, op, vec, m->max_m_tiles, s);
 #define F32_ROWS(OP)                                                                           \
@@ -255,7 +259,7 @@ hipError_t launch_product_f32(const omega_moe *m, int op, const float *x, const 
         case F32_UP: return f32_launch<F32_UP, F32_TILE_M_SMALL, 64>(p, vec, m->max_m_tiles, s);
         case F32_RAW: return f32_launch<F32_RAW, F32_TILE_M_SMALL, 64>(p, vec, m->max_m_tiles, s);
         case F32_DOWN: return F32_ROWS(F32_DOWN);
-        case F32_DA: return f32_launch<F32_DA, F32_TILE_M_SMALL, 32>(p, vec, m->max_m_tiles, s);
+        case F32_DA: return F32_ROWS(F32_DA);
         case F32_DXG: return F32_ROWS(F32_DXG);
         case F32_WG2: return f32_launch<F32_WG2, 64, 64>(p, vec, 0, s);
         default: return f32_launch<F32_WG13, 64, 64>(p, vec, 0, s);
